@@ -220,6 +220,16 @@ int slayer_res_bwd(float *g_re_in, float *g_im_in, float *grad_sin, float *grad_
                    int64_t M, int64_t neurons_per_batch, int64_t num_decays,
                    int64_t T, void *stream);
 
+/* slayer_res_bwd with the NaN scans of resonator.py:421-439 on the way: *nan_found (a word the device can write, e.g.
+ * pinned host memory; zeroed by the caller; NULL = slayer_res_bwd) is set when an incoming gradient or a result may
+ * hold a NaN.  It is set for every NaN, and also when infinities of both signs meet: a caller that finds it set after
+ * synchronising looks at the tensors themselves. */
+int slayer_res_bwd_checked(float *g_re_in, float *g_im_in, float *grad_sin, float *grad_cos,
+                           const float *g_re, const float *g_im, const float *re, const float *im,
+                           const float *sin_decay, const float *cos_decay, float *workspace,
+                           int64_t M, int64_t neurons_per_batch, int64_t num_decays,
+                           int64_t T, unsigned *nan_found, void *stream);
+
 /* Replaces AdResDynamicsFwd (neuron/dynamics/adaptive_resonator.cu:25-126 kernel and its host
  * function); arithmetic of _AdResDynamicsFwd (neuron/dynamics/adaptive_resonator.py:379-436):
  * the resonator recurrence without reset plus threshold / refractory recurrences whose spike
@@ -452,6 +462,14 @@ int slayer_rf_bwd(float *g_re_in, float *g_im_in, float *grad_sin, float *grad_c
                   const float *sin_decay, const float *cos_decay,
                   float spike_threshold, float tau_rho, float scale_rho, int graded, float *workspace,
                   int64_t M, int64_t neurons_per_batch, int64_t num_decays, int64_t T, const slayer_delays *delays, void *stream);
+
+/* slayer_rf_bwd with the NaN scans: nan_found as for slayer_res_bwd_checked. */
+int slayer_rf_bwd_checked(float *g_re_in, float *g_im_in, float *grad_sin, float *grad_cos,
+                          const float *grad_spikes, const float *re, const float *im,
+                          const float *sin_decay, const float *cos_decay,
+                          float spike_threshold, float tau_rho, float scale_rho, int graded, float *workspace,
+                          int64_t M, int64_t neurons_per_batch, int64_t num_decays, int64_t T,
+                          const slayer_delays *delays, unsigned *nan_found, void *stream);
 
 /* ---- fused adaptive-threshold LIF neuron ---------------------------------------------------- */
 

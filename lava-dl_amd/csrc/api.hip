@@ -41,6 +41,28 @@ void range_flag_raise_from_host() {
         *static_cast<volatile unsigned*>(g_range_host.load(std::memory_order_acquire)) = 1u;
 }
 
+// For tensors no other kernel has looked at on its way: the parameter gradients, and the small tensors whose backward
+// pass is not a scan (below 2^20 elements: latency-bound, 64 workgroups read them in one go).
+__global__ __launch_bounds__(256) void nan_check_kernel(unsigned* found, NanCheck t) {
+    bool bad = false;
+    for (int k = 0; k < 5; ++k) {
+        if (!t.p[k]) continue;
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < t.n[k]; i += (int64_t)gridDim.x * 256)
+            bad = bad || t.p[k][i] != t.p[k][i];
+    }
+    if (bad) *reinterpret_cast<volatile unsigned*>(found) = 1u;
+}
+
+int launch_nan_check(unsigned* found, const NanCheck& tensors, hipStream_t stream) {
+    int64_t most = 0;
+    for (int k = 0; k < 5; ++k)
+        if (tensors.p[k] && tensors.n[k] > most) most = tensors.n[k];
+    if (most == 0) return 0;
+    const int64_t blocks = (most + 255) / 256;
+    hipLaunchKernelGGL(nan_check_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, found, tensors);
+    return (int)hipGetLastError();
+}
+
 }  // namespace slayer
 
 extern "C" int slayer_abi_version(void) { return SLAYER_ABI_VERSION; }

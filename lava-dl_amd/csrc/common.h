@@ -56,6 +56,10 @@ inline int check_delays(const slayer_delays* d, int64_t M, int64_t npb) {
     return 0;
 }
 
+// Sets *found when one of the tensors holds a NaN (nullptr entries are skipped).  One launch for all of them.  (api.hip)
+struct NanCheck { const float* p[5]; int64_t n[5]; };
+int launch_nan_check(unsigned* found, const NanCheck& tensors, hipStream_t stream);
+
 // After the main kernel of a fused backward pass: the gradient of the output delay, when the caller asked for it.
 // in_scan: the backward scan has left the per-row sums in grad_workspace; else nothing has been summed yet and the
 // stand-alone kernel does the whole job.  (li.hip, shift.hip)

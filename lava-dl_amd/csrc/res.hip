@@ -176,7 +176,7 @@ bool bwd_scan_usable(int64_t M, int64_t npb, int64_t T);                // scan.
 int launch_res_bwd_scan(float* g_re_in, float* g_im_in, float* partial_sin, float* partial_cos, const float* g_re,
                         const float* g_im, const float* re, const float* im, const float* sin_decay,
                         const float* cos_decay, int surrogate, float spike_thr, float tau, float rho, int64_t M,
-                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts,
+                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts, unsigned* nan_found,
                         hipStream_t stream);       // scan.hip
 
 }  // namespace slayer
@@ -224,17 +224,18 @@ extern "C" int slayer_res_fwd(float* re_out, float* im_out, const float* re_in, 
 #undef SLAYER_RES_ARGS
 }
 
-extern "C" int slayer_res_bwd(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
-                              const float* g_re, const float* g_im, const float* re, const float* im,
-                              const float* sin_decay, const float* cos_decay, float* workspace,
-                              int64_t M, int64_t neurons_per_batch, int64_t num_decays,
-                              int64_t T, void* stream) {
+extern "C" int slayer_res_bwd_checked(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
+                                      const float* g_re, const float* g_im, const float* re, const float* im,
+                                      const float* sin_decay, const float* cos_decay, float* workspace,
+                                      int64_t M, int64_t neurons_per_batch, int64_t num_decays,
+                                      int64_t T, unsigned* nan_found, void* stream) {
     if (int e = check_rows(M, T)) return e;
     if (int e = check_params(M > 0 ? M : neurons_per_batch, neurons_per_batch, num_decays)) return e;
     if ((grad_sin == nullptr) != (grad_cos == nullptr)) return SLAYER_ENULL;
     const bool want = grad_sin != nullptr;
     if (want && !workspace && M > 0) return SLAYER_ENULL;
     hipStream_t st = (hipStream_t)stream;
+    bool in_scan = false;
     if (M > 0 && T > 0) {
         if (!g_re_in || !g_im_in || !g_re || !g_im || !re || !im || !sin_decay || !cos_decay) return SLAYER_ENULL;
         if (bwd_scan_usable(M, neurons_per_batch, T) && aligned16(g_re_in) && aligned16(g_im_in) && aligned16(g_re) &&
@@ -242,8 +243,9 @@ extern "C" int slayer_res_bwd(float* g_re_in, float* g_im_in, float* grad_sin, f
             // large tensors: the complex recurrence as a wave scan over a linear stream
             if (int e = launch_res_bwd_scan(g_re_in, g_im_in, want ? workspace : nullptr, want ? workspace + M : nullptr,
                                             g_re, g_im, re, im, sin_decay, cos_decay, 0, 0.0f, 1.0f, 0.0f, M,
-                                            neurons_per_batch, num_decays, T, nullptr, st))
+                                            neurons_per_batch, num_decays, T, nullptr, nan_found, st))
                 return e;
+            in_scan = true;
         } else {
             ResBwd::Params p{{g_re, g_im, re, im}, {g_re_in, g_im_in}, sin_decay, cos_decay,
                              want ? workspace : nullptr, want ? workspace + M : nullptr,
@@ -256,10 +258,23 @@ extern "C" int slayer_res_bwd(float* g_re_in, float* g_im_in, float* grad_sin, f
             if (int e = launch_zero_fill(grad_sin, num_decays, st)) return e;
             return launch_zero_fill(grad_cos, num_decays, st);
         }
-        return launch_reduce_param_grad_pair(grad_sin, grad_cos, workspace, workspace + 2 * M, M, neurons_per_batch, num_decays,
-                                             num_decays, st);
+        if (int e = launch_reduce_param_grad_pair(grad_sin, grad_cos, workspace, workspace + 2 * M, M, neurons_per_batch,
+                                                  num_decays, num_decays, st))
+            return e;
     }
-    return 0;
+    if (!nan_found || M == 0 || T == 0) return 0;
+    const float* unseen = in_scan ? nullptr : g_re_in;
+    return launch_nan_check(nan_found, NanCheck{{unseen, unseen ? g_im_in : nullptr, nullptr, grad_sin, grad_cos},
+                                                {M * T, M * T, 0, num_decays, num_decays}}, st);
+}
+
+extern "C" int slayer_res_bwd(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
+                              const float* g_re, const float* g_im, const float* re, const float* im,
+                              const float* sin_decay, const float* cos_decay, float* workspace,
+                              int64_t M, int64_t neurons_per_batch, int64_t num_decays,
+                              int64_t T, void* stream) {
+    return slayer_res_bwd_checked(g_re_in, g_im_in, grad_sin, grad_cos, g_re, g_im, re, im, sin_decay, cos_decay,
+                                  workspace, M, neurons_per_batch, num_decays, T, nullptr, stream);
 }
 
 extern "C" int slayer_adres_fwd(float* re_out, float* im_out, float* th_out, float* ref_out,

@@ -185,7 +185,7 @@ bool bwd_scan_usable(int64_t M, int64_t npb, int64_t T);                // scan.
 int launch_res_bwd_scan(float* g_re_in, float* g_im_in, float* partial_sin, float* partial_cos, const float* g_re,
                         const float* g_im, const float* re, const float* im, const float* sin_decay,
                         const float* cos_decay, int surrogate, float spike_thr, float tau, float rho, int64_t M,
-                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts,
+                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts, unsigned* nan_found,
                         hipStream_t stream);       // scan.hip
 
 }  // namespace slayer
@@ -235,12 +235,12 @@ extern "C" int slayer_rf_fwd(float* re_out, float* im_out, float* spk_out, float
 #undef SLAYER_RF_S
 }
 
-extern "C" int slayer_rf_bwd(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
-                             const float* grad_spikes, const float* re, const float* im,
-                             const float* sin_decay, const float* cos_decay,
-                             float spike_threshold, float tau_rho, float scale_rho, int graded, float* workspace,
-                             int64_t M, int64_t neurons_per_batch, int64_t num_decays, int64_t T,
-                             const slayer_delays* delays, void* stream) {
+extern "C" int slayer_rf_bwd_checked(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
+                                     const float* grad_spikes, const float* re, const float* im,
+                                     const float* sin_decay, const float* cos_decay,
+                                     float spike_threshold, float tau_rho, float scale_rho, int graded, float* workspace,
+                                     int64_t M, int64_t neurons_per_batch, int64_t num_decays, int64_t T,
+                                     const slayer_delays* delays, unsigned* nan_found, void* stream) {
     if (int e = check_rows(M, T)) return e;
     if (int e = check_delays(delays, M, neurons_per_batch)) return e;
     if (int e = check_params(M > 0 ? M : neurons_per_batch, neurons_per_batch, num_decays)) return e;
@@ -277,7 +277,7 @@ extern "C" int slayer_rf_bwd(float* g_re_in, float* g_im_in, float* grad_sin, fl
             if (int e = launch_res_bwd_scan(g_re_in, g_im_in, want ? workspace : nullptr, want ? workspace + M : nullptr,
                                             grad_spikes, nullptr, re, im, sin_decay, cos_decay, graded ? 2 : 1,
                                             spike_threshold, tau_rho, scale_rho, M, neurons_per_batch, num_decays,
-                                            T, delays ? &sh : nullptr, st))
+                                            T, delays ? &sh : nullptr, nan_found, st))
                 return e;
             done = true;
             in_scan = true;
@@ -295,8 +295,26 @@ extern "C" int slayer_rf_bwd(float* g_re_in, float* g_im_in, float* grad_sin, fl
             if (int e = launch_zero_fill(grad_sin, num_decays, st)) return e;
             return launch_zero_fill(grad_cos, num_decays, st);
         }
-        return launch_reduce_param_grad_pair(grad_sin, grad_cos, workspace, workspace + 2 * M, M, neurons_per_batch, num_decays,
-                                             num_decays, st);
+        if (int e = launch_reduce_param_grad_pair(grad_sin, grad_cos, workspace, workspace + 2 * M, M, neurons_per_batch,
+                                                  num_decays, num_decays, st))
+            return e;
     }
-    return 0;
+    if (!nan_found || M == 0 || T == 0) return 0;
+    // what the scan has not seen: all gradients of a step-by-step pass, and the part of the spike gradient that a
+    // delay shifts out of its row
+    const float* unseen = in_scan ? nullptr : g_re_in;
+    return launch_nan_check(nan_found, NanCheck{{unseen, unseen ? g_im_in : nullptr, delays ? grad_spikes : nullptr,
+                                                 grad_sin, grad_cos},
+                                                {M * T, M * T, M * T, num_decays, num_decays}}, st);
+}
+
+extern "C" int slayer_rf_bwd(float* g_re_in, float* g_im_in, float* grad_sin, float* grad_cos,
+                             const float* grad_spikes, const float* re, const float* im,
+                             const float* sin_decay, const float* cos_decay,
+                             float spike_threshold, float tau_rho, float scale_rho, int graded, float* workspace,
+                             int64_t M, int64_t neurons_per_batch, int64_t num_decays, int64_t T,
+                             const slayer_delays* delays, void* stream) {
+    return slayer_rf_bwd_checked(g_re_in, g_im_in, grad_sin, grad_cos, grad_spikes, re, im, sin_decay, cos_decay,
+                                 spike_threshold, tau_rho, scale_rho, graded, workspace, M, neurons_per_batch,
+                                 num_decays, T, delays, nullptr, stream);
 }

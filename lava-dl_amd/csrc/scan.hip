@@ -657,7 +657,7 @@ __global__ __launch_bounds__(kScanQuads) void res_bwd_scan_kernel(
         float* __restrict__ partial_cos, const float* __restrict__ g_re, const float* __restrict__ g_im,
         const float* __restrict__ re, const float* __restrict__ im, const float* __restrict__ sin_decay,
         const float* __restrict__ cos_decay, SpikeSurrogate surr, int64_t M, int T, int QR, int rpg, unsigned npb,
-        unsigned per_param, Shifts shifts) {
+        unsigned per_param, Shifts shifts, unsigned* nan_found) {
     constexpr bool SHIFT = MODE != 0, ANYT = MODE == 2;
     static_assert(MODE != 1 || SURR != 0, "delays are folded into the fused resonate-and-fire form only");
     static_assert(!DELAY || (SHIFT && SURR != 0), "the delay gradient belongs to the forms that read the spike gradient through a delay");
@@ -736,6 +736,7 @@ __global__ __launch_bounds__(kScanQuads) void res_bwd_scan_kernel(
         for (int rr = sp.lane; rr < sp.rows; rr += kWave) { sum_s[sp.wv][rr] = 0.0f; sum_c[sp.wv][rr] = 0.0f; }
     if (DELAY)
         for (int rr = sp.lane; rr < sp.rows; rr += kWave) sum_d[sp.wv][rr] = 0.0f;
+    float stored = 0.0f;                             // running sum of the gradients stored: NaN once one of them is
     int parity = (sp.npass - 1) & 1;
     if (sp.tid == 0) { L.cr[parity] = 0.0f; L.ci[parity] = 0.0f; }
     __syncthreads();
@@ -794,6 +795,7 @@ __global__ __launch_bounds__(kScanQuads) void res_bwd_scan_kernel(
             buf_store4<STREAM>(dst_r, off, make_float4(z0.re, z1.re, z2.re, z3.re));
             buf_store4<STREAM>(dst_i, off, make_float4(z0.im, z1.im, z2.im, z3.im));
         }
+        if (active) stored += ((z0.re + z0.im) + (z1.re + z1.im)) + ((z2.re + z2.im) + (z3.re + z3.im));
         if (sp.tid == kScanQuads - 1) { L.cr[parity ^ 1] = z0.re; L.ci[parity ^ 1] = z0.im; }
         if (PARTIAL) {
             // grad_sin: sum -gr[t+1] im[t] + gi[t+1] re[t];  grad_cos: sum gr[t+1] re[t] + gi[t+1] im[t]
@@ -819,6 +821,7 @@ __global__ __launch_bounds__(kScanQuads) void res_bwd_scan_kernel(
         pass(b[2]); if (--left == 0) break;
         if (NBUF == 4) { pass(b[NBUF - 1]); if (--left == 0) break; }
     }
+    if (nan_found && stored != stored) *reinterpret_cast<volatile unsigned*>(nan_found) = 1u;
     if (PARTIAL || DELAY) __syncthreads();
     if (PARTIAL) {
         store_row_sums(partial_sin, sum_s, sp);
@@ -928,10 +931,14 @@ int launch_cuba_bwd_scan(float* grad_in, float* partial_i, float* partial_v, con
 
 // surrogate: 0 = g_re / g_im are the gradients of the states; 1 / 2 = g_re is the gradient of binary / graded
 // spikes (g_im unused) and spike_thr, tau, rho parametrise the complex spike surrogate.
+// nan_found (or nullptr): a word the kernel sets when a gradient it stores may be NaN.  It adds up what it stores, eight
+// additions per quad, instead of leaving the search to a pass over each tensor of its own; opposite infinities look
+// like a NaN to the sum, so the word asks for a closer look and does not decide.
 int launch_res_bwd_scan(float* g_re_in, float* g_im_in, float* partial_sin, float* partial_cos, const float* g_re,
                         const float* g_im, const float* re, const float* im, const float* sin_decay,
                         const float* cos_decay, int surrogate, float spike_thr, float tau, float rho, int64_t M,
-                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts, hipStream_t stream) {
+                        int64_t npb, int64_t num_decays, int64_t T, const Shifts* shifts, unsigned* nan_found,
+                        hipStream_t stream) {
     const ScanGrid g = scan_grid(M, T);
     if (!g.ok) return SLAYER_ERANGE;
     if (shifts && surrogate == 0) return SLAYER_EINVAL;      // delays belong to the fused resonate-and-fire form
@@ -942,7 +949,7 @@ int launch_res_bwd_scan(float* g_re_in, float* g_im_in, float* partial_sin, floa
     hipLaunchKernelGGL((res_bwd_scan_kernel<P, S, U, SH, NB, DL>), g.grid, dim3(kScanQuads), 0, stream, g_re_in, g_im_in, \
                        partial_sin, partial_cos, g_re, g_im, re, im, sin_decay, cos_decay, k, M, (int)T, g.QR,   \
                        g.rpg,                                                                                    \
-                       (unsigned)npb, rows_per_param(npb, num_decays), sh)
+                       (unsigned)npb, rows_per_param(npb, num_decays), sh, nan_found)
 #define SLAYER_SCAN_N(P, S, U, SH, NB) do { if (SH != 0 && U != 0 && delay_grad) SLAYER_SCAN_L(P, S, U, SH, NB, (SH != 0 && U != 0)); else SLAYER_SCAN_L(P, S, U, SH, NB, false); } while (0)
 #define SLAYER_SCAN(P, S, U, SH) do { if (g.passes > 3) SLAYER_SCAN_N(P, S, U, SH, 4); else SLAYER_SCAN_N(P, S, U, SH, 3); } while (0)
 #define SLAYER_SCAN_S(P, U, SH) do { if (g.any_length) SLAYER_SCAN(P, false, U, 2); else if (g.streaming) SLAYER_SCAN(P, true, U, SH); else SLAYER_SCAN(P, false, U, SH); } while (0)

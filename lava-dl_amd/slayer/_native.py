@@ -50,6 +50,7 @@ _SIGNATURES = {
     'slayer_res_fwd': (_INT, [_P, _P, _P, _P, _P, _P, _P, _P, _D, _INT,
                               _I64, _I64, _I64, _I64, _I64, _I64, _P]),
     'slayer_res_bwd': (_INT, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P]),
+    'slayer_res_bwd_checked': (_INT, [_P] * 11 + [_I64] * 4 + [_P, _P]),
     'slayer_spike_fwd': (_INT, [_P, _P, _P, _I64, _F, _INT, _F, _I64, _P]),
     'slayer_spike_bwd': (_INT, [_P, _P, _P, _P, _I64, _F, _F, _F, _INT, _I64, _P]),
     'slayer_cspike_fwd': (_INT, [_P, _P, _P, _P, _I64, _F, _P, _I64, _F, _INT, _F, _I64, _I64, _P]),
@@ -72,6 +73,7 @@ _SIGNATURES = {
     'slayer_cuba_bwd': (_INT, [_P] * 8 + [_F, _F, _F, _INT, _P] + [_I64] * 5 + [_DP, _P]),
     'slayer_rf_fwd': (_INT, [_P] * 12 + [_F, _INT, _F, _INT] + [_I64] * 7 + [_DP, _P]),
     'slayer_rf_bwd': (_INT, [_P] * 9 + [_F, _F, _F, _INT, _P] + [_I64] * 4 + [_DP, _P]),
+    'slayer_rf_bwd_checked': (_INT, [_P] * 9 + [_F, _F, _F, _INT, _P] + [_I64] * 4 + [_DP, _P, _P]),
     'slayer_alif_fwd': (_INT, [_P] * 17 + [_I64, _I64, _INT, _F, _INT] + [_I64] * 11 + [_DP, _P]),
     'slayer_alif_bwd': (_INT, [_P] * 9 + [_F, _F, _INT, _P] + [_I64] * 5 + [_DP, _P]),
     'slayer_cuba_recurrent_fwd': (_INT, [_P] * 10 + [_F, _INT, _F, _INT] + [_I64] * 7 + [_P]),

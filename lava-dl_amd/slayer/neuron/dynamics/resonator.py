@@ -68,7 +68,7 @@ def _fwd(real_input, imag_input, sin_decay, cos_decay, real_state, imag_state, t
     return real, imag
 
 
-def _bwd(grad_real, grad_imag, real, imag, sin_decay, cos_decay, need_decay_grad=True):
+def _bwd(grad_real, grad_imag, real, imag, sin_decay, cos_decay, need_decay_grad=True, nan_found=None):
     dev = N.require_gpu(grad_real, grad_imag, real, imag, sin_decay, cos_decay)
     grad_real, grad_imag = grad_real.contiguous(), grad_imag.contiguous()
     sin_decay, cos_decay = sin_decay.contiguous(), cos_decay.contiguous()
@@ -81,11 +81,11 @@ def _bwd(grad_real, grad_imag, real, imag, sin_decay, cos_decay, need_decay_grad
         g_cos = torch.empty(cos_decay.numel(), dtype=torch.float32, device=dev)
         workspace = torch.empty(2 * M + 128 * sin_decay.numel(), dtype=torch.float32, device=dev)
     with N.device_guard(dev):
-        N.check(N.lib().slayer_res_bwd(
+        N.check(N.lib().slayer_res_bwd_checked(
             N.ptr(g_re_in), N.ptr(g_im_in), N.ptr(g_sin), N.ptr(g_cos),
             N.ptr(grad_real), N.ptr(grad_imag), N.ptr(real), N.ptr(imag),
             N.ptr(sin_decay), N.ptr(cos_decay), N.ptr(workspace),
-            M, N.neurons_per_batch(grad_real), sin_decay.numel(), T, N.stream_handle()))
+            M, N.neurons_per_batch(grad_real), sin_decay.numel(), T, N.ptr(nan_found), N.stream_handle()))
     return g_re_in, g_im_in, g_sin, g_cos
 
 
@@ -102,8 +102,21 @@ def _bwd_naive(grad_real, grad_imag, sin_decay, cos_decay):
     return g_re_in, g_im_in
 
 
-def _raise_on_nan(**tensors):
-    """The reference aborts the backward pass on NaN (resonator.py:421-439)."""
+def _nan_word():
+    """A word of pinned host memory for the backward kernels to report NaN in: this call's own (torch's pinned-memory
+    cache hands it out again only after the call has let go of it, by when ``_raise_on_nan`` has synchronised)."""
+    word = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    word[0] = 0
+    return word
+
+
+def _raise_on_nan(found=None, **tensors):
+    """The reference aborts the backward pass on NaN (resonator.py:421-439).  ``found``: the word the kernels have
+    reported to; the tensors themselves are read only when it is set."""
+    if found is not None:
+        torch.cuda.current_stream(next(t.device for t in tensors.values() if t is not None)).synchronize()
+        if found.item() == 0:
+            return
     for name, t in tensors.items():
         if t is not None and bool(torch.isnan(t).any()):
             raise Exception(f'{name} has NaN.')
@@ -130,13 +143,14 @@ class _ResDynamics(torch.autograd.Function):
     def backward(ctx, grad_real, grad_imag):
         real, imag, sin_decay, cos_decay = ctx.saved_tensors
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
+        found = _nan_word()
         g_re, g_im, g_sin, g_cos = _bwd(grad_real, grad_imag, real, imag,
-                                        sin_decay.detach(), cos_decay.detach(), need)
+                                        sin_decay.detach(), cos_decay.detach(), need, found)
         if ctx.debug:
             c_re, c_im = _bwd_naive(grad_real, grad_imag, sin_decay.detach(), cos_decay.detach())
             N.raise_on_mismatch('resonator grad real', g_re, c_re, rel=N.scan_tolerance(g_re))
             N.raise_on_mismatch('resonator grad imag', g_im, c_im, rel=N.scan_tolerance(g_im))
-        _raise_on_nan(grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
+        _raise_on_nan(found, grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
                       grad_imag_input=g_im, grad_sin_decay=g_sin, grad_cos_decay=g_cos)
         if g_sin is not None:
             g_sin = g_sin.reshape(sin_decay.shape)

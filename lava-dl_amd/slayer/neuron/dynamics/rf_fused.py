@@ -69,7 +69,7 @@ def _fwd(real_input, imag_input, sin_decay, cos_decay, real_state, imag_state, i
 
 
 def _bwd(grad_spikes, real, imag, sin_decay, cos_decay, threshold, tau_rho, scale_rho, graded,
-         need_decay_grad=True, folded=None):
+         need_decay_grad=True, folded=None, nan_found=None):
     dev = N.require_gpu(grad_spikes, real, imag, sin_decay, cos_decay)
     grad_spikes, sin_decay, cos_decay = grad_spikes.contiguous(), sin_decay.contiguous(), cos_decay.contiguous()
     M, T = N.rows_and_steps(grad_spikes)
@@ -80,11 +80,11 @@ def _bwd(grad_spikes, real, imag, sin_decay, cos_decay, threshold, tau_rho, scal
         g_cos = torch.empty(cos_decay.numel(), dtype=torch.float32, device=dev)
         workspace = torch.empty(2 * M + 128 * sin_decay.numel(), dtype=torch.float32, device=dev)
     with N.device_guard(dev):
-        N.check(N.lib().slayer_rf_bwd(
+        N.check(N.lib().slayer_rf_bwd_checked(
             N.ptr(g_re), N.ptr(g_im), N.ptr(g_sin), N.ptr(g_cos), N.ptr(grad_spikes), N.ptr(real), N.ptr(imag),
             N.ptr(sin_decay), N.ptr(cos_decay), float(threshold), float(tau_rho), float(scale_rho),
             1 if graded else 0, N.ptr(workspace),
-            M, N.neurons_per_batch(grad_spikes), sin_decay.numel(), T, D.ref(folded), N.stream_handle()))
+            M, N.neurons_per_batch(grad_spikes), sin_decay.numel(), T, D.ref(folded), N.ptr(nan_found), N.stream_handle()))
     return g_re, g_im, g_sin, g_cos
 
 
@@ -113,10 +113,11 @@ class _RfFused(torch.autograd.Function):
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
         grad_spikes = grad_spikes.contiguous()
         folded = D.fold(ctx.delays, grad_spikes, forward=False, delayed_spikes=spk) if ctx.delays else None
+        found = _res._nan_word()
         g_re, g_im, g_sin, g_cos = _bwd(grad_spikes, real, imag, sin_decay.detach(), cos_decay.detach(),
                                         threshold, tau_rho, scale_rho, graded, need,
-                                        folded)
-        _res._raise_on_nan(grad_spikes=grad_spikes, grad_real_input=g_re, grad_imag_input=g_im,
+                                        folded, found)
+        _res._raise_on_nan(found, grad_spikes=grad_spikes, grad_real_input=g_re, grad_imag_input=g_im,
                            grad_sin_decay=g_sin, grad_cos_decay=g_cos)
         if g_sin is not None:
             g_sin, g_cos = g_sin.reshape(sin_decay.shape), g_cos.reshape(cos_decay.shape)
