@@ -64,12 +64,15 @@ class _AdResDynamics(torch.autograd.Function):
             th_state.detach(), th_scale, th0, w_scale)
         ctx.save_for_backward(real, imag, sin_decay, cos_decay)
         ctx.mark_non_differentiable(threshold, refractory)
+        ctx.set_materialize_grads(False)             # no zero tensors for the traces nothing comes back through
         return real, imag, threshold, refractory
 
     @staticmethod
     def backward(ctx, grad_real, grad_imag, *_):
         real, imag, sin_decay, cos_decay = ctx.saved_tensors
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
+        grad_real = torch.zeros_like(real) if grad_real is None else grad_real
+        grad_imag = torch.zeros_like(imag) if grad_imag is None else grad_imag
         found = _res._nan_word()
         g_re, g_im, g_sin, g_cos = _res._bwd(grad_real, grad_imag, real, imag,
                                              sin_decay.detach(), cos_decay.detach(), need, found)

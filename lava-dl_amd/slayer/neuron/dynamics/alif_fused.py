@@ -125,6 +125,7 @@ class _AlifFused(torch.autograd.Function):
         ctx.delays = delays if folded else None
         spk_last = folded.spike_last if folded else None
         ctx.mark_non_differentiable(*[t for t in (cur, vol, theta, th_last, ref_last, spk_last) if t is not None])
+        ctx.set_materialize_grads(False)         # no zero tensors for the traces nothing comes back through
         return outs + (spk_last,)
 
     @staticmethod

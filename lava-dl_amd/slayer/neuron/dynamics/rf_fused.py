@@ -104,6 +104,7 @@ class _RfFused(torch.autograd.Function):
         ctx.delays = delays if folded else None
         spk_last = folded.spike_last if folded else None
         ctx.mark_non_differentiable(*[t for t in (real, imag, spk_last) if t is not None])
+        ctx.set_materialize_grads(False)         # no zero tensors for the traces nothing comes back through
         return real, imag, spk, spk_last
 
     @staticmethod
