@@ -68,9 +68,9 @@ def custom_recurrent(z, neuron, recurrent_synapse):
     last step.  Gradients reach ``z`` and the recurrent weights; as in the reference, the state the
     neuron carries from one step to the next is treated as a constant.
 
-    The one-launch kernel adds the feedback row by row in the order the neurons fired, 16 at a time, the
-    launch-per-step kernels in a fixed order of their own on the matrix cores (float32), where
-    the reference's loop calls ``torch.matmul``.  The sums are the same bits whenever every partial sum
+    The one-launch kernel adds the feedback of up to 256 neurons in a fixed order, that of wider layers row by row
+    in the order the neurons fired, 16 at a time, the launch-per-step kernels in a fixed order of their own on the
+    matrix cores (float32), where the reference's loop calls ``torch.matmul``.  The sums are the same bits whenever every partial sum
     is exactly representable in float32, which holds for quantised recurrent weights (multiples of a power
     of two of moderate size, what the synapse's ``pre_hook_fx`` quantiser produces).  With unquantised
     weights the sums can differ in the last bit and a dendrite value within that distance of the threshold
