@@ -11,6 +11,7 @@
 // per 8 samples, which makes the lane-stride-8 reads bank-conflict free.  Taps are read with
 // wave-uniform addresses (scalar loads) and accumulate in ascending order.
 #include "common.h"
+#include "split.h"
 #include "tile.h"
 
 namespace slayer {
@@ -128,20 +129,8 @@ typedef __bf16 mfma_bf8 __attribute__((ext_vector_type(8)));
 constexpr int kConvTile = 256;             // samples per tile
 constexpr int kConvRing = 4;               // tiles in the LDS ring = tiles per loop pass
 
-// A float as the sum of three bfloat16 numbers, each the rounding to nearest of what the parts before it leave
-// (|second| <= 2^-9, |third| <= 2^-18 of the value, what the three leave out <= 2^-27), four floats at a time:
-// part t of the quad as four bfloat16 in two dwords.
+// Four floats as three bfloat16 parts (split.h): part t of the quad as four bfloat16 in two dwords.
 struct SplitQuad { uint2 part[3]; };
-typedef __bf16 conv_bf2 __attribute__((ext_vector_type(2)));
-typedef float conv_f2 __attribute__((ext_vector_type(2)));
-// two floats rounded to bfloat16 in one dword; a and b become what the rounding left
-__device__ __forceinline__ unsigned round_pair(float& a, float& b) {
-    const conv_bf2 h = __builtin_convertvector(conv_f2{a, b}, conv_bf2);
-    const conv_f2 back = __builtin_convertvector(h, conv_f2);
-    a -= back.x;
-    b -= back.y;
-    return __builtin_bit_cast(unsigned, h);
-}
 // A finite float beyond the largest bfloat16 (3.3895e38 .. 3.4028e38) rounds to an infinite first part, and what
 // that leaves is an infinity of the other sign -- which nothing else produces (an infinite or NaN value leaves a
 // NaN), so it marks exactly this case.  Such a value then takes the largest bfloat16 as its first part instead; the

@@ -1,0 +1,47 @@
+// A float32 as the sum of three bfloat16 numbers, the operands of v_mfma_f32_16x16x32_bf16: each part is the rounding
+// to nearest of what the parts before it leave (|second| <= 2^-9, |third| <= 2^-18 of the value, what the three leave
+// out <= 2^-27).  The products of parts are exact in float32; of two split factors the products part i x part j with
+// i + j <= 2 are taken, what is left out is below 2^-26 of the product.
+//   A value that is not finite leaves a NaN (so does a finite one beyond the largest bfloat16, 3.3895e38): callers
+// either treat it (conv.hip) or recognise the NaN in the result and take the float32 instruction (synapse.hip).
+//   Parts below the smallest normal number are lost: a value under 3e-33 enters with an absolute error of 1e-38.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace slayer {
+
+typedef __bf16 split_bf2 __attribute__((ext_vector_type(2)));
+typedef __bf16 split_bf8 __attribute__((ext_vector_type(8)));
+typedef float split_f2 __attribute__((ext_vector_type(2)));
+typedef float split_f4 __attribute__((ext_vector_type(4)));
+
+// two floats rounded to bfloat16 in one dword
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(split_f2{a, b}, split_bf2));
+}
+// ... and a and b become what the rounding left
+__device__ __forceinline__ unsigned round_pair(float& a, float& b) {
+    const split_bf2 h = __builtin_convertvector(split_f2{a, b}, split_bf2);
+    const split_f2 back = __builtin_convertvector(h, split_f2);
+    a -= back.x;
+    b -= back.y;
+    return __builtin_bit_cast(unsigned, h);
+}
+// part t of eight floats (the k of one lane) as one operand of the instruction
+struct Split8 {
+    uint4 part[3];
+    __device__ __forceinline__ void set(float (&v)[8]) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            part[t].x = t < 2 ? round_pair(v[0], v[1]) : bf16_pair(v[0], v[1]);
+            part[t].y = t < 2 ? round_pair(v[2], v[3]) : bf16_pair(v[2], v[3]);
+            part[t].z = t < 2 ? round_pair(v[4], v[5]) : bf16_pair(v[4], v[5]);
+            part[t].w = t < 2 ? round_pair(v[6], v[7]) : bf16_pair(v[6], v[7]);
+        }
+    }
+};
+__device__ __forceinline__ split_f4 mfma_bf16(uint4 a, uint4 b, split_f4 d) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split_bf8, a), __builtin_bit_cast(split_bf8, b), d, 0, 0, 0);
+}
+
+}  // namespace slayer

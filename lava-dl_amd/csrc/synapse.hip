@@ -14,6 +14,7 @@
 // quad is the B operand of the e-th of four matrix products, whose column j stands for step 4j + e; lane (q, j) of a
 // result then holds output channels 4q .. 4q+3 of step 4j + e, i.e. over e a quad of consecutive steps per channel.
 #include "common.h"
+#include "split.h"
 #include "tile.h"
 
 namespace slayer {
@@ -543,133 +544,284 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 
 // The common case again (unit stride and dilation along the image row, KW taps per row): the taps of a tile are 16
 // (input channel, kernel row) pairs at one input column, and that column meets KW output pixels, one per tap of the
-// row -- so the wave walks the input columns of its image row, keeps the gradient quads of the last KW pixels in
-// registers (one new load per column), and a column costs 1 + NPT loads for KW * NPT * 4 products per 16 steps instead
-// of 1 + KW * NPT / ... loads of the form above.  Accumulator tile (x, pt): [16 channels x 16 pairs] for tap x.
+// row -- so the wave walks the input columns of its image row, keeps the gradient of the last KW pixels in registers
+// (one new visit per column), and a column costs 1 + NPT visits for KW * NPT tiles.
+// Accumulator tile (x, pt): [16 channels x 16 pairs] for tap x.
+//
+// The float32 instruction (16 steps of time in 4 x 32 cycles) was one bound of wide layers: 32 -> 64 channels on
+// [16,32,16,16,300] 539 us, 84 % of its peak.  Here the products run on the bfloat16
+// instruction (32 steps in 16 cycles): the gradient split into three parts (split.h), the input as it is where its
+// values are bfloat16 numbers -- spikes, and pooled spikes, always are; a visit that brings anything else splits it, too,
+// and takes six products instead of three.  The parts of the gradient are formed once per visit and stay in the window.
+// The other bound was the L1: in the operand's layout neighbouring lanes lie in sixteen different rows, so a load
+// of 1 KB looks up 64 lines.  Eight lanes now read the 128-byte line of a row together, and the split values
+// reach the operand's layout through 7.5 KB of LDS of the wave's own.
+//
+// The instruction rounds its sums down, not to nearest: a bias of some 2^-27 a product that a sum over 10^4 of them
+// collects (relative error of the result 1e-6, float32 instruction 1.3e-7 .. 5.7e-7).  A visit's products therefore start
+// from zero, every other column with the input negated, and the vector units add or subtract them: the biases cancel,
+// and the error is 0.8e-7 .. 1.2e-7 over spikes, graded spikes and real values.
+//   [16,32,16,16,300] -> 64 channels 539 -> 285 us, [32,8,32,32,300] -> 16 channels 374 -> 345 us (3 waves per SIMD; 64
+// steps per visit leave 2: 335 and 368 us).  What bounds it now: lines of the unaligned rows (T = 300) that two visits
+// share and fetch twice, and the vector instructions of the split.
+//
+// What is not finite (or beyond the largest bfloat16) shows as a NaN in a tile at the end: the wave then runs its
+// share again with the float32 instruction (float_products), whose results such inputs had before.
 #ifndef SLAYER_WGRAD_GROUPS
-#define SLAYER_WGRAD_GROUPS 4
+#define SLAYER_WGRAD_GROUPS 1
 #endif
-constexpr int kWgU = SLAYER_WGRAD_GROUPS;      // groups of 16 steps per visit of a column
+constexpr int kWgU = SLAYER_WGRAD_GROUPS;      // groups of 32 steps per visit of a column
+constexpr int kWgPitch = 80;                   // bytes of LDS per row of 32 bfloat16: no two quarters of a read collide
+constexpr int kWgSlot = 16 * kWgPitch;         // one part of one tile of 16 rows
+constexpr int kWgSlots = 6;                    // three parts of the gradient; the input's tiles, or three parts of one
 
 template <int KW, int NPT, bool TAIL>
-__global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_row_kernel(const SynapseWgrad p) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    constexpr int Pp = NPT * 16;
-    int* pair_off = reinterpret_cast<int*>(lds);        // [Pp] bytes, relative to the start of the wave's image row
-    int* pair_dy = pair_off + Pp;                       // [Pp]
-
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int groups = (p.items + kSynWaves - 1) / kSynWaves;
-    const int cobs = (p.Co + 15) / 16;
-    int b = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int ig = b % groups; b /= groups;
-    const int cob = b % cobs;
-    const int n = b / cobs;
-    const int co0 = cob * 16;
-    const int pass = blockIdx.y;
-    const int col = p.T * 4;
-
-    for (int pl = tid; pl < Pp; pl += kSynWaves * kWave) {
-        const int pr = pass * Pp + pl;
-        const int ci = pr / p.kh, y = pr - ci * p.kh;
-        const int dy = y * p.dh - p.ph;
-        pair_dy[pl] = pr < p.Ci * p.kh ? dy : (1 << 28);                 // a pair that does not exist: always outside
-        pair_off[pl] = ((ci * p.H + dy) * p.W) * col;
-    }
-    __syncthreads();
-
-    const int item = ig * kSynWaves + wave;
-    if (item >= p.items) return;
-    const int tpart = item % p.tparts;
-    const int ho = item / p.tparts;
-    const int kk = lane >> 4, j = lane & 15;
-    const int hin = ho * p.sh;
-    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
-    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
-    const int64_t out_plane = (int64_t)p.Co * p.Ho * p.Wo * p.T;
-    const __amdgpu_buffer_rsrc_t grd = make_rsrc(p.grad_out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
-    const bool co_ok = co0 + j < p.Co;
-    const int g_row = (co0 + j) * (p.Ho * p.Wo * col) + ho * p.Wo * col;  // gradient row of this lane's channel
-    const int s_row = hin * p.W * col;                                   // the wave's image row, before the pairs' offsets
-    int my_off[NPT];
-    bool my_row[NPT];
-#pragma unroll
-    for (int pt = 0; pt < NPT; ++pt) {
-        my_off[pt] = s_row + pair_off[16 * pt + j];
-        my_row[pt] = (unsigned)(hin + pair_dy[16 * pt + j]) < (unsigned)p.H;
-    }
+struct WgradRow {
+    const SynapseWgrad& p;
+    char* lds;                                 // kWgSlots slots of this wave
+    __amdgpu_buffer_rsrc_t src, grd;
+    int col, co0, ho, hin, pair0, t_lo, t_hi, lane;
     syn_f4 acc[KW][NPT];
-#pragma unroll
-    for (int x = 0; x < KW; ++x)
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt) acc[x][pt] = syn_f4{0.f, 0.f, 0.f, 0.f};
 
-    const int t_lo = tpart * p.tlen, t_hi = (t_lo + p.tlen) < p.T ? (t_lo + p.tlen) : p.T;
-    for (int t0 = t_lo; t0 < t_hi; t0 += 16 * kWgU) {                    // whole 128-byte lines of every row per visit
-        int toff[kWgU];
-        bool t_ok[kWgU];
-        SynQuad tq[kWgU];
+    // byte offset of the gradient row of channel co0 + r / of the input row of pair pair0 + r at column 0, or none
+    __device__ __forceinline__ int grad_row(int r) const {
+        return co0 + r < p.Co ? ((co0 + r) * p.Ho + ho) * p.Wo * col : kOutOfRange;
+    }
+    __device__ __forceinline__ int pair_row(int r) const {
+        const int pr = pair0 + r, ci = pr / p.kh, row = hin + (pr - ci * p.kh) * p.dh - p.ph;
+        return (pr < p.Ci * p.kh && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
+    }
+    // steps t .. t + 3 of the pixel (or column) x of such a row
+    __device__ __forceinline__ float4 grad_at(int row, int wo, const SynQuad& tq) const {
+        return tq.template place<TAIL>(buf_load4<false>(
+            grd, (tq.any() && row != kOutOfRange && (unsigned)wo < (unsigned)p.Wo) ? row + wo * col + tq.t_load * 4 : kOutOfRange));
+    }
+    __device__ __forceinline__ float4 pair_at(int row, int c, const SynQuad& tq) const {
+        return tq.template place<TAIL>(buf_load4<false>(
+            src, (tq.any() && row != kOutOfRange) ? row + c * col + tq.t_load * 4 : kOutOfRange));
+    }
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-        for (int u = 0; u < kWgU; ++u) {
-            const int t = t0 + 16 * u + 4 * kk;
-            tq[u].template set<TAIL>(t, t_hi);                                          // the shares are whole quads; a row's last quad may not be
-            t_ok[u] = tq[u].any();
-            toff[u] = tq[u].t_load * 4;
+        for (int x = 0; x < KW; ++x)
+#pragma unroll
+            for (int pt = 0; pt < NPT; ++pt) acc[x][pt] = syn_f4{0.f, 0.f, 0.f, 0.f};
+    }
+    // the wave's own LDS: its instructions run in order, the fences keep the compiler to that order
+    __device__ __forceinline__ static void settle() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    // Lane l holds a quad of steps 4 (l % 8) of row l / 8 (+ 8 in the second quad); the operand's lane (kk, j) takes
+    // steps 8 kk .. 8 kk + 7 of row j.
+    __device__ __forceinline__ void put(int slot, int half, uint2 v) const {
+        *reinterpret_cast<uint2*>(lds + slot * kWgSlot + ((lane >> 3) + 8 * half) * kWgPitch + (lane & 7) * 8) = v;
+    }
+    __device__ __forceinline__ uint4 get(int slot) const {
+        return *reinterpret_cast<const uint4*>(lds + slot * kWgSlot + (lane & 15) * kWgPitch + (lane >> 4) * 16);
+    }
+    __device__ __forceinline__ void put_parts(int slot, const float4 (&raw)[2]) const {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            float4 v = raw[h];
+            uint2 part;
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                part.x = t < 2 ? round_pair(v.x, v.y) : bf16_pair(v.x, v.y);
+                part.y = t < 2 ? round_pair(v.z, v.w) : bf16_pair(v.z, v.w);
+                put(slot + t, h, part);
+            }
         }
-        auto grad_at = [&](int wo, int u) {
-            return tq[u].template place<TAIL>(buf_load4<false>(
-                grd, (t_ok[u] && co_ok && (unsigned)wo < (unsigned)p.Wo) ? g_row + wo * col + toff[u] : kOutOfRange));
-        };
-        // gw[x][u]: the gradient at pixel c + pw - x for the column c at hand; gw[0] arrives with the column
-        float4 gw[KW][kWgU];
+    }
+
+    __device__ __forceinline__ void split_products() {
+        clear();
+        int g_row[2], q_row[NPT][2];
 #pragma unroll
-        for (int x = 1; x < KW; ++x)
+        for (int h = 0; h < 2; ++h) {
+            g_row[h] = grad_row((lane >> 3) + 8 * h);
 #pragma unroll
-            for (int u = 0; u < kWgU; ++u) gw[x][u] = grad_at(p.pw - x, u);
-        for (int c = 0; c < p.W; ++c) {
-            float4 q[kWgU][NPT];
+            for (int pt = 0; pt < NPT; ++pt) q_row[pt][h] = pair_row(16 * pt + (lane >> 3) + 8 * h);
+        }
+        for (int t0 = t_lo; t0 < t_hi; t0 += 32 * kWgU) {
+            SynQuad tq[kWgU];
 #pragma unroll
-            for (int u = 0; u < kWgU; ++u) {
-                gw[0][u] = grad_at(c + p.pw, u);
+            for (int u = 0; u < kWgU; ++u) tq[u].template set<TAIL>(t0 + 32 * u + 4 * (lane & 7), t_hi);
+            float4 raw_g[kWgU][2], raw_q[kWgU][NPT][2];
+            auto fetch_grad = [&](int wo, int u) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) raw_g[u][h] = grad_at(g_row[h], wo, tq[u]);
+            };
+            auto fetch = [&](int c, int u) {
+                fetch_grad(c + p.pw, u);
 #pragma unroll
                 for (int pt = 0; pt < NPT; ++pt)
-                    q[u][pt] = tq[u].template place<TAIL>(buf_load4<false>(
-                        src, (t_ok[u] && my_row[pt]) ? my_off[pt] + c * col + toff[u] : kOutOfRange));
-            }
 #pragma unroll
-            for (int u = 0; u < kWgU; ++u) {
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw[x][u].x, q[u][pt].x, acc[x][pt], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw[x][u].y, q[u][pt].y, acc[x][pt], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw[x][u].z, q[u][pt].z, acc[x][pt], 0, 0, 0);
-                    }
-#pragma unroll
-                for (int x = 0; x < KW; ++x)
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(gw[x][u].w, q[u][pt].w, acc[x][pt], 0, 0, 0);
-                    }
-            }
+                    for (int h = 0; h < 2; ++h) raw_q[u][pt][h] = pair_at(q_row[pt][h], c, tq[u]);
+            };
+            // gw[x]: the gradient at pixel c + pw - x for the column c at hand; gw[0] arrives with the column
+            uint4 gw[KW][kWgU][3];
 #pragma unroll
             for (int x = KW - 1; x >= 1; --x)
 #pragma unroll
-                for (int u = 0; u < kWgU; ++u) gw[x][u] = gw[x - 1][u];
+                for (int u = 0; u < kWgU; ++u) {
+                    fetch_grad(p.pw - x, u);
+                    put_parts(0, raw_g[u]);
+                    settle();
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) gw[x][u][t] = get(t);
+                    settle();
+                }
+#pragma unroll
+            for (int u = 0; u < kWgU; ++u) fetch(0, u);
+            for (int c = 0; c < p.W; ++c) {
+                const unsigned flip = (c & 1) ? 0x80008000u : 0u;
+                const float sign = (c & 1) ? -1.0f : 1.0f;
+                auto flipped = [&](uint4 v) { return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip); };
+#pragma unroll
+                for (int u = 0; u < kWgU; ++u) {
+                    put_parts(0, raw_g[u]);
+                    unsigned low = 0u;
+#pragma unroll
+                    for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const float4 v = raw_q[u][pt][h];
+                            low |= __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w);
+                        }
+                    const bool more = __any((low & 0xffffu) != 0u);      // more than bfloat16 holds
+                    if (!more) {
+#pragma unroll
+                        for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+                            for (int h = 0; h < 2; ++h)
+                                put(3 + pt, h, make_uint2(bf16_pair(raw_q[u][pt][h].x, raw_q[u][pt][h].y),
+                                                          bf16_pair(raw_q[u][pt][h].z, raw_q[u][pt][h].w)));
+                    }
+                    settle();
+#pragma unroll
+                    for (int t = 0; t < 3; ++t) gw[0][u][t] = get(t);
+                    if (more) {
+#pragma unroll
+                        for (int pt = 0; pt < NPT; ++pt) {
+                            put_parts(3, raw_q[u][pt]);
+                            settle();
+                            uint4 q[3];
+#pragma unroll
+                            for (int t = 0; t < 3; ++t) q[t] = flipped(get(3 + t));
+                            settle();
+#pragma unroll
+                            for (int x = 0; x < KW; ++x) {
+                                syn_f4 d{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                                for (int sum = 2; sum >= 0; --sum)       // the smallest products first
+#pragma unroll
+                                    for (int t = 0; t <= sum; ++t) d = mfma_bf16(gw[x][u][t], q[sum - t], d);
+                                for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[i], acc[x][pt][i]);
+                            }
+                        }
+                        if (c + 1 < p.W) fetch(c + 1, u);
+                    } else {
+                        if (c + 1 < p.W) fetch(c + 1, u);                // on its way during the products
+                        uint4 q[NPT];
+#pragma unroll
+                        for (int pt = 0; pt < NPT; ++pt) q[pt] = flipped(get(3 + pt));
+#pragma unroll
+                        for (int x = 0; x < KW; ++x) {
+                            syn_f4 d[NPT];
+#pragma unroll
+                            for (int pt = 0; pt < NPT; ++pt) d[pt] = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                            for (int t = 2; t >= 0; --t)
+#pragma unroll
+                                for (int pt = 0; pt < NPT; ++pt) d[pt] = mfma_bf16(gw[x][u][t], q[pt], d[pt]);
+#pragma unroll
+                            for (int pt = 0; pt < NPT; ++pt) {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[pt][i], acc[x][pt][i]);
+                            }
+                        }
+                    }
+                    settle();
+                }
+#pragma unroll
+                for (int x = KW - 1; x >= 1; --x)
+#pragma unroll
+                    for (int u = 0; u < kWgU; ++u)
+#pragma unroll
+                        for (int t = 0; t < 3; ++t) gw[x][u][t] = gw[x - 1][u][t];
+            }
         }
     }
+    // the same sums on the float32 instruction, 16 steps at a time
+    __device__ __forceinline__ void float_products() {
+        clear();
+        const int g_row = grad_row(lane & 15);
+        int q_row[NPT];
+#pragma unroll
+        for (int pt = 0; pt < NPT; ++pt) q_row[pt] = pair_row(16 * pt + (lane & 15));
+        for (int t0 = t_lo; t0 < t_hi; t0 += 16) {
+            SynQuad tq;
+            tq.template set<TAIL>(t0 + 4 * (lane >> 4), t_hi);
+            for (int c = 0; c < p.W; ++c) {
+#pragma unroll
+                for (int x = 0; x < KW; ++x) {
+                    const float4 g = grad_at(g_row, c + p.pw - x, tq);
+#pragma unroll
+                    for (int pt = 0; pt < NPT; ++pt) {
+                        const float4 q = pair_at(q_row[pt], c, tq);
+                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.x, q.x, acc[x][pt], 0, 0, 0);
+                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.y, q.y, acc[x][pt], 0, 0, 0);
+                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.z, q.z, acc[x][pt], 0, 0, 0);
+                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.w, q.w, acc[x][pt], 0, 0, 0);
+                    }
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ bool any_nan() const {
+        bool bad = false;
+#pragma unroll
+        for (int x = 0; x < KW; ++x)
+#pragma unroll
+            for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bad = bad || acc[x][pt][i] != acc[x][pt][i];
+        return __any(bad);
+    }
+};
+
+template <int KW, int NPT, bool TAIL>
+__global__ __launch_bounds__(kSynWaves * kWave) __attribute__((amdgpu_waves_per_eu(KW == 3 && !TAIL ? 3 : 2)))
+void synapse_wgrad_row_kernel(const SynapseWgrad p) {
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int cobs = (p.Co + 15) / 16;
+    // The waves of a workgroup, and neighbouring workgroups, take the channel blocks and passes of one share: they read
+    // the same input rows and gradient rows at about the same time and find them in the L1 and L2.
+    int b = xcd_contiguous(blockIdx.x, gridDim.x) * kSynWaves + wave;
+    const int cob = b % cobs; b /= cobs;
+    const int pass = b % p.passes; b /= p.passes;
+    const int item = b % p.items;
+    const int n = b / p.items;
+    if (n >= p.N) return;
+    const int co0 = cob * 16;
+    const int tpart = item % p.tparts;
+    const int ho = item / p.tparts;
+    __shared__ __attribute__((aligned(16))) char lds[kSynWaves][kWgSlots * kWgSlot];
+    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
+    const int64_t out_plane = (int64_t)p.Co * p.Ho * p.Wo * p.T;
+    WgradRow<KW, NPT, TAIL> w{p};
+    w.lds = lds[wave];
+    w.src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
+    w.grd = make_rsrc(p.grad_out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
+    w.col = p.T * 4;
+    w.lane = lane;
+    w.co0 = co0; w.ho = ho; w.hin = ho * p.sh;
+    w.pair0 = pass * NPT * 16;
+    w.t_lo = tpart * p.tlen;
+    w.t_hi = (w.t_lo + p.tlen) < p.T ? (w.t_lo + p.tlen) : p.T;
+    w.split_products();
+    if (w.any_nan()) w.float_products();
     // lane (q, j) of tile (x, pt): channels co0 + 4 q + i, pair 16 (pass NPT + pt) + j, tap x of its row
     float4* dst = reinterpret_cast<float4*>(p.partial) +
                   ((((int64_t)(n * cobs + cob) * p.items + item) * p.passes + pass) * (KW * NPT)) * kWave + lane;
@@ -677,7 +829,7 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_row_kernel(co
     for (int x = 0; x < KW; ++x)
 #pragma unroll
         for (int pt = 0; pt < NPT; ++pt)
-            dst[(x * NPT + pt) * kWave] = make_float4(acc[x][pt][0], acc[x][pt][1], acc[x][pt][2], acc[x][pt][3]);
+            dst[(x * NPT + pt) * kWave] = make_float4(w.acc[x][pt][0], w.acc[x][pt][1], w.acc[x][pt][2], w.acc[x][pt][3]);
 }
 
 // grad_w[co][k] = sum over batch entries and items of the waves' tiles, in double, in a fixed order, in two
@@ -940,10 +1092,10 @@ void wgrad_shape(int64_t N, int64_t Ci, int64_t Co, int64_t Ho, int64_t T, int64
                  SynapseWgrad& p) {
     if (f.row_kw) p.passes = (int)((Ci * kh + 16 * f.npt - 1) / (16 * f.npt));
     else p.passes = (int)((Ci * kh * kw + 16 * f.tiles - 1) / (16 * f.tiles));
-    // about four thousand waves (one per SIMD and occupancy slot), shares of whole visits of 64 steps: a wave's
+    // about eight thousand waves (4096: [16,32,16,16,300] -> 64 channels 310 instead of 285 us), shares of whole visits of 64 steps: a wave's
     // set-up (tables, the gradient window) is paid once per share
 #ifndef SLAYER_WGRAD_WAVES
-#define SLAYER_WGRAD_WAVES 4096
+#define SLAYER_WGRAD_WAVES 8192
 #endif
     const int64_t base = N * ((Co + 15) / 16) * Ho;
     const int64_t visits = (T + 63) / 64;
@@ -1015,7 +1167,9 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     double* stage = reinterpret_cast<double*>(workspace + tile_floats);
     const int64_t blocks = N * cobs * ((p.items + kSynWaves - 1) / kSynWaves);
     if (blocks > 0x7fffffffLL || p.passes > 65535) return SLAYER_ERANGE;
-    const dim3 grid((unsigned)blocks, (unsigned)p.passes), block(kSynWaves * kWave);
+    const int64_t row_blocks = (N * cobs * p.items * p.passes + kSynWaves - 1) / kSynWaves;
+    if (row_blocks > 0x7fffffffLL / kSynWaves) return SLAYER_ERANGE;
+    const dim3 grid((unsigned)blocks, (unsigned)p.passes), row_grid((unsigned)row_blocks), block(kSynWaves * kWave);
     const bool tail = (T % 4) != 0;                                       // rows that end inside a quad
 #define SLAYER_WGRAD(NTT)                                                                                              \
     do {                                                                                                               \
@@ -1024,8 +1178,8 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     } while (0)
 #define SLAYER_WGRAD_ROW(KW, NPT)                                                                                      \
     do {                                                                                                               \
-        if (tail) hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, true>), grid, block, NPT * 16 * 2 * sizeof(int), st, p); \
-        else hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, false>), grid, block, NPT * 16 * 2 * sizeof(int), st, p);    \
+        if (tail) hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, true>), row_grid, block, 0, st, p);             \
+        else hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, false>), row_grid, block, 0, st, p);                 \
     } while (0)
     if (f.row_kw == 3) { if (f.npt == 1) SLAYER_WGRAD_ROW(3, 1); else SLAYER_WGRAD_ROW(3, 2); }
     else if (f.row_kw == 5) { if (f.npt == 1) SLAYER_WGRAD_ROW(5, 1); else SLAYER_WGRAD_ROW(5, 2); }

@@ -1,0 +1,84 @@
+"""The convolution kernels that run on the bfloat16 matrix instruction with operands split into three parts: spikes
+(exact as they are), spikes with a few values in between that are not bfloat16 numbers, and real-valued inputs, against
+float64; and inputs and gradients that are not finite, which give what IEEE arithmetic on the same sums gives.
+
+Bar: 1e-5 of the sum of the magnitudes of an element's terms, as for the float32 kernels: what a split product leaves
+out is below 2^-26 of it, and a float32 sum of n terms in one chain is within n * 2^-24 of their magnitudes (chains
+here hold at most a few thousand)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from tests.util import assert_sum, dev
+
+pytestmark = pytest.mark.gpu
+
+# (batch, Ci, H, W, T), Co, kernel, stride, padding, dilation
+CASES = [
+    ((1, 1, 3, 3, 4), 2, (1, 3), (1, 1), (0, 1), (1, 1)),
+    ((2, 5, 6, 5, 31), 17, (3, 3), (1, 1), (1, 1), (1, 1)),          # 15 pairs: one tile
+    ((1, 6, 5, 7, 33), 16, (3, 3), (1, 1), (0, 0), (1, 1)),          # 18 pairs: two tiles
+    ((2, 11, 7, 4, 64), 33, (3, 3), (2, 1), (1, 1), (1, 1)),         # 33 pairs: two passes
+    ((1, 16, 6, 9, 65), 48, (3, 3), (1, 1), (1, 1), (2, 1)),
+    ((1, 4, 8, 8, 301), 8, (5, 5), (1, 1), (2, 2), (1, 1)),
+    ((1, 13, 7, 6, 36), 20, (5, 5), (1, 1), (2, 2), (1, 1)),         # 65 pairs
+    ((1, 32, 4, 6, 300), 64, (3, 3), (1, 1), (1, 1), (1, 1)),
+]
+
+
+def _run(x, w, g, stride, padding, dilation):
+    import lava_dl_amd.slayer as slayer
+    xg, wg = x.to(dev()).requires_grad_(), w.to(dev()).requires_grad_()
+    y = slayer.synapse.conv_synapse(xg, wg, stride, padding, dilation)
+    y.backward(g.to(dev()))
+    return y.detach(), xg.grad, wg.grad
+
+
+def _reference(x, w, g, stride, padding, dilation):
+    x, w = x.double().requires_grad_(), w.double().requires_grad_()
+    y = F.conv3d(x, w, None, stride + (1,), padding + (0,), dilation + (1,))
+    y.backward(g.double())
+    return y.detach(), x.grad, w.grad
+
+
+@pytest.mark.parametrize('case', CASES, ids=str)
+@pytest.mark.parametrize('kind', ['spikes', 'mixed', 'real'])
+@pytest.mark.parametrize('quantised', [True, False])
+def test_split_products_match_float64(case, kind, quantised):
+    shape, co, kernel, *geometry = case
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x = (torch.rand(shape, generator=gen) < 0.2).float()
+    if kind == 'mixed':                                              # some visits see more than bfloat16 holds
+        x += (torch.rand(shape, generator=gen) < 0.002) * torch.randn(shape, generator=gen)
+    elif kind == 'real':
+        x = torch.randn(shape, generator=gen)
+    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
+    if quantised:
+        w = (w * 32).round().clamp(-128, 127) / 64
+    y_shape = F.conv3d(x[..., :1], w, None, *(v + (i,) for v, i in zip(geometry, (1, 0, 1)))).shape[:-1] + shape[-1:]
+    g = torch.randn(y_shape, generator=gen)
+    got, want = _run(x, w, g, *geometry), _reference(x, w, g, *geometry)
+    size = _reference(x.abs(), w.abs(), g.abs(), *geometry)
+    for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
+        assert_sum(a, b, m + 1e-30, f'{kind} {name}')
+    if quantised and kind == 'spikes':
+        assert torch.equal(got[0].cpu().double(), want[0]), 'sums of spikes times quantised weights are exact'
+
+
+@pytest.mark.parametrize('where', ['input', 'gradient'])
+@pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan'), 3.4e38])
+def test_values_that_are_not_finite_or_overflow_a_part(where, value):
+    gen = torch.Generator().manual_seed(11)
+    x = torch.randint(1, 3, (2, 8, 6, 6, 40), generator=gen).float()
+    w = torch.randint(1, 5, (16, 8, 3, 3, 1), generator=gen).float() / 64
+    g = torch.rand(2, 16, 4, 4, 40, generator=gen) + 0.5
+    # an input pixel that every tap of its row meets inside the output
+    {'input': x[0, 0, 2, 2], 'gradient': g[0, 0, 1, 1]}[where].view(-1)[0] = value
+    geometry = (1, 1), (0, 0), (1, 1)
+    got, want = _run(x, w, g, *geometry), _reference(x, w, g, *geometry)
+    for name, a, b in zip(('output', 'grad input', 'grad weight'), got, want):
+        a, b = a.cpu(), b.float()                                    # what overflows float32 is infinite in float32
+        assert torch.equal(a.isnan(), b.isnan()), name
+        assert torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()]), name
+        ok = a.isfinite()
+        assert float((a[ok] - b[ok]).abs().max()) <= 1e-5 * float(b[ok].abs().max()), name
