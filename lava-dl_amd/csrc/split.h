@@ -27,19 +27,30 @@ __device__ __forceinline__ unsigned round_pair(float& a, float& b) {
     b -= back.y;
     return __builtin_bit_cast(unsigned, h);
 }
-// part t of eight floats (the k of one lane) as one operand of the instruction
-struct Split8 {
-    uint4 part[3];
-    __device__ __forceinline__ void set(float (&v)[8]) {
+// Eight floats (the k of one lane) as one operand of the instruction: rounded; rounded, leaving in v what the rounding
+// left; and for any value -- infinities and NaN are their own first part and leave nothing, a finite value is cut off
+// instead of rounded, which never overflows.
+__device__ __forceinline__ uint4 bf16_eight(const float (&v)[8]) {
+    return make_uint4(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]), bf16_pair(v[4], v[5]), bf16_pair(v[6], v[7]));
+}
+__device__ __forceinline__ uint4 round_eight(float (&v)[8]) {
+    uint4 r;
+    r.x = round_pair(v[0], v[1]);
+    r.y = round_pair(v[2], v[3]);
+    r.z = round_pair(v[4], v[5]);
+    r.w = round_pair(v[6], v[7]);
+    return r;
+}
+__device__ __forceinline__ uint4 cut_eight(float (&v)[8]) {
+    float first[8];
 #pragma unroll
-        for (int t = 0; t < 3; ++t) {
-            part[t].x = t < 2 ? round_pair(v[0], v[1]) : bf16_pair(v[0], v[1]);
-            part[t].y = t < 2 ? round_pair(v[2], v[3]) : bf16_pair(v[2], v[3]);
-            part[t].z = t < 2 ? round_pair(v[4], v[5]) : bf16_pair(v[4], v[5]);
-            part[t].w = t < 2 ? round_pair(v[6], v[7]) : bf16_pair(v[6], v[7]);
-        }
+    for (int i = 0; i < 8; ++i) {
+        const bool finite = fabsf(v[i]) < __builtin_inff();
+        first[i] = finite ? __uint_as_float(__float_as_uint(v[i]) & 0xffff0000u) : v[i];
+        v[i] = finite ? v[i] - first[i] : 0.f;
     }
-};
+    return bf16_eight(first);
+}
 __device__ __forceinline__ split_f4 mfma_bf16(uint4 a, uint4 b, split_f4 d) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split_bf8, a), __builtin_bit_cast(split_bf8, b), d, 0, 0, 0);
 }

@@ -327,6 +327,186 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kerne
     synapse_conv_row<KW, PIX, STREAM, true>(p);
 }
 
+// The row form on the bfloat16 matrix instruction, for layers with enough (input channel, kernel row) pairs to fill its 32
+// terms.  The float32 instruction bounds wide layers: 32 -> 64 channels on [16,32,16,16,300] 398 us forward (72 % of its
+// peak) and 429 us for the input gradient.  Operands are split into three parts (split.h) unless they are bfloat16
+// numbers as they are: the weights are looked at once per workgroup (those of an 8-bit quantiser always are), the input
+// once per column and group of 32 pairs (spikes are, gradients are not), and the products run to match: one for spikes
+// and quantised weights, three for one split operand, six for two.
+//
+// A wave walks the columns of its image row: lane (kk, j) loads steps 4j .. 4j+3 of pairs 32 g + 8 kk + {0 .. 7} at the
+// column, turns them into the operands of four products (one per step of the quad: eight pairs each), and uses these
+// for the KW output pixels the column meets, whose accumulators it keeps -- every column is loaded and split once.  A
+// pixel is complete, and stored, after its last column.  The next loads are on their way during the products.
+// [16,32,16,16,300] -> 64 channels forward 398 -> 232 us, input gradient 429 -> 319 us; [32,8,32,32,300] -> 16 channels 384
+// -> 320 us on average of both (161 registers, three waves per SIMD; five taps 193, two waves).  The error against float64
+// is 0.6 to 0.9 times that of the float32 form (real values 2.5e-7 and 2.9e-7 at 96 pairs).  What bounds it now: the
+// unaligned rows of the result (T = 300) for few channels, the vector instructions of the split for gradients.
+// LDS: the parts of the weights in the operand's layout, [group][tap][part][lane]; per wave the byte
+// offset of every pair's input row (or kOutOfRange).
+template <int KW, bool STREAM, bool TAIL>
+__global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const SynapseConv p) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int G = p.KG;                                 // groups of 32 pairs
+    const int pairs = p.Ci * p.kh;
+    uint4* wt = reinterpret_cast<uint4*>(lds);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), threads = blockDim.x, waves = threads / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int* row_off = reinterpret_cast<int*>(wt + G * KW * 3 * kWave) + wave * G * 32;
+    // neighbouring workgroups take the channel blocks of the same items: they share the input rows
+    const int cobs = (p.Co + 15) / 16;
+    const int groups = (p.items + waves - 1) / waves;
+    int b = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int cob = b % cobs; b /= cobs;
+    const int ig = b % groups;
+    const int n = b / groups;
+    const int co0 = cob * 16;
+    const int kk = lane >> 4, j = lane & 15;
+
+    const int64_t k_full = (int64_t)p.Ci * p.kh_full * p.kw_full;
+    unsigned low = 0u;
+    for (int i = tid; i < G * KW * kWave; i += threads) {
+        const int l = i & (kWave - 1), x = (i >> 6) % KW, g = (i >> 6) / KW;
+        const int co = co0 + (l & 15);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int pr = 32 * g + 8 * (l >> 4) + e, ci = pr / p.kh, y = pr - ci * p.kh;
+            v[e] = (pr < pairs && co < p.Co) ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.0f;
+            low |= __float_as_uint(v[e]);
+        }
+        uint4* to = wt + (i >> 6) * 3 * kWave + l;
+        to[0] = cut_eight(v);
+        to[kWave] = round_eight(v);
+        to[2 * kWave] = bf16_eight(v);
+    }
+    const int item = ig * waves + wave;
+    const bool on = item < p.items;
+    const int tile = item % p.ttiles;
+    const int piece = (item / p.ttiles) % p.wsplit;
+    const int ho = item / (p.ttiles * p.wsplit);
+    const int hin = ho * p.sh;
+    const int col = p.T * 4;                                             // bytes from a pixel to its right neighbour
+    for (int pr = lane; pr < 32 * G; pr += kWave) {
+        const int ci = pr / p.kh, row = hin + (pr - ci * p.kh) * p.dh - p.ph;
+        row_off[pr] = (pr < pairs && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
+    }
+    const bool split_w = __syncthreads_or((low & 0xffffu) != 0u);
+    if (!on) return;
+    const int t0 = tile * kSynTile;
+    SynQuad tq;
+    tq.template set<TAIL>(t0 + 4 * j, p.T);
+    const bool t_ok = tq.any();
+    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
+    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
+    const int64_t out_plane = (int64_t)p.Co * p.Ho_full * p.Wo_full * p.T;
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
+    const int per = (p.Wo + p.wsplit - 1) / p.wsplit;
+    const int w_lo = piece * per, w_hi = (w_lo + per) < p.Wo ? (w_lo + per) : p.Wo;
+    if (w_lo >= w_hi) return;
+
+    // column c (counted with the padding: tap x of output pixel wo lies at column wo + x) is image column c - pw
+    const int c_end = w_hi + KW - 1;
+    const int c_lo = w_lo > p.pw ? w_lo : p.pw;                          // the columns inside the image
+    const int c_hi = c_end < p.W + p.pw ? c_end : p.W + p.pw;
+    float4 raw[8];
+    auto fetch = [&](int c, int g) {
+        const int4* off = reinterpret_cast<const int4*>(row_off + 32 * g + 8 * kk);
+        const int4 o[2] = {off[0], off[1]};
+        const int at = (c - p.pw) * col + tq.t_load * 4;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            raw[4 * i] = buf_load4<false>(src, t_ok ? o[i].x + at : kOutOfRange);
+            raw[4 * i + 1] = buf_load4<false>(src, t_ok ? o[i].y + at : kOutOfRange);
+            raw[4 * i + 2] = buf_load4<false>(src, t_ok ? o[i].z + at : kOutOfRange);
+            raw[4 * i + 3] = buf_load4<false>(src, t_ok ? o[i].w + at : kOutOfRange);
+        }
+    };
+    syn_f4 acc[KW][4];
+    if (c_lo < c_hi) fetch(c_lo, 0);
+#pragma unroll
+    for (int x = 0; x < KW; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[x][e] = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = w_lo; c < c_end; ++c) {                                 // tap x of column c goes to pixel c - x: acc[x]
+        if (c >= c_lo && c < c_hi) {
+#pragma unroll 1
+            for (int g = 0; g < G; ++g) {
+                float v[4][8];                                       // [step of the quad][pair]
+                unsigned bits = 0u;
+                auto take = [&]() {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const float4 r = tq.template place<TAIL>(raw[i]);
+                        v[0][i] = r.x; v[1][i] = r.y; v[2][i] = r.z; v[3][i] = r.w;
+                        bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
+                    }
+                };
+                take();
+                const bool split_x = __any((bits & 0xffffu) != 0u);
+                const uint4* wg = wt + g * KW * 3 * kWave + lane;
+                // One copy of the products, in loops over the parts (branches around several copies cost the
+                // compiler a second set of accumulators: 256 registers and spills).
+                const int parts_x = split_x ? 3 : 1;
+#pragma unroll 1
+                for (int tx = 0; tx < parts_x; ++tx) {
+                    uint4 q[4];
+                    if (tx + 1 < parts_x) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) q[e] = round_eight(v[e]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) q[e] = bf16_eight(v[e]);
+                    }
+                    if (tx == 0) {
+                        if (split_x) {
+                            float left = 0.f;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                                for (int i = 0; i < 8; ++i) left += fabsf(v[e][i]);
+                            if (__any(!(left < __builtin_inff()))) { // a value that is not finite or rounds to infinity
+                                fetch(c, g);
+                                take();
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) q[e] = cut_eight(v[e]);
+                            }
+                        }
+                        const bool last = g + 1 == G;                // the next loads are on their way during the products
+                        if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
+                    }
+#pragma unroll 1
+                    for (int tw = split_w ? 2 - tx : 0; tw >= 0; --tw) {
+#pragma unroll
+                        for (int x = 0; x < KW; ++x) {
+                            const uint4 a = wg[(x * 3 + tw) * kWave];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[x][e] = mfma_bf16(a, q[e], acc[x][e]);
+                        }
+                    }
+                }
+            }
+        }
+        const int wo = c - (KW - 1);
+        if (wo >= w_lo) {
+            // lane (kk, j): output channels co0 + 16 o + 4 kk + i, steps t0 + 4 j + e
+            const int opix = p.out_pixel(ho, wo) * col + (t0 + 4 * j) * 4;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const syn_f4 (&d)[4] = acc[KW - 1];
+                const int co = co0 + 4 * kk + i;
+                syn_store_quad<STREAM, TAIL>(dst, co < p.Co, co * (p.Ho_full * p.Wo_full * col) + opix, tq.nv,
+                                             make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
+            }
+        }
+#pragma unroll
+        for (int x = KW - 1; x >= 0; --x)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[x][e] = x > 0 ? acc[x - 1][e] : syn_f4{0.f, 0.f, 0.f, 0.f};
+    }
+}
+
 // One input and one output channel (the pooling layers, which fold their channels into the image height,
 // synapse/layer.py:438-508 and :770-838 in the reference): there is no contraction for the matrix cores, and a wave
 // that owns 16 channels x 64 steps of one pixel would move 256 bytes per instruction.  One thread per quad of output
@@ -555,13 +735,13 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 // and takes six products instead of three.  The parts of the gradient are formed once per visit and stay in the window.
 // The other bound was the L1: in the operand's layout neighbouring lanes lie in sixteen different rows, so a load
 // of 1 KB looks up 64 lines.  Eight lanes now read the 128-byte line of a row together, and the split values
-// reach the operand's layout through 7.5 KB of LDS of the wave's own.
+// reach the operand's layout through LDS of the wave's own.
 //
 // The instruction rounds its sums down, not to nearest: a bias of some 2^-27 a product that a sum over 10^4 of them
 // collects (relative error of the result 1e-6, float32 instruction 1.3e-7 .. 5.7e-7).  A visit's products therefore start
 // from zero, every other column with the input negated, and the vector units add or subtract them: the biases cancel,
 // and the error is 0.8e-7 .. 1.2e-7 over spikes, graded spikes and real values.
-//   [16,32,16,16,300] -> 64 channels 539 -> 285 us, [32,8,32,32,300] -> 16 channels 374 -> 345 us (3 waves per SIMD; 64
+//   [16,32,16,16,300] -> 64 channels 539 -> 271 us, [32,8,32,32,300] -> 16 channels 374 -> 340 us (3 waves per SIMD; 64
 // steps per visit leave 2: 335 and 368 us).  What bounds it now: lines of the unaligned rows (T = 300) that two visits
 // share and fetch twice, and the vector instructions of the split.
 //
@@ -573,12 +753,12 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 constexpr int kWgU = SLAYER_WGRAD_GROUPS;      // groups of 32 steps per visit of a column
 constexpr int kWgPitch = 80;                   // bytes of LDS per row of 32 bfloat16: no two quarters of a read collide
 constexpr int kWgSlot = 16 * kWgPitch;         // one part of one tile of 16 rows
-constexpr int kWgSlots = 6;                    // three parts of the gradient; the input's tiles, or three parts of one
 
 template <int KW, int NPT, bool TAIL>
 struct WgradRow {
     const SynapseWgrad& p;
-    char* lds;                                 // kWgSlots slots of this wave
+    static constexpr int kSlots = 3 + 3 * NPT; // three parts of the gradient and of every tile of the input
+    char* lds;                                 // kSlots slots of this wave
     __amdgpu_buffer_rsrc_t src, grd;
     int col, co0, ho, hin, pair0, t_lo, t_hi, lane;
     syn_f4 acc[KW][NPT];
@@ -591,14 +771,13 @@ struct WgradRow {
         const int pr = pair0 + r, ci = pr / p.kh, row = hin + (pr - ci * p.kh) * p.dh - p.ph;
         return (pr < p.Ci * p.kh && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
     }
-    // steps t .. t + 3 of the pixel (or column) x of such a row
+    // steps t .. t + 3 of the pixel (or column) x of such a row, to be moved into place (SynQuad) where they are used
     __device__ __forceinline__ float4 grad_at(int row, int wo, const SynQuad& tq) const {
-        return tq.template place<TAIL>(buf_load4<false>(
-            grd, (tq.any() && row != kOutOfRange && (unsigned)wo < (unsigned)p.Wo) ? row + wo * col + tq.t_load * 4 : kOutOfRange));
+        return buf_load4<false>(
+            grd, (tq.any() && row != kOutOfRange && (unsigned)wo < (unsigned)p.Wo) ? row + wo * col + tq.t_load * 4 : kOutOfRange);
     }
     __device__ __forceinline__ float4 pair_at(int row, int c, const SynQuad& tq) const {
-        return tq.template place<TAIL>(buf_load4<false>(
-            src, (tq.any() && row != kOutOfRange) ? row + c * col + tq.t_load * 4 : kOutOfRange));
+        return buf_load4<false>(src, (tq.any() && row != kOutOfRange) ? row + c * col + tq.t_load * 4 : kOutOfRange);
     }
     __device__ __forceinline__ void clear() {
 #pragma unroll
@@ -619,10 +798,10 @@ struct WgradRow {
     __device__ __forceinline__ uint4 get(int slot) const {
         return *reinterpret_cast<const uint4*>(lds + slot * kWgSlot + (lane & 15) * kWgPitch + (lane >> 4) * 16);
     }
-    __device__ __forceinline__ void put_parts(int slot, const float4 (&raw)[2]) const {
+    __device__ __forceinline__ void put_parts(int slot, const float4 (&raw)[2], const SynQuad& tq) const {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            float4 v = raw[h];
+            float4 v = tq.template place<TAIL>(raw[h]);
             uint2 part;
 #pragma unroll
             for (int t = 0; t < 3; ++t) {
@@ -647,12 +826,9 @@ struct WgradRow {
 #pragma unroll
             for (int u = 0; u < kWgU; ++u) tq[u].template set<TAIL>(t0 + 32 * u + 4 * (lane & 7), t_hi);
             float4 raw_g[kWgU][2], raw_q[kWgU][NPT][2];
-            auto fetch_grad = [&](int wo, int u) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) raw_g[u][h] = grad_at(g_row[h], wo, tq[u]);
-            };
             auto fetch = [&](int c, int u) {
-                fetch_grad(c + p.pw, u);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) raw_g[u][h] = grad_at(g_row[h], c + p.pw, tq[u]);
 #pragma unroll
                 for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
@@ -660,12 +836,18 @@ struct WgradRow {
             };
             // gw[x]: the gradient at pixel c + pw - x for the column c at hand; gw[0] arrives with the column
             uint4 gw[KW][kWgU][3];
+            float4 first[KW][kWgU][2];
+#pragma unroll
+            for (int x = KW - 1; x >= 1; --x)
+#pragma unroll
+                for (int u = 0; u < kWgU; ++u)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) first[x][u][h] = grad_at(g_row[h], p.pw - x, tq[u]);
 #pragma unroll
             for (int x = KW - 1; x >= 1; --x)
 #pragma unroll
                 for (int u = 0; u < kWgU; ++u) {
-                    fetch_grad(p.pw - x, u);
-                    put_parts(0, raw_g[u]);
+                    put_parts(0, first[x][u], tq[u]);
                     settle();
 #pragma unroll
                     for (int t = 0; t < 3; ++t) gw[x][u][t] = get(t);
@@ -679,67 +861,59 @@ struct WgradRow {
                 auto flipped = [&](uint4 v) { return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip); };
 #pragma unroll
                 for (int u = 0; u < kWgU; ++u) {
-                    put_parts(0, raw_g[u]);
+                    put_parts(0, raw_g[u], tq[u]);
                     unsigned low = 0u;
 #pragma unroll
                     for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
-                            const float4 v = raw_q[u][pt][h];
+                            const float4 v = raw_q[u][pt][h] = tq[u].template place<TAIL>(raw_q[u][pt][h]);
                             low |= __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w);
                         }
                     const bool more = __any((low & 0xffffu) != 0u);      // more than bfloat16 holds
-                    if (!more) {
 #pragma unroll
-                        for (int pt = 0; pt < NPT; ++pt)
+                    for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
-                            for (int h = 0; h < 2; ++h)
-                                put(3 + pt, h, make_uint2(bf16_pair(raw_q[u][pt][h].x, raw_q[u][pt][h].y),
-                                                          bf16_pair(raw_q[u][pt][h].z, raw_q[u][pt][h].w)));
-                    }
+                        for (int h = 0; h < 2; ++h) {
+                            float4 v = raw_q[u][pt][h];
+                            if (!more) {
+                                put(3 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
+                            } else {
+                                uint2 part;
+                                part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
+                                put(3 + 3 * pt, h, part);
+                                part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
+                                put(4 + 3 * pt, h, part);
+                                put(5 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
+                            }
+                        }
                     settle();
+                    if (c + 1 < p.W) fetch(c + 1, u);                    // on its way during the products
 #pragma unroll
                     for (int t = 0; t < 3; ++t) gw[0][u][t] = get(t);
-                    if (more) {
 #pragma unroll
-                        for (int pt = 0; pt < NPT; ++pt) {
-                            put_parts(3, raw_q[u][pt]);
-                            settle();
-                            uint4 q[3];
+                    for (int pt = 0; pt < NPT; ++pt) {
+                        const uint4 q = flipped(get(3 + 3 * pt));
+                        syn_f4 d[KW];
 #pragma unroll
-                            for (int t = 0; t < 3; ++t) q[t] = flipped(get(3 + t));
-                            settle();
+                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][2], q, syn_f4{0.f, 0.f, 0.f, 0.f});
+                        if (more) {
+                            const uint4 q1 = flipped(get(4 + 3 * pt)), q2 = flipped(get(5 + 3 * pt));
 #pragma unroll
                             for (int x = 0; x < KW; ++x) {
-                                syn_f4 d{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                                for (int sum = 2; sum >= 0; --sum)       // the smallest products first
-#pragma unroll
-                                    for (int t = 0; t <= sum; ++t) d = mfma_bf16(gw[x][u][t], q[sum - t], d);
-                                for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[i], acc[x][pt][i]);
+                                d[x] = mfma_bf16(gw[x][u][0], q2, d[x]);
+                                d[x] = mfma_bf16(gw[x][u][1], q1, d[x]);
+                                d[x] = mfma_bf16(gw[x][u][0], q1, d[x]);
                             }
                         }
-                        if (c + 1 < p.W) fetch(c + 1, u);
-                    } else {
-                        if (c + 1 < p.W) fetch(c + 1, u);                // on its way during the products
-                        uint4 q[NPT];
 #pragma unroll
-                        for (int pt = 0; pt < NPT; ++pt) q[pt] = flipped(get(3 + pt));
+                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][1], q, d[x]);
 #pragma unroll
-                        for (int x = 0; x < KW; ++x) {
-                            syn_f4 d[NPT];
+                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][0], q, d[x]);
 #pragma unroll
-                            for (int pt = 0; pt < NPT; ++pt) d[pt] = syn_f4{0.f, 0.f, 0.f, 0.f};
+                        for (int x = 0; x < KW; ++x)
 #pragma unroll
-                            for (int t = 2; t >= 0; --t)
-#pragma unroll
-                                for (int pt = 0; pt < NPT; ++pt) d[pt] = mfma_bf16(gw[x][u][t], q[pt], d[pt]);
-#pragma unroll
-                            for (int pt = 0; pt < NPT; ++pt) {
-#pragma unroll
-                                for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[pt][i], acc[x][pt][i]);
-                            }
-                        }
+                            for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[x][i], acc[x][pt][i]);
                     }
                     settle();
                 }
@@ -765,10 +939,10 @@ struct WgradRow {
             for (int c = 0; c < p.W; ++c) {
 #pragma unroll
                 for (int x = 0; x < KW; ++x) {
-                    const float4 g = grad_at(g_row, c + p.pw - x, tq);
+                    const float4 g = tq.template place<TAIL>(grad_at(g_row, c + p.pw - x, tq));
 #pragma unroll
                     for (int pt = 0; pt < NPT; ++pt) {
-                        const float4 q = pair_at(q_row[pt], c, tq);
+                        const float4 q = tq.template place<TAIL>(pair_at(q_row[pt], c, tq));
                         acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.x, q.x, acc[x][pt], 0, 0, 0);
                         acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.y, q.y, acc[x][pt], 0, 0, 0);
                         acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.z, q.z, acc[x][pt], 0, 0, 0);
@@ -807,7 +981,7 @@ void synapse_wgrad_row_kernel(const SynapseWgrad p) {
     const int co0 = cob * 16;
     const int tpart = item % p.tparts;
     const int ho = item / p.tparts;
-    __shared__ __attribute__((aligned(16))) char lds[kSynWaves][kWgSlots * kWgSlot];
+    __shared__ __attribute__((aligned(16))) char lds[kSynWaves][WgradRow<KW, NPT, TAIL>::kSlots * kWgSlot];
     const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
     const int64_t out_plane = (int64_t)p.Co * p.Ho * p.Wo * p.T;
     WgradRow<KW, NPT, TAIL> w{p};
@@ -908,6 +1082,9 @@ using namespace slayer;
 
 namespace {
 
+#ifndef SLAYER_SPLIT_WAVES
+#define SLAYER_SPLIT_WAVES 6144
+#endif
 #ifndef SLAYER_SYN_PIX
 #define SLAYER_SYN_PIX 4
 #endif
@@ -942,6 +1119,41 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     if (blocks > 0x7fffffffLL) return SLAYER_ERANGE;
     const bool tail = (p.T % 4) != 0;                                     // rows that end inside a quad
     const dim3 grid((unsigned)blocks), block(kSynWaves * kWave);
+    // The split form from 17 (input channel, kernel row) pairs on -- it takes them 32 at a time -- if the parts of 16
+    // channels' weights fit LDS.  Spikes with quantised weights / real values with quantised weights / both real, us, here
+    // and in the float32 form below: 3x3, 24 pairs on [16,8,32,32,300] 165 / 164 / 171 and 180 / 180 / 180; 48 pairs on
+    // [8,16,24,24,300] 86 / 121 / 134 and 142 / 149 / 148; 5x5, 40 pairs on [8,8,32,32,300] 83 / 145 / 195 and 138 / 139 /
+    // 141; 80 pairs on [8,16,24,24,300] 131 / 195 / 275 and 360 / 365 / 364; 160
+    // pairs on [4,32,16,16,300] 103 / 214 / 311 and 277 / 281 / 280.  With 12 pairs ([16,4,32,32,300]) 59 / 95 / 115
+    // and 64 / 65 / 65: the float32 form.
+    const int g32 = (p.Ci * p.kh + 31) / 32;
+    const size_t split_lds = (size_t)g32 * p.kw * 3 * 1024;
+    if (rows && p.Ci * p.kh > 16 && split_lds <= 96 * 1024) {
+        const int waves = split_lds > 40 * 1024 ? 8 : 4;
+        const int64_t rows_all = (int64_t)p.N * cobs * p.Ho * p.ttiles;
+        int pieces = 1;                                                  // a piece visits kw - 1 columns more than it has pixels
+        while (rows_all * pieces < SLAYER_SPLIT_WAVES && p.Wo >= 16 * pieces) pieces *= 2;
+        p.wsplit = pieces;
+        p.KG = g32;
+        const int64_t all = (int64_t)p.Ho * pieces * p.ttiles;
+        const int64_t wgs = p.N * cobs * ((all + waves - 1) / waves);
+        if (all > 0x7fffffffLL || wgs * waves > 0x3fffffffLL) return SLAYER_ERANGE;
+        p.items = (int)all;
+        const dim3 sgrid((unsigned)wgs), sblock((unsigned)(waves * kWave));
+        const size_t bytes = split_lds + (size_t)waves * g32 * 32 * sizeof(int);
+#define SLAYER_SYN_SPLIT(KW)                                                                                        \
+        do {                                                                                                             \
+            if (tail) { if (streaming) hipLaunchKernelGGL((synapse_conv_split_kernel<KW, true, true>), sgrid, sblock, bytes, st, p); \
+                        else hipLaunchKernelGGL((synapse_conv_split_kernel<KW, false, true>), sgrid, sblock, bytes, st, p); } \
+            else { if (streaming) hipLaunchKernelGGL((synapse_conv_split_kernel<KW, true, false>), sgrid, sblock, bytes, st, p); \
+                   else hipLaunchKernelGGL((synapse_conv_split_kernel<KW, false, false>), sgrid, sblock, bytes, st, p); } \
+        } while (0)
+        if (p.kw == 2) SLAYER_SYN_SPLIT(2);
+        else if (p.kw == 3) { SLAYER_SYN_SPLIT(3); }
+        else SLAYER_SYN_SPLIT(5);
+#undef SLAYER_SYN_SPLIT
+        return (int)hipGetLastError();
+    }
     if (rows) {
         p.KG = (p.Ci * p.kh + 3) / 4;                                     // groups of four (channel, kernel row) pairs
         const size_t lds = (size_t)p.KG * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
@@ -1092,16 +1304,16 @@ void wgrad_shape(int64_t N, int64_t Ci, int64_t Co, int64_t Ho, int64_t T, int64
                  SynapseWgrad& p) {
     if (f.row_kw) p.passes = (int)((Ci * kh + 16 * f.npt - 1) / (16 * f.npt));
     else p.passes = (int)((Ci * kh * kw + 16 * f.tiles - 1) / (16 * f.tiles));
-    // about eight thousand waves (4096: [16,32,16,16,300] -> 64 channels 310 instead of 285 us), shares of whole visits of 64 steps: a wave's
+    // about eight thousand waves (4096: [16,32,16,16,300] -> 64 channels 310 instead of 285 us), shares of whole visits of 32 steps: a wave's
     // set-up (tables, the gradient window) is paid once per share
 #ifndef SLAYER_WGRAD_WAVES
 #define SLAYER_WGRAD_WAVES 8192
 #endif
     const int64_t base = N * ((Co + 15) / 16) * Ho;
-    const int64_t visits = (T + 63) / 64;
+    const int64_t visits = (T + 31) / 32;
     int64_t parts = (SLAYER_WGRAD_WAVES + base - 1) / base;
     parts = parts > visits ? visits : (parts < 1 ? 1 : parts);
-    const int64_t len = (visits + parts - 1) / parts * 64;
+    const int64_t len = (visits + parts - 1) / parts * 32;
     p.tparts = (int)((T + len - 1) / len);
     p.tlen = (int)len;
     p.items = (int)(Ho * p.tparts);

@@ -22,6 +22,8 @@ CASES = [
     ((1, 16, 6, 9, 65), 48, (3, 3), (1, 1), (1, 1), (2, 1)),
     ((1, 4, 8, 8, 301), 8, (5, 5), (1, 1), (2, 2), (1, 1)),
     ((1, 13, 7, 6, 36), 20, (5, 5), (1, 1), (2, 2), (1, 1)),         # 65 pairs
+    ((1, 32, 5, 6, 36), 8, (5, 5), (1, 1), (2, 2), (1, 1)),          # 160 pairs: the parts of the weights fill 75 KB
+    ((2, 16, 5, 5, 44), 8, (2, 2), (1, 1), (1, 1), (1, 1)),
     ((1, 32, 4, 6, 300), 64, (3, 3), (1, 1), (1, 1), (1, 1)),
 ]
 
