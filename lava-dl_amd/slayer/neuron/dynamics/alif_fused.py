@@ -133,7 +133,7 @@ class _AlifFused(torch.autograd.Function):
         cur, vol, theta, i_decay, v_decay, spk = ctx.saved_tensors
         tau_rho, scale_rho, graded = ctx.cfg
         need = (ctx.needs_input_grad[1] or ctx.needs_input_grad[2]) and cur is not None
-        grad_spikes = grad_spikes.contiguous()
+        grad_spikes = torch.zeros_like(vol) if grad_spikes is None else grad_spikes.contiguous()
         folded = D.fold(ctx.delays, grad_spikes, forward=False, delayed_spikes=spk) if ctx.delays else None
         g_in, g_i, g_v = _bwd(grad_spikes, vol, theta, cur, i_decay.detach(), v_decay.detach(),
                               tau_rho, scale_rho, graded, need,

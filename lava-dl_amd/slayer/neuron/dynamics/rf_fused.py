@@ -112,7 +112,7 @@ class _RfFused(torch.autograd.Function):
         real, imag, sin_decay, cos_decay, spk = ctx.saved_tensors
         threshold, tau_rho, scale_rho, graded = ctx.cfg
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
-        grad_spikes = grad_spikes.contiguous()
+        grad_spikes = torch.zeros_like(real) if grad_spikes is None else grad_spikes.contiguous()
         folded = D.fold(ctx.delays, grad_spikes, forward=False, delayed_spikes=spk) if ctx.delays else None
         found = _res._nan_word()
         g_re, g_im, g_sin, g_cos = _bwd(grad_spikes, real, imag, sin_decay.detach(), cos_decay.detach(),
