@@ -45,11 +45,7 @@ def custom_recurrent_ground_truth_2(z, neuron, recurrent_synapse):
 
 ONE_LAUNCH_MAX = 1024       # neurons per sample of the one-launch kernels (one thread per neuron)
 STEPS_MAX = 16384           # ... of the launch-per-step kernels (whole quads of neurons)
-# Width from which a launch per step is the faster form.  Up to 256 the one-launch kernels keep the matrix in registers:
-# 256 neurons, 300 steps, forward and backward, a launch per step / one launch, us: CUBA 8 samples 2530 / 570, 32 samples
-# 2560 / 602, 512 samples 4525 / 2130; ALIF 2670 / 653, 2700 / 695, 5090 / 2490.  Past it one launch reads the matrix from
-# the L2 in every step.
-STEPS_FROM = 257
+STEPS_FROM = 256            # width from which a launch per step is the faster form (measured at [32, C, 300])
 
 
 def _by_steps(c):
