@@ -3,7 +3,7 @@
 // out <= 2^-27).  The products of parts are exact in float32; of two split factors the products part i x part j with
 // i + j <= 2 are taken, what is left out is below 2^-26 of the product.
 //   A value that is not finite leaves a NaN (so does a finite one beyond the largest bfloat16, 3.3895e38): callers
-// either treat it (conv.hip) or recognise the NaN in the result and take the float32 instruction (synapse.hip).
+// either treat it (conv.hip) or recognise a result that is not finite and compute it again in float32 (synapse.hip).
 //   Parts below the smallest normal number are lost: a value under 3e-33 enters with an absolute error of 1e-38.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -27,9 +27,8 @@ __device__ __forceinline__ unsigned round_pair(float& a, float& b) {
     b -= back.y;
     return __builtin_bit_cast(unsigned, h);
 }
-// Eight floats (the k of one lane) as one operand of the instruction: rounded; rounded, leaving in v what the rounding
-// left; and for any value -- infinities and NaN are their own first part and leave nothing, a finite value is cut off
-// instead of rounded, which never overflows.
+// Eight floats (the k of one lane) as one operand of the instruction: rounded; and rounded, leaving in v what the rounding
+// left.
 __device__ __forceinline__ uint4 bf16_eight(const float (&v)[8]) {
     return make_uint4(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]), bf16_pair(v[4], v[5]), bf16_pair(v[6], v[7]));
 }
@@ -40,16 +39,6 @@ __device__ __forceinline__ uint4 round_eight(float (&v)[8]) {
     r.z = round_pair(v[4], v[5]);
     r.w = round_pair(v[6], v[7]);
     return r;
-}
-__device__ __forceinline__ uint4 cut_eight(float (&v)[8]) {
-    float first[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const bool finite = fabsf(v[i]) < __builtin_inff();
-        first[i] = finite ? __uint_as_float(__float_as_uint(v[i]) & 0xffff0000u) : v[i];
-        v[i] = finite ? v[i] - first[i] : 0.f;
-    }
-    return bf16_eight(first);
 }
 __device__ __forceinline__ split_f4 mfma_bf16(uint4 a, uint4 b, split_f4 d) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(split_bf8, a), __builtin_bit_cast(split_bf8, b), d, 0, 0, 0);

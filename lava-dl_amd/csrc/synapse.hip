@@ -342,10 +342,15 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kerne
 // -> 320 us on average of both (161 registers, three waves per SIMD; five taps 193, two waves).  The error against float64
 // is 0.6 to 0.9 times that of the float32 form (real values 2.5e-7 and 2.9e-7 at 96 pairs).  What bounds it now: the
 // unaligned rows of the result (T = 300) for few channels, the vector instructions of the split for gradients.
+//
+// A value that is not finite, or that rounds to an infinite first part, leaves parts of either sign, and infinity times
+// each of them is not infinity times their sum: a wave with a result that is not finite computes its row again from
+// the operands as they are, and so does every wave of a workgroup with such a weight.
 // LDS: the parts of the weights in the operand's layout, [group][tap][part][lane]; per wave the byte
 // offset of every pair's input row (or kOutOfRange).
 template <int KW, bool STREAM, bool TAIL>
-__global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const SynapseConv p) {
+__global__ __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(KW <= 3 ? 3 : 2)))
+void synapse_conv_split_kernel(const SynapseConv p) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int G = p.KG;                                 // groups of 32 pairs
     const int pairs = p.Ci * p.kh;
@@ -365,6 +370,7 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
 
     const int64_t k_full = (int64_t)p.Ci * p.kh_full * p.kw_full;
     unsigned low = 0u;
+    bool odd = false;                                   // a weight that is not finite
     for (int i = tid; i < G * KW * kWave; i += threads) {
         const int l = i & (kWave - 1), x = (i >> 6) % KW, g = (i >> 6) / KW;
         const int co = co0 + (l & 15);
@@ -374,9 +380,10 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
             const int pr = 32 * g + 8 * (l >> 4) + e, ci = pr / p.kh, y = pr - ci * p.kh;
             v[e] = (pr < pairs && co < p.Co) ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.0f;
             low |= __float_as_uint(v[e]);
+            odd = odd || !(fabsf(v[e]) < __builtin_inff());
         }
         uint4* to = wt + (i >> 6) * 3 * kWave + l;
-        to[0] = cut_eight(v);
+        to[0] = round_eight(v);
         to[kWave] = round_eight(v);
         to[2 * kWave] = bf16_eight(v);
     }
@@ -392,6 +399,7 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
         row_off[pr] = (pr < pairs && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
     }
     const bool split_w = __syncthreads_or((low & 0xffffu) != 0u);
+    const bool float_only = __syncthreads_or(odd);
     if (!on) return;
     const int t0 = tile * kSynTile;
     SynQuad tq;
@@ -422,6 +430,17 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
             raw[4 * i + 3] = buf_load4<false>(src, t_ok ? o[i].w + at : kOutOfRange);
         }
     };
+    // lane (kk, j): output channels co0 + 4 kk + i, steps t0 + 4 j + e
+    auto store = [&](int wo, const syn_f4 (&d)[4]) {
+        const int opix = p.out_pixel(ho, wo) * col + (t0 + 4 * j) * 4;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int co = co0 + 4 * kk + i;
+            syn_store_quad<STREAM, TAIL>(dst, co < p.Co, co * (p.Ho_full * p.Wo_full * col) + opix, tq.nv,
+                                         make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
+        }
+    };
+    float stored = 0.f;                                                  // not finite once a result is not
     syn_f4 acc[KW][4];
     if (c_lo < c_hi) fetch(c_lo, 0);
 #pragma unroll
@@ -435,15 +454,12 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
             for (int g = 0; g < G; ++g) {
                 float v[4][8];                                       // [step of the quad][pair]
                 unsigned bits = 0u;
-                auto take = [&]() {
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const float4 r = tq.template place<TAIL>(raw[i]);
-                        v[0][i] = r.x; v[1][i] = r.y; v[2][i] = r.z; v[3][i] = r.w;
-                        bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
-                    }
-                };
-                take();
+                for (int i = 0; i < 8; ++i) {
+                    const float4 r = tq.template place<TAIL>(raw[i]);
+                    v[0][i] = r.x; v[1][i] = r.y; v[2][i] = r.z; v[3][i] = r.w;
+                    bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
+                }
                 const bool split_x = __any((bits & 0xffffu) != 0u);
                 const uint4* wg = wt + g * KW * 3 * kWave + lane;
                 // One copy of the products, in loops over the parts (branches around several copies cost the
@@ -460,19 +476,6 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
                         for (int e = 0; e < 4; ++e) q[e] = bf16_eight(v[e]);
                     }
                     if (tx == 0) {
-                        if (split_x) {
-                            float left = 0.f;
-#pragma unroll
-                            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                                for (int i = 0; i < 8; ++i) left += fabsf(v[e][i]);
-                            if (__any(!(left < __builtin_inff()))) { // a value that is not finite or rounds to infinity
-                                fetch(c, g);
-                                take();
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) q[e] = cut_eight(v[e]);
-                            }
-                        }
                         const bool last = g + 1 == G;                // the next loads are on their way during the products
                         if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
                     }
@@ -490,20 +493,44 @@ __global__ __launch_bounds__(8 * kWave) void synapse_conv_split_kernel(const Syn
         }
         const int wo = c - (KW - 1);
         if (wo >= w_lo) {
-            // lane (kk, j): output channels co0 + 16 o + 4 kk + i, steps t0 + 4 j + e
-            const int opix = p.out_pixel(ho, wo) * col + (t0 + 4 * j) * 4;
+            const syn_f4 (&d)[4] = acc[KW - 1];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const syn_f4 (&d)[4] = acc[KW - 1];
-                const int co = co0 + 4 * kk + i;
-                syn_store_quad<STREAM, TAIL>(dst, co < p.Co, co * (p.Ho_full * p.Wo_full * col) + opix, tq.nv,
-                                             make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
-            }
+            for (int e = 0; e < 4; ++e) stored += (d[e][0] + d[e][1]) + (d[e][2] + d[e][3]);
+            store(wo, d);
         }
 #pragma unroll
         for (int x = KW - 1; x >= 0; --x)
 #pragma unroll
             for (int e = 0; e < 4; ++e) acc[x][e] = x > 0 ? acc[x - 1][e] : syn_f4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (!float_only && !__any(!(fabsf(stored) < __builtin_inff()))) return;
+
+    // once more in float32 multiplications and additions, taps outside the image as products with zero like the float32 form
+#pragma unroll 1
+    for (int wo = w_lo; wo < w_hi; ++wo) {
+        syn_f4 d[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[e] = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int pr = 0; pr < pairs; ++pr) {
+            const int ci = pr / p.kh, y = pr - ci * p.kh, row = row_off[pr];
+#pragma unroll 1
+            for (int x = 0; x < KW; ++x) {
+                const int c = wo + x - p.pw;
+                const bool in = t_ok && row != kOutOfRange && (unsigned)c < (unsigned)p.W;
+                const float4 q = tq.template place<TAIL>(buf_load4<false>(src, in ? row + c * col + tq.t_load * 4 : kOutOfRange));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int co = co0 + 4 * kk + i;
+                    const float w = co < p.Co ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.f;
+                    d[0][i] = __fmaf_rn(w, q.x, d[0][i]);
+                    d[1][i] = __fmaf_rn(w, q.y, d[1][i]);
+                    d[2][i] = __fmaf_rn(w, q.z, d[2][i]);
+                    d[3][i] = __fmaf_rn(w, q.w, d[3][i]);
+                }
+            }
+        }
+        store(wo, d);
     }
 }
 

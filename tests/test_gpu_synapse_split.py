@@ -84,3 +84,52 @@ def test_values_that_are_not_finite_or_overflow_a_part(where, value):
         assert torch.equal(a.isinf(), b.isinf()) and torch.equal(a[a.isinf()], b[b.isinf()]), name
         ok = a.isfinite()
         assert float((a[ok] - b[ok]).abs().max()) <= 1e-5 * float(b[ok].abs().max()), name
+
+
+def _padded_sums(x, w, g, stride, padding, dilation):
+    """The three passes in float64 as sums over every tap, taps outside the image as products with zero: what the float32
+    matrix instruction gives for operands that are not finite (0 * inf among them).  Unit stride and dilation, or none."""
+    x, w, g = x.double(), w.double()[..., 0], g.double()
+
+    def correlate(a, b, pad):                                        # a [N, Ci, H, W, T], b [Co, Ci, kh, kw]
+        kh, kw = b.shape[2:]
+        a = F.pad(a, (0, 0, pad[1], pad[1], pad[0], pad[0])).unfold(2, kh, 1).unfold(3, kw, 1)
+        return torch.stack([(a * b[co][None, :, None, None, None]).sum((1, 5, 6)) for co in range(b.shape[0])], 1)
+    kh, kw = w.shape[2:]
+    y = correlate(x, w, padding)
+    gx = correlate(g, w.flip(2, 3).transpose(0, 1), (kh - 1 - padding[0], kw - 1 - padding[1]))
+    taps = F.pad(x, (0, 0, padding[1], padding[1], padding[0], padding[0])).unfold(2, kh, 1).unfold(3, kw, 1)
+    gw = torch.stack([(taps * g[:, co, None, ..., None, None]).sum((0, 2, 3, 4)) for co in range(w.shape[0])])
+    return y, gx, gw[..., None]
+
+
+# both directions in the split form; 2, 3 and 5 taps; one group of pairs and two; a row that ends inside a quad; and the
+# float32 form (12 pairs forward)
+NOT_FINITE = [((2, 10, 5, 5, 36), 9, (2, 2)), ((1, 6, 6, 5, 37), 17, (3, 3)), ((1, 12, 5, 6, 70), 16, (3, 3)),
+              ((1, 4, 6, 6, 33), 7, (5, 5)), ((1, 4, 5, 6, 36), 16, (3, 3))]
+
+
+@pytest.mark.parametrize('case', NOT_FINITE, ids=str)
+@pytest.mark.parametrize('kind', ['spikes', 'real'])
+@pytest.mark.parametrize('where', ['input', 'gradient', 'weight'])
+@pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan'), 3.4e38])
+def test_not_finite_times_operands_of_several_parts(case, kind, where, value):
+    """The parts of a split operand are zero or of either sign: inf times each of them is not inf times their sum."""
+    shape, co, kernel = case
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x = torch.randn(shape, generator=gen) if kind == 'real' else (torch.rand(shape, generator=gen) < 0.5).float()
+    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
+    pad = (kernel[0] // 2, kernel[1] // 2)
+    g = torch.randn((shape[0], co) + tuple(s + 2 * p - k + 1 for s, p, k in zip(shape[2:4], pad, kernel)) + shape[4:],
+                    generator=gen)
+    # a pixel whose taps all lie inside the image: the weight gradient does not visit columns outside it
+    {'input': x[0, 1, 2, 3, 5:], 'gradient': g[0, 3, 2, 2, 9:], 'weight': w[2, 1, 1, 0]}[where].view(-1)[0] = value
+    geometry = (1, 1), pad, (1, 1)
+    got, want = _run(x, w, g, *geometry), _padded_sums(x, w, g, *geometry)
+    size = _padded_sums(x.abs(), w.abs(), g.abs(), *geometry)
+    for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
+        a, b32 = a.cpu(), b.float()                                  # what overflows float32 is infinite in float32
+        assert torch.equal(a.isnan(), b32.isnan()), name
+        assert torch.equal(a.isinf(), b32.isinf()) and torch.equal(a[a.isinf()], b32[b32.isinf()]), name
+        ok = a.isfinite()
+        assert bool(((a.double() - b).abs()[ok] <= 1e-5 * m[ok] + 1e-30).all()), name
