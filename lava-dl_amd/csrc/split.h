@@ -4,11 +4,17 @@
 // i + j <= 2 are taken, what is left out is below 2^-26 of the product.
 //   A value that is not finite leaves a NaN (so does a finite one beyond the largest bfloat16, 3.3895e38): callers
 // either treat it (conv.hip) or recognise a result that is not finite and compute it again in float32 (synapse.hip).
-//   Parts below the smallest normal number are lost: a value under 3e-33 enters with an absolute error of 1e-38.
+//   Parts below the smallest normal number are lost: a value under 3e-33 enters with an absolute error of 1e-38.  Every
+// float32 is a multiple of 2^-149, and so is what its parts leave: multiplied by kSplitScale first (exact), every part of
+// every value is zero or a normal number.  synapse.hip scales both operands; values from 1e31 on then overflow, like
+// values that are not finite.
 #pragma once
 #include <hip/hip_runtime.h>
 
 namespace slayer {
+
+constexpr float kSplitScale = 0x1p24f;
+constexpr float kSplitProductScale = 0x1p-48f;      // what takes the scale out of a product
 
 typedef __bf16 split_bf2 __attribute__((ext_vector_type(2)));
 typedef __bf16 split_bf8 __attribute__((ext_vector_type(8)));

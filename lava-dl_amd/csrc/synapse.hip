@@ -343,7 +343,7 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kerne
 // is 0.6 to 0.9 times that of the float32 form (real values 2.5e-7 and 2.9e-7 at 96 pairs).  What bounds it now: the
 // unaligned rows of the result (T = 300) for few channels, the vector instructions of the split for gradients.
 //
-// A value that is not finite, or that rounds to an infinite first part, leaves parts of either sign, and infinity times
+// A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
 // each of them is not infinity times their sum: a wave with a result that is not finite computes its row again from
 // the operands as they are, and so does every wave of a workgroup with such a weight.
 // LDS: the parts of the weights in the operand's layout, [group][tap][part][lane]; per wave the byte
@@ -381,6 +381,7 @@ void synapse_conv_split_kernel(const SynapseConv p) {
             v[e] = (pr < pairs && co < p.Co) ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.0f;
             low |= __float_as_uint(v[e]);
             odd = odd || !(fabsf(v[e]) < __builtin_inff());
+            v[e] *= kSplitScale;
         }
         uint4* to = wt + (i >> 6) * 3 * kWave + l;
         to[0] = round_eight(v);
@@ -457,7 +458,8 @@ void synapse_conv_split_kernel(const SynapseConv p) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float4 r = tq.template place<TAIL>(raw[i]);
-                    v[0][i] = r.x; v[1][i] = r.y; v[2][i] = r.z; v[3][i] = r.w;
+                    v[0][i] = r.x * kSplitScale; v[1][i] = r.y * kSplitScale;
+                    v[2][i] = r.z * kSplitScale; v[3][i] = r.w * kSplitScale;
                     bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
                 }
                 const bool split_x = __any((bits & 0xffffu) != 0u);
@@ -493,9 +495,14 @@ void synapse_conv_split_kernel(const SynapseConv p) {
         }
         const int wo = c - (KW - 1);
         if (wo >= w_lo) {
-            const syn_f4 (&d)[4] = acc[KW - 1];
+            syn_f4 d[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) stored += (d[e][0] + d[e][1]) + (d[e][2] + d[e][3]);
+            for (int e = 0; e < 4; ++e) {
+                d[e] = acc[KW - 1][e];
+                stored += (d[e][0] + d[e][1]) + (d[e][2] + d[e][3]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) d[e][i] *= kSplitProductScale;
+            }
             store(wo, d);
         }
 #pragma unroll
@@ -772,7 +779,7 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 // steps per visit leave 2: 335 and 368 us).  What bounds it now: lines of the unaligned rows (T = 300) that two visits
 // share and fetch twice, and the vector instructions of the split.
 //
-// What is not finite (or beyond the largest bfloat16) shows as a NaN in a tile at the end: the wave then runs its
+// What is not finite (or overflows when it is scaled or rounded) shows in a tile at the end: the wave then runs its
 // share again with the float32 instruction (float_products), whose results such inputs had before.
 #ifndef SLAYER_WGRAD_GROUPS
 #define SLAYER_WGRAD_GROUPS 1
@@ -825,10 +832,13 @@ struct WgradRow {
     __device__ __forceinline__ uint4 get(int slot) const {
         return *reinterpret_cast<const uint4*>(lds + slot * kWgSlot + (lane & 15) * kWgPitch + (lane >> 4) * 16);
     }
+    __device__ __forceinline__ static float4 scaled(float4 v) {
+        return make_float4(v.x * kSplitScale, v.y * kSplitScale, v.z * kSplitScale, v.w * kSplitScale);
+    }
     __device__ __forceinline__ void put_parts(int slot, const float4 (&raw)[2], const SynQuad& tq) const {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            float4 v = tq.template place<TAIL>(raw[h]);
+            float4 v = scaled(tq.template place<TAIL>(raw[h]));
             uint2 part;
 #pragma unroll
             for (int t = 0; t < 3; ++t) {
@@ -884,7 +894,7 @@ struct WgradRow {
             for (int u = 0; u < kWgU; ++u) fetch(0, u);
             for (int c = 0; c < p.W; ++c) {
                 const unsigned flip = (c & 1) ? 0x80008000u : 0u;
-                const float sign = (c & 1) ? -1.0f : 1.0f;
+                const float back = (c & 1) ? -kSplitProductScale : kSplitProductScale;
                 auto flipped = [&](uint4 v) { return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip); };
 #pragma unroll
                 for (int u = 0; u < kWgU; ++u) {
@@ -902,7 +912,7 @@ struct WgradRow {
                     for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
-                            float4 v = raw_q[u][pt][h];
+                            float4 v = scaled(raw_q[u][pt][h]);
                             if (!more) {
                                 put(3 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
                             } else {
@@ -940,7 +950,7 @@ struct WgradRow {
 #pragma unroll
                         for (int x = 0; x < KW; ++x)
 #pragma unroll
-                            for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(sign, d[x][i], acc[x][pt][i]);
+                            for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(back, d[x][i], acc[x][pt][i]);
                     }
                     settle();
                 }
@@ -979,14 +989,14 @@ struct WgradRow {
             }
         }
     }
-    __device__ __forceinline__ bool any_nan() const {
+    __device__ __forceinline__ bool not_finite() const {
         bool bad = false;
 #pragma unroll
         for (int x = 0; x < KW; ++x)
 #pragma unroll
             for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bad = bad || acc[x][pt][i] != acc[x][pt][i];
+                for (int i = 0; i < 4; ++i) bad = bad || !(fabsf(acc[x][pt][i]) < __builtin_inff());
         return __any(bad);
     }
 };
@@ -1022,7 +1032,7 @@ void synapse_wgrad_row_kernel(const SynapseWgrad p) {
     w.t_lo = tpart * p.tlen;
     w.t_hi = (w.t_lo + p.tlen) < p.T ? (w.t_lo + p.tlen) : p.T;
     w.split_products();
-    if (w.any_nan()) w.float_products();
+    if (w.not_finite()) w.float_products();
     // lane (q, j) of tile (x, pt): channels co0 + 4 q + i, pair 16 (pass NPT + pt) + j, tap x of its row
     float4* dst = reinterpret_cast<float4*>(p.partial) +
                   ((((int64_t)(n * cobs + cob) * p.items + item) * p.passes + pass) * (KW * NPT)) * kWave + lane;

@@ -133,3 +133,34 @@ def test_not_finite_times_operands_of_several_parts(case, kind, where, value):
         assert torch.equal(a.isinf(), b32.isinf()) and torch.equal(a[a.isinf()], b32[b32.isinf()]), name
         ok = a.isfinite()
         assert bool(((a.double() - b).abs()[ok] <= 1e-5 * m[ok] + 1e-30).all()), name
+
+
+@pytest.mark.parametrize('case', [((2, 10, 5, 5, 36), 9, (2, 2)), ((1, 12, 5, 6, 70), 16, (3, 3)), ((1, 7, 6, 6, 33), 7, (5, 5))],
+                         ids=str)
+@pytest.mark.parametrize('where', ['input', 'gradient', 'weight', 'input and weight', 'input and gradient'])
+@pytest.mark.parametrize('scale', [2.0 ** -126, 1e-36, 1e-33, 1e-30, 1e-20, 1e20, 1e33])
+def test_magnitudes_far_from_one(case, where, scale):
+    """A value keeps its 24 bits whatever its magnitude (a part of a split operand must not fall below the smallest normal
+    number), down to products and sums of float32's smallest numbers: the bar adds half a unit of these per term of a sum.
+    Sums whose terms leave float32's range are infinite or NaN, by their order, and not looked at."""
+    shape, co, kernel = case
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x = torch.randn(shape, generator=gen)
+    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
+    pad = (kernel[0] // 2, kernel[1] // 2)
+    g = torch.randn((shape[0], co) + tuple(s + 2 * p - k + 1 for s, p, k in zip(shape[2:4], pad, kernel)) + shape[4:],
+                    generator=gen)
+    if 'input' in where:
+        x *= scale
+    if 'gradient' in where:
+        g *= scale
+    if 'weight' in where:
+        w *= scale
+    geometry = (1, 1), pad, (1, 1)
+    got, want = _run(x, w, g, *geometry), _reference(x, w, g, *geometry)
+    size = _reference(x.abs(), w.abs(), g.abs(), *geometry)
+    for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
+        a, terms = a.cpu().double(), {'output': shape[1], 'grad input': co}.get(name, 0) * kernel[0] * kernel[1]
+        terms = terms or g.numel() // co
+        inside = m < 2.0 ** 127                                      # no order of the sum leaves the range
+        assert bool(((a - b).abs() <= 1e-5 * m + terms * 2.0 ** -150)[inside].all()), name
