@@ -1341,14 +1341,18 @@ void wgrad_shape(int64_t N, int64_t Ci, int64_t Co, int64_t Ho, int64_t T, int64
                  SynapseWgrad& p) {
     if (f.row_kw) p.passes = (int)((Ci * kh + 16 * f.npt - 1) / (16 * f.npt));
     else p.passes = (int)((Ci * kh * kw + 16 * f.tiles - 1) / (16 * f.tiles));
-    // about eight thousand waves (4096: [16,32,16,16,300] -> 64 channels 310 instead of 285 us), shares of whole visits of 32 steps: a wave's
-    // set-up (tables, the gradient window) is paid once per share
-#ifndef SLAYER_WGRAD_WAVES
-#define SLAYER_WGRAD_WAVES 8192
-#endif
+    // Shares of whole visits of 32 steps, about eight thousand waves: a wave's set-up (the gradient window) is paid once per
+    // share ([16,32,16,16,300] -> 64 channels 310 us with 4096 waves, 285 with 8192).  A row of up to 16 pairs has few
+    // products to a visit and is bound by its loads, and a line that two visits of one share have in common is gone
+    // from the caches when the second one comes, while the waves of neighbouring shares find it there: one visit a
+    // share, up to 32768 waves (float32 kernel before / 8192 / 32768 waves: [32,4,32,32,300] -> 16 channels 237 / 280 / 206 us,
+    // [64,1,32,32,300] -> 16 383 / 445 / 313, [8,4,64,64,300] -> 64 904 / 1008 / 685, 5x5 [32,2,32,32,300] -> 16
+    // 303 / 260 / 198, and where rows are whole lines [32,4,32,32,256] -> 16 147 / 147 / 146, [128,4,32,32,64] -> 16
+    // 167 / 176 / 177).
+    const int64_t waves = f.npt == 1 ? 32768 : 8192;
     const int64_t base = N * ((Co + 15) / 16) * Ho;
     const int64_t visits = (T + 31) / 32;
-    int64_t parts = (SLAYER_WGRAD_WAVES + base - 1) / base;
+    int64_t parts = (waves + base - 1) / base;
     parts = parts > visits ? visits : (parts < 1 ? 1 : parts);
     const int64_t len = (visits + parts - 1) / parts * 32;
     p.tparts = (int)((T + len - 1) / len);
