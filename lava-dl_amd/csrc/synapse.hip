@@ -1119,12 +1119,33 @@ using namespace slayer;
 
 namespace {
 
-#ifndef SLAYER_SPLIT_WAVES
-#define SLAYER_SPLIT_WAVES 6144
-#endif
 #ifndef SLAYER_SYN_PIX
 #define SLAYER_SYN_PIX 4
 #endif
+
+// What a launch of the row kernels takes, in us: every wave walks its piece of an image row -- the columns of the split
+// form with 32 (input channel, kernel row) pairs to a group, the blocks of four pixels of the float32 form with four -- and a
+// group costs a wait for its loads and its share of the SIMD, which all waves there divide up.  Fitted to 1900 layers
+// (2, 3 and 5 taps, 17 to 192 pairs, 3 to 64 output channels, 1 to 64 samples of 8x8 to 34x34 pixels, 50 to 302 steps; real
+// values times real weights) with an error of 12 to 15 % for the split and 13 to 22 % for the float32 form.
+// Split form over float32 form where it decides for the former (963 of 1741 layers), mean / 95 % of the layers / largest:
+//            spikes x quantised     real x quantised       real x real
+//   2 taps   0.60 / 0.83 / 1.25     0.71 / 0.96 / 1.28     0.79 / 1.11 / 1.30
+//   3 taps   0.61 / 0.90 / 1.05     0.72 / 0.93 / 1.06     0.83 / 1.03 / 1.30
+//   5 taps   0.46 / 0.70 / 0.84     0.65 / 0.88 / 1.01     0.85 / 1.12 / 1.44
+// Taken always from 17 pairs on, the split form lost up to 2.8 times on single samples of small images, up to 1.7
+// times with badly filled groups (5x5, 40 pairs, real x real 195 us against 141).
+double row_form_time(bool split, const SynapseConv& p, int64_t row_tiles, int pieces) {
+    struct Cost { double launch, step, wait, rate, tail; };               // tail: rows that end inside a quad
+    static constexpr Cost costs[2][3] = {{{0.0, 2.0, 0.21, 0.645, 0.85}, {4.5, 0.0, 0.10, 0.96, 0.71}, {1.0, 3.25, 0.62, 1.26, 0.69}},
+                                         {{1.7, 0.54, 0.03, 1.10, 0.70}, {0.0, 0.51, 0.30, 1.14, 0.63}, {0.0, 0.38, 0.71, 1.28, 0.92}}};
+    const Cost& c = costs[split][p.kw == 5 ? 2 : p.kw - 2];
+    const int pixels = (p.Wo + pieces - 1) / pieces, pairs = p.Ci * p.kh;
+    const int steps = split ? pixels + p.kw - 1 : (pixels + 3) / 4;
+    const int groups = split ? (pairs + 31) / 32 : (pairs + 3) / 4;
+    const double load = (double)(row_tiles * pieces) / 1024;              // waves per SIMD
+    return c.launch + steps * (c.step + groups * (c.wait + c.rate * (load > 1 ? load : 1))) * (p.T % 4 ? 1 + c.tail : 1);
+}
 
 // One launch of the convolution kernels for the geometry in p (tensors, sizes, taps and sub-lattices filled in by the
 // caller): the row kernel for unit stride and dilation along the image row with 2, 3 or 5 taps per row, else the
@@ -1156,20 +1177,17 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     if (blocks > 0x7fffffffLL) return SLAYER_ERANGE;
     const bool tail = (p.T % 4) != 0;                                     // rows that end inside a quad
     const dim3 grid((unsigned)blocks), block(kSynWaves * kWave);
-    // The split form from 17 (input channel, kernel row) pairs on -- it takes them 32 at a time -- if the parts of 16
-    // channels' weights fit LDS.  Spikes with quantised weights / real values with quantised weights / both real, us, here
-    // and in the float32 form below: 3x3, 24 pairs on [16,8,32,32,300] 165 / 164 / 171 and 180 / 180 / 180; 48 pairs on
-    // [8,16,24,24,300] 86 / 121 / 134 and 142 / 149 / 148; 5x5, 40 pairs on [8,8,32,32,300] 83 / 145 / 195 and 138 / 139 /
-    // 141; 80 pairs on [8,16,24,24,300] 131 / 195 / 275 and 360 / 365 / 364; 160
-    // pairs on [4,32,16,16,300] 103 / 214 / 311 and 277 / 281 / 280.  With 12 pairs ([16,4,32,32,300]) 59 / 95 / 115
-    // and 64 / 65 / 65: the float32 form.
-    const int g32 = (p.Ci * p.kh + 31) / 32;
+    // The split form where it is not the slower one with both operands real, its worst case (row_form_time), from 17 pairs
+    // on, and if the parts of 16 channels' weights fit LDS.  A piece of an image row visits kw - 1 columns more than it has
+    // pixels: rows are cut while there are few waves, for five taps (two waves per SIMD) below 1024 only
+    // ([4,16,16,16,300] -> 64 channels 182 us with 2560 waves, 140 with 1280).
+    const int pairs = p.Ci * p.kh;
+    const int g32 = (pairs + 31) / 32;
     const size_t split_lds = (size_t)g32 * p.kw * 3 * 1024;
-    if (rows && p.Ci * p.kh > 16 && split_lds <= 96 * 1024) {
+    int pieces = 1;
+    while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
+    if (rows && pairs > 16 && split_lds <= 96 * 1024 && row_form_time(true, p, base, pieces) <= 1.05 * row_form_time(false, p, base, wsplit)) {
         const int waves = split_lds > 40 * 1024 ? 8 : 4;
-        const int64_t rows_all = (int64_t)p.N * cobs * p.Ho * p.ttiles;
-        int pieces = 1;                                                  // a piece visits kw - 1 columns more than it has pixels
-        while (rows_all * pieces < SLAYER_SPLIT_WAVES && p.Wo >= 16 * pieces) pieces *= 2;
         p.wsplit = pieces;
         p.KG = g32;
         const int64_t all = (int64_t)p.Ho * pieces * p.ttiles;

@@ -103,29 +103,67 @@ def _padded_sums(x, w, g, stride, padding, dilation):
     return y, gx, gw[..., None]
 
 
-# both directions in the split form; 2, 3 and 5 taps; one group of pairs and two; a row that ends inside a quad; and the
-# float32 form (12 pairs forward)
-NOT_FINITE = [((2, 10, 5, 5, 36), 9, (2, 2)), ((1, 6, 6, 5, 37), 17, (3, 3)), ((1, 12, 5, 6, 70), 16, (3, 3)),
-              ((1, 4, 6, 6, 33), 7, (5, 5)), ((1, 4, 5, 6, 36), 16, (3, 3))]
+# Layers whose two directions fill the split form's groups of 32 pairs (24, 26; 24, 51; 48, 24; 25, 50 pairs), rows that end inside
+# a quad among them, and one with the float32 form forward (12 pairs).  It takes launches of 1024 waves and more, here
+# by a batch that is zero but for one sample.
+SPLIT = [((1, 12, 5, 5, 36), 13, (2, 2)), ((1, 8, 6, 5, 37), 17, (3, 3)), ((1, 16, 5, 6, 70), 8, (3, 3)), ((1, 5, 6, 6, 33), 10, (5, 5)),
+         ((1, 4, 5, 6, 36), 16, (3, 3))]
 
 
-@pytest.mark.parametrize('case', NOT_FINITE, ids=str)
+def _run_in_large_batch(x, w, g, stride, padding, dilation):
+    waves = g.shape[2] * ((g.shape[-1] + 63) // 64)
+    batch = 1024 // min(waves, x.shape[2] * ((x.shape[-1] + 63) // 64)) + 1
+    at = batch // 2
+
+    def embed(v):
+        return torch.zeros((batch,) + v.shape[1:]).index_copy(0, torch.tensor([at]), v)
+    y, gx, gw = _run(embed(x), w, embed(g), stride, padding, dilation)
+    return y[at:at + 1], gx[at:at + 1], gw
+
+
+def _operands(case, kind='real'):
+    shape, co, kernel = case
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x = torch.randn(shape, generator=gen)
+    if kind == 'spikes':
+        x = (torch.rand(shape, generator=gen) < 0.5).float()
+    elif kind == 'mixed':
+        x = (x > 1).float() + (torch.rand(shape, generator=gen) < 0.002) * x
+    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
+    pad = (kernel[0] // 2, kernel[1] // 2)
+    g = torch.randn((shape[0], co) + tuple(s + 2 * p - k + 1 for s, p, k in zip(shape[2:4], pad, kernel)) + shape[4:],
+                    generator=gen)
+    return x, w, g, ((1, 1), pad, (1, 1))
+
+
+# ... and the ends of a group of 32 pairs, several blocks of channels, an image row cut into pieces
+@pytest.mark.parametrize('case', SPLIT + [((1, 31, 4, 20, 64), 33, (1, 3)), ((1, 32, 4, 5, 65), 32, (1, 2)), ((1, 24, 5, 33, 301), 63, (1, 5)),
+                                          ((1, 6, 6, 6, 40), 12, (5, 5))],
+                         ids=str)
+@pytest.mark.parametrize('kind', ['spikes', 'mixed', 'real'])
+@pytest.mark.parametrize('quantised', [True, False])
+def test_split_form_of_large_launches(case, kind, quantised):
+    x, w, g, geometry = _operands(case, kind)
+    if quantised:
+        w = (w * 32).round().clamp(-128, 127) / 64
+    got, want = _run_in_large_batch(x, w, g, *geometry), _reference(x, w, g, *geometry)
+    size = _reference(x.abs(), w.abs(), g.abs(), *geometry)
+    for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
+        assert_sum(a, b, m + 1e-30, f'{kind} {name}')
+    if quantised and kind == 'spikes':
+        assert torch.equal(got[0].cpu().double(), want[0]), 'sums of spikes times quantised weights are exact'
+
+
+@pytest.mark.parametrize('case', SPLIT, ids=str)
 @pytest.mark.parametrize('kind', ['spikes', 'real'])
 @pytest.mark.parametrize('where', ['input', 'gradient', 'weight'])
 @pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan'), 3.4e38])
 def test_not_finite_times_operands_of_several_parts(case, kind, where, value):
     """The parts of a split operand are zero or of either sign: inf times each of them is not inf times their sum."""
-    shape, co, kernel = case
-    gen = torch.Generator().manual_seed(sum(shape) + co)
-    x = torch.randn(shape, generator=gen) if kind == 'real' else (torch.rand(shape, generator=gen) < 0.5).float()
-    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
-    pad = (kernel[0] // 2, kernel[1] // 2)
-    g = torch.randn((shape[0], co) + tuple(s + 2 * p - k + 1 for s, p, k in zip(shape[2:4], pad, kernel)) + shape[4:],
-                    generator=gen)
+    x, w, g, geometry = _operands(case, kind)
     # a pixel whose taps all lie inside the image: the weight gradient does not visit columns outside it
     {'input': x[0, 1, 2, 3, 5:], 'gradient': g[0, 3, 2, 2, 9:], 'weight': w[2, 1, 1, 0]}[where].view(-1)[0] = value
-    geometry = (1, 1), pad, (1, 1)
-    got, want = _run(x, w, g, *geometry), _padded_sums(x, w, g, *geometry)
+    got, want = _run_in_large_batch(x, w, g, *geometry), _padded_sums(x, w, g, *geometry)
     size = _padded_sums(x.abs(), w.abs(), g.abs(), *geometry)
     for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
         a, b32 = a.cpu(), b.float()                                  # what overflows float32 is infinite in float32
@@ -135,32 +173,24 @@ def test_not_finite_times_operands_of_several_parts(case, kind, where, value):
         assert bool(((a.double() - b).abs()[ok] <= 1e-5 * m[ok] + 1e-30).all()), name
 
 
-@pytest.mark.parametrize('case', [((2, 10, 5, 5, 36), 9, (2, 2)), ((1, 12, 5, 6, 70), 16, (3, 3)), ((1, 7, 6, 6, 33), 7, (5, 5))],
-                         ids=str)
+@pytest.mark.parametrize('case', SPLIT[:4], ids=str)
 @pytest.mark.parametrize('where', ['input', 'gradient', 'weight', 'input and weight', 'input and gradient'])
 @pytest.mark.parametrize('scale', [2.0 ** -126, 1e-36, 1e-33, 1e-30, 1e-20, 1e20, 1e33])
 def test_magnitudes_far_from_one(case, where, scale):
     """A value keeps its 24 bits whatever its magnitude (a part of a split operand must not fall below the smallest normal
     number), down to products and sums of float32's smallest numbers: the bar adds half a unit of these per term of a sum.
     Sums whose terms leave float32's range are infinite or NaN, by their order, and not looked at."""
-    shape, co, kernel = case
-    gen = torch.Generator().manual_seed(sum(shape) + co)
-    x = torch.randn(shape, generator=gen)
-    w = torch.randn((co, shape[1]) + kernel + (1,), generator=gen)
-    pad = (kernel[0] // 2, kernel[1] // 2)
-    g = torch.randn((shape[0], co) + tuple(s + 2 * p - k + 1 for s, p, k in zip(shape[2:4], pad, kernel)) + shape[4:],
-                    generator=gen)
+    x, w, g, geometry = _operands(case)
     if 'input' in where:
         x *= scale
     if 'gradient' in where:
         g *= scale
     if 'weight' in where:
         w *= scale
-    geometry = (1, 1), pad, (1, 1)
-    got, want = _run(x, w, g, *geometry), _reference(x, w, g, *geometry)
+    got, want = _run_in_large_batch(x, w, g, *geometry), _reference(x, w, g, *geometry)
     size = _reference(x.abs(), w.abs(), g.abs(), *geometry)
-    for name, a, b, m in zip(('output', 'grad input', 'grad weight'), got, want, size):
-        a, terms = a.cpu().double(), {'output': shape[1], 'grad input': co}.get(name, 0) * kernel[0] * kernel[1]
-        terms = terms or g.numel() // co
-        inside = m < 2.0 ** 127                                      # no order of the sum leaves the range
-        assert bool(((a - b).abs() <= 1e-5 * m + terms * 2.0 ** -150)[inside].all()), name
+    taps = w.shape[2] * w.shape[3]
+    terms = (x.shape[1] * taps, w.shape[0] * taps, g.numel() // w.shape[0])
+    for name, n, a, b, m in zip(('output', 'grad input', 'grad weight'), terms, got, want, size):
+        a, inside = a.cpu().double(), m < 2.0 ** 127                 # no order of the sum leaves the range
+        assert bool(((a - b).abs() <= 1e-5 * m + n * 2.0 ** -150)[inside].all()), name
