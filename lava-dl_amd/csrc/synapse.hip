@@ -1184,9 +1184,11 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     const int pairs = p.Ci * p.kh;
     const int g32 = (pairs + 31) / 32;
     const size_t split_lds = (size_t)g32 * p.kw * 3 * 1024;
+    const size_t row_lds = (size_t)((pairs + 3) / 4) * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
     int pieces = 1;
     while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
-    if (rows && pairs > 16 && split_lds <= 96 * 1024 && row_form_time(true, p, base, pieces) <= 1.05 * row_form_time(false, p, base, wsplit)) {
+    if (rows && pairs > 16 && split_lds <= 96 * 1024 &&
+        (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= 1.05 * row_form_time(false, p, base, wsplit))) {
         const int waves = split_lds > 40 * 1024 ? 8 : 4;
         p.wsplit = pieces;
         p.KG = g32;
@@ -1210,13 +1212,12 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
         return (int)hipGetLastError();
     }
     if (rows) {
-        p.KG = (p.Ci * p.kh + 3) / 4;                                     // groups of four (channel, kernel row) pairs
-        const size_t lds = (size_t)p.KG * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
-        if (lds > 64 * 1024) return SLAYER_ERANGE;
+        p.KG = (pairs + 3) / 4;                                           // groups of four (channel, kernel row) pairs
+        if (row_lds > 64 * 1024) return SLAYER_ERANGE;
 #define SLAYER_SYN_ROW_T(KERNEL, KW)                                                                      \
         do {                                                                                             \
-            if (streaming) hipLaunchKernelGGL((KERNEL<KW, kRowPix, true>), grid, block, lds, st, p);      \
-            else hipLaunchKernelGGL((KERNEL<KW, kRowPix, false>), grid, block, lds, st, p);               \
+            if (streaming) hipLaunchKernelGGL((KERNEL<KW, kRowPix, true>), grid, block, row_lds, st, p);  \
+            else hipLaunchKernelGGL((KERNEL<KW, kRowPix, false>), grid, block, row_lds, st, p);           \
         } while (0)
 #define SLAYER_SYN_ROW(KW)                                                                                \
         do { if (tail) SLAYER_SYN_ROW_T(synapse_conv_row_tail_kernel, KW); else SLAYER_SYN_ROW_T(synapse_conv_row_kernel, KW); } while (0)

@@ -194,3 +194,14 @@ def test_magnitudes_far_from_one(case, where, scale):
     for name, n, a, b, m in zip(('output', 'grad input', 'grad weight'), terms, got, want, size):
         a, inside = a.cpu().double(), m < 2.0 ** 127                 # no order of the sum leaves the range
         assert bool(((a - b).abs() <= 1e-5 * m + n * 2.0 ** -150)[inside].all()), name
+
+
+def test_filters_that_only_the_split_form_holds():
+    """500 (channel, kernel row) pairs of two taps: too many for the float32 row form's 64 KB of LDS at any launch size."""
+    from lava_dl_amd.slayer.synapse import layer
+    gen = torch.Generator().manual_seed(3)
+    x, w = torch.randn(1, 250, 2, 5, 8, generator=gen), torch.randn(250, 2, 4, 4, 1, generator=gen)
+    y = layer._launch_input_grad(x.to(dev()), w[..., 0].transpose(0, 1).contiguous().to(dev()), (1, 2, 4, 10, 8), (2, 2), (1, 1), (1, 1))
+    assert y is not None
+    args = None, (2, 2, 1), (1, 1, 0)
+    assert_sum(y, F.conv_transpose3d(x.double(), w.double(), *args), F.conv_transpose3d(x.double().abs(), w.double().abs(), *args), 'output')
