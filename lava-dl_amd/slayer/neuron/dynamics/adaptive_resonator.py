@@ -73,11 +73,11 @@ class _AdResDynamics(torch.autograd.Function):
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
         grad_real = torch.zeros_like(real) if grad_real is None else grad_real
         grad_imag = torch.zeros_like(imag) if grad_imag is None else grad_imag
-        found = _res._nan_word()
-        g_re, g_im, g_sin, g_cos = _res._bwd(grad_real, grad_imag, real, imag,
-                                             sin_decay.detach(), cos_decay.detach(), need, found)
-        _res._raise_on_nan(found, grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
-                           grad_imag_input=g_im, grad_sin_decay=g_sin, grad_cos_decay=g_cos)
+        with _res._nan_word(real.device) as found:
+            g_re, g_im, g_sin, g_cos = _res._bwd(grad_real, grad_imag, real, imag,
+                                                 sin_decay.detach(), cos_decay.detach(), need, found)
+            _res._raise_on_nan(found, grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
+                               grad_imag_input=g_im, grad_sin_decay=g_sin, grad_cos_decay=g_cos)
         if g_sin is not None:
             g_sin, g_cos = g_sin.reshape(sin_decay.shape), g_cos.reshape(cos_decay.shape)
         return (g_re, g_im, g_sin, g_cos) + (None,) * 9

@@ -4,6 +4,8 @@ Interface of lava.lib.dl.slayer.neuron.dynamics.resonator
 (neuron/dynamics/resonator.py:49-174 in the reference); the body is
 slayer_res_fwd / slayer_res_bwd of libslayer_hip.so.
 """
+import contextlib
+
 import torch
 
 from ... import _native as N
@@ -102,12 +104,18 @@ def _bwd_naive(grad_real, grad_imag, sin_decay, cos_decay):
     return g_re_in, g_im_in
 
 
-def _nan_word():
-    """A word of pinned host memory for the backward kernels to report NaN in: this call's own (torch's pinned-memory
-    cache hands it out again only after the call has let go of it, by when ``_raise_on_nan`` has synchronised)."""
+@contextlib.contextmanager
+def _nan_word(dev):
+    """A word of pinned host memory for the backward kernels on ``dev`` to report NaN in: this call's own.  No stream is
+    recorded for it, so torch's pinned-memory cache hands it out again as soon as it is let go of: by then
+    ``_raise_on_nan`` has synchronised, and so does a call that fails between its launches and there."""
     word = torch.empty(1, dtype=torch.int32, pin_memory=True)
     word[0] = 0
-    return word
+    try:
+        yield word
+    except BaseException:
+        torch.cuda.current_stream(dev).synchronize()
+        raise
 
 
 def _raise_on_nan(found=None, **tensors):
@@ -143,15 +151,15 @@ class _ResDynamics(torch.autograd.Function):
     def backward(ctx, grad_real, grad_imag):
         real, imag, sin_decay, cos_decay = ctx.saved_tensors
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
-        found = _nan_word()
-        g_re, g_im, g_sin, g_cos = _bwd(grad_real, grad_imag, real, imag,
-                                        sin_decay.detach(), cos_decay.detach(), need, found)
-        if ctx.debug:
-            c_re, c_im = _bwd_naive(grad_real, grad_imag, sin_decay.detach(), cos_decay.detach())
-            N.raise_on_mismatch('resonator grad real', g_re, c_re, rel=N.scan_tolerance(g_re))
-            N.raise_on_mismatch('resonator grad imag', g_im, c_im, rel=N.scan_tolerance(g_im))
-        _raise_on_nan(found, grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
-                      grad_imag_input=g_im, grad_sin_decay=g_sin, grad_cos_decay=g_cos)
+        with _nan_word(real.device) as found:
+            g_re, g_im, g_sin, g_cos = _bwd(grad_real, grad_imag, real, imag,
+                                            sin_decay.detach(), cos_decay.detach(), need, found)
+            if ctx.debug:
+                c_re, c_im = _bwd_naive(grad_real, grad_imag, sin_decay.detach(), cos_decay.detach())
+                N.raise_on_mismatch('resonator grad real', g_re, c_re, rel=N.scan_tolerance(g_re))
+                N.raise_on_mismatch('resonator grad imag', g_im, c_im, rel=N.scan_tolerance(g_im))
+            _raise_on_nan(found, grad_real=grad_real, grad_imag=grad_imag, grad_real_input=g_re,
+                          grad_imag_input=g_im, grad_sin_decay=g_sin, grad_cos_decay=g_cos)
         if g_sin is not None:
             g_sin = g_sin.reshape(sin_decay.shape)
             g_cos = g_cos.reshape(cos_decay.shape)

@@ -114,12 +114,12 @@ class _RfFused(torch.autograd.Function):
         need = ctx.needs_input_grad[2] or ctx.needs_input_grad[3]
         grad_spikes = torch.zeros_like(real) if grad_spikes is None else grad_spikes.contiguous()
         folded = D.fold(ctx.delays, grad_spikes, forward=False, delayed_spikes=spk) if ctx.delays else None
-        found = _res._nan_word()
-        g_re, g_im, g_sin, g_cos = _bwd(grad_spikes, real, imag, sin_decay.detach(), cos_decay.detach(),
-                                        threshold, tau_rho, scale_rho, graded, need,
-                                        folded, found)
-        _res._raise_on_nan(found, grad_spikes=grad_spikes, grad_real_input=g_re, grad_imag_input=g_im,
-                           grad_sin_decay=g_sin, grad_cos_decay=g_cos)
+        with _res._nan_word(real.device) as found:
+            g_re, g_im, g_sin, g_cos = _bwd(grad_spikes, real, imag, sin_decay.detach(), cos_decay.detach(),
+                                            threshold, tau_rho, scale_rho, graded, need,
+                                            folded, found)
+            _res._raise_on_nan(found, grad_spikes=grad_spikes, grad_real_input=g_re, grad_imag_input=g_im,
+                               grad_sin_decay=g_sin, grad_cos_decay=g_cos)
         if g_sin is not None:
             g_sin, g_cos = g_sin.reshape(sin_decay.shape), g_cos.reshape(cos_decay.shape)
         g_delay = D.delay_gradient(ctx.delays, folded)

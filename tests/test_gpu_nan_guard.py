@@ -54,3 +54,34 @@ def test_infinities_of_both_signs_are_not_reported(shape):
     g, = torch.autograd.grad(slayer.neuron.dynamics.resonator.dynamics(
         x, torch.zeros(shape).cuda(), sin, cos, zero, zero, 64), x, [grad, torch.zeros(shape).cuda()])
     assert torch.equal(g, grad)
+
+
+@pytest.mark.parametrize('model', ['rf', 'resonator', 'adaptive'])
+def test_a_call_that_fails_waits_for_its_launches(model, monkeypatch):
+    """The word the kernels report NaN in goes back to torch's pinned-memory cache when the call ends: a call that raises
+    after its launches (a raised range flag of an earlier call does) must not let go of it while they are still to run."""
+    import lava_dl_amd.slayer as slayer
+    from lava_dl_amd.slayer import _native
+    D, zero = slayer.neuron.dynamics, torch.zeros(1).cuda()
+    sin, cos = torch.full((1,), 100.0).cuda(), torch.full((1,), 2048.0).cuda()
+    x = [torch.randn(2, 3, 21).cuda().requires_grad_() for _ in range(2)]
+    if model == 'rf':
+        y = slayer.neuron.rf.Neuron(threshold=1.0, period=10, decay=0.1).cuda()(tuple(x))
+    elif model == 'resonator':
+        y = sum(D.resonator.dynamics(*x, sin, cos, zero, zero, 64))
+    else:
+        y = sum(D.adaptive_resonator.dynamics(*x, sin, cos, sin, sin, zero, zero, zero, zero, 1.0, 1.0, 64)[:2])
+
+    class Failed(Exception):
+        pass
+
+    def check(code):
+        assert code == 0
+        raise Failed()
+    grad = torch.ones_like(y)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(_native, 'check', check)
+    torch.cuda._sleep(200_000_000)                                   # the launches queue up behind this
+    with pytest.raises(Failed):
+        y.backward(grad)
+    assert torch.cuda.current_stream().query()
