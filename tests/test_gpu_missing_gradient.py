@@ -30,3 +30,22 @@ def test_no_gradient_for_the_spikes_is_a_zero_gradient(model, learn):
     _NoGradient.apply(neuron(tuple(inputs) if len(inputs) > 1 else inputs[0])).sum().backward()
     for x in inputs:
         assert x.grad is not None and not x.grad.any()
+
+
+def test_no_gradient_for_the_adaptive_resonator_is_a_zero_gradient():
+    import lava_dl_amd.slayer as slayer
+    shape, zero = (2, 3, 21), torch.zeros(1, device=dev())
+    x = [torch.randn(shape, device=dev(), requires_grad=True) for _ in range(2)]
+    sin, cos = (torch.full((1,), v, device=dev(), requires_grad=True) for v in (100.0, 2048.0))
+    decay = torch.full((1,), 400.0, device=dev())
+    dynamics = slayer.neuron.dynamics.adaptive_resonator.dynamics
+    re, im, *_ = dynamics(*x, sin, cos, decay, decay, zero, zero, zero, zero, 1.0, 1.0, 64)
+    (_NoGradient.apply(re) + _NoGradient.apply(im)).sum().backward()
+    for t in x + [sin, cos]:
+        assert t.grad is not None and not t.grad.any()
+    # a gradient of one of the two is what a gradient of zeros beside it gives
+    re, im, *_ = dynamics(*x, sin, cos, decay, decay, zero, zero, zero, zero, 1.0, 1.0, 64)
+    g = torch.randn(shape, device=dev())
+    one = torch.autograd.grad(re + _NoGradient.apply(im), x + [sin, cos], g, retain_graph=True)
+    both = torch.autograd.grad([re, im], x + [sin, cos], [g, torch.zeros_like(g)])
+    assert all(torch.equal(a, b) for a, b in zip(one, both))
