@@ -33,8 +33,9 @@ struct RecurrentFwd {
     unsigned* range_flag;                                     // see raise_range_flag in tile.h
 };
 
+// Any workgroup of whole waves with at least C threads.
 template <bool ALIF, bool GRADED, bool POW2, bool VEC4>
-__global__ __launch_bounds__(kMaxRecurrent) void recurrent_fwd_kernel(const RecurrentFwd p) {
+__device__ __forceinline__ void recurrent_fwd_gather(const RecurrentFwd& p) {
     // spikes of the previous step: per wave a count and the indices of its neurons that fired, padded
     // to a multiple of kGather with C, the index of the all-zero row that ends rec_t; graded spikes
     // bring their values along (0 in the padding)
@@ -188,6 +189,11 @@ __global__ __launch_bounds__(kMaxRecurrent) void recurrent_fwd_kernel(const Recu
     }
 }
 
+template <bool ALIF, bool GRADED, bool POW2, bool VEC4>
+__global__ __launch_bounds__(kMaxRecurrent) void recurrent_fwd_kernel(const RecurrentFwd p) {
+    recurrent_fwd_gather<ALIF, GRADED, POW2, VEC4>(p);
+}
+
 // Backward through the loop as the reference differentiates it (utils/recurrent.py:83-112): the
 // state carried between the one-step neuron calls is a constant, so a step contributes the spike
 // surrogate only, and the gradient reaches step t-1 through R.
@@ -273,7 +279,9 @@ __global__ __launch_bounds__(kMaxRecurrent) void recurrent_bwd_kernel(
 // four compute its step, and lane q of the quad moves the samples of time 4 i + q: any row length and alignment with
 // dword accesses that fill 16 bytes a neuron, loaded four steps ahead.
 //
-// A row sum is dense here (a neuron that did not fire contributes weight * 0), as it is in the reference's matmul.
+// A row sum is dense here: a neuron that did not fire contributes weight * 0.  Forward, where that is a NaN for a
+// weight that is not finite and would cost the receiving neuron its input, a workgroup with such a weight takes the
+// form above, which adds the weights of firing neurons only; backward that form is dense, too.
 constexpr int kRegisterNeurons = 256;
 
 template <int CTRL>
@@ -287,17 +295,22 @@ template <int KQ>
 struct RegisterMatrix {
     float w[4][4 * KQ];      // [neuron of the row of lanes][column]
 
-    // element (row n, column k) lies at mat[k * C + n]
-    __device__ void load(const float* __restrict__ mat, int C) {
+    // element (row n, column k) lies at mat[k * C + n]; false if one of this thread's elements is not finite
+    __device__ bool load(const float* __restrict__ mat, int C) {
         const int j = threadIdx.x & 15, n = (int)(threadIdx.x >> 4) * 4;
+        float zero = 0.f;                                     // a NaN after an element that is not finite
 #pragma unroll
         for (int i = 0; i < KQ; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int k = 64 * i + 4 * j + e;
 #pragma unroll
-                for (int a = 0; a < 4; ++a) w[a][4 * i + e] = (k < C && n + a < C) ? mat[k * C + n + a] : 0.f;
+                for (int a = 0; a < 4; ++a) {
+                    w[a][4 * i + e] = (k < C && n + a < C) ? mat[k * C + n + a] : 0.f;
+                    zero = __fmaf_rn(w[a][4 * i + e], 0.f, zero);
+                }
             }
+        return zero == 0.f;
     }
     // product with the vector at x; the result for neuron 4 * (thread / 16) + (thread / 4) % 4
     __device__ float times(const float4* x) const {
@@ -339,7 +352,7 @@ __global__ __launch_bounds__(256 * KQ) void recurrent_reg_fwd_kernel(const Recur
     auto from = [&](int y) -> float { const float f = (float)y; return POW2 ? f * inv_w : f / w; };
 
     RegisterMatrix<KQ> mat;
-    mat.load(p.rec_t, C);
+    if (__syncthreads_or(!mat.load(p.rec_t, C))) return recurrent_fwd_gather<ALIF, GRADED, POW2, false>(p);
     for (int i = threadIdx.x; i < 32 * KQ; i += blockDim.x) fired_s[0][i] = make_float4(0.f, 0.f, 0.f, 0.f);
 
     int yc = 0, yv = 0, th = 0, r = 0, mi = 0, mv = 0, mt = 0, mr = 0;

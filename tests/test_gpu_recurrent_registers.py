@@ -60,3 +60,31 @@ def test_register_kernels_match_the_oracle(c, t, kind, graded, monkeypatch):
     gz, gw = O.recurrent_cuba_bwd(g, spk, vol, w, theta, neuron.tau_rho * 100, neuron.scale_rho * 0.1, graded=graded)
     assert_rel(zg.grad, gz, 'grad z')
     assert_rel(syn.weight.grad.reshape(c, c), gw, 'grad weight')
+
+
+@pytest.mark.parametrize('c', [5, 70, 140, 255])
+@pytest.mark.parametrize('kind,graded', [('cuba', False), ('alif', False), ('alif', True)])
+@pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
+def test_a_weight_that_is_not_finite_counts_when_its_neuron_fires(c, kind, graded, value, monkeypatch):
+    """A silent neuron feeds nothing back whatever its weights (0 * inf would be a NaN, which the fixed-point current takes
+    as zero: the receiving neuron would lose its input); the wider layers' kernels gather the rows of the firing ones."""
+    import lava_dl_amd.slayer as slayer
+    monkeypatch.setattr(slayer.utils.recurrent, 'STEPS_FROM', 10 ** 9)
+    gen = torch.Generator().manual_seed(c)
+    z = torch.rand(2, c, 11, generator=gen) * 3
+    silent, to = c // 2, c - 1
+    z[:, silent] = -1.0
+    w = torch.randint(-2, 3, (c, c), generator=gen).float() / 64
+    w[silent] = 0.0
+    outs = []
+    for weight in (0.0, value):
+        w[to, silent] = weight
+        if kind == 'cuba':
+            neuron = slayer.neuron.cuba.Neuron(threshold=1.25, current_decay=0.25, voltage_decay=0.25, persistent_state=True)
+        else:
+            neuron = slayer.neuron.alif.Neuron(threshold=1.0, threshold_step=0.5, current_decay=0.5, voltage_decay=0.5,
+                                               threshold_decay=0.1, refractory_decay=0.2, persistent_state=True,
+                                               graded_spike=graded)
+        outs.append(slayer.utils.recurrent.custom_recurrent(z.to(dev()), neuron.to(dev()), _Dense(w).to(dev())).cpu())
+    assert not outs[0][:, silent].any() and outs[0][:, to].any()
+    assert torch.equal(*outs)
