@@ -506,7 +506,13 @@ int check_recurrent_sizes(int64_t N, int64_t C, int64_t T) {
 template <bool ALIF>
 int launch_recurrent_fwd(RecurrentFwd p, int graded, int w_scale, int64_t N, hipStream_t st) {
     const bool pow2 = is_pow2(w_scale);
-    if (p.C <= kRegisterNeurons) {
+    // Register form, except where its sixteen waves a sample (one sample at a time on a CU) have so many samples to do that
+    // the gathering form, which works on the firing neurons only, is no slower at usual rates: 250 neurons, 100 steps,
+    // 0.4 / 3 / 7 / 16 % of the neurons firing in a step, gathering 314 / 480 / 497 / 522 us for 1024 samples against 487, 556 / 854 /
+    // 916 / 974 for 2048 against 970; 512 samples 165 / 300 / 327 / 347 against 216.  Narrower layers: 192 neurons 204 / 267 /
+    // 293 / 306 for 1024 samples against 276, 128 neurons 127 / 175 / 190 / 198 against 129, fewer samples 1.5 to 3 times the register
+    // form's time.  (Backward the register form takes 0.2 to 0.8 of the other's time everywhere.)
+    if (p.C <= kRegisterNeurons && (p.C <= 192 || N < 1024)) {
         const dim3 threads((unsigned)((p.C + 15) / 16 * 64));
 #define SLAYER_REG(G, P, KQ) \
     hipLaunchKernelGGL((recurrent_reg_fwd_kernel<ALIF, G, P, KQ>), dim3((unsigned)N), threads, 0, st, p)

@@ -62,6 +62,24 @@ def test_register_kernels_match_the_oracle(c, t, kind, graded, monkeypatch):
     assert_rel(syn.weight.grad.reshape(c, c), gw, 'grad weight')
 
 
+@pytest.mark.parametrize('graded', [False, True])
+def test_large_batches_give_the_same_spikes_in_either_form(graded, monkeypatch):
+    """193 neurons, 1023 and 1024 samples: the batch from which the forward pass takes the gathering form."""
+    import lava_dl_amd.slayer as slayer
+    monkeypatch.setattr(slayer.utils.recurrent, 'STEPS_FROM', 10 ** 9)
+    gen = torch.Generator().manual_seed(7)
+    z, c = torch.randn(1024, 193, 5, generator=gen) * 3, 193
+    w = torch.randint(-2, 3, (c, c), generator=gen).float() / 32
+    w[torch.rand(c, c, generator=gen) > 4.0 / c] = 0.0               # graded products and sums exact
+    outs = []
+    for n in (1023, 1024):
+        neuron = slayer.neuron.alif.Neuron(threshold=1.0, threshold_step=0.5, current_decay=0.5, voltage_decay=0.5,
+                                           threshold_decay=0.1, refractory_decay=0.2, persistent_state=True,
+                                           graded_spike=graded).to(dev())
+        outs.append(slayer.utils.recurrent.custom_recurrent(z[:n].to(dev()), neuron, _Dense(w).to(dev())))
+    assert outs[0].any() and torch.equal(outs[0], outs[1][:1023])
+
+
 @pytest.mark.parametrize('c', [5, 70, 140, 255])
 @pytest.mark.parametrize('kind,graded', [('cuba', False), ('alif', False), ('alif', True)])
 @pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
