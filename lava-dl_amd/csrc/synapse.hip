@@ -781,10 +781,6 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 //
 // What is not finite (or overflows when it is scaled or rounded) shows in a tile at the end: the wave then runs its
 // share again with the float32 instruction (float_products), whose results such inputs had before.
-#ifndef SLAYER_WGRAD_GROUPS
-#define SLAYER_WGRAD_GROUPS 1
-#endif
-constexpr int kWgU = SLAYER_WGRAD_GROUPS;      // groups of 32 steps per visit of a column
 constexpr int kWgPitch = 80;                   // bytes of LDS per row of 32 bfloat16: no two quarters of a read collide
 constexpr int kWgSlot = 16 * kWgPitch;         // one part of one tile of 16 rows
 
@@ -858,108 +854,97 @@ struct WgradRow {
 #pragma unroll
             for (int pt = 0; pt < NPT; ++pt) q_row[pt][h] = pair_row(16 * pt + (lane >> 3) + 8 * h);
         }
-        for (int t0 = t_lo; t0 < t_hi; t0 += 32 * kWgU) {
-            SynQuad tq[kWgU];
+        for (int t0 = t_lo; t0 < t_hi; t0 += 32) {
+            SynQuad tq;
+            tq.template set<TAIL>(t0 + 4 * (lane & 7), t_hi);
+            float4 raw_g[2], raw_q[NPT][2];
+            auto fetch = [&](int c) {
 #pragma unroll
-            for (int u = 0; u < kWgU; ++u) tq[u].template set<TAIL>(t0 + 32 * u + 4 * (lane & 7), t_hi);
-            float4 raw_g[kWgU][2], raw_q[kWgU][NPT][2];
-            auto fetch = [&](int c, int u) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) raw_g[u][h] = grad_at(g_row[h], c + p.pw, tq[u]);
+                for (int h = 0; h < 2; ++h) raw_g[h] = grad_at(g_row[h], c + p.pw, tq);
 #pragma unroll
                 for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) raw_q[u][pt][h] = pair_at(q_row[pt][h], c, tq[u]);
+                    for (int h = 0; h < 2; ++h) raw_q[pt][h] = pair_at(q_row[pt][h], c, tq);
             };
             // gw[x]: the gradient at pixel c + pw - x for the column c at hand; gw[0] arrives with the column
-            uint4 gw[KW][kWgU][3];
-            float4 first[KW][kWgU][2];
+            uint4 gw[KW][3];
+            float4 first[KW][2];
 #pragma unroll
             for (int x = KW - 1; x >= 1; --x)
 #pragma unroll
-                for (int u = 0; u < kWgU; ++u)
+                for (int h = 0; h < 2; ++h) first[x][h] = grad_at(g_row[h], p.pw - x, tq);
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) first[x][u][h] = grad_at(g_row[h], p.pw - x, tq[u]);
+            for (int x = KW - 1; x >= 1; --x) {
+                put_parts(0, first[x], tq);
+                settle();
 #pragma unroll
-            for (int x = KW - 1; x >= 1; --x)
-#pragma unroll
-                for (int u = 0; u < kWgU; ++u) {
-                    put_parts(0, first[x][u], tq[u]);
-                    settle();
-#pragma unroll
-                    for (int t = 0; t < 3; ++t) gw[x][u][t] = get(t);
-                    settle();
-                }
-#pragma unroll
-            for (int u = 0; u < kWgU; ++u) fetch(0, u);
+                for (int t = 0; t < 3; ++t) gw[x][t] = get(t);
+                settle();
+            }
+            fetch(0);
             for (int c = 0; c < p.W; ++c) {
                 const unsigned flip = (c & 1) ? 0x80008000u : 0u;
                 const float back = (c & 1) ? -kSplitProductScale : kSplitProductScale;
                 auto flipped = [&](uint4 v) { return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip); };
+                put_parts(0, raw_g, tq);
+                unsigned low = 0u;
 #pragma unroll
-                for (int u = 0; u < kWgU; ++u) {
-                    put_parts(0, raw_g[u], tq[u]);
-                    unsigned low = 0u;
+                for (int pt = 0; pt < NPT; ++pt)
 #pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            const float4 v = raw_q[u][pt][h] = tq[u].template place<TAIL>(raw_q[u][pt][h]);
-                            low |= __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w);
-                        }
-                    const bool more = __any((low & 0xffffu) != 0u);      // more than bfloat16 holds
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                        for (int h = 0; h < 2; ++h) {
-                            float4 v = scaled(raw_q[u][pt][h]);
-                            if (!more) {
-                                put(3 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
-                            } else {
-                                uint2 part;
-                                part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
-                                put(3 + 3 * pt, h, part);
-                                part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
-                                put(4 + 3 * pt, h, part);
-                                put(5 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
-                            }
-                        }
-                    settle();
-                    if (c + 1 < p.W) fetch(c + 1, u);                    // on its way during the products
-#pragma unroll
-                    for (int t = 0; t < 3; ++t) gw[0][u][t] = get(t);
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        const uint4 q = flipped(get(3 + 3 * pt));
-                        syn_f4 d[KW];
-#pragma unroll
-                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][2], q, syn_f4{0.f, 0.f, 0.f, 0.f});
-                        if (more) {
-                            const uint4 q1 = flipped(get(4 + 3 * pt)), q2 = flipped(get(5 + 3 * pt));
-#pragma unroll
-                            for (int x = 0; x < KW; ++x) {
-                                d[x] = mfma_bf16(gw[x][u][0], q2, d[x]);
-                                d[x] = mfma_bf16(gw[x][u][1], q1, d[x]);
-                                d[x] = mfma_bf16(gw[x][u][0], q1, d[x]);
-                            }
-                        }
-#pragma unroll
-                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][1], q, d[x]);
-#pragma unroll
-                        for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][u][0], q, d[x]);
-#pragma unroll
-                        for (int x = 0; x < KW; ++x)
-#pragma unroll
-                            for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(back, d[x][i], acc[x][pt][i]);
+                    for (int h = 0; h < 2; ++h) {
+                        const float4 v = raw_q[pt][h] = tq.template place<TAIL>(raw_q[pt][h]);
+                        low |= __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w);
                     }
-                    settle();
+                const bool more = __any((low & 0xffffu) != 0u);          // more than bfloat16 holds
+#pragma unroll
+                for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        float4 v = scaled(raw_q[pt][h]);
+                        if (!more) {
+                            put(3 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
+                        } else {
+                            uint2 part;
+                            part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
+                            put(3 + 3 * pt, h, part);
+                            part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
+                            put(4 + 3 * pt, h, part);
+                            put(5 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
+                        }
+                    }
+                settle();
+                if (c + 1 < p.W) fetch(c + 1);                           // on its way during the products
+#pragma unroll
+                for (int t = 0; t < 3; ++t) gw[0][t] = get(t);
+#pragma unroll
+                for (int pt = 0; pt < NPT; ++pt) {
+                    const uint4 q = flipped(get(3 + 3 * pt));
+                    syn_f4 d[KW];
+#pragma unroll
+                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][2], q, syn_f4{0.f, 0.f, 0.f, 0.f});
+                    if (more) {
+                        const uint4 q1 = flipped(get(4 + 3 * pt)), q2 = flipped(get(5 + 3 * pt));
+#pragma unroll
+                        for (int x = 0; x < KW; ++x) {
+                            d[x] = mfma_bf16(gw[x][0], q2, d[x]);
+                            d[x] = mfma_bf16(gw[x][1], q1, d[x]);
+                            d[x] = mfma_bf16(gw[x][0], q1, d[x]);
+                        }
+                    }
+#pragma unroll
+                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][1], q, d[x]);
+#pragma unroll
+                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][0], q, d[x]);
+#pragma unroll
+                    for (int x = 0; x < KW; ++x)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(back, d[x][i], acc[x][pt][i]);
                 }
+                settle();
 #pragma unroll
                 for (int x = KW - 1; x >= 1; --x)
 #pragma unroll
-                    for (int u = 0; u < kWgU; ++u)
-#pragma unroll
-                        for (int t = 0; t < 3; ++t) gw[x][u][t] = gw[x - 1][u][t];
+                    for (int t = 0; t < 3; ++t) gw[x][t] = gw[x - 1][t];
             }
         }
     }
@@ -1002,7 +987,7 @@ struct WgradRow {
 };
 
 template <int KW, int NPT, bool TAIL>
-__global__ __launch_bounds__(kSynWaves * kWave) __attribute__((amdgpu_waves_per_eu(KW == 3 && !TAIL ? 3 : 2)))
+__global__ __launch_bounds__(kSynWaves * kWave) __attribute__((amdgpu_waves_per_eu(KW == 3 || NPT == 1 ? 3 : 2)))
 void synapse_wgrad_row_kernel(const SynapseWgrad p) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
