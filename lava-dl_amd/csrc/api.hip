@@ -41,8 +41,10 @@ void range_flag_raise_from_host() {
         *static_cast<volatile unsigned*>(g_range_host.load(std::memory_order_acquire)) = 1u;
 }
 
-// For tensors no other kernel has looked at on its way: the parameter gradients, and the small tensors whose backward
-// pass is not a scan (below 2^20 elements: latency-bound, 64 workgroups read them in one go).
+// For tensors no other kernel has looked at on its way: the parameter gradients; the input gradients of a backward pass that
+// is not a scan (tensors below 2^20 elements, and larger ones the scan does not take); and, with a delay, the
+// gradient of the spikes, of which the scan does not see what the delay shifts out of its row.  The last two can be
+// tensors of full size: one more read of them (the searches this stands for read every tensor twice).
 __global__ __launch_bounds__(256) void nan_check_kernel(unsigned* found, NanCheck t) {
     bool bad = false;
     for (int k = 0; k < 5; ++k) {

@@ -45,7 +45,10 @@ def custom_recurrent_ground_truth_2(z, neuron, recurrent_synapse):
 
 ONE_LAUNCH_MAX = 1024       # neurons per sample of the one-launch kernels (one thread per neuron)
 STEPS_MAX = 16384           # ... of the launch-per-step kernels (whole quads of neurons)
-STEPS_FROM = 256            # width from which a launch per step is the faster form (measured at [32, C, 300])
+# Width from which layers take a launch per step.  It is the faster form from 260 neurons on (measured at [32, C, 300]); at 256 the
+# one-launch kernels still hold the matrix in registers and are faster (forward and backward, 300 steps, CUBA: 602 us against 2560
+# for 32 samples, 2130 against 4525 for 512).
+STEPS_FROM = 256
 
 
 def _by_steps(c):
@@ -68,13 +71,15 @@ def custom_recurrent(z, neuron, recurrent_synapse):
     last step.  Gradients reach ``z`` and the recurrent weights; as in the reference, the state the
     neuron carries from one step to the next is treated as a constant.
 
-    The one-launch kernel adds the feedback of up to 256 neurons in a fixed order, that of wider layers row by row
-    in the order the neurons fired, 16 at a time, the launch-per-step kernels in a fixed order of their own on the
-    matrix cores (float32), where the reference's loop calls ``torch.matmul``.  The sums are the same bits whenever every partial sum
-    is exactly representable in float32, which holds for quantised recurrent weights (multiples of a power
-    of two of moderate size, what the synapse's ``pre_hook_fx`` quantiser produces).  With unquantised
-    weights the sums can differ in the last bit and a dendrite value within that distance of the threshold
-    may spike in one and not in the other; no fixture of the reference pins that case."""
+    The one-launch kernel adds the feedback of up to 256 neurons in a fixed order, that of wider layers (and of 193 and
+    more neurons in batches from 1024 samples on) row by row in the order the neurons fired, 16 at a time, the
+    launch-per-step kernels in a fixed order of their own on the matrix cores (float32), where the reference's loop calls
+    ``torch.matmul``.  The sums are the same bits whenever every partial sum is exactly representable in float32, which
+    holds for quantised recurrent weights (multiples of a power of two of moderate size, what the synapse's
+    ``pre_hook_fx`` quantiser produces).  With unquantised weights the sums can differ in the last bit and a dendrite
+    value within that distance of the threshold may spike in one and not in the other; no fixture of the reference pins
+    that case.  A weight that is not finite counts in the one-launch kernels when its neuron fires; as a product with
+    a silent neuron, which the loop's ``torch.matmul`` and the launch-per-step kernels form, it is a NaN."""
     recurrent_mat = _recurrent_matrix(recurrent_synapse)
     if _fusable(z, neuron):
         return _FusedRecurrent.apply(z, neuron, recurrent_mat)
