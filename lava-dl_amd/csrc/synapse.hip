@@ -1113,9 +1113,9 @@ namespace {
 // group costs a wait for its loads and its share of the SIMD, which all waves there divide up.  Fitted to 1900 layers
 // (2, 3 and 5 taps, 17 to 192 pairs, 3 to 64 output channels, 1 to 64 samples of 8x8 to 34x34 pixels, 50 to 302 steps; real
 // values times real weights) with an error of 12 to 15 % for the split and 13 to 22 % for the float32 form.
-// Split form over float32 form where it decides for the former (963 of 1741 layers), mean / 95 % of the layers / largest:
+// Split form over float32 form where it decides for the former (991 of 1741 layers), mean / 95 % of the layers / largest:
 //            spikes x quantised     real x quantised       real x real
-//   2 taps   0.60 / 0.83 / 1.25     0.71 / 0.96 / 1.28     0.79 / 1.11 / 1.30
+//   2 taps   0.62 / 0.86 / 1.23     0.73 / 0.97 / 1.26     0.81 / 1.11 / 1.29
 //   3 taps   0.61 / 0.90 / 1.05     0.72 / 0.93 / 1.06     0.83 / 1.03 / 1.30
 //   5 taps   0.46 / 0.70 / 0.84     0.65 / 0.88 / 1.01     0.85 / 1.12 / 1.44
 // Taken always from 17 pairs on, the split form lost up to 2.8 times on single samples of small images, up to 1.7
@@ -1172,8 +1172,10 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     const size_t row_lds = (size_t)((pairs + 3) / 4) * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
     int pieces = 1;
     while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
+    // (the estimate is a little hard on two taps, less so in small launches)
+    const double margin = p.kw != 2 ? 1.05 : base * pieces >= 640 ? 1.2 : 1.1;
     if (rows && pairs > 16 && split_lds <= 96 * 1024 &&
-        (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= 1.05 * row_form_time(false, p, base, wsplit))) {
+        (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= margin * row_form_time(false, p, base, wsplit))) {
         const int waves = split_lds > 40 * 1024 ? 8 : 4;
         p.wsplit = pieces;
         p.KG = g32;
