@@ -322,8 +322,10 @@ int slayer_corr(float *out, const float *in, const float *filt, int64_t K, float
  * out[n][co][ho][wo][t] = sum over ci, y, x of weight[co][ci][y][x] *
  *                         in[n][ci][ho * stride_h + y * dil_h - pad_h][wo * stride_w + x * dil_w - pad_w][t]
  * (zero outside the image), Ho = (H + 2 pad_h - dil_h (kh - 1) - 1) / stride_h + 1, Wo likewise; weight is
- * [Co][Ci][kh][kw] (the reference's [Co][Ci][kh][kw][1]).  float32 operands and accumulation on the matrix cores
- * (on the vector units when Ci = Co = 1: the pooling layers, which fold their channels into the image height).
+ * [Co][Ci][kh][kw] (the reference's [Co][Ci][kh][kw][1]).  float32 operands and accumulation on the matrix cores:
+ * on the float32 instruction, or, where that is faster, on the bfloat16 instruction with operands in up to three parts
+ * that keep all 24 bits (on the vector units when Ci = Co = 1: the pooling layers, which fold their channels into the
+ * image height).
  * The gradient of the input is the same call on the gradient with the weights transposed and flipped.
  * Rows of any length from four steps on, float-aligned tensors.  SLAYER_ERANGE for what the kernel does not take
  * (T < 4, a batch entry of 2 GiB or more, more than about 860 taps Ci * kh * kw): the caller keeps its library
@@ -351,7 +353,7 @@ int slayer_conv_synapse_input_grad(float *grad_in, const float *grad_out, const 
 /* The gradient of the synapse's weights (what autograd obtains from conv3d's backward, synapse/layer.py:297-323):
  * grad_weight[co][ci][y][x] = sum over n, ho, wo, t of grad_out[n][co][ho][wo][t] *
  *                             in[n][ci][ho * stride_h + y * dil_h - pad_h][wo * stride_w + x * dil_w - pad_w][t],
- * reduced along time on the matrix cores (float32), the partial tiles of the waves added in double in a fixed
+ * reduced along time on the matrix cores (as slayer_conv_synapse), the partial tiles of the waves added in double in a fixed
  * order.  workspace: slayer_conv_synapse_wgrad_workspace(...) floats of device memory, 16-byte aligned, contents
  * undefined afterwards (that function returns a negative error code for sizes the entry point refuses).  Same
  * limits as slayer_conv_synapse, up to 4096 taps. */
