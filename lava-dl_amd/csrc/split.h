@@ -33,17 +33,21 @@ __device__ __forceinline__ unsigned round_pair(float& a, float& b) {
     b -= back.y;
     return __builtin_bit_cast(unsigned, h);
 }
-// Eight floats (the k of one lane) as one operand of the instruction: rounded; and rounded, leaving in v what the rounding
-// left.
+// Eight floats (the k of one lane) as one operand of the instruction: rounded; what that rounding leaves; both.
 __device__ __forceinline__ uint4 bf16_eight(const float (&v)[8]) {
     return make_uint4(bf16_pair(v[0], v[1]), bf16_pair(v[2], v[3]), bf16_pair(v[4], v[5]), bf16_pair(v[6], v[7]));
 }
+__device__ __forceinline__ void leave_eight(float (&v)[8], uint4 rounded) {
+    const unsigned pair[4] = {rounded.x, rounded.y, rounded.z, rounded.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        v[2 * i] -= __uint_as_float(pair[i] << 16);
+        v[2 * i + 1] -= __uint_as_float(pair[i] & 0xffff0000u);
+    }
+}
 __device__ __forceinline__ uint4 round_eight(float (&v)[8]) {
-    uint4 r;
-    r.x = round_pair(v[0], v[1]);
-    r.y = round_pair(v[2], v[3]);
-    r.z = round_pair(v[4], v[5]);
-    r.w = round_pair(v[6], v[7]);
+    const uint4 r = bf16_eight(v);
+    leave_eight(v, r);
     return r;
 }
 __device__ __forceinline__ split_f4 mfma_bf16(uint4 a, uint4 b, split_f4 d) {

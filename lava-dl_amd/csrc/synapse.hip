@@ -338,10 +338,15 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kerne
 // column, turns them into the operands of four products (one per step of the quad: eight pairs each), and uses these
 // for the KW output pixels the column meets, whose accumulators it keeps -- every column is loaded and split once.  A
 // pixel is complete, and stored, after its last column.  The next loads are on their way during the products.
-// [16,32,16,16,300] -> 64 channels forward 398 -> 232 us, input gradient 429 -> 319 us; [32,8,32,32,300] -> 16 channels 384
-// -> 320 us on average of both (161 registers, three waves per SIMD; five taps 193, two waves).  The error against float64
-// is 0.6 to 0.9 times that of the float32 form (real values 2.5e-7 and 2.9e-7 at 96 pairs).  What bounds it now: the
-// unaligned rows of the result (T = 300) for few channels, the vector instructions of the split for gradients.
+// The instruction rounds every sum it leaves, so the products of the lower parts, 2^-8 of the whole at most, are added up
+// from zero and join the sum in one addition: it is rounded twice for 32 terms, not up to six times.  The error against
+// float64 is 0.3 to 0.6 times that of the float32 form, sparse (graded) inputs included (96 pairs: real x real 1.0e-7 and
+// 2.9e-7, graded x real 0.7e-7 and 1.2e-7, real x quantised over 192 pairs 1.3e-7 and 4.2e-7; every product into the one sum:
+// 2.6e-7, 2.1e-7, 2.4e-7).
+// [16,32,16,16,300] -> 64 channels forward 402 -> 259 us, input gradient 418 -> 286 us with quantised weights, 365 without;
+// [32,8,32,32,300] -> 16 channels 352 -> 297 and 415 -> 330 us (168 registers, three waves per SIMD; five taps 213, two waves).
+// What bounds it now: the unaligned rows of the result (T = 300) for few channels, the vector instructions of the split
+// for gradients.
 //
 // A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
 // each of them is not infinity times their sum: a wave with a result that is not finite computes its row again from
@@ -464,31 +469,55 @@ void synapse_conv_split_kernel(const SynapseConv p) {
                 }
                 const bool split_x = __any((bits & 0xffffu) != 0u);
                 const uint4* wg = wt + g * KW * 3 * kWave + lane;
-                // One copy of the products, in loops over the parts (branches around several copies cost the
-                // compiler a second set of accumulators: 256 registers and spills).
-                const int parts_x = split_x ? 3 : 1;
-#pragma unroll 1
-                for (int tx = 0; tx < parts_x; ++tx) {
-                    uint4 q[4];
-                    if (tx + 1 < parts_x) {
+                const bool last = g + 1 == G;                            // the next loads are on their way during the products
+                if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
+                // kH steps of the quad at a time (the parts of all four do not fit beside the accumulators), and branches
+                // around the products of the lower parts only: around several copies of the whole they cost the compiler a
+                // second set of accumulators and spills.
+                constexpr int kH = KW == 5 ? 4 : 2;
+                const syn_f4 zero = syn_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) q[e] = round_eight(v[e]);
-                    } else {
+                for (int h = 0; h < 4; h += kH) {
+                    uint4 q[kH][3];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) q[e] = bf16_eight(v[e]);
-                    }
-                    if (tx == 0) {
-                        const bool last = g + 1 == G;                // the next loads are on their way during the products
-                        if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
-                    }
-#pragma unroll 1
-                    for (int tw = split_w ? 2 - tx : 0; tw >= 0; --tw) {
-#pragma unroll
-                        for (int x = 0; x < KW; ++x) {
-                            const uint4 a = wg[(x * 3 + tw) * kWave];
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) acc[x][e] = mfma_bf16(a, q[e], acc[x][e]);
+                    for (int e = 0; e < kH; ++e) {
+                        q[e][0] = bf16_eight(v[h + e]);
+                        if (split_x) {
+                            leave_eight(v[h + e], q[e][0]);
+                            q[e][1] = round_eight(v[h + e]);
+                            q[e][2] = bf16_eight(v[h + e]);
                         }
+                    }
+#pragma unroll
+                    for (int x = 0; x < KW; ++x) {
+                        const uint4 w0 = wg[x * 3 * kWave];
+                        syn_f4 d[kH];
+                        if (split_x) {
+                            if (split_w) {
+                                const uint4 w1 = wg[(x * 3 + 1) * kWave], w2 = wg[(x * 3 + 2) * kWave];
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][1], d[e]);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][0], d[e]);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], d[e]);
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], zero);
+                            }
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) acc[x][h + e] += mfma_bf16(w0, q[e][1], d[e]);
+                        } else if (split_w) {
+                            const uint4 w1 = wg[(x * 3 + 1) * kWave], w2 = wg[(x * 3 + 2) * kWave];
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) acc[x][h + e] += mfma_bf16(w1, q[e][0], d[e]);
+                        }
+#pragma unroll
+                        for (int e = 0; e < kH; ++e) acc[x][h + e] = mfma_bf16(w0, q[e][0], acc[x][h + e]);
                     }
                 }
             }
