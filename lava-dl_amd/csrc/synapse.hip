@@ -1142,11 +1142,12 @@ namespace {
 // group costs a wait for its loads and its share of the SIMD, which all waves there divide up.  Fitted to 1900 layers
 // (2, 3 and 5 taps, 17 to 192 pairs, 3 to 64 output channels, 1 to 64 samples of 8x8 to 34x34 pixels, 50 to 302 steps; real
 // values times real weights) with an error of 12 to 15 % for the split and 13 to 22 % for the float32 form.
-// Split form over float32 form where it decides for the former (991 of 1741 layers), mean / 95 % of the layers / largest:
+// Split form over float32 form where it decides for the former, margins of the caller included (1026 of 1741 layers), mean /
+// 95 % of the layers / largest:
 //            spikes x quantised     real x quantised       real x real
-//   2 taps   0.62 / 0.86 / 1.23     0.73 / 0.97 / 1.26     0.81 / 1.11 / 1.29
-//   3 taps   0.61 / 0.90 / 1.05     0.72 / 0.93 / 1.06     0.83 / 1.03 / 1.30
-//   5 taps   0.46 / 0.70 / 0.84     0.65 / 0.88 / 1.01     0.85 / 1.12 / 1.44
+//   2 taps   0.63 / 0.85 / 1.24     0.75 / 1.01 / 1.27     0.82 / 1.12 / 1.30
+//   3 taps   0.63 / 0.91 / 1.04     0.76 / 0.98 / 1.11     0.88 / 1.11 / 1.42
+//   5 taps   0.49 / 0.72 / 0.82     0.67 / 0.87 / 0.97     0.84 / 1.08 / 1.28
 // Taken always from 17 pairs on, the split form lost up to 2.8 times on single samples of small images, up to 1.7
 // times with badly filled groups (5x5, 40 pairs, real x real 195 us against 141).
 double row_form_time(bool split, const SynapseConv& p, int64_t row_tiles, int pieces) {
@@ -1191,7 +1192,7 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     if (blocks > 0x7fffffffLL) return SLAYER_ERANGE;
     const bool tail = (p.T % 4) != 0;                                     // rows that end inside a quad
     const dim3 grid((unsigned)blocks), block(kSynWaves * kWave);
-    // The split form where it is not the slower one with both operands real, its worst case (row_form_time), from 17 pairs
+    // The split form where it is about as fast with both operands real, its worst case (row_form_time), from 17 pairs
     // on, and if the parts of 16 channels' weights fit LDS.  A piece of an image row visits kw - 1 columns more than it has
     // pixels: rows are cut while there are few waves, for five taps (two waves per SIMD) below 1024 only
     // ([4,16,16,16,300] -> 64 channels 182 us with 2560 waves, 140 with 1280).
@@ -1201,8 +1202,11 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     const size_t row_lds = (size_t)((pairs + 3) / 4) * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
     int pieces = 1;
     while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
-    // (the estimate is a little hard on two taps, less so in small launches)
-    const double margin = p.kw != 2 ? 1.05 : base * pieces >= 640 ? 1.2 : 1.1;
+    // In all but small launches a margin for what it gains with spikes and quantised weights, which the host cannot see:
+    // layers estimated at 1.0 to 1.1 of the float32 form take 0.4 to 0.7 of it with both, 0.7 to 0.9 with one, 1.0 to 1.1 with
+    // neither.
+    const bool small = base * pieces < 640;
+    const double margin = p.kw == 2 ? (small ? 1.1 : 1.2) : small ? 1.0 : p.kw == 3 ? 1.12 : 1.07;
     if (rows && pairs > 16 && split_lds <= 96 * 1024 &&
         (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= margin * row_form_time(false, p, base, wsplit))) {
         const int waves = split_lds > 40 * 1024 ? 8 : 4;
