@@ -1142,12 +1142,12 @@ namespace {
 // group costs a wait for its loads and its share of the SIMD, which all waves there divide up.  Fitted to 1900 layers
 // (2, 3 and 5 taps, 17 to 192 pairs, 3 to 64 output channels, 1 to 64 samples of 8x8 to 34x34 pixels, 50 to 302 steps; real
 // values times real weights) with an error of 12 to 15 % for the split and 13 to 22 % for the float32 form.
-// Split form over float32 form where it decides for the former, margins of the caller included (1026 of 1741 layers), mean /
-// 95 % of the layers / largest:
+// Split form over float32 form for 500 layers of these ranges that it decides for the former, margins of the caller included,
+// mean / 95 % of the layers / largest:
 //            spikes x quantised     real x quantised       real x real
-//   2 taps   0.63 / 0.85 / 1.24     0.75 / 1.01 / 1.27     0.82 / 1.12 / 1.30
-//   3 taps   0.63 / 0.91 / 1.04     0.76 / 0.98 / 1.11     0.88 / 1.11 / 1.42
-//   5 taps   0.49 / 0.72 / 0.82     0.67 / 0.87 / 0.97     0.84 / 1.08 / 1.28
+//   2 taps   0.60 / 0.84 / 0.97     0.76 / 1.01 / 1.12     0.85 / 1.18 / 1.27
+//   3 taps   0.52 / 0.77 / 1.11     0.72 / 0.99 / 1.29     0.85 / 1.16 / 1.40
+//   5 taps   0.42 / 0.68 / 0.74     0.60 / 0.90 / 1.05     0.75 / 1.11 / 1.28
 // Taken always from 17 pairs on, the split form lost up to 2.8 times on single samples of small images, up to 1.7
 // times with badly filled groups (5x5, 40 pairs, real x real 195 us against 141).
 double row_form_time(bool split, const SynapseConv& p, int64_t row_tiles, int pieces) {
@@ -1203,13 +1203,18 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     int pieces = 1;
     while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
     // In all but small launches a margin for what it gains with spikes and quantised weights, which the host cannot see:
-    // layers estimated at 1.0 to 1.1 of the float32 form take 0.4 to 0.7 of it with both, 0.7 to 0.9 with one, 1.0 to 1.1 with
+    // layers estimated at 1.0 to 1.1 of the float32 form take 0.5 to 0.7 of it with both, 0.8 to 1.0 with one, 1.0 to 1.15 with
     // neither.
     const bool small = base * pieces < 640;
     const double margin = p.kw == 2 ? (small ? 1.1 : 1.2) : small ? 1.0 : p.kw == 3 ? 1.12 : 1.07;
     if (rows && pairs > 16 && split_lds <= 96 * 1024 &&
         (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= margin * row_form_time(false, p, base, wsplit))) {
-        const int waves = split_lds > 40 * 1024 ? 8 : 4;
+        // Workgroups of four waves: the registers hold three of them on a CU (five taps: two), but one of eight.  Eight where the
+        // LDS has room for one workgroup only and there are more than four waves to a CU.  Both operands real, us, float32
+        // form / four / eight waves: 3x3 on [5,43,31,31,64] -> 40 channels 127 / 153 / 192, [2,43,32,32,300] -> 27 144 / 159 /
+        // 215, 5x5 on [10,25,11,11,100] -> 2 97 / 98 / 128; with room for one, 5x5 on [1,33,35,35,300] -> 3 (700 waves)
+        // 249 / 166 / 220, 3x3 on [3,86,23,23,159] -> 47 (1242 waves) 758 / 1006 / 553.
+        const int waves = 2 * (split_lds + 4 * g32 * 32 * sizeof(int)) > 160 * 1024 && base * pieces > 4 * 256 ? 8 : 4;
         p.wsplit = pieces;
         p.KG = g32;
         const int64_t all = (int64_t)p.Ho * pieces * p.ttiles;

@@ -224,3 +224,17 @@ def test_products_of_the_lower_parts_do_not_round_the_sum(kind):
     for name, groups, a, b in zip(('output', 'grad input'), (9, 18), got, want):
         error = float((a.cpu().double() - b).norm() / b.norm())
         assert error <= groups ** 0.5 * 2.0 ** -23 / 3 ** 0.5 * 0.72, (name, error)
+
+
+@pytest.mark.parametrize('batch', [204, 205])
+@pytest.mark.parametrize('ci,kernel', [(43, 3), (85, 3), (86, 3), (32, 5), (33, 5)])
+def test_workgroups_of_either_size(batch, ci, kernel):
+    """Weights of which two workgroups share the LDS of a compute unit, and of which one fills it: four waves each, or eight
+    from 1025 waves on (five rows an image, so the last workgroup of a sample has waves without work)."""
+    from lava_dl_amd.slayer.synapse import layer
+    gen = torch.Generator().manual_seed(ci + batch)
+    x, w = torch.randn(batch, ci, 5, 8, 8, generator=gen), torch.randn(3, ci, kernel, kernel, 1, generator=gen)
+    pad = kernel // 2
+    y = layer._launch(x.to(dev()), w[..., 0].contiguous().to(dev()), (1, 1), (pad, pad), (1, 1))
+    args = None, 1, (pad, pad, 0)
+    assert_sum(y, F.conv3d(x.double(), w.double(), *args), F.conv3d(x.double().abs(), w.double().abs(), *args), 'output')
