@@ -343,8 +343,8 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kerne
 // float64 is 0.3 to 0.6 times that of the float32 form, sparse (graded) inputs included (96 pairs: real x real 1.0e-7 and
 // 2.9e-7, graded x real 0.7e-7 and 1.2e-7, real x quantised over 192 pairs 1.3e-7 and 4.2e-7; every product into the one sum:
 // 2.6e-7, 2.1e-7, 2.4e-7).
-// [16,32,16,16,300] -> 64 channels forward 402 -> 259 us, input gradient 418 -> 286 us with quantised weights, 365 without;
-// [32,8,32,32,300] -> 16 channels 352 -> 297 and 415 -> 330 us (168 registers, three waves per SIMD; five taps 213, two waves).
+// [16,32,16,16,300] -> 64 channels forward 402 -> 262 us, input gradient 418 -> 287 us with quantised weights, 357 without;
+// [32,8,32,32,300] -> 16 channels 352 -> 297 and 415 -> 328 us (168 registers, three waves per SIMD; five taps 213, two waves).
 // What bounds it now: the unaligned rows of the result (T = 300) for few channels, the vector instructions of the split
 // for gradients.
 //
