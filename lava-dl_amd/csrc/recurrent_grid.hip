@@ -1,0 +1,718 @@
+// Recurrent layer of CUBA or ALIF neurons, the whole time loop in one launch spread over the chip.
+//
+//   feedback[t] = R s[t-1];  s[t] = neuron(z[t] + feedback[t])          (utils/recurrent.py:45-112 in the reference)
+//
+// A launch per time step (recurrent_steps.hip) reads the [C x C] matrix from the caches and starts and drains the chip
+// once a step: 7.6 us forward at [32, 2048, 300].  The registers of the chip hold the matrix (2048 neurons:
+// 16.8 MB as float32, against 128 MB): a workgroup owns 16 neurons x 16 samples, keeps its rows of R in registers for all
+// steps, and what a step hands to the next crosses the chip through the caches.
+//
+// Forward exchange: one 32-bit word per sample and tile of 16 neurons, the spikes in the low half, the step's number
+// in the high half, in two sets used in turn.  A wave polls the words it multiplies until all carry the
+// previous step's number, so the data is its own flag: one store and one load across the chip per step, no barrier, no
+// counter.  Two sets are enough: a workgroup writes step t after it has read all words of step t-1, and whoever
+// published t-1 had read all of t-2.
+//
+// The product runs on the bfloat16 matrix instruction: a spike is the bfloat16 number 2.0 (one bit, which a shift and a
+// mask put in place), a weight is halved and cut into three parts of 8 bits -- its 24 bits, nothing is
+// rounded -- and the parts beyond the first are skipped by a wave whose weights have none (8-bit quantisers).
+//
+// The workgroups wait for one another, so all of them must be on the chip at once: the launch is a cooperative one,
+// which the runtime refuses beyond what the device holds, does not run beside another and grants to one process at a time
+// (a refused call takes a launch per step).  Every wait is bounded all the same (kSpinLimit polls); a workgroup that
+// gives up leaves a mark, and the kernel that is launched behind computes the layer again, one workgroup per sample,
+// when it finds it.
+//
+// Measured against a launch per step, whole layer, forward and backward: CUBA [32, 2048, 300] 5 121 -> 3 117 us (forward
+// kernel 2 430 -> 493, backward 2 075 -> 1 751), [32, 256, 300] 2 527 -> 951, ALIF [32, 512, 300] 2 651 -> 1 237,
+// [64, 2048, 100] 2 982 -> 2 189; ALIF [32, 1024, 100] forward alone 623 -> 221.  A forward step of 2048 neurons is 1.5 us:
+// 0.9 of them the way of the words across the chip, 0.7 the product, the sum over the waves and the neuron, a chain of
+// dependent instructions.
+#include "recurrent_step.h"
+#include "split.h"
+
+namespace slayer {
+
+constexpr int kGridWaves = 8;                        // waves of a workgroup: each takes an eighth of the sum over k
+constexpr int kGridThreads = kGridWaves * kWave;
+constexpr int kGridMaxC = 2048;                      // the parts of 16 rows in the registers of eight waves
+constexpr int kGridMaxT = 1 << 26;                   // 32-bit byte offsets of four rows
+constexpr int kGridChunk = 16;                       // steps of the tensors a wave stages in LDS at a time
+constexpr int kGridPitch = kGridChunk + 1;
+#ifndef SLAYER_GRID_POLLS
+#define SLAYER_GRID_POLLS (1 << 18)                   // about a third of a second
+#endif
+constexpr int kSpinLimit = SLAYER_GRID_POLLS;        // polls before a wave gives up
+constexpr int kSoloThreads = 1024;
+
+__device__ __forceinline__ void wave_lds_order() {   // LDS written by some lanes of this wave, read by others
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ void lds_barrier() {      // orders LDS only: stores to memory stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Which workgroup does what.  Workgroups go to the chip's eight XCDs round-robin by index; those of one sample group
+// share what they exchange, so they are put on as few XCDs as hold them (`xcds`, a power of two), `per_xcd` on each:
+// [32, 2048, 300] forward 645 us with both groups on all eight XCDs, 520 with four XCDs to a group.  Where they
+// really run changes only the time.
+struct GridMap {
+    int xcds, per_xcd;
+    __device__ __forceinline__ int tile(int id) const { return ((id >> 3) % per_xcd) * xcds + (id & 7) % xcds; }
+    __device__ __forceinline__ int group(int id) const { return (id >> 3) / per_xcd * (8 / xcds) + (id & 7) / xcds; }
+};
+
+struct GridFwd {
+    StepFwd p;                                       // its time-major tensors and packed operands are not used
+    float *spk, *vol, *theta;                        // [N][C][T]
+    const float *z, *rec;
+    unsigned* words;                                 // [2][S][words_of(KB)]
+    GridMap map;
+    unsigned* gave_up;
+};
+// words of one sample tile, [KB][16 samples], whole units
+__host__ __device__ inline int words_of(int KB) { return (KB + 7) / 8 * 8 * 16; }
+
+__global__ __launch_bounds__(256) void grid_fill_kernel(unsigned* dst, int64_t n, unsigned value, unsigned* gave_up) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = value;
+    if (i == 0) *gave_up = 0u;
+}
+
+// the upper 8 bits of the significand as a bfloat16 in the upper half of a word; v keeps the rest
+__device__ __forceinline__ unsigned cut(float& v) {
+    const unsigned u = __float_as_uint(v);
+    if ((u & 0x7f800000u) == 0x7f800000u) {          // infinities and NaN have no rest
+        v = 0.f;
+        return (u & 0x007fffffu) ? 0x7fc00000u : (u & 0xffff0000u);
+    }
+    const unsigned h = u & 0xffff0000u;
+    v -= __uint_as_float(h);
+    return h;
+}
+
+// Thread (wave v, lane 16 i + nn) of the first four waves runs neuron nn of the tile for sample 4 v + i; the ballot of its
+// wave then holds the 16 spikes of a sample in one 16-bit field.
+template <bool ALIF, bool POW2, int U, int NT>
+__global__ __launch_bounds__(kGridThreads) void recurrent_grid_fwd_kernel(const GridFwd g) {
+    constexpr int kPlane = 68;                       // pitch of a plane of red: reads of a wave meet 64 banks
+    __shared__ float red[2][kGridWaves][4][kPlane];
+    __shared__ float zbuf[NT][4][kWave * kGridPitch], vbuf[NT][4][kWave * kGridPitch];
+    __shared__ float tbuf[ALIF ? NT : 1][4][ALIF ? kWave * kGridPitch : 1];
+    __shared__ unsigned sbits[4][kWave];
+    __shared__ int dead[2];
+    const StepFwd& p = g.p;
+    const int C = p.C, N = p.N, T = p.T, KB = p.KB;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kk = lane >> 4, j = lane & 15;
+    const int P = g.map.tile(blockIdx.x), c0 = P * 16, group = g.map.group(blockIdx.x);
+    if (P >= KB || group * NT >= p.S) return;
+    const int words = words_of(KB);
+    const int64_t set = (int64_t)p.S * words;
+    if (tid < 2) dead[tid] = 0;
+
+    // rows c0 .. c0 + 15 of R as A operands.  Unit u = 8 neuron tiles = 128 presynaptic neurons = four products; lane
+    // (kk, j) has tiles 8u + 2kk and 8u + 2kk + 1 of row c0 + j, element 2i (2i + 1) of product a is neuron 4a + i of
+    // the first (second) tile.
+    uint4 wh[U][4], wm[U][4], wl[U][4];
+    unsigned rest = 0u;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k0 = 16 * (8 * (wave + kGridWaves * u) + 2 * kk);
+        float v[32];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const bool ok = c0 + j < C && k0 + 4 * q < C;            // C is a multiple of 4
+            const float4 f = ok ? load_quad_dword_aligned(g.rec + (int64_t)(c0 + j) * C + k0 + 4 * q)
+                                : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[4 * q] = 0.5f * f.x; v[4 * q + 1] = 0.5f * f.y; v[4 * q + 2] = 0.5f * f.z; v[4 * q + 3] = 0.5f * f.w;
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            unsigned h[4], m[4], l[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float &x = v[4 * a + i], &y = v[16 + 4 * a + i];
+                h[i] = cut(x) >> 16; h[i] |= cut(y);
+                m[i] = cut(x) >> 16; m[i] |= cut(y);
+                l[i] = cut(x) >> 16; l[i] |= cut(y);
+                rest |= m[i] | l[i];
+            }
+            wh[u][a] = make_uint4(h[0], h[1], h[2], h[3]);
+            wm[u][a] = make_uint4(m[0], m[1], m[2], m[3]);
+            wl[u][a] = make_uint4(l[0], l[1], l[2], l[3]);
+        }
+    }
+    const bool lower = __any(rest != 0u);
+    // where this lane finds the words of its units, and which of the two tiles there are (an address beyond them is moved
+    // to the first tiles; its words are of no consequence, the weights there are zero)
+    int word_at[U];
+    unsigned need_lo[U], need_hi[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int first = 8 * (wave + kGridWaves * u) + 2 * kk;
+        word_at[u] = 16 * (16 * first < words ? first : 0) + j;
+        need_lo[u] = first < KB ? 0xffff0000u : 0u;
+        need_hi[u] = first + 1 < KB ? 0xffff0000u : 0u;
+    }
+
+    // this thread's neuron, one sample of each of the workgroup's sample tiles
+    const int nn = lane & 15, c = c0 + nn;
+    StepNeuron<ALIF, false, POW2> nrn[NT];
+    unsigned fired[NT];
+    bool mine[NT];
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+        const int n = (group * NT + s) * 16 + 4 * wave + kk;
+        mine[s] = wave < 4 && n < N && c < C;
+        nrn[s] = StepNeuron<ALIF, false, POW2>{};
+        if (mine[s]) {
+            nrn[s].load_decays(p, c);
+            nrn[s].load_states(p, (int64_t)n * C + c);
+            nrn[s].check(p.range_flag);
+        }
+        nrn[s].decay(p);
+    }
+    // staging of a wave's 64 rows, 16 steps at a time: access q covers rows 4q .. 4q + 3, lane (kk, j) step j of row 4q + kk
+    auto row_ok = [&](int s, int q) -> bool {
+        return (group * NT + s) * 16 + 4 * wave + (q >> 2) < N && c0 + 4 * (q & 3) < C;
+    };
+    // The address is a scalar, one addition further for every access, and the lane's 32-bit offset; what the empty asm keeps
+    // the compiler from is holding all of them in registers at once.
+    const unsigned lane_at = (unsigned)kk * (unsigned)T + (unsigned)j;
+    auto first_row = [&](int s, int t0) -> int64_t {
+        return ((int64_t)((group * NT + s) * 16 + 4 * wave) * C + c0) * T + t0;
+    };
+    auto next_rows = [&](int64_t& at, int q) {
+        at += (int64_t)((q & 3) == 3 ? C - 12 : 4) * T;
+        asm volatile("" : "+s"(at));
+    };
+    float zn[NT][16];
+    auto fetch = [&](int t0) {
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            int64_t at = first_row(s, t0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q, next_rows(at, q - 1))
+                zn[s][q] = (row_ok(s, q) && t0 + j < T) ? (g.z + at)[lane_at] : 0.f;
+        }
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) zbuf[s][wave][(4 * q + kk) * kGridPitch + j] = zn[s][q];
+        wave_lds_order();
+    };
+    if (wave < 4) { fetch(0); put(); }
+    lds_barrier();
+
+    bool stop = false;
+    for (int t0 = 0; t0 < T && !stop; t0 += kGridChunk) {
+        if (wave < 4 && t0 + kGridChunk < T) fetch(t0 + kGridChunk);
+        const int steps = T - t0 < kGridChunk ? T - t0 : kGridChunk;
+#pragma unroll
+        for (int s = 0; s < NT; ++s) fired[s] = 0u;
+        for (int e = 0; e < steps && !stop; ++e) {
+            const int t = t0 + e;
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                const int sel = NT == 1 ? (t & 1) : s & 1;
+                const int tile = group * NT + s;
+                float z = wave < 4 ? zbuf[s][wave][lane * kGridPitch + e] : 0.f;
+                if (t > 0) {
+                    const unsigned tag = (unsigned)t << 16;
+                    const unsigned* src = g.words + ((t - 1) & 1) * set + (int64_t)tile * words;
+                    unsigned W[U];
+                    for (int spin = 0;; ++spin) {
+                        unsigned late = 0u, lo[U], hi[U];
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            lo[u] = __hip_atomic_load(src + word_at[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            hi[u] = __hip_atomic_load(src + word_at[u] + 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+#pragma unroll
+                        for (int u = 0; u < U; ++u) {
+                            late |= ((lo[u] ^ tag) & need_lo[u]) | ((hi[u] ^ tag) & need_hi[u]);
+                            W[u] = __builtin_amdgcn_perm(hi[u], lo[u], 0x05040100u); // the low halves side by side
+                        }
+                        if (!__any(late != 0u)) break;
+                        if (spin == kSpinLimit ||
+                            ((spin & 1023) == 1023 &&
+                             __hip_atomic_load(g.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
+                            dead[sel] = 1;
+                            break;
+                        }
+                    }
+                    split_f4 acc[2] = {split_f4{0.f, 0.f, 0.f, 0.f}, split_f4{0.f, 0.f, 0.f, 0.f}};
+                    split_f4 low = split_f4{0.f, 0.f, 0.f, 0.f};
+                    auto spikes = [&](int u, int a) -> uint4 {
+                        unsigned b[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const int bit = 4 * a + i;                    // neuron `bit` of both tiles, to bits 14 and 30
+                            b[i] = (bit <= 14 ? W[u] << (14 - bit) : W[u] >> 1) & 0x40004000u;
+                        }
+                        return make_uint4(b[0], b[1], b[2], b[3]);
+                    };
+                    if (!lower) {
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+#pragma unroll
+                            for (int a = 0; a < 4; ++a) acc[a & 1] = mfma_bf16(wh[u][a], spikes(u, a), acc[a & 1]);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < U; ++u)
+#pragma unroll
+                            for (int a = 0; a < 4; ++a) {
+                                const uint4 b = spikes(u, a);
+                                acc[a & 1] = mfma_bf16(wh[u][a], b, acc[a & 1]);
+                                low = mfma_bf16(wm[u][a], b, low);
+                                low = mfma_bf16(wl[u][a], b, low);
+                            }
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) red[sel][wave][i][lane] = acc[0][i] + acc[1][i] + low[i];
+                }
+                lds_barrier();
+                if (wave < 4) {
+                    if (t > 0) {
+                        float fb = 0.f;
+#pragma unroll
+                        for (int v = 0; v < kGridWaves; ++v) fb += red[sel][v][nn & 3][(nn >> 2) * 16 + 4 * wave + kk];
+                        z += fb;
+                    }
+                    const float spike = nrn[s].fire(z, p);
+                    const bool spiked = mine[s] && spike > 0.0f;
+                    const unsigned long long mask = __ballot(spiked);
+                    if (lane < 4)                                              // sample 4 wave + lane
+                        __hip_atomic_store(g.words + (t & 1) * set + (int64_t)tile * words +
+                                               P * 16 + 4 * wave + lane,
+                                           ((unsigned)(t + 1) << 16) | (unsigned)((mask >> (16 * lane)) & 0xffffull),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    fired[s] |= (spiked ? 1u : 0u) << e;
+                    vbuf[s][wave][lane * kGridPitch + e] = nrn[s].vol;
+                    if (ALIF) tbuf[s][wave][lane * kGridPitch + e] = nrn[s].theta;
+                    if (mine[s] && t == T - 1) {
+                        const int64_t m = (int64_t)(tile * 16 + 4 * wave + kk) * C + c;
+                        p.cur_last[m] = nrn[s].cur;
+                        p.vol_last[m] = nrn[s].vol;
+                        if (ALIF) { p.th_last[m] = nrn[s].thf; p.ref_last[m] = nrn[s].rf; }
+                    }
+                    nrn[s].carry(spike, p);
+                    if (t < T - 1) nrn[s].decay(p);
+                }
+                stop = stop || dead[sel] != 0;
+                // The waves without neurons wait here for those with: polling early, they hold up the words on their
+                // way (763 us without this barrier, 520 with it).
+                lds_barrier();
+            }
+        }
+        if (wave < 4) {
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                sbits[wave][lane] = fired[s];
+                wave_lds_order();
+                int64_t at = first_row(s, t0);
+#pragma unroll
+                for (int q = 0; q < 16; ++q, next_rows(at, q - 1)) {
+                    const int r = 4 * q + kk;
+                    if (!row_ok(s, q) || j >= steps) continue;
+                    (g.spk + at)[lane_at] = (sbits[wave][r] >> j) & 1u ? 1.0f : 0.0f;
+                    (g.vol + at)[lane_at] = vbuf[s][wave][r * kGridPitch + j];
+                    if (ALIF) (g.theta + at)[lane_at] = tbuf[s][wave][r * kGridPitch + j];
+                }
+                wave_lds_order();
+            }
+            if (t0 + kGridChunk < T) put();
+        }
+    }
+    if (stop) {
+        if (tid == 0) __hip_atomic_store(g.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return;
+    }
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+        if (mine[s] && (range_exceeded(nrn[s].acc_lif, 30) || range_exceeded(nrn[s].acc_th, 28))) raise_range_flag(p.range_flag);
+}
+
+// The same layer, one workgroup per sample, when a workgroup of the kernel above gave up waiting.
+template <bool ALIF, bool POW2>
+__global__ __launch_bounds__(kSoloThreads) void recurrent_solo_fwd_kernel(const GridFwd g) {
+    __shared__ float spikes[2][kGridMaxC];
+    if (*g.gave_up == 0u) return;
+    const StepFwd& p = g.p;
+    const int C = p.C, T = p.T;
+    constexpr int kEach = kGridMaxC / kSoloThreads;
+    StepNeuron<ALIF, false, POW2> nrn[kEach];
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        const int c = threadIdx.x + i * kSoloThreads;
+        nrn[i] = StepNeuron<ALIF, false, POW2>{};
+        if (c < C) {
+            nrn[i].load_decays(p, c);
+            nrn[i].load_states(p, (int64_t)blockIdx.x * C + c);
+            nrn[i].check(p.range_flag);
+        }
+    }
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+        for (int i = 0; i < kEach; ++i) {
+            const int c = threadIdx.x + i * kSoloThreads;
+            if (c >= C) continue;
+            const int64_t m = (int64_t)blockIdx.x * C + c, at = m * T + t;
+            float fb = 0.f;
+            if (t > 0)
+                for (int k = 0; k < C; ++k) fb += g.rec[(int64_t)c * C + k] * spikes[(t - 1) & 1][k];
+            const StepValues o = nrn[i].step(g.z[at] + fb, p);
+            spikes[t & 1][c] = o.spike;
+            g.spk[at] = o.spike;
+            g.vol[at] = o.voltage;
+            if (ALIF) g.theta[at] = o.theta;
+            if (t == T - 1) {
+                p.cur_last[m] = o.current;
+                p.vol_last[m] = o.voltage;
+                if (ALIF) { p.th_last[m] = o.threshold; p.ref_last[m] = o.refractory; }
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < kEach; ++i)
+        if (threadIdx.x + i * kSoloThreads < (unsigned)C &&
+            (range_exceeded(nrn[i].acc_lif, 30) || range_exceeded(nrn[i].acc_th, 28)))
+            raise_range_flag(p.range_flag);
+}
+
+// ---- backward -----------------------------------------------------------------------------------------------------
+//
+//   grad_z[t] = surrogate(v[t], theta[t]) * (grad_s[t] + grad_z[t+1] R)     (the carried state is a constant)
+//
+// The same split of the work; the product of two real operands stays on the float32 matrix instruction.  What a step
+// hands on are 16 x 16 floats per workgroup in the order the product's lanes load them (a contiguous kilobyte), in
+// a ring of four sets.  A float is its own flag here: a set is filled with kUnwritten, a NaN pattern that is never
+// published, before it is used again.  A workgroup clears its part of the set of step t+3 when it begins step t: it has
+// read all of t+2, whose publishers had read all of t+3; the clearing store has arrived before it publishes t, and
+// nobody looks at the set again, for step t-1, before having read t.
+//   Bound at [32, 2048, 300] by the float32 matrix rate (1.7 us a step) and by the 128 KB each compute unit
+// reads a step (1.1 us from the L2).
+constexpr unsigned kUnwritten = 0xffffffffu;
+
+struct GridBwd {
+    float* gz;                                       // [N][C][T]
+    const float *g, *v, *theta, *rec;                // theta: nullptr for one threshold
+    unsigned* ring;                                  // [4][S][KB][256]
+    unsigned* gave_up;
+    GridMap map;
+    int KB, S, N, C, T, graded;
+    float spike_thr, tau, rho;
+};
+
+__device__ __forceinline__ float surrogate_factor(const GridBwd& p, float v, float th) {
+    const float lead = (p.rho / 2.0f) / p.tau, inv_tau = 1.0f / p.tau;
+    const float d = v - th;
+    return p.graded ? p.rho * expf(fminf(d, 0.0f) * inv_tau) : lead * expf(-fabsf(d) * inv_tau);
+}
+
+// Thread (wave v, lane 4 j + i) of the first four waves has neuron 4 v + i of the tile and sample j.
+template <bool THETA, int U, int NT>
+__global__ __launch_bounds__(kGridThreads) void recurrent_grid_bwd_kernel(const GridBwd p) {
+    constexpr int kPlane = 80;                       // pitch of a plane of red: reads of a wave meet 64 banks
+    __shared__ float red[2][kGridWaves][4][kPlane];
+    __shared__ float gbuf[NT][4][kWave * kGridPitch], fbuf[NT][4][kWave * kGridPitch], obuf[NT][4][kWave * kGridPitch];
+    __shared__ int dead[2];
+    const int C = p.C, N = p.N, T = p.T, KB = p.KB;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kk = lane >> 4, j = lane & 15;
+    const int P = p.map.tile(blockIdx.x), c0 = P * 16, group = p.map.group(blockIdx.x);
+    if (P >= KB || group * NT >= p.S) return;
+    if (tid < 2) dead[tid] = 0;
+
+    // columns c0 .. c0 + 15 of R as A operands: lane (kk, j) has rows 16 kb + 4 kk .. + 3 of column c0 + j
+    float4 w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k = 16 * (wave + kGridWaves * u) + 4 * kk;
+        const bool ok = c0 + j < C && k < C;                     // C is a multiple of 4
+        const float* at = p.rec + (ok ? (int64_t)k * C + c0 + j : 0);
+        w[u] = make_float4(at[0], at[ok ? C : 0], at[ok ? 2 * (int64_t)C : 0], at[ok ? 3 * (int64_t)C : 0]);
+        if (!ok) w[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    const __amdgpu_buffer_rsrc_t ring = make_rsrc(reinterpret_cast<const float*>(p.ring), 4u * p.S * KB * 1024u);
+
+    // staging as in the forward kernel: access q covers the four rows of sample q, lane (kk, j) step j of neuron 4 wave + kk
+    const unsigned lane_at = (unsigned)kk * (unsigned)T + (unsigned)j;
+    auto row_ok = [&](int s, int q) -> bool { return (group * NT + s) * 16 + q < N && c0 + 4 * wave < C; };
+    auto first_row = [&](int s, int t0) -> int64_t {
+        return ((int64_t)((group * NT + s) * 16) * C + c0 + 4 * wave) * T + t0;
+    };
+    auto next_rows = [&](int64_t& at) {
+        at += (int64_t)C * T;
+        asm volatile("" : "+s"(at));
+    };
+    float gn[NT][16], vn[NT][16], tn[THETA ? NT : 1][16];
+    auto fetch = [&](int t0) {
+#pragma unroll
+        for (int s = 0; s < NT; ++s) {
+            int64_t at = first_row(s, t0);
+#pragma unroll
+            for (int q = 0; q < 16; ++q, next_rows(at)) {
+                const bool ok = row_ok(s, q) && t0 + j < T;
+                gn[s][q] = ok ? (p.g + at)[lane_at] : 0.f;
+                vn[s][q] = ok ? (p.v + at)[lane_at] : 0.f;
+                if (THETA) tn[s][q] = ok ? (p.theta + at)[lane_at] : 0.f;
+            }
+        }
+    };
+    auto put = [&]() {
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                gbuf[s][wave][(4 * q + kk) * kGridPitch + j] = gn[s][q];
+                fbuf[s][wave][(4 * q + kk) * kGridPitch + j] =
+                    row_ok(s, q) ? surrogate_factor(p, vn[s][q], THETA ? tn[s][q] : p.spike_thr) : 0.f;
+            }
+        wave_lds_order();
+    };
+    const int t_last = (T - 1) / kGridChunk * kGridChunk;
+    if (wave < 4) { fetch(t_last); put(); }
+    lds_barrier();
+
+    bool stop = false;
+    for (int t0 = t_last; t0 >= 0 && !stop; t0 -= kGridChunk) {
+        if (wave < 4 && t0 > 0) fetch(t0 - kGridChunk);
+        const int steps = T - t0 < kGridChunk ? T - t0 : kGridChunk;
+        for (int e = steps - 1; e >= 0 && !stop; --e) {
+            const int t = t0 + e;
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                const int sel = NT == 1 ? (t & 1) : s & 1;
+                const int tile = group * NT + s;
+                auto set_at = [&](int step) -> int { return (((step & 3) * p.S + tile) * KB) * 1024; };   // bytes
+                unsigned* mine = p.ring + set_at(0) / 4 + P * 256 + tid;                    // of set 0; tid < 256
+                const int per_set = p.S * KB * 256;
+                float gs = 0.f, factor = 0.f;
+                if (wave < 4) {
+                    gs = gbuf[s][wave][lane * kGridPitch + e];
+                    factor = fbuf[s][wave][lane * kGridPitch + e];
+                    if (t + 3 < T)
+                        __hip_atomic_store(mine + (int64_t)((t + 3) & 3) * per_set, kUnwritten, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                if (t + 1 < T) {
+                    const int base = set_at(t + 1) + lane * 16;
+                    auto load = [&](int u) -> v4u {
+                        const int kb = wave + kGridWaves * u;
+                        return __builtin_amdgcn_raw_buffer_load_b128(ring, base + kb * 1024, 0, 16);     // agent scope
+                    };
+                    auto unwritten = [&](v4u q) -> bool {
+                        return q.x == kUnwritten || q.y == kUnwritten || q.z == kUnwritten || q.w == kUnwritten;
+                    };
+                    v4u a[U];
+                    int spin = 0;
+                    auto wait = [&](int u) {                     // until block u of this wave is there
+                        while (__any(unwritten(a[u]))) {
+                            if (spin == kSpinLimit ||
+                                ((spin & 1023) == 1023 &&
+                                 __hip_atomic_load(p.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
+                                dead[sel] = 1;
+                                spin = kSpinLimit;
+                                break;
+                            }
+                            ++spin;
+                            asm volatile("" ::: "memory");
+                            a[u] = load(u);
+                        }
+                    };
+                    // the first block is polled, the others are requested when it is there
+                    if (wave < KB) { a[0] = load(0); wait(0); }
+#pragma unroll
+                    for (int u = 1; u < U; ++u)
+                        if (wave + kGridWaves * u < KB) a[u] = load(u);
+                    split_f4 acc[2] = {split_f4{0.f, 0.f, 0.f, 0.f}, split_f4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (wave + kGridWaves * u >= KB) continue;                        // the same for the whole wave
+                        if (u > 0) wait(u);
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u].x, __uint_as_float(a[u].x), acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u].y, __uint_as_float(a[u].y), acc[1], 0, 0, 0);
+                        acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u].z, __uint_as_float(a[u].z), acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u].w, __uint_as_float(a[u].w), acc[1], 0, 0, 0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) red[sel][wave][i][lane] = acc[0][i] + acc[1][i];
+                }
+                lds_barrier();
+                if (wave < 4) {
+                    if (t + 1 < T) {
+                        float carry = 0.f;
+#pragma unroll
+                        for (int v = 0; v < kGridWaves; ++v) carry += red[sel][v][lane & 3][wave * 16 + (lane >> 2)];
+                        gs = carry + gs;
+                    }
+                    const float gz = factor * gs;
+                    if (t > 0) {
+                        const unsigned bits = __float_as_uint(gz);
+                        __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): the clearing store has arrived
+                        __hip_atomic_store(mine + (int64_t)(t & 3) * per_set, bits == kUnwritten ? 0x7fffffffu : bits,
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                    obuf[s][wave][lane * kGridPitch + e] = gz;
+                }
+                stop = stop || dead[sel] != 0;
+                lds_barrier();                                   // see the forward kernel
+            }
+        }
+        if (wave < 4) {
+#pragma unroll
+            for (int s = 0; s < NT; ++s) {
+                wave_lds_order();
+                int64_t at = first_row(s, t0);
+#pragma unroll
+                for (int q = 0; q < 16; ++q, next_rows(at))
+                    if (row_ok(s, q) && j < steps) (p.gz + at)[lane_at] = obuf[s][wave][(4 * q + kk) * kGridPitch + j];
+            }
+            wave_lds_order();
+            if (t0 > 0) put();
+        }
+    }
+    if (stop && tid == 0) __hip_atomic_store(p.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(kSoloThreads) void recurrent_solo_bwd_kernel(const GridBwd p) {
+    __shared__ float next[2][kGridMaxC];
+    if (*p.gave_up == 0u) return;
+    for (int t = p.T - 1; t >= 0; --t) {
+        for (int c = threadIdx.x; c < p.C; c += kSoloThreads) {
+            const int64_t at = ((int64_t)blockIdx.x * p.C + c) * p.T + t;
+            float carry = 0.f;
+            if (t + 1 < p.T)
+                for (int k = 0; k < p.C; ++k) carry += next[(t + 1) & 1][k] * p.rec[(int64_t)k * p.C + c];
+            const float gz = surrogate_factor(p, p.v[at], p.theta ? p.theta[at] : p.spike_thr) * (carry + p.g[at]);
+            next[t & 1][c] = gz;
+            p.gz[at] = gz;
+        }
+        __syncthreads();
+    }
+}
+
+namespace {
+
+struct GridPlan {
+    int KB, S, NT;
+    GridMap map;
+    unsigned grid;
+};
+
+// One workgroup per compute unit: 16 neurons by one or two sample tiles.  A handful of steps costs more as a
+// cooperative launch (14 us more than a plain one) than as separate launches (7 us each).
+bool grid_plan(int64_t N, int64_t C, int64_t T, hipStream_t st, GridPlan* plan) {
+    if (C > kGridMaxC || T < 8 || T > kGridMaxT) return false;
+    int dev = 0, units = 0, coop = 0;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop ||
+        hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const int64_t KB = (C + 15) / 16, tiles = (N + 15) / 16;
+    for (int nt = 1; nt <= 2; ++nt) {
+        const int64_t groups = (tiles + nt - 1) / nt;
+        for (int xcds = 1; xcds <= 8; xcds *= 2) {
+            const int64_t per_xcd = (KB + xcds - 1) / xcds, rounds = (groups + 8 / xcds - 1) / (8 / xcds);
+            if (8 * per_xcd * rounds > units) continue;
+            plan->KB = (int)KB; plan->S = (int)(groups * nt); plan->NT = nt;
+            plan->map.xcds = xcds; plan->map.per_xcd = (int)per_xcd;
+            plan->grid = (unsigned)(8 * per_xcd * rounds);
+            return true;
+        }
+    }
+    return false;
+}
+
+// false: the runtime does not take the grid as a cooperative one
+bool launch_grid(const void* kernel, unsigned grid, void* args, hipStream_t st) {
+    void* list[] = {args};
+    if (hipLaunchCooperativeKernel(kernel, dim3(grid), dim3(kGridThreads), list, 0, st) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
+template <bool ALIF, bool POW2>
+bool launch_grid_fwd(const GridFwd& g, const GridPlan& plan, hipStream_t st) {
+    const bool narrow = plan.KB <= 8 * kGridWaves;               // one unit a wave
+    const void* k = plan.NT == 1
+        ? (narrow ? (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 1, 1> : (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 2, 1>)
+        : (narrow ? (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 1, 2> : (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 2, 2>);
+    if (!launch_grid(k, plan.grid, (void*)&g, st)) return false;
+    hipLaunchKernelGGL((recurrent_solo_fwd_kernel<ALIF, POW2>), dim3((unsigned)g.p.N), dim3(kSoloThreads), 0, st, g);
+    return true;
+}
+
+void launch_grid_fill(unsigned* dst, int64_t n, unsigned value, unsigned* gave_up, hipStream_t st) {
+    hipLaunchKernelGGL(grid_fill_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dst, n, value, gave_up);
+}
+
+}  // namespace
+
+bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* theta, const float* z, const float* rec,
+              float* workspace, int64_t workspace_floats, hipStream_t st, int* error) {
+    GridPlan plan;
+    if (!grid_plan(p.N, p.C, p.T, st, &plan)) return false;
+    const int64_t words = (int64_t)2 * plan.S * words_of(plan.KB);
+    if (workspace_floats < words + 4) return false;
+    GridFwd g{};
+    g.p = p;
+    g.p.KB = plan.KB; g.p.S = plan.S;
+    g.map = plan.map;
+    g.spk = spk; g.vol = vol; g.theta = theta; g.z = z; g.rec = rec;
+    g.gave_up = reinterpret_cast<unsigned*>(workspace);
+    g.words = reinterpret_cast<unsigned*>(workspace) + 4;
+    launch_grid_fill(g.words, words, 0u, g.gave_up, st);
+    const bool taken = alif ? (pow2 ? launch_grid_fwd<true, true>(g, plan, st) : launch_grid_fwd<true, false>(g, plan, st))
+                            : (pow2 ? launch_grid_fwd<false, true>(g, plan, st) : launch_grid_fwd<false, false>(g, plan, st));
+    if (taken) *error = (int)hipGetLastError();
+    return taken;
+}
+
+namespace {
+template <bool THETA, int NT>
+const void* grid_bwd_kernel(int KB) {
+    if (KB <= 4 * kGridWaves) return (const void*)recurrent_grid_bwd_kernel<THETA, 4, NT>;
+    if (KB <= 8 * kGridWaves) return (const void*)recurrent_grid_bwd_kernel<THETA, 8, NT>;
+    return (const void*)recurrent_grid_bwd_kernel<THETA, 16, NT>;
+}
+}  // namespace
+
+bool grid_bwd(float* gz, const float* grad_spikes, const float* voltage, const float* theta, const float* rec,
+              float spike_thr, float tau, float rho, int graded, int64_t N, int64_t C, int64_t T,
+              float* workspace, int64_t workspace_floats, hipStream_t st, int* error) {
+    GridPlan plan;
+    if (!grid_plan(N, C, T, st, &plan)) return false;
+    const int64_t ring = (int64_t)4 * plan.S * plan.KB * 256;
+    if (workspace_floats < ring + 4) return false;
+    GridBwd p{};
+    p.gz = gz; p.g = grad_spikes; p.v = voltage; p.theta = theta; p.rec = rec;
+    p.gave_up = reinterpret_cast<unsigned*>(workspace);
+    p.ring = reinterpret_cast<unsigned*>(workspace) + 4;
+    p.map = plan.map;
+    p.KB = plan.KB; p.S = plan.S; p.N = (int)N; p.C = (int)C; p.T = (int)T; p.graded = graded;
+    p.spike_thr = spike_thr; p.tau = tau; p.rho = rho;
+    launch_grid_fill(p.ring, ring, kUnwritten, p.gave_up, st);
+    const void* k = theta ? (plan.NT == 1 ? grid_bwd_kernel<true, 1>(plan.KB) : grid_bwd_kernel<true, 2>(plan.KB))
+                          : (plan.NT == 1 ? grid_bwd_kernel<false, 1>(plan.KB) : grid_bwd_kernel<false, 2>(plan.KB));
+    if (!launch_grid(k, plan.grid, (void*)&p, st)) return false;
+    hipLaunchKernelGGL(recurrent_solo_bwd_kernel, dim3((unsigned)N), dim3(kSoloThreads), 0, st, p);
+    *error = (int)hipGetLastError();
+    return true;
+}
+
+}  // namespace slayer

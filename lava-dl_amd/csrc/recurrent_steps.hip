@@ -1,5 +1,7 @@
 // Recurrent layer of CUBA or ALIF neurons, one launch per time step: the form for layers too wide for one
-// workgroup per sample (recurrent.hip), where re-reading the weight matrix per sample is what a step costs.
+// workgroup per sample (recurrent.hip), where re-reading the weight matrix per sample is what a step costs, that
+// recurrent_grid.hip does not take: more than 2048 neurons or a batch beyond what the chip holds at once, graded spikes
+// forward, a handful of steps, a stream under capture.
 //
 //   feedback[t] = R s[t-1];  s[t] = neuron(z[t] + feedback[t])          (utils/recurrent.py:45-112 in the reference)
 //
@@ -27,8 +29,7 @@
 // The backward pass has the same shape (the reference's convention, utils/recurrent.py:83-112: the state carried
 // between two steps is a constant): grad_dendrite[t] = surrogate(v[t], theta[t]) * (grad_spike[t] + grad_dendrite[t+1] R),
 // the product taken with the transposed matrix so that both directions read weight rows along the summed index.
-#include "common.h"
-#include "tile.h"
+#include "recurrent_step.h"
 
 namespace slayer {
 
@@ -142,22 +143,6 @@ __device__ __forceinline__ float4 step_product(const float4* __restrict__ wp, co
     return sum;
 }
 
-struct StepFwd {
-    float *spk_t, *vol_t, *theta_t;                           // [T][N][C]; theta: ALIF only
-    const float* z_t;                                         // [T][N][C]
-    int* carried;                                             // [4][N][C]: current, voltage, threshold, refractory
-    float *cur_last, *vol_last, *th_last, *ref_last;          // [N*C]; th / ref: ALIF only
-    const float4* rec_packed;                                 // see pack_weights_kernel
-    float4* spk_packed;                                       // two buffers of [KB][S][64] quads, written in turn
-    int KB, S;                                                // blocks of 16 neurons, sample tiles
-    const float *i_decay, *v_decay, *th_decay, *ref_decay, *i_state, *v_state, *th_state, *ref_state;
-    int64_t n_id, n_vd, n_td, n_rd, n_is, n_vs, n_ts, n_rs;
-    float w, inv_w, spike_thr, spike_scale, th_step_f;
-    int base;
-    int N, C, T;
-    unsigned* range_flag;                                     // see raise_range_flag in tile.h
-};
-
 // One step of the layer for 16 neurons x 16 NT samples.  The neuron step is that of recurrent_fwd_kernel
 // (recurrent.hip), state by state: each starts from the float32 value the previous step left and hands a float32
 // value on, as between two one-step neuron calls.
@@ -174,8 +159,7 @@ __global__ __launch_bounds__(kStepWaves * kWave) void recurrent_step_fwd_kernel(
     const int n = n0 + 16 * (tid >> 6) + (lane & 15), c = c0 + 4 * (lane >> 4);
     const bool valid = worker && n < N && c < C;
     const int64_t m = valid ? (int64_t)n * C + c : 0;         // first of this thread's four neurons
-    const float w = p.w, inv_w = p.inv_w;
-    auto from = [&](int y) -> float { const float f = (float)y; return POW2 ? f * inv_w : f / w; };
+    const float w = p.w;
     // what the neuron step reads is on its way while the product runs
     float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     int yc[4] = {0, 0, 0, 0}, yv[4] = {0, 0, 0, 0}, th[4] = {0, 0, 0, 0}, r[4] = {0, 0, 0, 0};
@@ -231,39 +215,12 @@ __global__ __launch_bounds__(kStepWaves * kWave) void recurrent_step_fwd_kernel(
     float so[4], vo[4], to[4], co[4], tho[4], ro[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        if (t == 0) {
-            check_multiplier(mi[i], p.range_flag); check_multiplier(mv[i], p.range_flag);
-            if (ALIF) { check_multiplier(mt[i], p.range_flag); check_multiplier(mr[i], p.range_flag); }
-            acc_lif |= ((unsigned)yc[i] + (1u << 30)) | ((unsigned)yv[i] + (1u << 30));
-            acc_th |= ((unsigned)th[i] + (1u << 28)) | ((unsigned)r[i] + (1u << 28));
-        }
-        const float dend = zs[i] + fbs[i];
-        yc[i] = add_sat(rs0_12(yc[i], mi[i]), trunc_i32(w * dend));
-        const float cur = from(yc[i]);
-        yc[i] = trunc_i32(w * cur);
-        const int yn = add_sat(rs0_12(yv[i], mv[i]), yc[i]);
-        acc_lif |= ((unsigned)yc[i] + (1u << 30)) | ((unsigned)yn + (1u << 30));
-        const float vol = from(yn);
-        float theta = p.spike_thr, thf = 0.f, rf = 0.f;
-        if (ALIF) {
-            r[i] = rs0_12(r[i], mr[i]);
-            th[i] = rs0_12(th[i] - p.base, mt[i]) + p.base;
-            acc_th |= ((unsigned)th[i] + (1u << 28)) | ((unsigned)r[i] + (1u << 28));
-            thf = from(th[i]);
-            rf = from(r[i]);
-            theta = thf + rf;
-        }
-        const bool fired = vol >= theta;
-        const float s = GRADED ? ((fired ? 1.0f : 0.0f) * vol) / p.spike_scale : (fired ? 1.0f : 0.0f);
-        const bool spiked = s > 0.0f;                          // what the carried states see
-        if (ALIF) {
-            yv[i] = trunc_i32(w * vol);
-            r[i] = trunc_i32((spiked ? rf + 2.0f * thf : rf) * w);
-            th[i] = trunc_i32((spiked ? thf + p.th_step_f : thf) * w);
-        } else {
-            yv[i] = spiked ? 0 : trunc_i32(w * vol);
-        }
-        so[i] = s; vo[i] = vol; to[i] = theta; co[i] = cur; tho[i] = thf; ro[i] = rf;
+        StepNeuron<ALIF, GRADED, POW2> nrn{yc[i], yv[i], th[i], r[i], mi[i], mv[i], mt[i], mr[i], 0u, 0u};
+        if (t == 0) nrn.check(p.range_flag);
+        const StepValues o = nrn.step(zs[i] + fbs[i], p);
+        yc[i] = nrn.yc; yv[i] = nrn.yv; th[i] = nrn.th; r[i] = nrn.r;
+        acc_lif |= nrn.acc_lif; acc_th |= nrn.acc_th;
+        so[i] = o.spike; vo[i] = o.voltage; to[i] = o.theta; co[i] = o.current; tho[i] = o.threshold; ro[i] = o.refractory;
     }
     if (range_exceeded(acc_lif, 30) || range_exceeded(acc_th, 28)) raise_range_flag(p.range_flag);
     *reinterpret_cast<float4*>(p.spk_t + t * slab + m) = make_float4(so[0], so[1], so[2], so[3]);
@@ -439,6 +396,9 @@ int run_steps_fwd(StepFwd p, float* spk, float* vol, float* theta, const float* 
     if (!aligned16(workspace) || !aligned16(p.cur_last) || !aligned16(p.vol_last) ||
         (ALIF && (!aligned16(p.th_last) || !aligned16(p.ref_last))))
         return SLAYER_ERANGE;
+    int error = 0;
+    if (!graded && grid_fwd(p, ALIF, is_pow2(w_scale), spk, vol, theta, z, rec, workspace, workspace_floats, st, &error))
+        return error;
     float* zt = workspace;
     p.z_t = zt;
     p.spk_t = workspace + nct;
@@ -546,6 +506,10 @@ extern "C" int slayer_recurrent_steps_bwd(float* grad_z, const float* grad_spike
     if (workspace_floats < l.total(tensors)) return SLAYER_ERANGE;
     if (!aligned16(workspace)) return SLAYER_ERANGE;
     hipStream_t st = (hipStream_t)stream;
+    int error = 0;
+    if (grid_bwd(grad_z, grad_spikes, voltage, theta, rec, spike_threshold, tau_rho, scale_rho, graded, N, C, T, workspace,
+                 workspace_floats, st, &error))
+        return error;
     const int64_t nct = l.nct;
     float* g_t = workspace;
     float* v_t = workspace + nct;

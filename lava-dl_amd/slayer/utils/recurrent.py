@@ -4,8 +4,9 @@ Interface of lava.lib.dl.slayer.utils.recurrent (utils/recurrent.py:7-112 in the
 For a CUBA or an ALIF neuron on the GPU (binary or graded spikes) the time loop runs inside the library: narrow
 layers (and widths up to ``ONE_LAUNCH_MAX`` that are not a multiple of 4) as one kernel launch per direction
 (slayer_cuba_recurrent_fwd / slayer_alif_recurrent_fwd / slayer_recurrent_bwd), layers from ``STEPS_FROM`` neurons
-on (a multiple of 4 up to 16384) as one launch per time step that multiplies the recurrent matrix with the whole
-batch (slayer_*_recurrent_steps_*); any other neuron runs the reference's loop of one-step neuron calls.
+on (a multiple of 4 up to 16384) through slayer_*_recurrent_steps_*: one launch spread over the chip that keeps the
+matrix in registers (up to 2048 neurons, spikes without values, while the batch fits), else one launch per time step
+that multiplies the matrix with the whole batch; any other neuron runs the reference's loop of one-step neuron calls.
 """
 import torch
 

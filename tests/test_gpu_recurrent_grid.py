@@ -1,0 +1,114 @@
+"""Recurrent layers whose time loop is one launch spread over the chip (csrc/recurrent_grid.hip): at the edges of its
+tiles -- one and two sample tiles per workgroup, units of 128 presynaptic neurons, chunks of 16 steps, the shortest
+sequence it takes -- against the CPU oracle, and with weights that are not on a quantiser's grid."""
+import os
+import subprocess
+
+import pytest
+import torch
+
+from oracle import slayer_oracle as O
+from tests import test_gpu_recurrent as base
+from tests.util import dev, assert_exact, assert_rel
+
+pytestmark = pytest.mark.gpu
+
+BINARY = os.path.join(os.path.dirname(os.path.abspath(__file__)), 'native', 'recurrent_solo_check')
+
+
+@pytest.fixture(scope='module')
+def slayer():
+    import lava_dl_amd.slayer as s
+    return s
+
+
+# 16 and 17 samples; whole and partial tiles of 16 neurons; 8 steps (the fewest), 16 and 17; 33 samples of 2048 neurons
+# and 129 of 516 take two sample tiles per workgroup
+@pytest.mark.parametrize('n,c,t', [(16, 256, 8), (17, 260, 16), (1, 1028, 17), (5, 2036, 33), (33, 2048, 9), (129, 516, 18)])
+def test_layer_matches_the_oracle(slayer, n, c, t):
+    R = slayer.utils.recurrent
+    gen = torch.Generator().manual_seed(1000 * c + n)
+    z = torch.randn(n, c, t, generator=gen) * 1.5
+    g = torch.rand(n, c, t, generator=gen)
+    neuron = base._neuron(slayer)
+    syn = base._Dense(c, torch.Generator().manual_seed(5)).to(dev())
+    with torch.no_grad():
+        syn.weight.mul_(6.0 / c ** 0.5)
+    syn.pre_hook_fx = neuron.quantize_8bit
+    zg = z.to(dev()).requires_grad_()
+    out = R.custom_recurrent(zg, neuron, syn)
+    assert 0.01 < float(out.detach().mean()) < 0.9
+    rec = neuron.quantize_8bit(syn.weight.detach().reshape(c, c)).cpu()
+    d_i, d_v = neuron.current_decay.detach().round().cpu(), neuron.voltage_decay.detach().round().cpu()
+    thr, zero = neuron.threshold + neuron.threshold_eps, torch.tensor([0.0])
+    r_spk, r_vol, r_cs, r_vs = O.recurrent_cuba_fwd(z, rec, d_i, d_v, zero, zero, 4096, thr)
+    assert_exact(out, r_spk, 'spikes')
+    assert_exact(neuron.current_state, r_cs, 'carried current')
+    assert_exact(neuron.voltage_state, r_vs, 'carried voltage')
+    out.backward(g.to(dev()))
+    r_gz, _ = O.recurrent_cuba_bwd(g, r_spk, r_vol, rec, thr, neuron.tau_rho * 100, neuron.scale_rho * 0.1)
+    assert_rel(zg.grad, r_gz, 'grad z')
+
+
+@pytest.mark.parametrize('c', [260, 2048])
+def test_feedback_of_weights_off_the_grid(slayer, c):
+    """Weights with all their 24 bits: with decays of 4096 and a scale of 2^22 the voltage of step t is the feedback of the
+    spikes of step t - 1 to 2^-24, compared with a float64 sum.  Bound: the three parts hold every bit of a weight, the
+    sum of c terms is rounded about c / 32 + 16 times to 2^-24 of its running value, which stays below the sum of the
+    magnitudes: c / 32 * 2^-24 of that sum, at most 5e-6 of it (measured: 3e-8)."""
+    from lava_dl_amd.slayer import _native as N
+    n, t = 20, 8
+    gen = torch.Generator().manual_seed(c)
+    rec = (torch.randn(c, c, generator=gen) * 3 / c ** 0.5).to(dev())
+    z = torch.randn(n, c, t, generator=gen).mul(4)
+    z[..., 1:] *= 1e-3
+    z = z.to(dev())
+    spk, vol = torch.empty_like(z), torch.empty_like(z)
+    last = [torch.empty(n, c, device=dev()) for _ in range(2)]
+    full, zero = torch.full((1,), 4096.0, device=dev()), torch.zeros(1, device=dev())
+    floats = N.lib().slayer_recurrent_steps_workspace(n, c, t, 0)
+    ws = torch.empty(floats, device=dev())
+    N.check(N.lib().slayer_cuba_recurrent_steps_fwd(
+        N.ptr(spk), N.ptr(vol), N.ptr(last[0]), N.ptr(last[1]), N.ptr(z), N.ptr(rec), N.ptr(full), N.ptr(full), N.ptr(zero),
+        N.ptr(zero), 0.5, 0, 1.0, 1 << 22, n, c, 1, 1, 1, 1, t, N.ptr(ws), floats, N.stream_handle()))
+    assert 0.05 < float(spk.mean()) < 0.95
+    s, w = spk.cpu().double(), rec.cpu().double()
+    for step in range(1, t):
+        want = z[..., step].cpu().double() + s[..., step - 1] @ w.t()
+        magnitude = s[..., step - 1] @ w.abs().t() + z[..., step].cpu().double().abs()
+        err = ((vol[..., step].cpu().double() - want).abs() / (magnitude + 1)).max()
+        assert float(err) <= 5e-6, float(err)
+
+
+def test_weights_that_are_not_finite(slayer, monkeypatch):
+    """An infinite weight times a silent neuron is a NaN, and so is a NaN weight times any: what the two receiving neurons
+    do is lost, the other neurons' feedback is untouched."""
+    from lava_dl_amd.slayer import _native as N
+    monkeypatch.setattr(N, '_range_policy', 'ignore')              # an infinite feedback leaves a state at its limit
+    R = slayer.utils.recurrent
+    n, c, t = 3, 300, 12
+    gen = torch.Generator().manual_seed(3)
+    z = (torch.randn(n, c, t, generator=gen) * 1.5).to(dev())
+    weight = torch.round(torch.randn(c, c, generator=gen) * 12) / 64
+    weight[:, 5] = weight[:, 9] = 0                                # what neurons 5 and 9 do reaches nobody
+    results = []
+    for bad in (0.0, float('inf'), float('nan')):
+        neuron = base._neuron(slayer)
+        weight[5, 7] = weight[9, 11] = bad
+        with torch.no_grad():
+            results.append(R._FusedRecurrent.apply(z, neuron, weight.to(dev())))
+    assert 0.01 < float(results[0].mean()) < 0.9
+    rows = [i for i in range(c) if i not in (5, 9)]
+    for out in results[1:]:
+        assert torch.equal(out[:, rows], results[0][:, rows])
+        assert not torch.equal(out, results[0])
+    torch.cuda.synchronize()
+    N.clear_range_flag()
+
+
+def test_workgroups_that_give_up_waiting():
+    if not os.path.exists(BINARY):
+        pytest.skip('tests/native/recurrent_solo_check has not been built (python -c "import __graft_entry__ as g; g.build()")')
+    run = subprocess.run([BINARY], capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stdout + run.stderr
+    assert 'solo kernels agree' in run.stdout
