@@ -34,7 +34,12 @@ struct AlifFwd {
     static constexpr int kIn = 1, kOut = KEEP_CURRENT ? 4 : 3;   // out: [current,] voltage, threshold + refractory, spikes
     static constexpr int kVol = kOut - 3, kTheta = kOut - 2, kSpk = kOut - 1;
     static constexpr unsigned kShiftIn = SHIFT ? 1u : 0u, kShiftOut = SHIFT ? (1u << kSpk) : 0u;
-    static constexpr int kCopyWaves = SHIFT ? 4 : 2;     // the shifted copies cost the copy waves more instructions
+    // The shifted copies cost the copy waves more instructions, and so do rows that are not whole quads: [16,512,1450] with
+    // two / eight copy waves 111 / 81 us in the staged kernel, [32,256,1500] with two / four 74.7 / 72.2.  In the two-wave kernel
+    // two stay: [64,512,1000] 121 / 137, [32,16,32,32,300] 545 / 810 with four.
+    static constexpr int copy_waves(bool, bool unaligned, bool staged) {
+        return staged && !SHIFT && unaligned ? 8 : (staged || SHIFT ? 4 : 2);
+    }
     static constexpr bool kReverse = false;
     static constexpr bool kTransforms = true;
     static constexpr int64_t kRows32Below = 32768, kRows16Below = 32768;
@@ -53,6 +58,7 @@ struct AlifFwd {
     static constexpr bool kRangeChecked = true;
     static constexpr int range_log2(int o) { return o >= kTheta ? 28 : 30; }   // threshold / refractory : current, voltage
     int yc, yv, th, r, th_out, r_out, mi, mv, mt, mr, th_step, base;
+    bool nonneg;
     float w, inv_w, spike_scale;
 
     __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
@@ -72,6 +78,7 @@ struct AlifFwd {
             check_state(yc, 30, p.range_flag); check_state(yv, 30, p.range_flag);
             check_state(th, 28, p.range_flag); check_state(r, 28, p.range_flag);
         }
+        nonneg = all_nonneg(mi | mv | mt | mr);
     }
     // what the next operator reads of a state: trunc(w * (float(y) / w)); for a power of two the scaling
     // is exact and only the int -> float32 rounding remains
@@ -80,11 +87,13 @@ struct AlifFwd {
         return POW2 ? trunc_i32(f) : trunc_i32(w * (f / w));
     }
     __device__ __forceinline__ void pre(float4 (&x)[1]) const { x[0] = to_state(x[0], w); }
-    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) {
-        yc = add_sat(rs0_12(yc, mi), __float_as_int(x[0]));
-        yv = add_sat(rs0_12(yv, mv), reread(yc));               // the voltage op reads the float32 current
-        r = rs0_12(r, mr);
-        th = rs0_12(th - base, mt) + base;
+    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) { step_as<false>(x, o); }
+    template <bool NONNEG>
+    __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[kOut]) {
+        yc = add_sat(decayed<NONNEG>(yc, mi), __float_as_int(x[0]));
+        yv = add_sat(decayed<NONNEG>(yv, mv), reread(yc));      // the voltage op reads the float32 current
+        r = decayed<NONNEG>(r, mr);
+        th = decayed<NONNEG>(th - base, mt) + base;
         th_out = th; r_out = r;
         const bool fired = reread(yv) >= th + r;                // the threshold op reads the float32 voltage
         r += fired ? 2 * th : 0;
@@ -103,6 +112,7 @@ struct AlifFwd {
         static constexpr int in_tile(int) { return 0; }
         static constexpr int out_tile(int o) { return o; }       // [current,] voltage: tiles 0 .. kVol
         int yc, yv, mi, mv;
+        bool nonneg;
         float w, inv_w;
         __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
             w = p.w; inv_w = p.inv_w; yc = yv = mi = mv = 0;
@@ -114,11 +124,14 @@ struct AlifFwd {
                 check_multiplier(mi, p.range_flag); check_multiplier(mv, p.range_flag);
                 check_state(yc, 30, p.range_flag); check_state(yv, 30, p.range_flag);
             }
+            nonneg = all_nonneg(mi | mv);
         }
-        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) {
-            yc = add_sat(rs0_12(yc, mi), __float_as_int(x[0]));
+        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) { step_as<false>(x, o); }
+        template <bool NONNEG>
+        __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[kOut]) {
+            yc = add_sat(decayed<NONNEG>(yc, mi), __float_as_int(x[0]));
             const float cf = (float)yc;
-            yv = add_sat(rs0_12(yv, mv), POW2 ? trunc_i32(cf) : trunc_i32(w * (cf / w)));
+            yv = add_sat(decayed<NONNEG>(yv, mv), POW2 ? trunc_i32(cf) : trunc_i32(w * (cf / w)));
             if (KEEP_CURRENT) o[0] = __int_as_float(yc);
             o[kVol] = __int_as_float(yv);
         }
@@ -133,6 +146,7 @@ struct AlifFwd {
         static constexpr int in_tile(int) { return kVol; }
         static constexpr int out_tile(int o) { return kTheta + o; }   // threshold, refractory state
         int th, r, th_out, r_out, yv_last, mt, mr, th_step, base;
+        bool nonneg;
         float w, inv_w, spike_scale;
         __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
             w = p.w; inv_w = p.inv_w; spike_scale = p.spike_scale; th_step = p.step; base = p.base;
@@ -146,12 +160,15 @@ struct AlifFwd {
                 check_multiplier(mt, p.range_flag); check_multiplier(mr, p.range_flag);
                 check_state(th, 28, p.range_flag); check_state(r, 28, p.range_flag);
             }
+            nonneg = all_nonneg(mt | mr);
         }
-        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[2]) {
+        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[2]) { step_as<false>(x, o); }
+        template <bool NONNEG>
+        __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[2]) {
             const int yv = __float_as_int(x[0]);
             const float vf = (float)yv;
-            r = rs0_12(r, mr);
-            th = rs0_12(th - base, mt) + base;
+            r = decayed<NONNEG>(r, mr);
+            th = decayed<NONNEG>(th - base, mt) + base;
             th_out = th; r_out = r; yv_last = yv;
             const bool fired = (POW2 ? trunc_i32(vf) : trunc_i32(w * (vf / w))) >= th + r;
             r += fired ? 2 * th : 0;

@@ -48,8 +48,14 @@ struct CubaFwd {
     static constexpr bool kRangeChecked = true;
     static constexpr int range_log2(int) { return 30; }
     static constexpr bool kTransforms = true;        // integer tiles, see to_state / from_state
-    static constexpr int kCopyWaves = SHIFT ? 8 : 2;     // the shifted copies cost the copy waves more instructions
+    // The shifted copies cost the copy waves more instructions, and so do rows that are not whole quads: [16,512,1450] with
+    // two / four / eight copy waves 81 / 59 / 49 us, [32,256,1500] 43.7 / 41.7 / 41.9.  Large tensors, two / four: [32,16,32,32,300]
+    // 503 / 533 with the current trace, 237 / 249 without any trace, [.., 301] 751 / 939 and (no current) 492 / 449.
+    static constexpr int copy_waves(bool large, bool unaligned, bool) {
+        return SHIFT || (unaligned && !large) ? 8 : (large ? (unaligned && !KEEP_CURRENT ? 4 : 2) : 4);
+    }
     int yc, yv, yv_out, mi, mv, fire_above;
+    bool nonneg;
     float w, inv_w, spike_thr, spike_scale;
 
     __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
@@ -64,18 +70,21 @@ struct CubaFwd {
             check_multiplier(mi, p.range_flag); check_multiplier(mv, p.range_flag);
             check_state(yc, 30, p.range_flag); check_state(yv, 30, p.range_flag);
         }
+        nonneg = all_nonneg(mi | mv);
     }
     __device__ __forceinline__ void pre(float4 (&x)[1]) const { x[0] = to_state(x[0], w); }
     __device__ __forceinline__ void post(float4 (&o)[kOut]) const {
 #pragma unroll
         for (int i = 0; i < kOut; ++i) o[i] = from_state<POW2>(o[i], w, inv_w);
     }
-    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) {
-        yc = add_sat(rs0_12(yc, mi), __float_as_int(x[0]));
+    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) { step_as<false>(x, o); }
+    template <bool NONNEG>
+    __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[kOut]) {
+        yc = add_sat(decayed<NONNEG>(yc, mi), __float_as_int(x[0]));
         // the voltage op reads the float32 current: trunc(w * (float(yc) / w)); for a power of two
         // the scaling is exact and only the int -> float32 rounding remains
         const float cf = (float)yc;
-        const int yn = add_sat(rs0_12(yv, mv), POW2 ? trunc_i32(cf) : trunc_i32(w * (cf / w)));
+        const int yn = add_sat(decayed<NONNEG>(yv, mv), POW2 ? trunc_i32(cf) : trunc_i32(w * (cf / w)));
         yv = (yn > fire_above) ? 0 : yn;             // float(yn) >= threshold, decided on the integer
         yv_out = yn;
         if (KEEP_CURRENT) o[0] = __int_as_float(yc);
@@ -84,7 +93,7 @@ struct CubaFwd {
     // The same step as two Ops for the staged multi-wave kernel: the current recurrence, and the voltage
     // recurrence one chunk later.  What the voltage op reads of the current (the float32 round trip) is worked
     // out by the first wave and left in the voltage tile, where the second wave replaces it with the voltage:
-    // that evens out the two steps (8 and 9 instructions instead of 6 and 11).
+    // that evens out the two steps (6 instructions each in their short form, see rs0_12_nonneg, instead of 4 and 8).
     static constexpr int kStages = 2;
     static constexpr bool kStagedWhenLarge = true;
     struct Stage0 {
@@ -93,6 +102,7 @@ struct CubaFwd {
         static constexpr int in_tile(int) { return 0; }
         static constexpr int out_tile(int o) { return o; }       // [current,] what the voltage op reads of it
         int yc, mi;
+        bool nonneg;
         float w, inv_w;
         __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
             w = p.w; inv_w = p.inv_w; yc = mi = 0;
@@ -101,9 +111,12 @@ struct CubaFwd {
                 mi = 4096 - trunc_i32(rintf(p.i_decay[param_index(m, p.npb, p.n_id)]));
                 check_multiplier(mi, p.range_flag); check_state(yc, 30, p.range_flag);
             }
+            nonneg = all_nonneg(mi);
         }
-        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) {
-            yc = add_sat(rs0_12(yc, mi), __float_as_int(x[0]));
+        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[kOut]) { step_as<false>(x, o); }
+        template <bool NONNEG>
+        __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[kOut]) {
+            yc = add_sat(decayed<NONNEG>(yc, mi), __float_as_int(x[0]));
             const float cf = (float)yc;
             if (KEEP_CURRENT) o[0] = __int_as_float(yc);
             o[kVol] = __int_as_float(POW2 ? trunc_i32(cf) : trunc_i32(w * (cf / w)));
@@ -118,6 +131,7 @@ struct CubaFwd {
         static constexpr int in_tile(int) { return kVol; }
         static constexpr int out_tile(int) { return kVol; }      // in place
         int yv, yv_out, mv, fire_above;
+        bool nonneg;
         float w, inv_w, spike_thr, spike_scale;
         __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
             w = p.w; inv_w = p.inv_w; fire_above = p.fire_above; spike_thr = p.spike_thr; spike_scale = p.spike_scale;
@@ -127,9 +141,12 @@ struct CubaFwd {
                 mv = 4096 - trunc_i32(rintf(p.v_decay[param_index(m, p.npb, p.n_vd)]));
                 check_multiplier(mv, p.range_flag); check_state(yv, 30, p.range_flag);
             }
+            nonneg = all_nonneg(mv);
         }
-        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[1]) {
-            const int yn = add_sat(rs0_12(yv, mv), __float_as_int(x[0]));
+        __device__ __forceinline__ void step(const float (&x)[1], float (&o)[1]) { step_as<false>(x, o); }
+        template <bool NONNEG>
+        __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[1]) {
+            const int yn = add_sat(decayed<NONNEG>(yv, mv), __float_as_int(x[0]));
             yv = (yn > fire_above) ? 0 : yn;
             yv_out = yn;
             o[0] = __int_as_float(yn);

@@ -31,8 +31,11 @@ struct LiFwd {
     // on its way into LDS, the state is converted and scaled back on its way out, and the
     // sequential loop is left with the recurrence alone.
     static constexpr bool kTransforms = true;
-    static constexpr int kCopyWaves = 2;
+    // [32,256,1500] 35 -> 32 us with four instead of two (43 -> 40 with a threshold), [16,512,1450] 54 -> 35 with eight,
+    // [32,16,32,32,300] 239 -> 233, [32,16,32,32,301] 299 -> 287 (eight: 325)
+    static constexpr int copy_waves(bool large, bool unaligned, bool) { return unaligned && !large ? 8 : 4; }
     int y, mult, fire_above;
+    bool nonneg;
     float w, inv_w;
 
     __device__ __forceinline__ void init(const Params& p, int64_t m, bool valid) {
@@ -44,11 +47,14 @@ struct LiFwd {
             check_multiplier(mult, p.range_flag);
             check_state(y, 30, p.range_flag);
         }
+        nonneg = all_nonneg(mult);
     }
     __device__ __forceinline__ void pre(float4 (&x)[1]) const { x[0] = to_state(x[0], w); }
     __device__ __forceinline__ void post(float4 (&o)[1]) const { o[0] = from_state<POW2>(o[0], w, inv_w); }
-    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[1]) {
-        const int yn = add_sat(rs0_12(y, mult), __float_as_int(x[0]));
+    __device__ __forceinline__ void step(const float (&x)[1], float (&o)[1]) { step_as<false>(x, o); }
+    template <bool NONNEG>
+    __device__ __forceinline__ void step_as(const float (&x)[1], float (&o)[1]) {
+        const int yn = add_sat(decayed<NONNEG>(y, mult), __float_as_int(x[0]));
         o[0] = __int_as_float(yn);
         y = (RESET && yn > fire_above) ? 0 : yn;     // (float)yn >= threshold, decided on the integer
     }

@@ -32,6 +32,18 @@ __device__ __forceinline__ int rs0_12(int a, int b) {
     return (int)(((long long)a * (long long)b + bias) >> 12);
 }
 
+// The same for a multiplier 0 <= b < 2^26 (a decay of at most 4096), two instructions less: with the multiplier scaled to
+// a shift by 16 the bias of a negative product is sixteen copies of a's sign bit, which one byte permutation makes out of a.
+// The multiply-add, the shift and the permutation are all that is left in front of the addition of the input.
+__device__ __forceinline__ int rs0_12_nonneg(int a, int b) {
+    const unsigned bias = __builtin_amdgcn_perm((unsigned)a, (unsigned)a, 0x0c0c0909u);     // 0, 0, sign, sign
+    return (int)(((long long)a * (long long)(b << 4) + (long long)bias) >> 16);
+}
+template <bool NONNEG>
+__device__ __forceinline__ int decayed(int a, int b) { return NONNEG ? rs0_12_nonneg(a, b) : rs0_12(a, b); }
+// true when every lane's multiplier takes that form
+__device__ __forceinline__ bool all_nonneg(int b) { return __all((unsigned)b < (1u << 26)); }
+
 // a + b held inside the int32 range (v_add_i32 with clamp: one instruction, as the wrapping add).  The state
 // updates use it so that a sum that leaves the range ends at the limit, where the range check of the copy-out
 // sees it, instead of wrapping to an innocent-looking value.
@@ -208,6 +220,8 @@ struct TileGeom {
 //     in[] entry other than in[0] reads as zeros: a slot for pre() to fill)
 //   __device__ void init(const Params&, int64_t m, bool valid);
 //   __device__ void step(const float (&x)[kIn], float (&y)[kOut]);
+//   optionally bool nonneg, set by init, and template <bool NONNEG> step_as(x, y): what step() does, in a shorter form
+//     that the interior chunks take when nonneg is set (see rs0_12_nonneg)
 //   __device__ void finish(const Params&, int64_t m, bool valid);
 
 template <class Op, class = void>
@@ -728,6 +742,16 @@ struct TileMap<Op, decltype((void)Op::kTileMapped)> {
     static constexpr int out(int o) { return Op::out_tile(o); }
 };
 
+template <class Op, class = void>
+struct HasShortStep { static constexpr bool value = false; };
+template <class Op>
+struct HasShortStep<Op, decltype((void)sizeof(((Op*)nullptr)->nonneg))> { static constexpr bool value = true; };
+// std::true_type: the short form
+template <class Op, class X, class Y>
+__device__ __forceinline__ void op_step(Op& op, const X& x, Y& y, std::false_type) { op.step(x, y); }
+template <class Op, class X, class Y>
+__device__ __forceinline__ void op_step(Op& op, const X& x, Y& y, std::true_type) { op.template step_as<true>(x, y); }
+
 // The sequential part: lane = neuron, one chunk of the tiles in place.
 // EXACT: rows may begin and end inside a quad (see Copier, UNAL); on the edge chunks the steps of a quad that lie
 // outside the row are then skipped one by one.
@@ -736,7 +760,7 @@ __device__ __forceinline__ void run_chunk(Op& op, float (*tile)[TileGeom<R, S>::
                                           bool inner, int a_lane, int T) {
     using G = TileGeom<R, S>;
     constexpr int NI = Op::kIn, NO = Op::kOut;
-    auto run_quad = [&](int qq) {
+    auto run_quad = [&](int qq, auto short_form) {
         float xin[NI][4], yout[NO][4];
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
@@ -749,7 +773,7 @@ __device__ __forceinline__ void run_chunk(Op& op, float (*tile)[TileGeom<R, S>::
             float x[NI], y[NO];
 #pragma unroll
             for (int i = 0; i < NI; ++i) x[i] = xin[i][ss];
-            op.step(x, y);
+            op_step(op, x, y, short_form);
 #pragma unroll
             for (int o = 0; o < NO; ++o) yout[o][ss] = y[o];
         }
@@ -760,14 +784,21 @@ __device__ __forceinline__ void run_chunk(Op& op, float (*tile)[TileGeom<R, S>::
     };
     if (inner) {
         if (lane < R) {
+            if constexpr (HasShortStep<Op>::value) {
+                if (op.nonneg) {
 #pragma unroll UNROLL
-            for (int q = 0; q < G::kQuads; ++q) run_quad(Op::kReverse ? G::kQuads - 1 - q : q);
+                    for (int q = 0; q < G::kQuads; ++q) run_quad(Op::kReverse ? G::kQuads - 1 - q : q, std::true_type{});
+                    return;
+                }
+            }
+#pragma unroll UNROLL
+            for (int q = 0; q < G::kQuads; ++q) run_quad(Op::kReverse ? G::kQuads - 1 - q : q, std::false_type{});
         }
     } else if (!EXACT) {
         const int tl = chunk * G::kChunk - a_lane;       // step held by column 0 of this lane's row
         for (int q = 0; q < G::kQuads; ++q) {
             const int qq = Op::kReverse ? G::kQuads - 1 - q : q;
-            if (lane < R && (unsigned)(tl + 4 * qq) < (unsigned)T) run_quad(qq);
+            if (lane < R && (unsigned)(tl + 4 * qq) < (unsigned)T) run_quad(qq, std::false_type{});
         }
     } else {
         const int tl = chunk * G::kChunk - a_lane;
@@ -776,7 +807,7 @@ __device__ __forceinline__ void run_chunk(Op& op, float (*tile)[TileGeom<R, S>::
             const int t0 = tl + 4 * qq;                  // step of the quad's first column
             if (lane < R && t0 > -4 && t0 < T) {
                 if (t0 >= 0 && t0 <= T - 4) {
-                    run_quad(qq);
+                    run_quad(qq, std::false_type{});
                 } else {
                     float xin[NI][4], yout[NO][4];
 #pragma unroll
@@ -1186,13 +1217,25 @@ struct CopyWaves { static constexpr int value = 1; };
 template <class Op>
 struct CopyWaves<Op, decltype((void)Op::kCopyWaves)> { static constexpr int value = Op::kCopyWaves; };
 
+// An Op may set them for each kernel it takes: copy_waves(large tensor, rows that are not whole quads, staged kernel).
+// While all workgroups are resident the sequential waves should not wait for their tiles, and a copy wave, which issues an
+// instruction every few cycles whatever it does, cannot keep up with the short form of a step; on large tensors
+// more of them only add to what is in flight.
+template <class Op, bool STREAM, bool UNAL, bool STAGED, class = void>
+struct CopyWavesOf { static constexpr int value = CopyWaves<Op>::value; };
+template <class Op, bool STREAM, bool UNAL, bool STAGED>
+struct CopyWavesOf<Op, STREAM, UNAL, STAGED, decltype((void)Op::copy_waves(STREAM, UNAL, STAGED))> {
+    static constexpr int value = Op::copy_waves(STREAM, UNAL, STAGED);
+};
+
 // Workgroups of the multi-wave kernel that one compute unit holds at a time (LDS and registers).
 template <class Op, int R, bool STREAM, bool UNAL = false>
 int duo_groups_per_cu() {
     static const int n = [] {
+        constexpr int NC = CopyWavesOf<Op, STREAM, UNAL, false>::value;
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, stream_kernel_duo<Op, R, STREAM, CopyWaves<Op>::value, kTileSamples, UNAL>,
-                                                         (1 + CopyWaves<Op>::value) * kWave, 0) != hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, stream_kernel_duo<Op, R, STREAM, NC, kTileSamples, UNAL>,
+                                                         (1 + NC) * kWave, 0) != hipSuccess)
             v = 0;
         return v;
     }();
@@ -1307,7 +1350,7 @@ template <class Op, int R, bool STREAM, bool UNAL = false>
 unsigned duo_pad_when_large() {
     static const unsigned pad = [] {
         hipFuncAttributes a;
-        if (hipFuncGetAttributes(&a, (const void*)stream_kernel_duo<Op, R, STREAM, CopyWaves<Op>::value, kTileSamples, UNAL>) != hipSuccess)
+        if (hipFuncGetAttributes(&a, (const void*)stream_kernel_duo<Op, R, STREAM, CopyWavesOf<Op, STREAM, UNAL, false>::value, kTileSamples, UNAL>) != hipSuccess)
             return 0u;
         return lds_pad_for(kGroupsPerCuWhenLarge, a.sharedSizeBytes);
     }();
@@ -1324,9 +1367,10 @@ struct StageCount<Op, decltype((void)Op::kStages)> { static constexpr int value 
 template <class Op, bool STREAM, bool UNAL = false>
 int staged_groups_per_cu() {
     static const int n = [] {
+        constexpr int NC = CopyWavesOf<Op, STREAM, UNAL, true>::value;
         int v = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, stream_kernel_staged<Op, 64, STREAM, CopyWaves<Op>::value, UNAL>,
-                                                         (2 + CopyWaves<Op>::value) * kWave, 0) != hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, stream_kernel_staged<Op, 64, STREAM, NC, UNAL>, (2 + NC) * kWave,
+                                                         0) != hipSuccess)
             v = 0;
         return v;
     }();
@@ -1347,7 +1391,7 @@ template <class Op, bool STREAM, bool UNAL = false>
 unsigned staged_pad_when_large() {
     static const unsigned pad = [] {
         hipFuncAttributes a;
-        if (hipFuncGetAttributes(&a, (const void*)stream_kernel_staged<Op, 64, STREAM, CopyWaves<Op>::value, UNAL>) != hipSuccess)
+        if (hipFuncGetAttributes(&a, (const void*)stream_kernel_staged<Op, 64, STREAM, CopyWavesOf<Op, STREAM, UNAL, true>::value, UNAL>) != hipSuccess)
             return 0u;
         return lds_pad_for(kStagedGroupsPerCuWhenLarge, a.sharedSizeBytes);
     }();
@@ -1364,8 +1408,8 @@ constexpr int64_t kUnalignedMinSteps = 256;
 
 template <class Op, bool STREAM>
 int launch_stream_unaligned(const typename Op::Params& prm, int64_t M, int64_t T, hipStream_t stream) {
-    constexpr int NC = CopyWaves<Op>::value;
     if constexpr (StageCount<Op>::value == 2) {
+        constexpr int NC = CopyWavesOf<Op, STREAM, true, true>::value;
         const int per_cu = staged_groups_per_cu<Op, STREAM, true>();
         const bool fits = (M + 63) / 64 <= (int64_t)per_cu * compute_units();
         if (per_cu > 0 && (fits || StagedWhenLarge<Op>::value)) {
@@ -1376,6 +1420,7 @@ int launch_stream_unaligned(const typename Op::Params& prm, int64_t M, int64_t T
         }
     }
     constexpr int RD = DuoRows<Op>::value;
+    constexpr int NC = CopyWavesOf<Op, STREAM, true, false>::value;
     const int64_t groups = (M + RD - 1) / RD;
     const bool resident = groups <= (int64_t)duo_groups_per_cu<Op, RD, STREAM, true>() * compute_units();
     const dim3 grid((unsigned)groups), block((1 + NC) * kWave);
@@ -1397,14 +1442,14 @@ int launch_stream(const typename Op::Params& prm, int64_t M, int64_t T, hipStrea
         const int per_cu = streaming ? staged_groups_per_cu<Op, true>() : staged_groups_per_cu<Op, false>();
         const bool fits = (M + 63) / 64 <= (int64_t)per_cu * compute_units();
         if (vec && per_cu > 0 && (fits || (StagedWhenLarge<Op>::value && !long_pieces && T >= kMultiwaveWhenLargeMinSteps))) {
-            constexpr int NC = CopyWaves<Op>::value;
-            const dim3 grid((unsigned)((M + 63) / 64)), block((2 + NC) * kWave);
+            constexpr int NL = CopyWavesOf<Op, true, false, true>::value, NS = CopyWavesOf<Op, false, false, true>::value;
+            const dim3 grid((unsigned)((M + 63) / 64));
             if (streaming) {
                 const unsigned pad = fits ? 0u : staged_pad_when_large<Op, true>();
-                hipLaunchKernelGGL((stream_kernel_staged<Op, 64, true, NC>), grid, block, pad, stream, prm, M, (int)T);
+                hipLaunchKernelGGL((stream_kernel_staged<Op, 64, true, NL>), grid, dim3((2 + NL) * kWave), pad, stream, prm, M, (int)T);
             } else {
                 const unsigned pad = fits ? 0u : staged_pad_when_large<Op, false>();
-                hipLaunchKernelGGL((stream_kernel_staged<Op, 64, false, NC>), grid, block, pad, stream, prm, M, (int)T);
+                hipLaunchKernelGGL((stream_kernel_staged<Op, 64, false, NS>), grid, dim3((2 + NS) * kWave), pad, stream, prm, M, (int)T);
             }
             return (int)hipGetLastError();
         }
@@ -1412,14 +1457,14 @@ int launch_stream(const typename Op::Params& prm, int64_t M, int64_t T, hipStrea
     const bool resident = stream_fits_multiwave<Op>(prm, M, T);
     if (resident || (vec && MultiwaveWhenLarge<Op>::value && !long_pieces && T >= kMultiwaveWhenLargeMinSteps)) {
         constexpr int RD = DuoRows<Op>::value;
-        constexpr int NC = CopyWaves<Op>::value;
-        const dim3 grid((unsigned)((M + RD - 1) / RD)), block((1 + NC) * kWave);
+        constexpr int NL = CopyWavesOf<Op, true, false, false>::value, NS = CopyWavesOf<Op, false, false, false>::value;
+        const dim3 grid((unsigned)((M + RD - 1) / RD));
         if (streaming) {
             const unsigned pad = resident ? 0u : duo_pad_when_large<Op, RD, true>();
-            hipLaunchKernelGGL((stream_kernel_duo<Op, RD, true, NC>), grid, block, pad, stream, prm, M, (int)T);
+            hipLaunchKernelGGL((stream_kernel_duo<Op, RD, true, NL>), grid, dim3((1 + NL) * kWave), pad, stream, prm, M, (int)T);
         } else {
             const unsigned pad = resident ? 0u : duo_pad_when_large<Op, RD, false>();
-            hipLaunchKernelGGL((stream_kernel_duo<Op, RD, false, NC>), grid, block, pad, stream, prm, M, (int)T);
+            hipLaunchKernelGGL((stream_kernel_duo<Op, RD, false, NS>), grid, dim3((1 + NS) * kWave), pad, stream, prm, M, (int)T);
         }
         return (int)hipGetLastError();
     }
