@@ -600,6 +600,16 @@ int slayer_recurrent_steps_bwd(float *grad_z, const float *grad_spikes, const fl
                                int64_t N, int64_t C, int64_t T,
                                float *workspace, int64_t workspace_floats, void *stream);
 
+/* ---- weight quantiser ------------------------------------------------------------------------- */
+
+/* out = clamp(rint(in / step) * step, lo, hi) * scale (utils/quantize.py:84-115), a NaN stays one; the division is the
+ * multiplication by the float32 reciprocal of step.  inside[i] (or NULL): whether the rounded value lies in [lo, hi]. */
+int slayer_quantize(float *out, unsigned char *inside, const float *in, float step, float lo, float hi, float scale,
+                    int64_t n, void *stream);
+/* grad_in = inside ? grad_out * scale : 0 */
+int slayer_quantize_bwd(float *grad_in, const float *grad_out, const unsigned char *inside, float scale, int64_t n,
+                        void *stream);
+
 /* ---- cross-check implementations (debug mode) ------------------------------------------------ */
 
 /* The reference's debug mode runs its CPU loop next to its kernel and raises on a difference

@@ -1,0 +1,52 @@
+// Weight quantiser of the synapse layers (utils/quantize.py:84-115 in the reference): round to a multiple of `step`, limit to
+// [lo, hi], scale; backward the gradient of the weights inside the limits.  One launch each way for what the element-wise
+// operators take four and five for (some 4 us apiece on weights of any usual size: nothing but the launches), operation by
+// operation the same: the division is the multiplication by the reciprocal the operator makes of it.
+#include "common.h"
+
+namespace slayer {
+
+__global__ __launch_bounds__(256) void quantize_kernel(float* __restrict__ out, unsigned char* __restrict__ inside,
+                                                       const float* __restrict__ in, float inv_step, float step, float lo,
+                                                       float hi, float scale, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float q = rintf(in[i] * inv_step) * step;
+    if (inside) inside[i] = q >= lo && q <= hi;
+    out[i] = (q != q ? q : fminf(fmaxf(q, lo), hi)) * scale;
+}
+
+__global__ __launch_bounds__(256) void quantize_bwd_kernel(float* __restrict__ grad_in, const float* __restrict__ grad_out,
+                                                           const unsigned char* __restrict__ inside, float scale, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) grad_in[i] = inside[i] ? grad_out[i] * scale : 0.f;
+}
+
+}  // namespace slayer
+
+using namespace slayer;
+
+namespace {
+int check_count(int64_t n) { return n < 0 ? SLAYER_EINVAL : (n > ((int64_t)1 << 38) ? SLAYER_ERANGE : 0); }
+}  // namespace
+
+extern "C" int slayer_quantize(float* out, unsigned char* inside, const float* in, float step, float lo, float hi, float scale,
+                               int64_t n, void* stream) {
+    if (int e = check_count(n)) return e;
+    if (step == 0.0f) return SLAYER_EINVAL;
+    if (n == 0) return 0;
+    if (!out || !in) return SLAYER_ENULL;
+    hipLaunchKernelGGL(quantize_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, out, inside, in,
+                       1.0f / step, step, lo, hi, scale, n);
+    return (int)hipGetLastError();
+}
+
+extern "C" int slayer_quantize_bwd(float* grad_in, const float* grad_out, const unsigned char* inside, float scale, int64_t n,
+                                   void* stream) {
+    if (int e = check_count(n)) return e;
+    if (n == 0) return 0;
+    if (!grad_in || !grad_out || !inside) return SLAYER_ENULL;
+    hipLaunchKernelGGL(quantize_bwd_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, grad_in,
+                       grad_out, inside, scale, n);
+    return (int)hipGetLastError();
+}

@@ -9,7 +9,7 @@ constants, and the hardware view of the parameters (cx_* integers, device_params
 import numpy as np
 import torch
 
-from ..utils.quantize import quantize
+from ..utils.quantize import limit, quantize
 
 P_SCALE = 1 << 12      # decays are stored as 12-bit integers
 
@@ -72,8 +72,7 @@ class Neuron(torch.nn.Module):
     def quantize_8bit(self, weight, descale=False):
         """Weight quantiser to link with a synapse (``synapse.pre_hook_fx = neuron.quantize_8bit``):
         steps of 2 / scale, clamped to the 8-bit range; ``descale`` returns integers."""
-        q = quantize(weight, step=2 / self.w_scale).clamp(-256 / self.w_scale, 254 / self.w_scale)
-        return q * self.w_scale if descale else q
+        return limit(weight, 2 / self.w_scale, -256 / self.w_scale, 254 / self.w_scale, self.w_scale if descale else 1)
 
     # --------------------------------------------------------------- hardware view
     @property

@@ -1,6 +1,6 @@
 from . import time, filter, int_utils, recurrent
 from .int_utils import right_shift_to_zero
-from .quantize import quantize, quantize_hook_fx, MODE
+from .quantize import limit, quantize, quantize_hook_fx, MODE
 from .quantize import MODE as QUANTIZE_MODE
 from .utils import staticproperty, diagonal_mask, event_rate, dotdict
 

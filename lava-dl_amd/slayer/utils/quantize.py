@@ -2,6 +2,9 @@
 from enum import IntEnum, unique
 
 import torch
+from torch.autograd import forward_ad
+
+from .. import _native as N
 
 
 @unique
@@ -33,10 +36,58 @@ def quantize(input, step=1, mode=MODE.ROUND):
     return _StraightThrough.apply(input, step, mode == MODE.FLOOR)
 
 
+class _Limited(torch.autograd.Function):
+    """limit() in one launch each way (slayer_quantize)."""
+
+    @staticmethod
+    def forward(ctx, input, step, lo, hi, scale):
+        inside = torch.empty(input.shape, dtype=torch.bool, device=input.device)
+        ctx.save_for_backward(inside)
+        ctx.scale = scale
+        return _launch(input, step, lo, hi, scale, inside)
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        inside, = ctx.saved_tensors
+        if torch.is_grad_enabled() or grad_output.dtype != torch.float32:          # create_graph=True
+            return torch.where(inside, grad_output * ctx.scale, 0.0), None, None, None, None
+        grad_output = grad_output.contiguous()
+        grad = torch.empty_like(grad_output)
+        with N.device_guard(grad.device):
+            N.check(N.lib().slayer_quantize_bwd(N.ptr(grad), N.ptr(grad_output), N.ptr(inside), ctx.scale, grad.numel(),
+                                                N.stream_handle()))
+        return grad, None, None, None, None
+
+
+def _launch(input, step, lo, hi, scale, inside):
+    out = torch.empty_like(input)
+    with N.device_guard(out.device):
+        N.check(N.lib().slayer_quantize(N.ptr(out), N.ptr(inside), N.ptr(input), step, lo, hi, scale, out.numel(),
+                                        N.stream_handle()))
+    return out
+
+
+def _takes_kernel(input):
+    """float32 weights on the GPU as they lie in memory, and nobody who wants to see the single operations: tracing,
+    compilation, function transforms, forward-mode differentiation."""
+    return (type(input) in (torch.Tensor, torch.nn.Parameter) and input.is_cuda and input.dtype == torch.float32
+            and input.is_contiguous() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0)
+
+
+def limit(input, step, lo, hi, scale=1):
+    """``quantize(input, step).clamp(lo, hi) * scale``."""
+    if not _takes_kernel(input):
+        q = quantize(input, step=step).clamp(lo, hi)
+        return q if scale == 1 else q * scale
+    if torch.is_grad_enabled() and input.requires_grad:
+        return _Limited.apply(input, float(step), float(lo), float(hi), float(scale))
+    return _launch(input, float(step), float(lo), float(hi), float(scale), None)
+
+
 def quantize_hook_fx(x, scale=1 << 6, num_bits=8, descale=False):
     """Synapse pre-hook quantiser (utils/quantize.py:84-115 in the reference): even multiples of
     1 / scale, limited to the signed ``num_bits`` weight range; ``descale`` returns integers."""
     lo = -2 * (1 << num_bits) / scale
     hi = 2 * ((1 << num_bits) - 1) / scale
-    q = quantize(x, step=2 / scale).clamp(lo, hi)
-    return q * scale if descale else q
+    return limit(x, 2 / scale, lo, hi, scale if descale else 1)

@@ -1,0 +1,68 @@
+"""The weight quantiser's one launch (csrc/quantize.hip) against the operators it stands for, bit for bit."""
+import pytest
+import torch
+
+from tests.util import dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def slayer():
+    import lava_dl_amd.slayer as s
+    return s
+
+
+def _chain(slayer, x, step, lo, hi, scale):
+    q = slayer.utils.quantize(x, step=step).clamp(lo, hi)
+    return q if scale == 1 else q * scale
+
+
+# powers of two and scales whose step and reciprocal are rounded; ties, both limits, infinities, NaN, negative zero
+@pytest.mark.parametrize('scale', [64, 1, 50, 3.7])
+@pytest.mark.parametrize('descale', [False, True])
+@pytest.mark.parametrize('shape', [(1,), (257,), (16, 8, 3, 3, 1)])
+def test_quantizer_is_the_chain_of_operators(slayer, scale, descale, shape):
+    gen = torch.Generator().manual_seed(int(scale * 10) + len(shape))
+    x = torch.randn(shape, generator=gen) * 3 * 64 / scale
+    flat = x.view(-1)
+    special = [0.5 * 2 / scale, 1.5 * 2 / scale, -0.3 / scale, 254 / scale, 255 / scale, 256 / scale, -256 / scale, -257 / scale,
+               float('inf'), float('-inf'), float('nan'), 1e-40]
+    flat[:min(len(special), flat.numel())] = torch.tensor(special)[:flat.numel()]
+    g = torch.randn(shape, generator=gen).to(dev())
+    results = []
+    for fused in (True, False):
+        xg = x.to(dev()).requires_grad_()
+        args = (xg, 2 / scale, -256 / scale, 254 / scale, scale if descale else 1)
+        out = slayer.utils.limit(*args) if fused else _chain(slayer, *args)
+        grad, = torch.autograd.grad(out, xg, g)
+        with torch.no_grad():
+            plain = slayer.utils.limit(*args) if fused else _chain(slayer, *args)
+        results.append([t.detach().cpu().view(torch.int32) for t in (out, grad, plain)])
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+def test_calls_that_keep_the_operators(slayer):
+    """Layouts, types and devices the kernel does not take, and users of the single operations."""
+    limit = slayer.utils.limit
+    gen = torch.Generator().manual_seed(1)
+    w = torch.randn(6, 10, generator=gen).to(dev())
+    args = (2 / 64, -4.0, 254 / 64)
+    want = _chain(slayer, w, *args, 1)
+    assert torch.equal(limit(w.t(), *args), want.t())
+    assert torch.equal(limit(w.cpu(), *args), want.cpu())
+    assert limit(w.double(), *args).dtype == torch.float64
+    assert limit(w[:0], *args).shape == (0, 10)
+    assert torch.equal(torch.func.vmap(lambda r: limit(r, *args))(w), want)
+    assert torch.equal(torch.jit.trace(lambda r: limit(r, *args), (w,))(w + 1), _chain(slayer, w + 1, *args, 1))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(w, torch.ones_like(w))
+        limit(dual, *args)
+    x = w.clone().requires_grad_()
+    grad, = torch.autograd.grad((limit(x, *args) ** 2).sum(), x, create_graph=True)
+    second, = torch.autograd.grad(grad.sum(), x)
+    y = w.clone().requires_grad_()
+    grad_y, = torch.autograd.grad((_chain(slayer, y, *args, 1) ** 2).sum(), y, create_graph=True)
+    second_y, = torch.autograd.grad(grad_y.sum(), y)
+    assert torch.equal(grad, grad_y) and torch.equal(second, second_y)
