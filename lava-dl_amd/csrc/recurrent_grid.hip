@@ -77,9 +77,9 @@ struct GridFwd {
 // words of one sample tile, [KB][16 samples], whole units
 __host__ __device__ inline int words_of(int KB) { return (KB + 7) / 8 * 8 * 16; }
 
-__global__ __launch_bounds__(256) void grid_fill_kernel(unsigned* dst, int64_t n, unsigned value, unsigned* gave_up) {
+__global__ __launch_bounds__(256) void grid_fill_kernel(unsigned* dst, int64_t n, unsigned* gave_up) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = value;
+    if (i < n) dst[i] = 0u;
     if (i == 0) *gave_up = 0u;
 }
 
@@ -366,10 +366,10 @@ __global__ __launch_bounds__(kSoloThreads) void recurrent_solo_fwd_kernel(const 
             const int c = threadIdx.x + i * kSoloThreads;
             if (c >= C) continue;
             const int64_t m = (int64_t)blockIdx.x * C + c, at = m * T + t;
-            float fb = 0.f;
+            double fb = 0.0;                         // one sum after the other: float32 would lose to the sums of the matrix cores
             if (t > 0)
-                for (int k = 0; k < C; ++k) fb += g.rec[(int64_t)c * C + k] * spikes[(t - 1) & 1][k];
-            const StepValues o = nrn[i].step(g.z[at] + fb, p);
+                for (int k = 0; k < C; ++k) fb += (double)g.rec[(int64_t)c * C + k] * (double)spikes[(t - 1) & 1][k];
+            const StepValues o = nrn[i].step(g.z[at] + (float)fb, p);
             spikes[t & 1][c] = o.spike;
             g.spk[at] = o.spike;
             g.vol[at] = o.voltage;
@@ -411,7 +411,30 @@ struct GridBwd {
     GridMap map;
     int KB, S, N, C, T, graded;
     float spike_thr, tau, rho;
+    // groups of four samples and workgroups of 64 neurons to a group (0: not for these sizes), see grid_bwd_local; what
+    // the blocks of grid_bwd_fill_kernel found
+    int groups4, tiles64;
+    const unsigned* inexact;                         // [kFillBlocks]
 };
+constexpr int kFillBlocks = 256;
+constexpr float kLocalScale = 0x1p24f;               // small gradients keep their bits
+constexpr float kLocalLargest = 0x1p85f;             // beyond it a scaled sum could leave the range
+
+// Clears the ring, and looks whether every weight is a bfloat16 number of a size that leaves room for the scale.
+__global__ __launch_bounds__(1024) void grid_bwd_fill_kernel(unsigned* ring, int64_t n, unsigned* gave_up, const float* rec,
+                                                             int64_t weights, unsigned* inexact) {
+    const int64_t first = (int64_t)blockIdx.x * 1024 + threadIdx.x, stride = (int64_t)kFillBlocks * 1024;
+    for (int64_t i = first; i < n; i += stride) ring[i] = kUnwritten;
+    bool bad = false;
+#pragma unroll 8
+    for (int64_t i = first; i < weights; i += stride) {
+        const float w = rec[i], size = fabsf(w);
+        bad = bad || (__float_as_uint(w) & 0xffffu) != 0u || !(size <= 256.0f) || (size != 0.0f && size < 0x1p-40f);
+    }
+    const int any = __syncthreads_or(bad);
+    if (threadIdx.x == 0) inexact[blockIdx.x] = any ? 1u : 0u;
+    if (first == 0) *gave_up = 0u;
+}
 
 __device__ __forceinline__ float surrogate_factor(const GridBwd& p, float v, float th) {
     const float lead = (p.rho / 2.0f) / p.tau, inv_tau = 1.0f / p.tau;
@@ -419,20 +442,233 @@ __device__ __forceinline__ float surrogate_factor(const GridBwd& p, float v, flo
     return p.graded ? p.rho * expf(fminf(d, 0.0f) * inv_tau) : lead * expf(-fabsf(d) * inv_tau);
 }
 
+__device__ __forceinline__ float quad_swapped(float x) {         // that of the other lane of the pair
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xb1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ unsigned quad_swapped(unsigned x) { return (unsigned)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true); }
+__device__ __forceinline__ float quad_third(float x) {           // that of the third lane of the quad
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xaa, 0xf, 0xf, true));
+}
+
+// Weights that are bfloat16 numbers (8-bit quantisers): half the bytes, so a workgroup holds 64 columns of R, and the
+// 32 workgroups that cover 2048 neurons are one XCD -- a group of four samples stays on one XCD, whose L2 is all a step
+// crosses.  The gradients travel as three bfloat16 parts of 8 bits (cut: 24 bits, nothing is rounded) and the parts are
+// columns of the product: column 4 s + q of the B operand is part q of sample s, so one product per 16 rows of weights and
+// 32 k does all three (column 4 s + 3 is never written and never looked at).  [32, 2048, 300] 1 751 -> 1 170 us: of a
+// step's 3.7 us the way of the gradients across the XCD takes 2.3, the products 0.4, the sum over the waves, the neuron
+// and the barriers 1.0.
+//   ring: [4][groups4][2 tiles64 blocks of 32 k][64 lanes][8 bfloat16]; thread (wave v, lane) of the first four waves has
+// sample v of the group and neuron `lane` of the tile.
+template <bool THETA, int U>
+__device__ __forceinline__ void grid_bwd_local(const GridBwd& p, float (*red)[kGridWaves][4 * 68], float* gbuf, float* fbuf,
+                                               float* obuf, int* dead) {
+    const int C = p.C, N = p.N, T = p.T, W = p.tiles64, blocks = 2 * W;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kk = lane >> 4, j = lane & 15, part = j & 3;
+    const int group = (blockIdx.x & 7) + 8 * ((blockIdx.x >> 3) / W), P = (blockIdx.x >> 3) % W, c0 = 64 * P;
+    if (group >= p.groups4) return;
+
+    uint4 w[U][4];                                   // columns c0 + 16 r + j, rows 32 b + 8 kk .. + 7 of block b = wave + 8 u
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        asm volatile("" ::: "memory");               // a block's loads at a time: all of them at once would not fit the registers
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int c = c0 + 16 * r + j, k = 32 * (wave + kGridWaves * u) + 8 * kk;
+            unsigned h[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) h[e] = (c < C && k + e < C) ? __float_as_uint(p.rec[(int64_t)(k + e) * C + c]) : 0u;
+            w[u][r] = make_uint4(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u), __builtin_amdgcn_perm(h[3], h[2], 0x07060302u),
+                                 __builtin_amdgcn_perm(h[5], h[4], 0x07060302u), __builtin_amdgcn_perm(h[7], h[6], 0x07060302u));
+        }
+    }
+    const __amdgpu_buffer_rsrc_t ring = make_rsrc(reinterpret_cast<const float*>(p.ring), 4u * p.groups4 * blocks * 1024u);
+    const int64_t per_set = (int64_t)p.groups4 * blocks * 256;                        // words
+    // this thread's word of part (lane & 1); that of the third part, which the even lanes write, is part 2
+    unsigned* mine = p.ring + ((int64_t)group * blocks + 2 * P + (lane >> 5)) * 256 +
+                     (((lane >> 3) & 3) * 16 + 4 * (wave & 3)) * 4 + ((lane & 7) >> 1);
+    const int own = (lane & 1) * 4, third = 2 * 4;
+
+    // staging: all eight waves, a sample and 32 of its rows each (sixteen rows more in registers would not fit beside the
+    // weights); access q covers neurons first + 4 q .. first + 4 q + 3
+    const int n = 4 * group + (wave & 3), first_row = 32 * (wave >> 2);
+    const unsigned lane_at = (unsigned)kk * (unsigned)T + (unsigned)j;
+    auto row_ok = [&](int q) -> bool { return n < N && c0 + first_row + 4 * q < C; };
+    auto next_rows = [&](int64_t& at) {
+        at += 4 * (int64_t)T;
+        asm volatile("" : "+s"(at));
+    };
+    float gn[8], vn[8], tn[THETA ? 8 : 1];
+    auto fetch = [&](int t0) {
+        int64_t at = ((int64_t)n * C + c0 + first_row) * T + t0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q, next_rows(at)) {
+            const bool ok = row_ok(q) && t0 + j < T;
+            gn[q] = ok ? (p.g + at)[lane_at] : 0.f;
+            vn[q] = ok ? (p.v + at)[lane_at] : 0.f;
+            if (THETA) tn[q] = ok ? (p.theta + at)[lane_at] : 0.f;
+        }
+    };
+    const int rows_of = (wave & 3) * kWave * kGridPitch;         // this wave's sample in the buffers
+    float *gb = gbuf + rows_of, *fb = fbuf + rows_of, *ob = obuf + rows_of;
+    auto put = [&]() {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            gb[(first_row + 4 * q + kk) * kGridPitch + j] = gn[q];
+            fb[(first_row + 4 * q + kk) * kGridPitch + j] =
+                row_ok(q) ? surrogate_factor(p, vn[q], THETA ? tn[q] : p.spike_thr) : 0.f;
+        }
+    };
+    const int t_last = (T - 1) / kGridChunk * kGridChunk;
+    fetch(t_last);
+    put();
+    lds_barrier();
+
+    bool stop = false;
+    int patience = kSpinLimit;                       // polls of a wait; none once one of this wave's has run out
+    for (int t0 = t_last; t0 >= 0 && !stop; t0 -= kGridChunk) {
+        if (t0 > 0) fetch(t0 - kGridChunk);
+        const int steps = T - t0 < kGridChunk ? T - t0 : kGridChunk;
+        for (int e = steps - 1; e >= 0; --e) {
+            const int t = t0 + e, sel = t & 1;
+            float gs = 0.f, factor = 0.f;
+            if (wave < 4) {
+                gs = gb[lane * kGridPitch + e];
+                factor = fb[lane * kGridPitch + e];
+                if (t + 3 < T) {
+                    unsigned* at = mine + ((t + 3) & 3) * per_set;
+                    __hip_atomic_store(at + own, kUnwritten, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if ((lane & 1) == 0) __hip_atomic_store(at + third, kUnwritten, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            if (t + 1 < T) {
+                const int base = (((t + 1) & 3) * p.groups4 + group) * blocks * 1024 + lane * 16;
+                auto load = [&](int u) -> v4u {
+                    return __builtin_amdgcn_raw_buffer_load_b128(ring, base + (wave + kGridWaves * u) * 1024, 0, 16);
+                };
+                auto late = [&](v4u q) -> bool {
+                    const unsigned m = max(max(max(q.x, q.y), q.z), q.w);        // kUnwritten is the largest word
+                    return __any(part != 3 && m == kUnwritten);
+                };
+                v4u a[U];
+                int spin = patience;
+                auto wait = [&](int u) {
+                    while (late(a[u])) {
+                        if (spin == 0 || ((spin & 1023) == 1 &&
+                                          __hip_atomic_load(p.gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u)) {
+                            dead[(t0 / kGridChunk) & 1] = 1;
+                            patience = spin = 0;
+                            break;
+                        }
+                        --spin;
+                        asm volatile("" ::: "memory");
+                        a[u] = load(u);
+                    }
+                };
+                // Eight blocks are requested at once ([32, 2048, 300] 1 170 us, one polled first and the others behind it 1 250),
+                // fewer behind the first ([64, 1024, 100], whole layer 674 us, all at once 754).
+                if (U < 8 && wave < blocks) { a[0] = load(0); wait(0); }
+#pragma unroll
+                for (int u = U < 8 ? 1 : 0; u < U; ++u)
+                    if (wave + kGridWaves * u < blocks) a[u] = load(u);
+                split_f4 acc[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[r] = split_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (wave + kGridWaves * u >= blocks) continue;
+                    if (U >= 8 || u > 0) wait(u);
+                    const uint4 b = make_uint4(a[u].x, a[u].y, a[u].z, a[u].w);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[r] = mfma_bf16(w[u][r], b, acc[r]);
+                }
+                // the three parts added up in the first two lanes of a quad, which keep two of the four row tiles each
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float x = acc[r][i];
+                        x = (x + quad_swapped(x)) + quad_third(x);
+                        asm volatile("" : "+v"(x));              // not moved behind the branch, so that the lanes are part of the addition
+                        acc[r][i] = x;
+                    }
+                if (part < 2) {
+                    float* at = &red[sel][wave][(j >> 2) * 68 + part * 32 + 4 * kk];
+                    const split_f4 first = part == 0 ? acc[0] : acc[2], second = part == 0 ? acc[1] : acc[3];
+                    *reinterpret_cast<float4*>(at) = make_float4(first[0], first[1], first[2], first[3]);
+                    *reinterpret_cast<float4*>(at + 16) = make_float4(second[0], second[1], second[2], second[3]);
+                }
+            }
+            lds_barrier();
+            if (wave < 4) {
+                if (t + 1 < T) {
+                    float from[kGridWaves], carry = 0.f;
+#pragma unroll
+                    for (int v = 0; v < kGridWaves; ++v) from[v] = red[sel][v][wave * 68 + lane];
+                    __builtin_amdgcn_sched_barrier(0);           // all eight under way before the first is waited for
+#pragma unroll
+                    for (int v = 0; v < kGridWaves; ++v) carry += from[v];
+                    gs = carry * (1.0f / kLocalScale) + gs;
+                }
+                const float gz = factor * gs;
+                if (t > 0) {
+                    // this neuron's parts, those of the pair's other neuron, and the words of both
+                    const float x = gz * kLocalScale, size = fabsf(gz);
+                    const unsigned bits = __float_as_uint(x);
+                    unsigned h = bits & 0xffff0000u;
+                    const float left = x - __uint_as_float(h);
+                    unsigned m = __float_as_uint(left) & 0xffff0000u, l = __float_as_uint(left - __uint_as_float(m));
+                    if (!(fabsf(x) <= 3.402823466e38f)) {        // infinities and NaN have no rest
+                        h = x != x ? 0x7fc00000u : h;
+                        m = l = 0u;
+                    }
+                    const unsigned sent = (lane & 1) ? h : m, got = quad_swapped(sent), l_odd = quad_swapped(l);
+                    const unsigned first = (lane & 1) ? __builtin_amdgcn_perm(m, got, 0x07060302u)
+                                                      : __builtin_amdgcn_perm(got, h, 0x07060302u);
+                    unsigned* at = mine + (t & 3) * per_set;
+                    __builtin_amdgcn_s_waitcnt(0x0f70);          // vmcnt(0): the clearing stores have arrived
+                    __hip_atomic_store(at + own, first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if ((lane & 1) == 0)
+                        __hip_atomic_store(at + third, __builtin_amdgcn_perm(l_odd, l, 0x07060302u), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+                    if (size >= kLocalLargest && size <= 3.402823466e38f) dead[(t0 / kGridChunk) & 1] = 1;      // left to the kernel behind
+                }
+                ob[lane * kGridPitch + e] = gz;
+            }
+            lds_barrier();                                       // see the forward kernel
+        }
+        int64_t at = ((int64_t)n * C + c0 + first_row) * T + t0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q, next_rows(at))
+            if (row_ok(q) && j < steps) (p.gz + at)[lane_at] = ob[(first_row + 4 * q + kk) * kGridPitch + j];
+        if (t0 > 0) put();
+        lds_barrier();
+        stop = dead[(t0 / kGridChunk) & 1] != 0;                 // looked at once a chunk: the next step does not wait for it
+    }
+    if (stop && tid == 0) __hip_atomic_store(p.gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Thread (wave v, lane 4 j + i) of the first four waves has neuron 4 v + i of the tile and sample j.
 template <bool THETA, int U, int NT>
 __global__ __launch_bounds__(kGridThreads) void recurrent_grid_bwd_kernel(const GridBwd p) {
     constexpr int kPlane = 80;                       // pitch of a plane of red: reads of a wave meet 64 banks
-    __shared__ float red[2][kGridWaves][4][kPlane];
+    __shared__ __attribute__((aligned(16))) float red[2][kGridWaves][4][kPlane];
     __shared__ float gbuf[NT][4][kWave * kGridPitch], fbuf[NT][4][kWave * kGridPitch], obuf[NT][4][kWave * kGridPitch];
     __shared__ int dead[2];
     const int C = p.C, N = p.N, T = p.T, KB = p.KB;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid < 2) dead[tid] = 0;
+    if constexpr (NT == 1)
+        if (p.tiles64 > 0 && !__syncthreads_or(tid < kFillBlocks && p.inexact[tid] != 0u)) {
+            grid_bwd_local<THETA, U / 2>(p, reinterpret_cast<float (*)[kGridWaves][4 * 68]>(&red[0][0][0][0]), gbuf[0][0], fbuf[0][0],
+                                         obuf[0][0], dead);
+            return;
+        }
     const int kk = lane >> 4, j = lane & 15;
     const int P = p.map.tile(blockIdx.x), c0 = P * 16, group = p.map.group(blockIdx.x);
     if (P >= KB || group * NT >= p.S) return;
-    if (tid < 2) dead[tid] = 0;
 
     // columns c0 .. c0 + 15 of R as A operands: lane (kk, j) has rows 16 kb + 4 kk .. + 3 of column c0 + j
     float4 w[U];
@@ -591,10 +827,10 @@ __global__ __launch_bounds__(kSoloThreads) void recurrent_solo_bwd_kernel(const 
     for (int t = p.T - 1; t >= 0; --t) {
         for (int c = threadIdx.x; c < p.C; c += kSoloThreads) {
             const int64_t at = ((int64_t)blockIdx.x * p.C + c) * p.T + t;
-            float carry = 0.f;
+            double carry = 0.0;
             if (t + 1 < p.T)
-                for (int k = 0; k < p.C; ++k) carry += next[(t + 1) & 1][k] * p.rec[(int64_t)k * p.C + c];
-            const float gz = surrogate_factor(p, p.v[at], p.theta ? p.theta[at] : p.spike_thr) * (carry + p.g[at]);
+                for (int k = 0; k < p.C; ++k) carry += (double)next[(t + 1) & 1][k] * (double)p.rec[(int64_t)k * p.C + c];
+            const float gz = surrogate_factor(p, p.v[at], p.theta ? p.theta[at] : p.spike_thr) * ((float)carry + p.g[at]);
             next[t & 1][c] = gz;
             p.gz[at] = gz;
         }
@@ -608,6 +844,7 @@ struct GridPlan {
     int KB, S, NT;
     GridMap map;
     unsigned grid;
+    int compute_units;
 };
 
 // One workgroup per compute unit: 16 neurons by one or two sample tiles.  A handful of steps costs more as a
@@ -632,6 +869,7 @@ bool grid_plan(int64_t N, int64_t C, int64_t T, hipStream_t st, GridPlan* plan) 
             plan->KB = (int)KB; plan->S = (int)(groups * nt); plan->NT = nt;
             plan->map.xcds = xcds; plan->map.per_xcd = (int)per_xcd;
             plan->grid = (unsigned)(8 * per_xcd * rounds);
+            plan->compute_units = units;
             return true;
         }
     }
@@ -657,10 +895,6 @@ bool launch_grid_fwd(const GridFwd& g, const GridPlan& plan, hipStream_t st) {
     return true;
 }
 
-void launch_grid_fill(unsigned* dst, int64_t n, unsigned value, unsigned* gave_up, hipStream_t st) {
-    hipLaunchKernelGGL(grid_fill_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, dst, n, value, gave_up);
-}
-
 }  // namespace
 
 bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* theta, const float* z, const float* rec,
@@ -676,7 +910,7 @@ bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* th
     g.spk = spk; g.vol = vol; g.theta = theta; g.z = z; g.rec = rec;
     g.gave_up = reinterpret_cast<unsigned*>(workspace);
     g.words = reinterpret_cast<unsigned*>(workspace) + 4;
-    launch_grid_fill(g.words, words, 0u, g.gave_up, st);
+    hipLaunchKernelGGL(grid_fill_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, g.words, words, g.gave_up);
     const bool taken = alif ? (pow2 ? launch_grid_fwd<true, true>(g, plan, st) : launch_grid_fwd<true, false>(g, plan, st))
                             : (pow2 ? launch_grid_fwd<false, true>(g, plan, st) : launch_grid_fwd<false, false>(g, plan, st));
     if (taken) *error = (int)hipGetLastError();
@@ -697,19 +931,32 @@ bool grid_bwd(float* gz, const float* grad_spikes, const float* voltage, const f
               float* workspace, int64_t workspace_floats, hipStream_t st, int* error) {
     GridPlan plan;
     if (!grid_plan(N, C, T, st, &plan)) return false;
-    const int64_t ring = (int64_t)4 * plan.S * plan.KB * 256;
-    if (workspace_floats < ring + 4) return false;
+    int64_t ring = (int64_t)4 * plan.S * plan.KB * 256;
+    const int64_t head = 4 + kFillBlocks;
+    if (workspace_floats < ring + head) return false;
     GridBwd p{};
     p.gz = gz; p.g = grad_spikes; p.v = voltage; p.theta = theta; p.rec = rec;
     p.gave_up = reinterpret_cast<unsigned*>(workspace);
-    p.ring = reinterpret_cast<unsigned*>(workspace) + 4;
+    p.ring = reinterpret_cast<unsigned*>(workspace) + head;
     p.map = plan.map;
+    // four samples to an XCD, as long as the chip holds them all
+    const int64_t groups4 = (N + 3) / 4, tiles64 = (C + 63) / 64, rounds = (groups4 + 7) / 8;
+    const int64_t local_ring = (int64_t)4 * groups4 * 2 * tiles64 * 256;
+    unsigned grid = plan.grid;
+    if (plan.NT == 1 && 8 * rounds * tiles64 <= plan.compute_units && workspace_floats >= local_ring + head) {
+        p.groups4 = (int)groups4;
+        p.tiles64 = (int)tiles64;
+        if (grid < 8 * rounds * tiles64) grid = (unsigned)(8 * rounds * tiles64);
+        if (ring < local_ring) ring = local_ring;
+    }
+    unsigned* inexact = reinterpret_cast<unsigned*>(workspace) + 4;
+    p.inexact = inexact;
     p.KB = plan.KB; p.S = plan.S; p.N = (int)N; p.C = (int)C; p.T = (int)T; p.graded = graded;
     p.spike_thr = spike_thr; p.tau = tau; p.rho = rho;
-    launch_grid_fill(p.ring, ring, kUnwritten, p.gave_up, st);
+    hipLaunchKernelGGL(grid_bwd_fill_kernel, dim3(kFillBlocks), dim3(1024), 0, st, p.ring, ring, p.gave_up, rec, C * C, inexact);
     const void* k = theta ? (plan.NT == 1 ? grid_bwd_kernel<true, 1>(plan.KB) : grid_bwd_kernel<true, 2>(plan.KB))
                           : (plan.NT == 1 ? grid_bwd_kernel<false, 1>(plan.KB) : grid_bwd_kernel<false, 2>(plan.KB));
-    if (!launch_grid(k, plan.grid, (void*)&p, st)) return false;
+    if (!launch_grid(k, grid, (void*)&p, st)) return false;
     hipLaunchKernelGGL(recurrent_solo_bwd_kernel, dim3((unsigned)N), dim3(kSoloThreads), 0, st, p);
     *error = (int)hipGetLastError();
     return true;

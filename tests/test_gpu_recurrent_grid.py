@@ -80,6 +80,43 @@ def test_feedback_of_weights_off_the_grid(slayer, c):
         assert float(err) <= 5e-6, float(err)
 
 
+# 2048 neurons fill 32 workgroups of 64, 68 leave most of the second one empty; 33 samples of 1300 neurons do not fit the
+# form for weights that are bfloat16 numbers, [4 samples] x [64 neurons] a workgroup; 18 steps are two chunks
+@pytest.mark.parametrize('n,c,t', [(5, 68, 18), (32, 2048, 9), (33, 1300, 20), (7, 260, 33)])
+@pytest.mark.parametrize('weights,scale', [('grid', 1.0), ('grid', 1e-34), ('grid', 1e27), ('real', 1.0), ('real', 1e-34),
+                                           ('large', 1.0)])
+def test_gradients_of_weights_on_and_off_the_grid(slayer, n, c, t, weights, scale):
+    """The input gradient against a float64 evaluation, with weights that are bfloat16 numbers and others, among them one
+    too large for the first form; gradients near both ends of float32's range.  Both forms keep 24 bits of either factor and sum
+    in float32.  Bound: a step's float32 factor is off by the rounding of its exponent (of magnitude 2), of exp and of three
+    products, 6 x 2^-24, and what comes back through all t steps carries t of them: 4e-7 t of the largest magnitude.  The
+    surrogate's scale of 0.04 keeps a gradient from leaving float32 on its way (0.9 times a step without the large weight)."""
+    from lava_dl_amd.slayer import _native as N
+    gen = torch.Generator().manual_seed(c + n)
+    rec = torch.randn(c, c, generator=gen) * 3 / c ** 0.5
+    if weights != 'real':
+        rec = (rec * 32).round().clamp(-128, 127) / 32
+        if weights == 'large':
+            rec[c // 2, c // 3] = 1024.0
+    v = torch.randn(n, c, t, generator=gen) * 0.02 + 1.25
+    g = torch.randn(n, c, t, generator=gen) * scale
+    d = [x.to(dev()) for x in (g, v, rec)]
+    gz = torch.empty_like(d[0])
+    floats = N.lib().slayer_recurrent_steps_workspace(n, c, t, 0)
+    ws = torch.empty(floats, device=dev())
+    N.check(N.lib().slayer_recurrent_steps_bwd(N.ptr(gz), N.ptr(d[0]), N.ptr(d[1]), None, N.ptr(d[2]), 1.25, 0.05, 0.04, 0,
+                                               n, c, t, N.ptr(ws), floats, N.stream_handle()))
+    factor = (0.04 / 2 / 0.05) * torch.exp(-(v.double() - 1.25).abs() / 0.05)
+    want, carry = torch.empty_like(factor), torch.zeros(n, c, dtype=torch.float64)
+    for step in reversed(range(t)):
+        want[..., step] = factor[..., step] * (g[..., step].double() + carry)
+        carry = want[..., step] @ rec.double()
+    err = (gz.cpu().double() - want).abs()
+    if scale == 1e27:
+        assert bool((want.abs() > 4e25).any())
+    assert bool((err <= 4e-7 * t * want.abs().amax()).all()), float(err.max() / want.abs().max())
+
+
 def test_weights_that_are_not_finite(slayer, monkeypatch):
     """An infinite weight times a silent neuron is a NaN, and so is a NaN weight times any: what the two receiving neurons
     do is lost, the other neurons' feedback is untouched."""
