@@ -606,6 +606,9 @@ int slayer_recurrent_steps_bwd(float *grad_z, const float *grad_spikes, const fl
  * multiplication by the float32 reciprocal of step.  inside[i] (or NULL): whether the rounded value lies in [lo, hi]. */
 int slayer_quantize(float *out, unsigned char *inside, const float *in, float step, float lo, float hi, float scale,
                     int64_t n, void *stream);
+/* Rotation parameters of a resonate-and-fire neuron limited in place (neuron/rf.py:136-257): gain sqrt(sin^2 + cos^2) at most
+ * gain_max, sin at least 1, cos at least 0.  n: entries of either tensor. */
+int slayer_rf_limit(float *sin_decay, float *cos_decay, float gain_max, int64_t n, void *stream);
 /* grad_in = inside ? grad_out * scale : 0 */
 int slayer_quantize_bwd(float *grad_in, const float *grad_out, const unsigned char *inside, float scale, int64_t n,
                         void *stream);

@@ -22,6 +22,22 @@ __global__ __launch_bounds__(256) void quantize_bwd_kernel(float* __restrict__ g
     if (i < n) grad_in[i] = inside[i] ? grad_out[i] * scale : 0.f;
 }
 
+// The rotation parameters of a resonate-and-fire neuron, in place: gain limited to `gain_max`, sin at least 1, cos at least 0
+// (neuron/rf.py:136-257 in the reference) -- nine element-wise operators otherwise, on one value per channel, at the head of
+// every forward pass of a neuron that learns.  The same operations in the same order, so the same bits.
+__global__ __launch_bounds__(256) void rf_limit_kernel(float* __restrict__ sin_decay, float* __restrict__ cos_decay, float gain_max,
+                                                       int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float s = sin_decay[i], c = cos_decay[i];
+    const float gain = sqrtf(s * s + c * c);
+    const float ratio = (gain != gain ? gain : fminf(fmaxf(gain, 0.f), gain_max)) / gain;
+    s *= ratio;
+    c *= ratio;
+    sin_decay[i] = s != s ? s : fmaxf(s, 1.f);
+    cos_decay[i] = c != c ? c : fmaxf(c, 0.f);
+}
+
 }  // namespace slayer
 
 using namespace slayer;
@@ -48,5 +64,14 @@ extern "C" int slayer_quantize_bwd(float* grad_in, const float* grad_out, const 
     if (!grad_in || !grad_out || !inside) return SLAYER_ENULL;
     hipLaunchKernelGGL(quantize_bwd_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, grad_in,
                        grad_out, inside, scale, n);
+    return (int)hipGetLastError();
+}
+
+extern "C" int slayer_rf_limit(float* sin_decay, float* cos_decay, float gain_max, int64_t n, void* stream) {
+    if (int e = check_count(n)) return e;
+    if (n == 0) return 0;
+    if (!sin_decay || !cos_decay) return SLAYER_ENULL;
+    hipLaunchKernelGGL(rf_limit_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, sin_decay, cos_decay,
+                       gain_max, n);
     return (int)hipGetLastError();
 }

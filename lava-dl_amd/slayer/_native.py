@@ -83,6 +83,7 @@ _SIGNATURES = {
     'slayer_cuba_recurrent_steps_fwd': (_INT, [_P] * 10 + [_F, _INT, _F, _INT] + [_I64] * 7 + [_P, _I64, _P]),
     'slayer_alif_recurrent_steps_fwd': (_INT, [_P] * 17 + [_F, _I64, _INT, _F, _INT] + [_I64] * 11 + [_P, _I64, _P]),
     'slayer_quantize': (_INT, [_P] * 3 + [_F] * 4 + [_I64, _P]),
+    'slayer_rf_limit': (_INT, [_P] * 2 + [_F, _I64, _P]),
     'slayer_quantize_bwd': (_INT, [_P] * 3 + [_F, _I64, _P]),
     'slayer_recurrent_steps_bwd': (_INT, [_P] * 5 + [_F, _F, _F, _INT] + [_I64] * 3 + [_P, _I64, _P]),
     'slayer_li_fwd_naive': (_INT, [_P, _P, _P, _P, _D, _INT, _I64, _I64, _I64, _I64, _I64, _P]),

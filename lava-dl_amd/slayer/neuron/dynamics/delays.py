@@ -124,7 +124,10 @@ def delay_gradient(delays, folded):
     (axon/delay.py:201-221 in the reference: the sum times the sampling time times ``grad_scale``)."""
     if folded is None or folded.grad_sum is None:
         return None
-    grad = folded.grad_sum * delays.sampling_time * delays.grad_scale
+    grad = folded.grad_sum
+    for factor in (delays.sampling_time, delays.grad_scale):
+        if not (type(factor) in (int, float) and factor == 1):      # a product by one is a launch for nothing
+            grad = grad * factor
     if delays.output_delay.numel() == 1:
         grad = grad.sum()
     return grad.reshape(delays.output_delay.shape)

@@ -6,8 +6,9 @@ import torch
 from .base import Neuron as _Base, hardware_decay
 from .dynamics import resonator, rf_fused
 from .dynamics import delays as D
+from .. import _native as N
 from ..spike import complex as complex_spike
-from ..utils.quantize import quantize
+from ..utils.quantize import quantize, takes_kernel
 
 TAU_RHO_MULT = 0.5      # surrogate-gradient constants of the RF family (neuron/rf.py:19-20)
 SCALE_RHO_MULT = 10
@@ -72,6 +73,11 @@ class ResonatorNeuron(_Base):
             for name, prm in self.named_parameters(recurse=False):
                 if name not in ('sin_decay', 'cos_decay'):
                     prm.data.clamp_(0, self.p_scale)
+            s, c = self.sin_decay, self.cos_decay
+            if takes_kernel(s) and takes_kernel(c) and s.device == c.device and s.shape == c.shape:
+                with N.device_guard(s.device):                       # the lines below in one launch
+                    N.check(N.lib().slayer_rf_limit(N.ptr(s), N.ptr(c), float(self.p_scale - 1), s.numel(), N.stream_handle()))
+                return
             gain = torch.sqrt(self.sin_decay ** 2 + self.cos_decay ** 2)
             ratio = gain.clamp(0, self.p_scale - 1) / gain
             self.sin_decay.data *= ratio

@@ -18,6 +18,8 @@ class _StraightThrough(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, input, step, use_floor):
+        if step == 1:                                               # what follows, without the two products by one
+            return torch.floor(input) if use_floor else torch.round(input)
         scaled = input / step
         return (torch.floor(scaled) if use_floor else torch.round(scaled)) * step
 
@@ -67,7 +69,7 @@ def _launch(input, step, lo, hi, scale, inside):
     return out
 
 
-def _takes_kernel(input):
+def takes_kernel(input):
     """float32 weights on the GPU as they lie in memory, and nobody who wants to see the single operations: tracing,
     compilation, function transforms, forward-mode differentiation."""
     return (type(input) in (torch.Tensor, torch.nn.Parameter) and input.is_cuda and input.dtype == torch.float32
@@ -77,7 +79,7 @@ def _takes_kernel(input):
 
 def limit(input, step, lo, hi, scale=1):
     """``quantize(input, step).clamp(lo, hi) * scale``."""
-    if not _takes_kernel(input):
+    if not takes_kernel(input):
         q = quantize(input, step=step).clamp(lo, hi)
         return q if scale == 1 else q * scale
     if torch.is_grad_enabled() and input.requires_grad:

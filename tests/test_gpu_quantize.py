@@ -66,3 +66,28 @@ def test_calls_that_keep_the_operators(slayer):
     grad_y, = torch.autograd.grad((_chain(slayer, y, *args, 1) ** 2).sum(), y, create_graph=True)
     second_y, = torch.autograd.grad(grad_y.sum(), y)
     assert torch.equal(grad, grad_y) and torch.equal(second, second_y)
+
+
+def test_rotation_limits_are_the_chain_of_operators(slayer):
+    """ResonatorNeuron.clamp in one launch: gains on either side of the limit, negative and vanishing parts, NaN, infinity."""
+    gen = torch.Generator().manual_seed(3)
+    neuron = slayer.neuron.rf.Neuron(threshold=1.0, period=[20, 200], decay=[0.01, 0.9], shared_param=False).to(dev())
+    s, c = torch.randn(600, generator=gen) * 4000, torch.randn(600, generator=gen) * 4000
+    s[:6] = torch.tensor([0.0, float('nan'), float('inf'), 4095.0, 1e-30, 3e38])
+    c[:6] = torch.tensor([0.0, 1.0, 2.0, 0.0, -1e-30, 3e38])
+    results = []
+    for fused in (True, False):
+        neuron.sin_decay.data, neuron.cos_decay.data = s.clone().to(dev()), c.clone().to(dev())
+        if fused:
+            neuron.clamp()
+        else:
+            with torch.no_grad():
+                gain = torch.sqrt(neuron.sin_decay ** 2 + neuron.cos_decay ** 2)
+                ratio = gain.clamp(0, 4095) / gain
+                neuron.sin_decay.data.mul_(ratio).clamp_(1)
+                neuron.cos_decay.data.mul_(ratio).clamp_(0)
+        results.append([p.data.cpu().clone() for p in (neuron.sin_decay, neuron.cos_decay)])
+    for a, b in zip(*results):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+        ok = ~torch.isnan(a)
+        assert torch.equal(a[ok].view(torch.int32), b[ok].view(torch.int32))
