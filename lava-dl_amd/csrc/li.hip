@@ -31,9 +31,9 @@ struct LiFwd {
     // on its way into LDS, the state is converted and scaled back on its way out, and the
     // sequential loop is left with the recurrence alone.
     static constexpr bool kTransforms = true;
-    // [32,256,1500] 35 -> 32 us with four instead of two (43 -> 40 with a threshold), [16,512,1450] 54 -> 35 with eight,
-    // [32,16,32,32,300] 239 -> 233, [32,16,32,32,301] 299 -> 287 (eight: 325)
-    static constexpr int copy_waves(bool large, bool unaligned, bool) { return unaligned && !large ? 8 : 4; }
+    // [32,256,1500] 35 -> 32 us with four instead of two (43 -> 40 with a threshold), [16,512,1450] 54 -> 37 (eight: 35),
+    // [32,16,32,32,300] 239 -> 233, [32,16,32,32,301] 299 -> 287 (eight: 325), [225,256,257] 31 with two (eight: 39)
+    static constexpr int kCopyWaves = 4;
     int y, mult, fire_above;
     bool nonneg;
     float w, inv_w;
