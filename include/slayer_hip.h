@@ -557,10 +557,10 @@ int slayer_recurrent_bwd(float *grad_z, const float *grad_spikes, const float *v
                          const float *rec, float spike_threshold, float tau_rho, float scale_rho, int graded,
                          int64_t N, int64_t C, int64_t T, void *stream);
 
-/* The same loops, one launch per time step: for layers of any width up to 16384 neurons (C a multiple of 4).
- * A step multiplies the weight matrix with the spikes of the previous step for the whole batch (the matrix is read
- * once per step, on the matrix cores in float32) and runs one neuron step on the result; the launches follow each
- * other on `stream`.  Same arguments, results and arithmetic as slayer_cuba_recurrent_fwd / slayer_alif_recurrent_fwd
+/* The same loops for layers of any width up to 16384 neurons (C a multiple of 4), the whole batch together.
+ * Up to 2048 neurons, binary spikes and a batch that the device holds at once run as one cooperative launch that keeps
+ * the matrix in registers; other calls, and calls on a stream under capture, as one launch per time step that reads
+ * the matrix once (on the matrix cores in float32).  Everything runs on `stream`.  Same arguments, results and arithmetic as slayer_cuba_recurrent_fwd / slayer_alif_recurrent_fwd
  * except: `rec` is R itself, [C][C] (row c = the weights that reach neuron c); the *_last outputs are 16-byte
  * aligned; the feedback of a step is summed in a fixed order of its own (equal bits whenever the sums are exact in
  * float32, e.g. quantised weights and binary spikes); `workspace` is device memory of at least

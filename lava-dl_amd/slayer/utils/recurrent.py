@@ -46,9 +46,9 @@ def custom_recurrent_ground_truth_2(z, neuron, recurrent_synapse):
 
 ONE_LAUNCH_MAX = 1024       # neurons per sample of the one-launch kernels (one thread per neuron)
 STEPS_MAX = 16384           # ... of the launch-per-step kernels (whole quads of neurons)
-# Width from which layers take a launch per step.  It is the faster form from 260 neurons on (measured at [32, C, 300]); at 256 the
-# one-launch kernels still hold the matrix in registers and are faster (forward and backward, 300 steps, CUBA: 602 us against 2560
-# for 32 samples, 2130 against 4525 for 512).
+# Width from which layers take the kernels for the whole batch, the faster form from 260 neurons on (measured at [32, C, 300]);
+# at 256 one workgroup per sample still holds the matrix in registers and is faster (forward and backward, 300 steps, CUBA, 32
+# samples: 602 us against 990).
 STEPS_FROM = 256
 
 
@@ -74,7 +74,7 @@ def custom_recurrent(z, neuron, recurrent_synapse):
 
     The one-launch kernel adds the feedback of up to 256 neurons in a fixed order, that of wider layers (and of 193 and
     more neurons in batches from 1024 samples on) row by row in the order the neurons fired, 16 at a time, the
-    launch-per-step kernels in a fixed order of their own on the matrix cores (float32), where the reference's loop calls
+    kernels for the whole batch in a fixed order of their own on the matrix cores, where the reference's loop calls
     ``torch.matmul``.  The sums are the same bits whenever every partial sum is exactly representable in float32, which
     holds for quantised recurrent weights (multiples of a power of two of moderate size, what the synapse's
     ``pre_hook_fx`` quantiser produces).  With unquantised weights the sums can differ in the last bit and a dendrite
@@ -140,7 +140,7 @@ def _steps_workspace(n, c, t, with_theta, dev):
 
 class _FusedRecurrent(torch.autograd.Function):
     """The whole time loop of a CUBA or an ALIF layer inside the library: one launch per direction, or one per
-    time step for wide layers."""
+    time step for layers that do not fit the chip at once."""
 
     @staticmethod
     def forward(ctx, z, neuron, recurrent_mat):
