@@ -1,6 +1,7 @@
 """Straight-through parameter quantiser (utils/quantize.py:18-94 in the reference)."""
 from enum import IntEnum, unique
 
+import numpy as np
 import torch
 from torch.autograd import forward_ad
 
@@ -13,12 +14,17 @@ class MODE(IntEnum):
     FLOOR = 1
 
 
+def _is_number(*values):
+    """Plain numbers: not tensors or arrays, whose elements differ, may be trained, or lie on the GPU."""
+    return all(isinstance(v, (int, float, np.integer, np.floating)) for v in values)
+
+
 class _StraightThrough(torch.autograd.Function):
     """Snap to a grid of ``step`` in the forward pass, identity in the backward pass."""
 
     @staticmethod
     def forward(ctx, input, step, use_floor):
-        if step == 1:                                               # what follows, without the two products by one
+        if _is_number(step) and step == 1:                          # what follows, without the two products by one
             return torch.floor(input) if use_floor else torch.round(input)
         scaled = input / step
         return (torch.floor(scaled) if use_floor else torch.round(scaled)) * step
@@ -34,7 +40,7 @@ def quantize(input, step=1, mode=MODE.ROUND):
         raise ValueError(f'{mode=} is not recognized.')
     if not (torch.is_grad_enabled() and input.requires_grad):      # nothing to pass a gradient to
         snap = torch.floor if mode == MODE.FLOOR else torch.round
-        return snap(input) if step == 1 else snap(input / step) * step
+        return snap(input) if _is_number(step) and step == 1 else snap(input / step) * step
     return _StraightThrough.apply(input, step, mode == MODE.FLOOR)
 
 
