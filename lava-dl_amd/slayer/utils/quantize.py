@@ -19,6 +19,9 @@ def _is_number(*values):
     return all(isinstance(v, (int, float, np.integer, np.floating)) for v in values)
 
 
+_FLOAT32_MAX = torch.finfo(torch.float32).max
+
+
 class _StraightThrough(torch.autograd.Function):
     """Snap to a grid of ``step`` in the forward pass, identity in the backward pass."""
 
@@ -83,11 +86,18 @@ def takes_kernel(input):
             and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0)
 
 
+def _fits_kernel(step, lo, hi, scale):
+    """Plain numbers that are float32 numbers too, and a step whose reciprocal is one."""
+    return (_is_number(step, lo, hi, scale) and 2.0 ** -126 <= abs(step) <= 2.0 ** 126
+            and all(abs(v) <= _FLOAT32_MAX for v in (lo, hi, scale)))
+
+
 def limit(input, step, lo, hi, scale=1):
-    """``quantize(input, step).clamp(lo, hi) * scale``."""
-    if not takes_kernel(input):
+    """``quantize(input, step).clamp(lo, hi) * scale``.  A step, a limit or a scale may be a tensor (one per channel, or one that is
+    trained); those take the operators."""
+    if not (takes_kernel(input) and _fits_kernel(step, lo, hi, scale)):
         q = quantize(input, step=step).clamp(lo, hi)
-        return q if scale == 1 else q * scale
+        return q if _is_number(scale) and scale == 1 else q * scale
     if torch.is_grad_enabled() and input.requires_grad:
         return _Limited.apply(input, float(step), float(lo), float(hi), float(scale))
     return _launch(input, float(step), float(lo), float(hi), float(scale), None)
