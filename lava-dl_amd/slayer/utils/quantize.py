@@ -60,7 +60,7 @@ class _Limited(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         inside, = ctx.saved_tensors
-        if torch.is_grad_enabled() or grad_output.dtype != torch.float32:          # create_graph=True
+        if torch.is_grad_enabled() or not takes_kernel(grad_output, contiguous=False):      # create_graph=True, batched gradients
             return torch.where(inside, grad_output * ctx.scale, 0.0), None, None, None, None
         grad_output = grad_output.contiguous()
         grad = torch.empty_like(grad_output)
@@ -78,12 +78,16 @@ def _launch(input, step, lo, hi, scale, inside):
     return out
 
 
-def takes_kernel(input):
+def takes_kernel(input, contiguous=True):
     """float32 weights on the GPU as they lie in memory, and nobody who wants to see the single operations: tracing,
-    compilation, function transforms, forward-mode differentiation."""
+    compilation, function transforms (those of ``is_grads_batched`` too, whose tensors have no memory of their own),
+    forward-mode differentiation."""
     return (type(input) in (torch.Tensor, torch.nn.Parameter) and input.is_cuda and input.dtype == torch.float32
-            and input.is_contiguous() and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
-            and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0)
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
+            and not torch._C._functorch.is_legacy_batchedtensor(input)
+            and not torch._C._functorch.is_functorch_wrapped_tensor(input)
+            and (not contiguous or input.is_contiguous()))
 
 
 def _fits_kernel(step, lo, hi, scale):

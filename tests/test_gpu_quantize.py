@@ -68,6 +68,21 @@ def test_calls_that_keep_the_operators(slayer):
     assert torch.equal(grad, grad_y) and torch.equal(second, second_y)
 
 
+@pytest.mark.parametrize('form', ['is_grads_batched', 'vmap'])
+def test_batched_gradients(slayer, form):
+    """Gradients without memory of their own take the operators; what each entry of the batch gives alone is the kernel's."""
+    gen = torch.Generator().manual_seed(4)
+    w = (torch.randn(6, 10, generator=gen) * 3).to(dev()).requires_grad_()
+    g = torch.randn(5, 6, 10, generator=gen).to(dev())
+    out = slayer.utils.limit(w, 2 / 64, -4.0, 254 / 64, 64)
+    single = torch.stack([torch.autograd.grad(out, w, r, retain_graph=True)[0] for r in g])
+    if form == 'vmap':
+        batched = torch.func.vmap(lambda r: torch.autograd.grad(out, w, r, retain_graph=True)[0])(g)
+    else:
+        batched, = torch.autograd.grad(out, w, g, is_grads_batched=True, retain_graph=True)
+    assert torch.equal(single, batched)
+
+
 def test_rotation_limits_are_the_chain_of_operators(slayer):
     """ResonatorNeuron.clamp in one launch: gains on either side of the limit, negative and vanishing parts, NaN, infinity."""
     gen = torch.Generator().manual_seed(3)
