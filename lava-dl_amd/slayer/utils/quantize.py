@@ -80,10 +80,11 @@ def _launch(input, step, lo, hi, scale, inside):
 
 def takes_kernel(input, contiguous=True):
     """float32 weights on the GPU as they lie in memory, and nobody who wants to see the single operations: tracing,
-    compilation, function transforms (those of ``is_grads_batched`` too, whose tensors have no memory of their own),
-    forward-mode differentiation."""
+    compilation, dispatch modes (make_fx), function transforms (those of ``is_grads_batched`` too, whose tensors have no
+    memory of their own), forward-mode differentiation."""
     return (type(input) in (torch.Tensor, torch.nn.Parameter) and input.is_cuda and input.dtype == torch.float32
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
             and not torch._C._functorch.is_legacy_batchedtensor(input)
             and not torch._C._functorch.is_functorch_wrapped_tensor(input)

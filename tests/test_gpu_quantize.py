@@ -57,8 +57,11 @@ def test_calls_that_keep_the_operators(slayer):
     assert torch.equal(torch.func.vmap(lambda r: limit(r, *args))(w), want)
     assert torch.equal(torch.jit.trace(lambda r: limit(r, *args), (w,))(w + 1), _chain(slayer, w + 1, *args, 1))
     with torch.autograd.forward_ad.dual_level():
-        dual = torch.autograd.forward_ad.make_dual(w, torch.ones_like(w))
-        limit(dual, *args)
+        dual = torch.autograd.forward_ad.make_dual(w, torch.full_like(w, 0.75))
+        primal, tangent = torch.autograd.forward_ad.unpack_dual(limit(dual, *args))
+        want_tangent = torch.autograd.forward_ad.unpack_dual(_chain(slayer, dual, *args, 1)).tangent
+        assert torch.equal(primal, want)
+        assert (tangent is None) == (want_tangent is None) and (tangent is None or torch.equal(tangent, want_tangent))
     x = w.clone().requires_grad_()
     grad, = torch.autograd.grad((limit(x, *args) ** 2).sum(), x, create_graph=True)
     second, = torch.autograd.grad(grad.sum(), x)
@@ -66,6 +69,14 @@ def test_calls_that_keep_the_operators(slayer):
     grad_y, = torch.autograd.grad((_chain(slayer, y, *args, 1) ** 2).sum(), y, create_graph=True)
     second_y, = torch.autograd.grad(grad_y.sum(), y)
     assert torch.equal(grad, grad_y) and torch.equal(second, second_y)
+
+
+def test_a_recorded_graph_holds_the_operators(slayer):
+    from torch.fx.experimental.proxy_tensor import make_fx
+    limit = slayer.utils.limit
+    w = (torch.randn(6, 10, generator=torch.Generator().manual_seed(5)) * 3).to(dev())
+    graph = make_fx(lambda r: limit(r, 2 / 64, -4.0, 254 / 64))(w)
+    assert torch.equal(graph(w * 0.7), _chain(slayer, w * 0.7, 2 / 64, -4.0, 254 / 64, 1))
 
 
 @pytest.mark.parametrize('form', ['is_grads_batched', 'vmap'])
