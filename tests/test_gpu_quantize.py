@@ -71,6 +71,26 @@ def test_calls_that_keep_the_operators(slayer):
     assert torch.equal(grad, grad_y) and torch.equal(second, second_y)
 
 
+def test_more_weights_than_a_launch_has_threads(slayer):
+    """2^32 + 300 entries through the C interface; looked at near both ends and in the middle, where a thread's second entry lies."""
+    from lava_dl_amd.slayer import _native as N
+    n, scale = (1 << 32) + 300, 64.0
+    gen = torch.Generator().manual_seed(6)
+    parts = [slice(0, 600), slice((1 << 31) - 300, (1 << 31) + 300), slice(n - 600, n)]
+    x, out = (torch.empty(n, device=dev()) for _ in range(2))
+    inside = torch.empty(n, dtype=torch.uint8, device=dev())
+    for p in parts:
+        x[p] = (torch.randn(600, generator=gen) * 3).to(dev())
+    N.check(N.lib().slayer_quantize(N.ptr(out), N.ptr(inside), N.ptr(x), 2 / 64, -4.0, 254 / 64, scale, n, N.stream_handle()))
+    wants = [_chain(slayer, x[p], 2 / 64, -4.0, 254 / 64, scale) for p in parts]
+    for p, want in zip(parts, wants):
+        assert torch.equal(out[p], want)
+    N.check(N.lib().slayer_quantize_bwd(N.ptr(out), N.ptr(x), N.ptr(inside), scale, n, N.stream_handle()))
+    for p in parts:
+        q = slayer.utils.quantize(x[p], step=2 / 64)
+        assert torch.equal(out[p], torch.where((q >= -4.0) & (q <= 254 / 64), x[p] * scale, 0.0))
+
+
 def test_a_recorded_graph_holds_the_operators(slayer):
     from torch.fx.experimental.proxy_tensor import make_fx
     limit = slayer.utils.limit
