@@ -611,7 +611,7 @@ __device__ __forceinline__ void grid_bwd_local(const GridBwd& p, float (*red)[kG
                     for (int v = 0; v < kGridWaves; ++v) carry += from[v];
                     gs = carry * (1.0f / kLocalScale) + gs;
                 }
-                const float gz = factor * gs;
+                const float gz = c0 + lane < C ? factor * gs : 0.f;      // nothing beyond the layer: 0 times an infinity is none
                 if (t > 0) {
                     // this neuron's parts, those of the pair's other neuron, and the words of both
                     const float x = gz * kLocalScale, size = fabsf(gz);
@@ -792,7 +792,7 @@ __global__ __launch_bounds__(kGridThreads) void recurrent_grid_bwd_kernel(const 
                         for (int v = 0; v < kGridWaves; ++v) carry += red[sel][v][lane & 3][wave * 16 + (lane >> 2)];
                         gs = carry + gs;
                     }
-                    const float gz = factor * gs;
+                    const float gz = c0 + 4 * wave < C ? factor * gs : 0.f;      // nothing beyond the layer: 0 times an infinity is none
                     if (t > 0) {
                         const unsigned bits = __float_as_uint(gz);
                         __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): the clearing store has arrived

@@ -117,6 +117,41 @@ def test_gradients_of_weights_on_and_off_the_grid(slayer, n, c, t, weights, scal
     assert bool((err <= 4e-7 * t * want.abs().amax()).all()), float(err.max() / want.abs().max())
 
 
+# 68 and 260 neurons leave twelve columns of a tile of 16 and sixty of a tile of 64 empty, in either form of the kernel
+@pytest.mark.parametrize('c', [68, 260])
+@pytest.mark.parametrize('weights', ['grid', 'real'])
+@pytest.mark.parametrize('bad', [float('inf'), float('-inf'), float('nan')])
+def test_gradients_that_are_not_finite(slayer, c, weights, bad):
+    """Positive weights: an infinite gradient of one neuron leaves every earlier one of its sample infinite and of its sign, as in the
+    float64 loop; a NaN makes them NaN; the other samples are untouched (bound as above)."""
+    from lava_dl_amd.slayer import _native as N
+    n, t = 5, 18
+    gen = torch.Generator().manual_seed(c)
+    rec = torch.rand(c, c, generator=gen) + 0.25
+    if weights == 'grid':
+        rec = (rec * 32).round() / 32
+    rec /= 256
+    v = torch.randn(n, c, t, generator=gen) * 0.02 + 1.25
+    g = torch.randn(n, c, t, generator=gen)
+    g[1, 3, t - 2] = bad
+    d = [x.to(dev()) for x in (g, v, rec)]
+    gz = torch.empty_like(d[0])
+    floats = N.lib().slayer_recurrent_steps_workspace(n, c, t, 0)
+    ws = torch.empty(floats, device=dev())
+    N.check(N.lib().slayer_recurrent_steps_bwd(N.ptr(gz), N.ptr(d[0]), N.ptr(d[1]), None, N.ptr(d[2]), 1.25, 0.05, 0.04, 0,
+                                               n, c, t, N.ptr(ws), floats, N.stream_handle()))
+    factor = (0.04 / 2 / 0.05) * torch.exp(-(v.double() - 1.25).abs() / 0.05)
+    want, carry = torch.empty_like(factor), torch.zeros(n, c, dtype=torch.float64)
+    for step in reversed(range(t)):
+        want[..., step] = factor[..., step] * (g[..., step].double() + carry)
+        carry = want[..., step] @ rec.double()
+    got = gz.cpu().double()
+    assert not torch.isfinite(want[1, :, :t - 2]).any() and torch.isfinite(want).sum() == want.numel() - c * (t - 2) - 1
+    finite = torch.isfinite(want)
+    assert torch.equal(got[~finite].nan_to_num(5.0, 6.0, 7.0), want[~finite].nan_to_num(5.0, 6.0, 7.0))
+    assert bool(((got - want)[finite].abs() <= 4e-7 * t * want[finite].abs().amax()).all())
+
+
 def test_weights_that_are_not_finite(slayer, monkeypatch):
     """An infinite weight times a silent neuron is a NaN, and so is a NaN weight times any: what the two receiving neurons
     do is lost, the other neurons' feedback is untouched."""
