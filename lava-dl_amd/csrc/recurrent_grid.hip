@@ -30,6 +30,7 @@
 // dependent instructions.
 #include "recurrent_step.h"
 #include "split.h"
+#include <initializer_list>
 
 namespace slayer {
 
@@ -876,6 +877,18 @@ bool grid_plan(int64_t N, int64_t C, int64_t T, hipStream_t st, GridPlan* plan) 
     return false;
 }
 
+struct Floats { const float* at; int64_t n; };                    // at = nullptr: none
+// Whether results lie over inputs.  The kernel behind computes a layer again from its inputs, so such a call takes a launch per step,
+// which copies its inputs first.
+bool overlap(std::initializer_list<Floats> results, std::initializer_list<Floats> inputs) {
+    for (const Floats& a : results)
+        for (const Floats& b : inputs) {
+            const uintptr_t p = (uintptr_t)a.at, q = (uintptr_t)b.at;
+            if (a.at && b.at && p < q + 4 * (uintptr_t)b.n && q < p + 4 * (uintptr_t)a.n) return true;
+        }
+    return false;
+}
+
 // false: the runtime does not take the grid as a cooperative one
 bool launch_grid(const void* kernel, unsigned grid, void* args, hipStream_t st) {
     void* list[] = {args};
@@ -903,6 +916,11 @@ bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* th
     if (!grid_plan(p.N, p.C, p.T, st, &plan)) return false;
     const int64_t words = (int64_t)2 * plan.S * words_of(plan.KB);
     if (workspace_floats < words + 4) return false;
+    const int64_t nc = (int64_t)p.N * p.C, nct = nc * p.T;
+    if (overlap({{spk, nct}, {vol, nct}, {theta, nct}, {p.cur_last, nc}, {p.vol_last, nc}, {p.th_last, nc}, {p.ref_last, nc}},
+                {{z, nct}, {rec, (int64_t)p.C * p.C}, {p.i_decay, p.n_id}, {p.v_decay, p.n_vd}, {p.th_decay, p.n_td},
+                 {p.ref_decay, p.n_rd}, {p.i_state, p.n_is}, {p.v_state, p.n_vs}, {p.th_state, p.n_ts}, {p.ref_state, p.n_rs}}))
+        return false;
     GridFwd g{};
     g.p = p;
     g.p.KB = plan.KB; g.p.S = plan.S;
@@ -934,6 +952,8 @@ bool grid_bwd(float* gz, const float* grad_spikes, const float* voltage, const f
     int64_t ring = (int64_t)4 * plan.S * plan.KB * 256;
     const int64_t head = 4 + kFillBlocks;
     if (workspace_floats < ring + head) return false;
+    const int64_t nct = N * C * T;
+    if (overlap({{gz, nct}}, {{grad_spikes, nct}, {voltage, nct}, {theta, nct}, {rec, C * C}})) return false;
     GridBwd p{};
     p.gz = gz; p.g = grad_spikes; p.v = voltage; p.theta = theta; p.rec = rec;
     p.gave_up = reinterpret_cast<unsigned*>(workspace);

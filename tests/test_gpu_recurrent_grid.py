@@ -117,6 +117,28 @@ def test_gradients_of_weights_on_and_off_the_grid(slayer, n, c, t, weights, scal
     assert bool((err <= 4e-7 * t * want.abs().amax()).all()), float(err.max() / want.abs().max())
 
 
+@pytest.mark.parametrize('where', [0, 1])
+def test_gradients_in_place(slayer, where):
+    """grad_z over grad_spikes or over the voltage, with gradients so large that the layer is computed a second time."""
+    from lava_dl_amd.slayer import _native as N
+    n, c, t = 5, 68, 18
+    gen = torch.Generator().manual_seed(8)
+    rec = (torch.randn(c, c, generator=gen) * 12 / c ** 0.5).round().to(dev()) / 4
+    v = (torch.randn(n, c, t, generator=gen) * 0.02 + 1.25).to(dev())
+    g = (torch.randn(n, c, t, generator=gen) * 1e27).to(dev())
+    floats = N.lib().slayer_recurrent_steps_workspace(n, c, t, 0)
+    ws = torch.empty(floats, device=dev())
+
+    def run(gz, g, v):
+        N.check(N.lib().slayer_recurrent_steps_bwd(N.ptr(gz), N.ptr(g), N.ptr(v), None, N.ptr(rec), 1.25, 0.05, 0.04, 0, n, c, t,
+                                                   N.ptr(ws), floats, N.stream_handle()))
+        return gz
+    want = run(torch.empty_like(g), g, v)
+    ins = [g.clone(), v.clone()]
+    assert float(want.abs().max()) > 1e26
+    assert_rel(run(ins[where], *ins), want.cpu(), 'grad z in place')
+
+
 # 68 and 260 neurons leave twelve columns of a tile of 16 and sixty of a tile of 64 empty, in either form of the kernel
 @pytest.mark.parametrize('c', [68, 260])
 @pytest.mark.parametrize('weights', ['grid', 'real'])
