@@ -20,8 +20,8 @@
 // The workgroups wait for one another, so all of them must be on the chip at once: the launch is a cooperative one,
 // which the runtime refuses beyond what the device holds, does not run beside another and grants to one process at a time
 // (a refused call takes a launch per step).  Every wait is bounded all the same (kSpinLimit polls); a workgroup that
-// gives up leaves a mark, and the kernel that is launched behind computes the layer again, one workgroup per sample,
-// when it finds it.
+// gives up leaves a mark, and the kernel that is launched behind computes the layer again when it finds it: forward with the same
+// bits, one workgroup per sample tile; backward one workgroup per sample, its sums in double and so equal to rounding.
 //
 // Measured against a launch per step, whole layer, forward and backward: CUBA [32, 2048, 300] 5 121 -> 3 117 us (forward
 // kernel 2 430 -> 493, backward 2 075 -> 1 751), [32, 256, 300] 2 527 -> 951, ALIF [32, 512, 300] 2 651 -> 1 237,
@@ -72,6 +72,7 @@ struct GridFwd {
     float *spk, *vol, *theta;                        // [N][C][T]
     const float *z, *rec;
     unsigned* words;                                 // [2][S][words_of(KB)]
+    int* carried;                                    // [4][N][C], see recurrent_solo_fwd_kernel
     GridMap map;
     unsigned* gave_up;
 };
@@ -96,6 +97,47 @@ __device__ __forceinline__ unsigned cut(float& v) {
     return h;
 }
 
+// Unit u of 16 rows of R as A operands, halved, in three parts.  A unit is 8 neuron tiles = 128 presynaptic neurons = four
+// products; lane (kk, j) has tiles 8u + 2kk and 8u + 2kk + 1 of row c, element 2i (2i + 1) of product a is neuron 4a + i of
+// the first (second) tile, k0 its first neuron.  Returns whether a part beyond the first has a bit.
+__device__ __forceinline__ bool weight_parts(const float* rec, int C, int c, int k0, uint4 (&wh)[4], uint4 (&wm)[4], uint4 (&wl)[4]) {
+    float v[32];
+    unsigned rest = 0u;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const bool ok = c < C && k0 + 4 * q < C;                         // C is a multiple of 4
+        const float4 f = ok ? load_quad_dword_aligned(rec + (int64_t)c * C + k0 + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
+        v[4 * q] = 0.5f * f.x; v[4 * q + 1] = 0.5f * f.y; v[4 * q + 2] = 0.5f * f.z; v[4 * q + 3] = 0.5f * f.w;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        unsigned h[4], m[4], l[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float &x = v[4 * a + i], &y = v[16 + 4 * a + i];
+            h[i] = cut(x) >> 16; h[i] |= cut(y);
+            m[i] = cut(x) >> 16; m[i] |= cut(y);
+            l[i] = cut(x) >> 16; l[i] |= cut(y);
+            rest |= m[i] | l[i];
+        }
+        wh[a] = make_uint4(h[0], h[1], h[2], h[3]);
+        wm[a] = make_uint4(m[0], m[1], m[2], m[3]);
+        wl[a] = make_uint4(l[0], l[1], l[2], l[3]);
+    }
+    return rest != 0u;
+}
+
+// The B operand of product a: the spikes of two tiles, side by side in a word, as the numbers 2.0 and 0.
+__device__ __forceinline__ uint4 spike_parts(unsigned both, int a) {
+    unsigned b[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int bit = 4 * a + i;                                       // neuron `bit` of both tiles, to bits 14 and 30
+        b[i] = (bit <= 14 ? both << (14 - bit) : both >> 1) & 0x40004000u;
+    }
+    return make_uint4(b[0], b[1], b[2], b[3]);
+}
+
 // Thread (wave v, lane 16 i + nn) of the first four waves runs neuron nn of the tile for sample 4 v + i; the ballot of its
 // wave then holds the 16 spikes of a sample in one 16-bit field.
 template <bool ALIF, bool POW2, int U, int NT>
@@ -117,39 +159,12 @@ __global__ __launch_bounds__(kGridThreads) void recurrent_grid_fwd_kernel(const 
     const int64_t set = (int64_t)p.S * words;
     if (tid < 2) dead[tid] = 0;
 
-    // rows c0 .. c0 + 15 of R as A operands.  Unit u = 8 neuron tiles = 128 presynaptic neurons = four products; lane
-    // (kk, j) has tiles 8u + 2kk and 8u + 2kk + 1 of row c0 + j, element 2i (2i + 1) of product a is neuron 4a + i of
-    // the first (second) tile.
-    uint4 wh[U][4], wm[U][4], wl[U][4];
-    unsigned rest = 0u;
+    uint4 wh[U][4], wm[U][4], wl[U][4];              // rows c0 .. c0 + 15 of R
+    bool rest = false;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int k0 = 16 * (8 * (wave + kGridWaves * u) + 2 * kk);
-        float v[32];
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            const bool ok = c0 + j < C && k0 + 4 * q < C;            // C is a multiple of 4
-            const float4 f = ok ? load_quad_dword_aligned(g.rec + (int64_t)(c0 + j) * C + k0 + 4 * q)
-                                : make_float4(0.f, 0.f, 0.f, 0.f);
-            v[4 * q] = 0.5f * f.x; v[4 * q + 1] = 0.5f * f.y; v[4 * q + 2] = 0.5f * f.z; v[4 * q + 3] = 0.5f * f.w;
-        }
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-            unsigned h[4], m[4], l[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float &x = v[4 * a + i], &y = v[16 + 4 * a + i];
-                h[i] = cut(x) >> 16; h[i] |= cut(y);
-                m[i] = cut(x) >> 16; m[i] |= cut(y);
-                l[i] = cut(x) >> 16; l[i] |= cut(y);
-                rest |= m[i] | l[i];
-            }
-            wh[u][a] = make_uint4(h[0], h[1], h[2], h[3]);
-            wm[u][a] = make_uint4(m[0], m[1], m[2], m[3]);
-            wl[u][a] = make_uint4(l[0], l[1], l[2], l[3]);
-        }
-    }
-    const bool lower = __any(rest != 0u);
+    for (int u = 0; u < U; ++u)
+        rest |= weight_parts(g.rec, C, c0 + j, 16 * (8 * (wave + kGridWaves * u) + 2 * kk), wh[u], wm[u], wl[u]);
+    const bool lower = __any(rest);
     // where this lane finds the words of its units, and which of the two tiles there are (an address beyond them is moved
     // to the first tiles; its words are of no consequence, the weights there are zero)
     int word_at[U];
@@ -252,26 +267,17 @@ __global__ __launch_bounds__(kGridThreads) void recurrent_grid_fwd_kernel(const 
                     }
                     split_f4 acc[2] = {split_f4{0.f, 0.f, 0.f, 0.f}, split_f4{0.f, 0.f, 0.f, 0.f}};
                     split_f4 low = split_f4{0.f, 0.f, 0.f, 0.f};
-                    auto spikes = [&](int u, int a) -> uint4 {
-                        unsigned b[4];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const int bit = 4 * a + i;                    // neuron `bit` of both tiles, to bits 14 and 30
-                            b[i] = (bit <= 14 ? W[u] << (14 - bit) : W[u] >> 1) & 0x40004000u;
-                        }
-                        return make_uint4(b[0], b[1], b[2], b[3]);
-                    };
                     if (!lower) {
 #pragma unroll
                         for (int u = 0; u < U; ++u)
 #pragma unroll
-                            for (int a = 0; a < 4; ++a) acc[a & 1] = mfma_bf16(wh[u][a], spikes(u, a), acc[a & 1]);
+                            for (int a = 0; a < 4; ++a) acc[a & 1] = mfma_bf16(wh[u][a], spike_parts(W[u], a), acc[a & 1]);
                     } else {
 #pragma unroll
                         for (int u = 0; u < U; ++u)
 #pragma unroll
                             for (int a = 0; a < 4; ++a) {
-                                const uint4 b = spikes(u, a);
+                                const uint4 b = spike_parts(W[u], a);
                                 acc[a & 1] = mfma_bf16(wh[u][a], b, acc[a & 1]);
                                 low = mfma_bf16(wm[u][a], b, low);
                                 low = mfma_bf16(wl[u][a], b, low);
@@ -342,52 +348,91 @@ __global__ __launch_bounds__(kGridThreads) void recurrent_grid_fwd_kernel(const 
         if (mine[s] && (range_exceeded(nrn[s].acc_lif, 30) || range_exceeded(nrn[s].acc_th, 28))) raise_range_flag(p.range_flag);
 }
 
-// The same layer, one workgroup per sample, when a workgroup of the kernel above gave up waiting.
+// The same layer, one workgroup per sample tile, when a workgroup of the kernel above gave up waiting: every product and sum in the
+// same order (a part that is zero adds nothing), so which of the two computed a layer cannot be told from its bits.  The carried
+// states lie in memory between two steps, and a workgroup reads the whole matrix every step, which is what bounds it: 0.28 ms a step at
+// 1300 neurons (one workgroup per sample and a thread per row: 0.70).
 template <bool ALIF, bool POW2>
-__global__ __launch_bounds__(kSoloThreads) void recurrent_solo_fwd_kernel(const GridFwd g) {
-    __shared__ float spikes[2][kGridMaxC];
+__global__ __launch_bounds__(kGridThreads) void recurrent_solo_fwd_kernel(const GridFwd g) {
+    __shared__ unsigned bits[2][kGridMaxC / 16][16];     // the spikes of a neuron tile and sample
+    __shared__ float red[kGridWaves][4][68];
     if (*g.gave_up == 0u) return;
     const StepFwd& p = g.p;
-    const int C = p.C, T = p.T;
-    constexpr int kEach = kGridMaxC / kSoloThreads;
-    StepNeuron<ALIF, false, POW2> nrn[kEach];
-#pragma unroll
-    for (int i = 0; i < kEach; ++i) {
-        const int c = threadIdx.x + i * kSoloThreads;
-        nrn[i] = StepNeuron<ALIF, false, POW2>{};
-        if (c < C) {
-            nrn[i].load_decays(p, c);
-            nrn[i].load_states(p, (int64_t)blockIdx.x * C + c);
-            nrn[i].check(p.range_flag);
-        }
-    }
+    const int C = p.C, N = p.N, T = p.T, KB = p.KB;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6, kk = lane >> 4, j = lane & 15;
+    const int n = 16 * blockIdx.x + 4 * wave + kk;       // of the first four waves
+    const int64_t nc = (int64_t)N * C;
+    for (int i = tid; i < 2 * (kGridMaxC / 16) * 16; i += kGridThreads) (&bits[0][0][0])[i] = 0u;
+    __syncthreads();
+    unsigned acc_lif = 0u, acc_th = 0u;
     for (int t = 0; t < T; ++t) {
+        for (int P = 0; P < KB; ++P) {
+            if (t > 0) {
+                split_f4 acc[2] = {split_f4{0.f, 0.f, 0.f, 0.f}, split_f4{0.f, 0.f, 0.f, 0.f}};
+                split_f4 low = split_f4{0.f, 0.f, 0.f, 0.f};
+                for (int u = wave; 8 * u < KB; u += kGridWaves) {
+                    uint4 wh[4], wm[4], wl[4];
+                    const int first = 8 * u + 2 * kk;
+                    weight_parts(g.rec, C, 16 * P + j, 16 * first, wh, wm, wl);
+                    const unsigned both = bits[(t - 1) & 1][first][j] | bits[(t - 1) & 1][first + 1][j] << 16;
 #pragma unroll
-        for (int i = 0; i < kEach; ++i) {
-            const int c = threadIdx.x + i * kSoloThreads;
-            if (c >= C) continue;
-            const int64_t m = (int64_t)blockIdx.x * C + c, at = m * T + t;
-            double fb = 0.0;                         // one sum after the other: float32 would lose to the sums of the matrix cores
-            if (t > 0)
-                for (int k = 0; k < C; ++k) fb += (double)g.rec[(int64_t)c * C + k] * (double)spikes[(t - 1) & 1][k];
-            const StepValues o = nrn[i].step(g.z[at] + (float)fb, p);
-            spikes[t & 1][c] = o.spike;
-            g.spk[at] = o.spike;
-            g.vol[at] = o.voltage;
-            if (ALIF) g.theta[at] = o.theta;
-            if (t == T - 1) {
-                p.cur_last[m] = o.current;
-                p.vol_last[m] = o.voltage;
-                if (ALIF) { p.th_last[m] = o.threshold; p.ref_last[m] = o.refractory; }
+                    for (int a = 0; a < 4; ++a) {
+                        const uint4 b = spike_parts(both, a);
+                        acc[a & 1] = mfma_bf16(wh[a], b, acc[a & 1]);
+                        low = mfma_bf16(wm[a], b, low);
+                        low = mfma_bf16(wl[a], b, low);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) red[wave][i][lane] = acc[0][i] + acc[1][i] + low[i];
             }
-        }
-        __syncthreads();
-    }
+            __syncthreads();
+            const int c = 16 * P + j;
+            if (wave < 4) {
+                const bool mine = n < N && c < C;
+                bool spiked = false;
+                if (mine) {
+                    const int64_t m = (int64_t)n * C + c, at = m * T + t;
+                    StepNeuron<ALIF, false, POW2> nrn{};
+                    nrn.load_decays(p, c);
+                    if (t == 0) {
+                        nrn.load_states(p, m);
+                        nrn.check(p.range_flag);
+                    } else {
+                        nrn.yc = g.carried[m];
+                        nrn.yv = g.carried[nc + m];
+                        if (ALIF) { nrn.th = g.carried[2 * nc + m]; nrn.r = g.carried[3 * nc + m]; }
+                    }
+                    float z = g.z[at];
+                    if (t > 0) {
+                        float fb = 0.f;
 #pragma unroll
-    for (int i = 0; i < kEach; ++i)
-        if (threadIdx.x + i * kSoloThreads < (unsigned)C &&
-            (range_exceeded(nrn[i].acc_lif, 30) || range_exceeded(nrn[i].acc_th, 28)))
-            raise_range_flag(p.range_flag);
+                        for (int v = 0; v < kGridWaves; ++v) fb += red[v][j & 3][(j >> 2) * 16 + 4 * wave + kk];
+                        z += fb;
+                    }
+                    const StepValues o = nrn.step(z, p);
+                    spiked = o.spike > 0.0f;
+                    g.spk[at] = o.spike;
+                    g.vol[at] = o.voltage;
+                    if (ALIF) g.theta[at] = o.theta;
+                    g.carried[m] = nrn.yc;
+                    g.carried[nc + m] = nrn.yv;
+                    if (ALIF) { g.carried[2 * nc + m] = nrn.th; g.carried[3 * nc + m] = nrn.r; }
+                    if (t == T - 1) {
+                        p.cur_last[m] = o.current;
+                        p.vol_last[m] = o.voltage;
+                        if (ALIF) { p.th_last[m] = o.threshold; p.ref_last[m] = o.refractory; }
+                    }
+                    acc_lif |= nrn.acc_lif;
+                    acc_th |= nrn.acc_th;
+                }
+                const unsigned long long mask = __ballot(spiked);
+                if (lane < 4) bits[t & 1][P][4 * wave + lane] = (unsigned)((mask >> (16 * lane)) & 0xffffull);
+            }
+            __syncthreads();
+        }
+    }
+    if (range_exceeded(acc_lif, 30) || range_exceeded(acc_th, 28)) raise_range_flag(p.range_flag);
 }
 
 // ---- backward -----------------------------------------------------------------------------------------------------
@@ -904,7 +949,7 @@ bool launch_grid_fwd(const GridFwd& g, const GridPlan& plan, hipStream_t st) {
         ? (narrow ? (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 1, 1> : (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 2, 1>)
         : (narrow ? (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 1, 2> : (const void*)recurrent_grid_fwd_kernel<ALIF, POW2, 2, 2>);
     if (!launch_grid(k, plan.grid, (void*)&g, st)) return false;
-    hipLaunchKernelGGL((recurrent_solo_fwd_kernel<ALIF, POW2>), dim3((unsigned)g.p.N), dim3(kSoloThreads), 0, st, g);
+    hipLaunchKernelGGL((recurrent_solo_fwd_kernel<ALIF, POW2>), dim3((unsigned)(g.p.N + 15) / 16), dim3(kGridThreads), 0, st, g);
     return true;
 }
 
@@ -915,8 +960,8 @@ bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* th
     GridPlan plan;
     if (!grid_plan(p.N, p.C, p.T, st, &plan)) return false;
     const int64_t words = (int64_t)2 * plan.S * words_of(plan.KB);
-    if (workspace_floats < words + 4) return false;
     const int64_t nc = (int64_t)p.N * p.C, nct = nc * p.T;
+    if (workspace_floats < 4 + words + 4 * nc) return false;
     if (overlap({{spk, nct}, {vol, nct}, {theta, nct}, {p.cur_last, nc}, {p.vol_last, nc}, {p.th_last, nc}, {p.ref_last, nc}},
                 {{z, nct}, {rec, (int64_t)p.C * p.C}, {p.i_decay, p.n_id}, {p.v_decay, p.n_vd}, {p.th_decay, p.n_td},
                  {p.ref_decay, p.n_rd}, {p.i_state, p.n_is}, {p.v_state, p.n_vs}, {p.th_state, p.n_ts}, {p.ref_state, p.n_rs}}))
@@ -928,6 +973,7 @@ bool grid_fwd(StepFwd p, bool alif, bool pow2, float* spk, float* vol, float* th
     g.spk = spk; g.vol = vol; g.theta = theta; g.z = z; g.rec = rec;
     g.gave_up = reinterpret_cast<unsigned*>(workspace);
     g.words = reinterpret_cast<unsigned*>(workspace) + 4;
+    g.carried = reinterpret_cast<int*>(workspace) + 4 + words;
     hipLaunchKernelGGL(grid_fill_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, g.words, words, g.gave_up);
     const bool taken = alif ? (pow2 ? launch_grid_fwd<true, true>(g, plan, st) : launch_grid_fwd<true, false>(g, plan, st))
                             : (pow2 ? launch_grid_fwd<false, true>(g, plan, st) : launch_grid_fwd<false, false>(g, plan, st));
