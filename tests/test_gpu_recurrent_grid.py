@@ -3,6 +3,8 @@ tiles -- one and two sample tiles per workgroup, units of 128 presynaptic neuron
 sequence it takes -- against the CPU oracle, and with weights that are not on a quantiser's grid."""
 import os
 import subprocess
+import sys
+import threading
 
 import pytest
 import torch
@@ -206,3 +208,79 @@ def test_workgroups_that_give_up_waiting():
     run = subprocess.run([BINARY], capture_output=True, text=True, timeout=100)
     assert run.returncode == 0, run.stdout + run.stderr
     assert 'solo kernels agree' in run.stdout
+
+
+def _layer(slayer, n, c, t, seed):
+    gen = torch.Generator().manual_seed(seed)
+    neuron = base._neuron(slayer)
+    syn = base._Dense(c, gen).to(dev())
+    with torch.no_grad():
+        syn.weight.mul_(6.0 / c ** 0.5)
+    syn.pre_hook_fx = neuron.quantize_8bit
+    z = (torch.randn(n, c, t, generator=gen) * 1.5).to(dev()).requires_grad_()
+    return neuron, syn, z, torch.rand(n, c, t, generator=gen).to(dev())
+
+
+def _run_layer(slayer, neuron, syn, z, g):
+    out = slayer.utils.recurrent.custom_recurrent(z, neuron, syn)
+    grads = torch.autograd.grad(out, (z, syn.weight), g)
+    return (out.detach(), neuron.current_state, neuron.voltage_state) + grads
+
+
+def test_layers_on_two_streams_from_two_threads(slayer):
+    """Both fill the chip, so they cannot run side by side: each gives what it gives alone."""
+    sizes = [(32, 2048, 24), (40, 1028, 33)]
+    wants = [_run_layer(slayer, *_layer(slayer, *size, 3)) for size in sizes]
+    rounds = 4
+    layers = [[_layer(slayer, *size, 3) for _ in range(rounds)] for size in sizes]
+    torch.cuda.synchronize()
+    results, errors = [[], []], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for layer in layers[i]:
+                    results[i].append(_run_layer(slayer, *layer))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:                                     # shown by the main thread
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for got, want in zip(results, wants):
+        assert len(got) == rounds and 0.01 < float(want[0].mean()) < 0.9
+        for r in got:
+            for k, what in enumerate(('spikes', 'current', 'voltage')):
+                assert torch.equal(r[k], want[k]), what
+            assert_rel(r[3], want[3].cpu(), 'grad z')
+            assert_rel(r[4], want[4].cpu(), 'grad weight')
+
+
+CHILD = """
+import sys
+import torch
+import lava_dl_amd.slayer as slayer
+from tests import test_gpu_recurrent_grid as T
+torch.save([x.cpu() for x in T._run_layer(slayer, *T._layer(slayer, 5, 260, 20, 4))], sys.argv[1])
+"""
+
+
+def test_layer_in_a_process_beside_another(slayer, tmp_path):
+    """The runtime grants cooperative launches to one process at a time (here this one): the other's layer takes a launch per
+    step where it is refused, with the same spikes (quantised weights) and gradients."""
+    want = _run_layer(slayer, *_layer(slayer, 5, 260, 20, 4))
+    torch.cuda.synchronize()
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    path = str(tmp_path / 'child.pt')
+    run = subprocess.run([sys.executable, '-c', CHILD, path], cwd=root, env=dict(os.environ, PYTHONPATH=root),
+                         capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stdout + run.stderr
+    got = torch.load(path, weights_only=True)
+    for k, what in enumerate(('spikes', 'current', 'voltage')):
+        assert torch.equal(got[k], want[k].cpu()), what
+    assert_rel(got[3], want[3].cpu(), 'grad z')
+    assert_rel(got[4], want[4].cpu(), 'grad weight')

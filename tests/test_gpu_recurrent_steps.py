@@ -1,6 +1,8 @@
-"""Recurrent CUBA / ALIF layers through the launch-per-step kernels (layers wider than one workgroup per sample
-holds): the checks of the one-launch kernels repeated on this path (CPU oracle bit for bit with quantised weights,
-the loops of one-step calls), the two paths against each other, and wide layers at their natural size."""
+"""Recurrent CUBA / ALIF layers through the kernels for the whole batch (slayer_*_recurrent_steps_*): one launch spread over
+the chip, or one launch per time step for what that does not take -- layers beyond 2048 neurons, batches beyond the chip, graded
+spikes forward, fewer than 8 steps, streams under capture.  The checks of the kernels with one workgroup per sample repeated on
+these entry points (CPU oracle bit for bit with quantised weights, the loops of one-step calls), the two against each other,
+wide layers at their natural size, and each kernel of the launch-per-step form by sizes that must take it."""
 import pytest
 import torch
 
@@ -17,20 +19,44 @@ def slayer():
     return s
 
 
+PATTERN = 0x3f9e0652                       # what a workspace holds before the call
+
+
+def workspace_with_pattern(slayer, n, c, t, with_theta):
+    floats = slayer._native.lib().slayer_recurrent_steps_workspace(n, c, t, 1 if with_theta else 0)
+    return torch.full((floats,), PATTERN, dtype=torch.int32, device=dev()).view(torch.float32)
+
+
+def form_of(ws, n, c, t, with_theta):
+    """'steps' when the call that had this workspace took a launch per step, 'grid' for the one launch.  The launch per step
+    packs the weights behind the time-major tensors and the states; the one launch uses the front of the workspace only."""
+    kb, tiles, tiles64 = (c + 15) // 16, (n + 15) // 16 + 1, (c + 63) // 64
+    at = (4 if with_theta else 3) * n * c * t + 4 * n * c + kb * kb * 256 - 1
+    grid_end = 260 + max(4 * tiles * kb * 256, 4 * ((n + 3) // 4) * 2 * tiles64 * 256, 2 * tiles * (kb + 7) * 16 + 4 * n * c)
+    if t >= 8 and c <= 2048:
+        assert grid_end <= at, 'the two forms cannot be told apart at this size'
+    return 'grid' if int(ws.view(torch.int32)[at]) == PATTERN else 'steps'
+
+
+class Calls(list):
+    def forms(self):
+        return {form_of(ws, *size) for ws, size in self}
+
+
 @pytest.fixture()
 def by_steps(slayer, monkeypatch):
-    """Every layer whose width is a multiple of 4 takes the launch-per-step kernels; counts their calls."""
+    """Every layer whose width is a multiple of 4 takes the entry points for the whole batch; keeps the workspace of
+    each call, whose contents tell the form that it took."""
     R = slayer.utils.recurrent
-    calls = []
-    plain = R._steps_workspace
+    calls = Calls()
 
-    def counted(*a):
-        calls.append(a)
-        return plain(*a)
+    def kept(n, c, t, with_theta, device):
+        calls.append((workspace_with_pattern(slayer, n, c, t, with_theta), (n, c, t, with_theta)))
+        return calls[-1][0]
     monkeypatch.setattr(R, 'STEPS_FROM', 0)
-    monkeypatch.setattr(R, '_steps_workspace', counted)
+    monkeypatch.setattr(R, '_steps_workspace', kept)
     yield calls
-    assert calls, 'the launch-per-step path was not taken'
+    assert calls, 'the entry points for the whole batch were not taken'
 
 
 # batch sizes on either side of 16, 32 and 64 samples (one, two, four sample tiles, two workgroups along the batch),
@@ -52,6 +78,87 @@ def test_graded_cuba_layer_by_steps_matches_the_oracle(slayer, by_steps, n, c, t
     base.test_fused_cuba_loop_with_graded_spikes_matches_the_oracle(slayer, n, c, t)
 
 
+# What the one launch does not take: wider layers; 530 samples of 260 neurons, four sample tiles to a workgroup (2052: one,
+# 33 of 20: one per tile); fewer than 8 steps
+MUST_TAKE_STEPS = [(2, 2052, 9), (530, 260, 8), (3, 68, 7), (33, 20, 5), (70, 1028, 6)]
+
+
+@pytest.mark.parametrize('n,c,t', MUST_TAKE_STEPS)
+def test_cuba_layer_that_must_take_a_launch_per_step(slayer, by_steps, n, c, t):
+    base.test_fused_loop_matches_the_oracle(slayer, n, c, t, True)
+    assert by_steps.forms() == {'steps'} and len(by_steps) == 3
+
+
+@pytest.mark.parametrize('n,c,t', MUST_TAKE_STEPS)
+@pytest.mark.parametrize('graded', [False, True])
+def test_alif_layer_that_must_take_a_launch_per_step(slayer, by_steps, n, c, t, graded):
+    base.test_fused_alif_loop_matches_the_oracle(slayer, n, c, t, graded)
+    assert by_steps.forms() == {'steps'} and len(by_steps) == 3
+
+
+@pytest.mark.parametrize('n,c,t', MUST_TAKE_STEPS)
+def test_graded_cuba_layer_that_must_take_a_launch_per_step(slayer, by_steps, n, c, t):
+    base.test_fused_cuba_loop_with_graded_spikes_matches_the_oracle(slayer, n, c, t)
+    assert by_steps.forms() == {'steps'} and len(by_steps) == 2
+
+
+# one and two sample tiles to a workgroup
+@pytest.mark.parametrize('n,c,t', [(9, 516, 18), (33, 2048, 9), (129, 516, 10)])
+def test_alif_layer_in_one_launch(slayer, by_steps, n, c, t):
+    base.test_fused_alif_loop_matches_the_oracle(slayer, n, c, t, False)
+    assert by_steps.forms() == {'grid'} and len(by_steps) == 3
+
+
+@pytest.mark.parametrize('n,c,t', [(33, 2048, 9), (5, 68, 33)])
+def test_graded_gradients_in_one_launch(slayer, by_steps, n, c, t):
+    """Forward a launch per step, backward one launch."""
+    base.test_fused_cuba_loop_with_graded_spikes_matches_the_oracle(slayer, n, c, t)
+    assert [form_of(ws, *size) for ws, size in by_steps] == ['steps', 'grid']
+
+
+def test_layer_on_a_stream_under_capture(slayer):
+    """A captured call is one launch per step; its replays, with new inputs and eager calls between them, give what eager
+    calls (one launch) give: the same bits forward (quantised weights), the gradient to summation order."""
+    from lava_dl_amd.slayer import _native as N
+    n, c, t = 5, 260, 12
+    gen = torch.Generator().manual_seed(17)
+    zs = [(torch.randn(n, c, t, generator=gen) * 1.5).to(dev()) for _ in range(3)]
+    g = torch.rand(n, c, t, generator=gen).to(dev())
+    rec = ((torch.randn(c, c, generator=gen) * 32 * 6 / c ** 0.5).round() / 64).to(dev())
+    decay, zero = torch.full((1,), 1024.0, device=dev()), torch.zeros(1, device=dev())
+
+    def buffers():
+        return [torch.empty_like(g) for _ in range(3)] + [torch.empty(n, c, device=dev()) for _ in range(2)] + \
+            [workspace_with_pattern(slayer, n, c, t, False) for _ in range(2)]
+
+    def run(z, spk, vol, gz, cur, last, ws, ws_bwd):
+        N.check(N.lib().slayer_cuba_recurrent_steps_fwd(
+            N.ptr(spk), N.ptr(vol), N.ptr(cur), N.ptr(last), N.ptr(z), N.ptr(rec), N.ptr(decay), N.ptr(decay), N.ptr(zero),
+            N.ptr(zero), 1.25, 0, 1.0, 4096, n, c, 1, 1, 1, 1, t, N.ptr(ws), ws.numel(), N.stream_handle()))
+        N.check(N.lib().slayer_recurrent_steps_bwd(N.ptr(gz), N.ptr(g), N.ptr(vol), None, N.ptr(rec), 1.25, 1.0, 0.1, 0, n, c, t,
+                                                   N.ptr(ws_bwd), ws_bwd.numel(), N.stream_handle()))
+    wants = []
+    for z in zs:
+        eager = buffers()
+        run(z, *eager)
+        wants.append(eager)
+        assert {form_of(ws, n, c, t, False) for ws in eager[5:]} == {'grid'} and 0.01 < float(eager[0].mean()) < 0.9
+    z, captured = torch.zeros_like(g), buffers()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(z, *captured)
+    for k in (0, 1, 2, 0):
+        z.copy_(zs[k])
+        graph.replay()
+        run(zs[k - 1], *buffers())
+        torch.cuda.synchronize()
+        for i, what in ((0, 'spikes'), (1, 'voltage'), (3, 'carried current'), (4, 'carried voltage')):
+            assert torch.equal(captured[i], wants[k][i]), what
+        assert_rel(captured[2], wants[k][2].cpu(), 'grad z')
+    assert {form_of(ws, n, c, t, False) for ws in captured[5:]} == {'steps'}
+
+
 @pytest.mark.parametrize('kind,graded', [('alif', False), ('alif', True), ('cuba', True)])
 def test_layer_by_steps_matches_the_loops_of_one_step_calls(slayer, by_steps, kind, graded):
     base.test_fused_loop_of_other_neurons_matches_the_loops_of_one_step_calls(slayer, kind, graded)
@@ -59,7 +166,7 @@ def test_layer_by_steps_matches_the_loops_of_one_step_calls(slayer, by_steps, ki
 
 @pytest.mark.parametrize('kind', ['cuba', 'alif'])
 def test_the_two_kernel_paths_agree(slayer, monkeypatch, kind):
-    """One layer through the one-launch kernels and through the launch-per-step kernels: the same spikes and carried
+    """One layer through the kernels with one workgroup per sample and through those for the whole batch: the same spikes and carried
     states bit for bit (quantised weights), the same gradients to summation order."""
     R = slayer.utils.recurrent
     gen = torch.Generator().manual_seed(90210)
@@ -88,7 +195,7 @@ def test_the_two_kernel_paths_agree(slayer, monkeypatch, kind):
 
 @pytest.mark.parametrize('n,c,t', [(2, 1100, 12), (8, 2048, 24)])
 def test_wide_layers_match_the_oracle_and_the_generic_loop(slayer, n, c, t):
-    """Layers beyond 1024 neurons take the launch-per-step kernels by themselves."""
+    """Layers beyond 1024 neurons take the entry points for the whole batch by themselves."""
     R = slayer.utils.recurrent
     gen = torch.Generator().manual_seed(c + t)
     z = torch.randn(n, c, t, generator=gen)
@@ -147,7 +254,7 @@ def test_sizes_the_step_kernels_refuse(slayer):
 @pytest.mark.parametrize('c', [24, 260])
 def test_recurrent_layer_with_the_dense_synapse_module(slayer, c):
     """The recurrent synapse as the package's own Dense layer (what the reference's Recurrent blocks hold,
-    block/cuba.py:166-176): the kernels (one launch for 24 neurons, a launch per step for 260) and the plain loop
+    block/cuba.py:166-176): the kernels (one workgroup per sample for 24 neurons, the whole batch together for 260) and the plain loop
     that calls the synapse module step by step give the same spikes and weight gradients."""
     R = slayer.utils.recurrent
     gen = torch.Generator().manual_seed(c)
