@@ -869,12 +869,12 @@ class Recurrent(Workload):
     """A recurrent CUBA layer (utils/recurrent.py:45-112 in the reference: s[t] = neuron(z[t] + R s[t-1]), one neuron
     call per time step in a Python loop), forward and backward with the gradient of the recurrent weights, through
     the module interface (custom_recurrent).  The algorithmic bytes per neuron-timestep are those of the tensors
-    (z, spikes, voltage; gradient, voltage, gradient of z) plus 4 C / N for a [C x C] matrix read once a step for the
-    whole batch; the kernels that 2048 neurons take keep the matrix in registers and read it once a call."""
+    (z, spikes, voltage; gradient, voltage, gradient of z) plus 4 C / (N T) for the [C x C] matrix, read once a call as
+    the kernels that 2048 neurons take do, which keep it in registers."""
     name = 'Recurrent CUBA layer, 2048 neurons, fwd+bwd (module interface)'
     shape = (32, 2048, 300)
-    ops = [('recurrent_fwd', 'recurrent_grid_fwd_kernel, one launch', 12 + 4 * 2048 // 32),
-           ('recurrent_bwd', 'recurrent_grid_bwd_kernel, one launch, + weight-gradient GEMM', 12 + 4 * 2048 // 32)]
+    ops = [('recurrent_fwd', 'recurrent_grid_fwd_kernel, one launch', round(12 + 4 * 2048 / (32 * 300), 2)),
+           ('recurrent_bwd', 'recurrent_grid_bwd_kernel, one launch, + weight-gradient GEMM', round(12 + 4 * 2048 / (32 * 300), 2))]
     note = ('CUBA decays 0.25 / 0.25, threshold 1.25, z ~ 1.5 N(0,1), weights N(0, 0.6) * 6 / sqrt(C) quantised to '
             '8 bits (the synapse pre-hook), about 40 % of the neurons spike per step')
     generic_loop = False
@@ -932,8 +932,8 @@ class RecurrentLoop(Recurrent):
     """The same layer through the reference's loop of one-step neuron calls (CustomRecurrent, the path layers take
     that the kernels do not cover)."""
     name = 'Recurrent CUBA layer, 2048 neurons, fwd+bwd: loop of one-step neuron calls'
-    ops = [('recurrent_fwd', 'a dozen launches per time step (one-step neuron calls + torch.matmul)', 12 + 4 * 2048 // 32),
-           ('recurrent_bwd', 'autograd of every step + torch.matmul', 12 + 4 * 2048 // 32)]
+    ops = [('recurrent_fwd', 'a dozen launches per time step (one-step neuron calls + torch.matmul)', round(12 + 4 * 2048 / (32 * 300), 2)),
+           ('recurrent_bwd', 'autograd of every step + torch.matmul', round(12 + 4 * 2048 / (32 * 300), 2))]
     generic_loop = True
 
 
