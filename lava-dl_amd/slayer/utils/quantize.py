@@ -14,12 +14,10 @@ class MODE(IntEnum):
     FLOOR = 1
 
 
-def _is_number(*values):
-    """Plain numbers: not tensors or arrays, whose elements differ, may be trained, or lie on the GPU."""
-    return all(isinstance(v, (int, float, np.integer, np.floating)) for v in values)
-
-
+# Plain numbers: not tensors or arrays, whose elements differ, may be trained, or lie on the GPU.
+_NUMBER = (int, float, np.integer, np.floating)
 _FLOAT32_MAX = torch.finfo(torch.float32).max
+_STEP_MIN, _STEP_MAX = 2.0 ** -126, 2.0 ** 126                      # steps whose reciprocal is a float32 number too
 
 
 class _StraightThrough(torch.autograd.Function):
@@ -27,7 +25,7 @@ class _StraightThrough(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, input, step, use_floor):
-        if _is_number(step) and step == 1:                          # what follows, without the two products by one
+        if isinstance(step, _NUMBER) and step == 1:                          # what follows, without the two products by one
             return torch.floor(input) if use_floor else torch.round(input)
         scaled = input / step
         return (torch.floor(scaled) if use_floor else torch.round(scaled)) * step
@@ -43,7 +41,7 @@ def quantize(input, step=1, mode=MODE.ROUND):
         raise ValueError(f'{mode=} is not recognized.')
     if not (torch.is_grad_enabled() and input.requires_grad):      # nothing to pass a gradient to
         snap = torch.floor if mode == MODE.FLOOR else torch.round
-        return snap(input) if _is_number(step) and step == 1 else snap(input / step) * step
+        return snap(input) if isinstance(step, _NUMBER) and step == 1 else snap(input / step) * step
     return _StraightThrough.apply(input, step, mode == MODE.FLOOR)
 
 
@@ -87,14 +85,14 @@ def takes_kernel(input, contiguous=True):
             and torch._C._len_torch_dispatch_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and forward_ad._current_level < 0
             and not torch._C._functorch.is_legacy_batchedtensor(input)
-            and not torch._C._functorch.is_functorch_wrapped_tensor(input)
             and (not contiguous or input.is_contiguous()))
 
 
 def _fits_kernel(step, lo, hi, scale):
-    """Plain numbers that are float32 numbers too, and a step whose reciprocal is one."""
-    return (_is_number(step, lo, hi, scale) and 2.0 ** -126 <= abs(step) <= 2.0 ** 126
-            and all(abs(v) <= _FLOAT32_MAX for v in (lo, hi, scale)))
+    """Plain numbers inside the range of float32."""
+    return (isinstance(step, _NUMBER) and isinstance(lo, _NUMBER) and isinstance(hi, _NUMBER) and isinstance(scale, _NUMBER)
+            and _STEP_MIN <= abs(step) <= _STEP_MAX and -_FLOAT32_MAX <= lo <= _FLOAT32_MAX
+            and -_FLOAT32_MAX <= hi <= _FLOAT32_MAX and -_FLOAT32_MAX <= scale <= _FLOAT32_MAX)
 
 
 def limit(input, step, lo, hi, scale=1):
@@ -102,7 +100,7 @@ def limit(input, step, lo, hi, scale=1):
     trained); those take the operators."""
     if not (takes_kernel(input) and _fits_kernel(step, lo, hi, scale)):
         q = quantize(input, step=step).clamp(lo, hi)
-        return q if _is_number(scale) and scale == 1 else q * scale
+        return q if isinstance(scale, _NUMBER) and scale == 1 else q * scale
     if torch.is_grad_enabled() and input.requires_grad:
         return _Limited.apply(input, float(step), float(lo), float(hi), float(scale))
     return _launch(input, float(step), float(lo), float(hi), float(scale), None)
