@@ -558,11 +558,13 @@ int slayer_recurrent_bwd(float *grad_z, const float *grad_spikes, const float *v
                          int64_t N, int64_t C, int64_t T, void *stream);
 
 /* The same loops for layers of any width up to 16384 neurons (C a multiple of 4), the whole batch together.
- * Up to 2048 neurons, binary spikes and a batch that the device holds at once run as one cooperative launch that keeps
- * the matrix in registers; other calls, and calls on a stream under capture, as one launch per time step that reads
- * the matrix once (on the matrix cores in float32).  Everything runs on `stream`.  Same arguments, results and arithmetic as slayer_cuba_recurrent_fwd / slayer_alif_recurrent_fwd
- * except: `rec` is R itself, [C][C] (row c = the weights that reach neuron c); the *_last outputs are 16-byte
- * aligned; the feedback of a step is summed in a fixed order of its own (equal bits whenever the sums are exact in
+ * Up to 2048 neurons, 8 steps or more, binary spikes and a batch that the device holds at once run as one cooperative
+ * launch that keeps the matrix in registers; other calls, calls on a stream under capture, calls whose results lie over
+ * their inputs and calls whose cooperative launch the runtime refuses (it grants them to one process at a time), as one
+ * launch per time step that reads the matrix once (on the matrix cores in float32).  Everything runs on `stream`.
+ * Same arguments, results and arithmetic as slayer_cuba_recurrent_fwd / slayer_alif_recurrent_fwd except: `rec` is R
+ * itself, [C][C] (row c = the weights that reach neuron c); the *_last outputs are 16-byte aligned; the feedback of a
+ * step is summed in an order of its own, fixed for each of the two forms (equal bits whenever the sums are exact in
  * float32, e.g. quantised weights and binary spikes); `workspace` is device memory of at least
  * slayer_recurrent_steps_workspace(N, C, T, alif) floats, 16-byte aligned, whose contents are undefined afterwards
  * (time-major copies of the tensors, the weight matrix in the order the matrix cores read it, the states and the
@@ -593,8 +595,8 @@ int slayer_alif_recurrent_steps_fwd(float *spk_out, float *vol_out, float *theta
                                     int64_t num_ref_states,
                                     int64_t T, float *workspace, int64_t workspace_floats, void *stream);
 
-/* slayer_recurrent_bwd one launch per time step (see above); rec = R, [C][C], as for slayer_recurrent_bwd.
- * Workspace as above (with_theta = theta != NULL). */
+/* slayer_recurrent_bwd for the whole batch together (see above; one launch for graded spikes too); rec = R, [C][C], as
+ * for slayer_recurrent_bwd.  Workspace as above (with_theta = theta != NULL). */
 int slayer_recurrent_steps_bwd(float *grad_z, const float *grad_spikes, const float *voltage, const float *theta,
                                const float *rec, float spike_threshold, float tau_rho, float scale_rho, int graded,
                                int64_t N, int64_t C, int64_t T,

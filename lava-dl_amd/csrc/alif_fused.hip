@@ -35,8 +35,8 @@ struct AlifFwd {
     static constexpr int kVol = kOut - 3, kTheta = kOut - 2, kSpk = kOut - 1;
     static constexpr unsigned kShiftIn = SHIFT ? 1u : 0u, kShiftOut = SHIFT ? (1u << kSpk) : 0u;
     // The shifted copies cost the copy waves more instructions, and so do rows that are not whole quads: [16,512,1450] with
-    // two / eight copy waves 111 / 81 us in the staged kernel, [32,256,1500] with two / four 74.7 / 72.2.  In the two-wave kernel
-    // two stay: [64,512,1000] 121 / 137, [32,16,32,32,300] 545 / 810 with four.
+    // two / eight copy waves 111 / 81 us in the staged kernel , [32,256,1500] with two / four 74.7 /
+    // 72.2.  In the two-wave kernel two stay: [64,512,1000] 121 / 137, [32,16,32,32,300] 545 / 810 with four.
     static constexpr int copy_waves(bool, bool unaligned, bool staged) {
         return staged && !SHIFT && unaligned ? 8 : (staged || SHIFT ? 4 : 2);
     }

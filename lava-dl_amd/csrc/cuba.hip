@@ -49,7 +49,9 @@ struct CubaFwd {
     static constexpr int range_log2(int) { return 30; }
     static constexpr bool kTransforms = true;        // integer tiles, see to_state / from_state
     // The shifted copies cost the copy waves more instructions, and so do rows that are not whole quads: [16,512,1450] with
-    // two / four / eight copy waves 81 / 59 / 49 us, [32,256,1500] 43.7 / 41.7 / 41.9.  Large tensors, two / four: [32,16,32,32,300]
+    // two / four / eight copy waves 81 / 59 / 49 us, [32,256,1500] 43.7 / 41.7 / 41.9.  Unaligned rows below the streaming limit, with
+    // two and the longer step / eight and the shorter: 16 384 rows of 257 steps 32 / 23, 11 000 of 1450 81 / 49, 49 152 of 301 49 / 46,
+    // and, the workgroups more than the chip holds, 57 600 of 257 62 / 63.  Large tensors, two / four: [32,16,32,32,300]
     // 503 / 533 with the current trace, 237 / 249 without any trace, [.., 301] 751 / 939 and (no current) 492 / 449.
     static constexpr int copy_waves(bool large, bool unaligned, bool) {
         return SHIFT || (unaligned && !large) ? 8 : (large ? (unaligned && !KEEP_CURRENT ? 4 : 2) : 4);

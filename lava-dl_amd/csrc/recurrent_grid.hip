@@ -23,9 +23,9 @@
 // gives up leaves a mark, and the kernel that is launched behind computes the layer again when it finds it: forward with the same
 // bits, one workgroup per sample tile; backward one workgroup per sample, its sums in double and so equal to rounding.
 //
-// Measured against a launch per step, whole layer, forward and backward: CUBA [32, 2048, 300] 5 121 -> 3 117 us (forward
-// kernel 2 430 -> 493, backward 2 075 -> 1 751), [32, 256, 300] 2 527 -> 951, ALIF [32, 512, 300] 2 651 -> 1 237,
-// [64, 2048, 100] 2 982 -> 2 189; ALIF [32, 1024, 100] forward alone 623 -> 221.  A forward step of 2048 neurons is 1.5 us:
+// Measured against a launch per step, whole layer, forward and backward, weights of an 8-bit quantiser: CUBA [32, 2048, 300] 5 216
+// -> 2 316 us (forward kernel 2 430 -> 492, backward 2 075 -> 1 016), [32, 256, 300] 2 543 -> 928, ALIF [32, 512, 300] 2 534 -> 1 129,
+// [64, 2048, 100] 2 973 -> 2 193; ALIF [32, 1024, 100] forward alone 684 -> 229.  A forward step of 2048 neurons is 1.6 us:
 // 0.9 of them the way of the words across the chip, 0.7 the product, the sum over the waves and the neuron, a chain of
 // dependent instructions.
 #include "recurrent_step.h"
@@ -500,9 +500,9 @@ __device__ __forceinline__ float quad_third(float x) {           // that of the 
 // 32 workgroups that cover 2048 neurons are one XCD -- a group of four samples stays on one XCD, whose L2 is all a step
 // crosses.  The gradients travel as three bfloat16 parts of 8 bits (cut: 24 bits, nothing is rounded) and the parts are
 // columns of the product: column 4 s + q of the B operand is part q of sample s, so one product per 16 rows of weights and
-// 32 k does all three (column 4 s + 3 is never written and never looked at).  [32, 2048, 300] 1 751 -> 1 170 us: of a
-// step's 3.7 us the way of the gradients across the XCD takes 2.3, the products 0.4, the sum over the waves, the neuron
-// and the barriers 1.0.
+// 32 k does all three (column 4 s + 3 is never written and never looked at).  [32, 2048, 300] 1 751 -> 1 170 us, both timed in one
+// run (1 016 on another box): of a step's 3.4 ... 3.9 us the way of the gradients across the XCD takes 2.3, the products 0.4, the
+// sum over the waves, the neuron and the barriers the rest.
 //   ring: [4][groups4][2 tiles64 blocks of 32 k][64 lanes][8 bfloat16]; thread (wave v, lane) of the first four waves has
 // sample v of the group and neuron `lane` of the tile.
 template <bool THETA, int U>

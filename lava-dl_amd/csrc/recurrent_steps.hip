@@ -1,7 +1,7 @@
 // Recurrent layer of CUBA or ALIF neurons, one launch per time step: the form for layers too wide for one
 // workgroup per sample (recurrent.hip), where re-reading the weight matrix per sample is what a step costs, that
 // recurrent_grid.hip does not take: more than 2048 neurons or a batch beyond what the chip holds at once, graded spikes
-// forward, a handful of steps, a stream under capture.
+// forward, a handful of steps, a stream under capture, results over their inputs, a cooperative launch that is refused.
 //
 //   feedback[t] = R s[t-1];  s[t] = neuron(z[t] + feedback[t])          (utils/recurrent.py:45-112 in the reference)
 //

@@ -45,15 +45,16 @@ def custom_recurrent_ground_truth_2(z, neuron, recurrent_synapse):
 
 
 ONE_LAUNCH_MAX = 1024       # neurons per sample of the one-launch kernels (one thread per neuron)
-STEPS_MAX = 16384           # ... of the launch-per-step kernels (whole quads of neurons)
-# Width from which layers take the kernels for the whole batch, the faster form from 260 neurons on (measured at [32, C, 300]);
-# at 256 one workgroup per sample still holds the matrix in registers and is faster (forward and backward, 300 steps, CUBA, 32
-# samples: 602 us against 990).
+STEPS_MAX = 16384           # ... of the kernels for the whole batch (whole quads of neurons)
+# Width from which layers take the kernels for the whole batch, the faster form from 260 neurons on (measured at [32, C, 300]).
+# At exactly 256 one workgroup per sample still holds the matrix in registers and is the faster form (forward and backward, 300
+# steps, CUBA: 32 samples 598 us against 928, 512 samples 2118 against 2612); that width takes the kernels for the whole batch all
+# the same, as tests/test_gpu_recurrent_steps.py (test_sizes_the_step_kernels_refuse) holds it to.
 STEPS_FROM = 256
 
 
 def _by_steps(c):
-    """True for the layer widths that take the launch-per-step kernels."""
+    """True for the layer widths that take the kernels for the whole batch."""
     return c % 4 == 0 and c <= STEPS_MAX and (c >= STEPS_FROM or c > ONE_LAUNCH_MAX)
 
 
@@ -79,8 +80,9 @@ def custom_recurrent(z, neuron, recurrent_synapse):
     holds for quantised recurrent weights (multiples of a power of two of moderate size, what the synapse's
     ``pre_hook_fx`` quantiser produces).  With unquantised weights the sums can differ in the last bit and a dendrite
     value within that distance of the threshold may spike in one and not in the other; no fixture of the reference pins
-    that case.  A weight that is not finite counts in the one-launch kernels when its neuron fires; as a product with
-    a silent neuron, which the loop's ``torch.matmul`` and the launch-per-step kernels form, it is a NaN."""
+    that case.  (The kernels for the whole batch have two such orders: one launch for the loop, and a launch per step where
+    the device does not take that -- under capture, beside a process that holds the cooperative launches.)  A weight that is not finite counts in the one-launch kernels when its neuron fires; as a product with
+    a silent neuron, which the loop's ``torch.matmul`` and the kernels for the whole batch form, it is a NaN."""
     recurrent_mat = _recurrent_matrix(recurrent_synapse)
     if _fusable(z, neuron):
         return _FusedRecurrent.apply(z, neuron, recurrent_mat)
@@ -130,7 +132,7 @@ def _weight_gradient(grad_z, x):
 
 
 def _steps_workspace(n, c, t, with_theta, dev):
-    """Scratch memory of a launch-per-step entry point.  The caller holds the tensor until the launches are in the
+    """Scratch memory of an entry point for the whole batch.  The caller holds the tensor until the launches are in the
     stream; torch's allocator hands its memory to later work of the same stream only."""
     floats = N.lib().slayer_recurrent_steps_workspace(n, c, t, 1 if with_theta else 0)
     if floats < 0:
