@@ -501,7 +501,7 @@ __device__ __forceinline__ float quad_third(float x) {           // that of the 
 // crosses.  The gradients travel as three bfloat16 parts of 8 bits (cut: 24 bits, nothing is rounded) and the parts are
 // columns of the product: column 4 s + q of the B operand is part q of sample s, so one product per 16 rows of weights and
 // 32 k does all three (column 4 s + 3 is never written and never looked at).  [32, 2048, 300] 1 751 -> 1 170 us, both timed in one
-// run (1 016 on another box): of a step's 3.4 ... 3.9 us the way of the gradients across the XCD takes 2.3, the products 0.4, the
+// run (1 016 on another card): of a step's 3.4 ... 3.9 us the way of the gradients across the XCD takes 2.3, the products 0.4, the
 // sum over the waves, the neuron and the barriers the rest.
 //   ring: [4][groups4][2 tiles64 blocks of 32 k][64 lanes][8 bfloat16]; thread (wave v, lane) of the first four waves has
 // sample v of the group and neuron `lane` of the tile.
