@@ -668,8 +668,8 @@ class ConvSynapse(Cuba):
     place.  Weights are multiples of 1/64 (quantised, as a SLAYER synapse's are), so the weighted spikes are exact
     and the forward parity check stays bit for bit.  Bytes per neuron-timestep of the output tensor."""
     name = 'Conv synapse (3x3, 8 -> 16 channels) -> fused CUBA neuron, fwd+bwd (input and weight gradients)'
-    ops = [('conv_synapse', 'synapse_conv_split_kernel', 6), ('cuba_fwd', 'stream_kernel_staged<CubaFwd>', 16),
-           ('cuba_bwd', 'cuba_bwd_scan_kernel', 16), ('conv_synapse_bwd', 'synapse_conv_split_kernel', 6),
+    ops = [('conv_synapse', 'synapse_walk_kernel', 6), ('cuba_fwd', 'stream_kernel_staged<CubaFwd>', 16),
+           ('cuba_bwd', 'cuba_bwd_scan_kernel', 16), ('conv_synapse_bwd', 'synapse_walk_kernel', 6),
            ('conv_synapse_wgrad', 'synapse_wgrad_row_kernel', 6)]
     weight_gradient = True
     note = Cuba.note + '; input spikes Bernoulli(0.05) on 8 channels, weights round(N(0, 0.3) * 64) / 64'
@@ -789,7 +789,7 @@ class ConvTransposeSynapse(Workload):
     quarter of the pixels)."""
     name = 'ConvTranspose synapse 4x4 stride 2, 16 -> 8 channels, 16x16 -> 32x32, fwd + input and weight gradients'
     shape = (32, 8, 32, 32, 300)
-    ops = [('conv_transpose', 'synapse_conv_split_kernel<2> x 4 residue classes', 6), ('conv_transpose_bwd', 'synapse_conv_kernel (stride 2)', 6),
+    ops = [('conv_transpose', 'synapse_walk_kernel', 6), ('conv_transpose_bwd', 'synapse_walk_kernel', 6),
            ('conv_transpose_wgrad', 'synapse_wgrad_kernel', 6)]
     note = 'input spikes Bernoulli(0.05) on 16 channels of 16x16, weights round(N(0, 0.3) * 64) / 64, upstream gradient N(0, 1)'
 

@@ -3,104 +3,27 @@
 // A SLAYER conv synapse is a spatial convolution applied at every time step (synapse/layer.py:297-323 in the
 // reference: F.conv3d with a kernel of (kh, kw, 1) on [N, C, H, W, T]).  A library conv3d wants channels last: it
 // transposes the tensor there and back around its kernel, three passes over tensors whose innermost axis is already
-// the one the neuron kernels walk.  Here the tensors stay as they are: for an output pixel (n, h, w) and a tile of
-// 64 time steps the [Co x 64] result is the [Co x K] weight matrix (K = Ci * kh * kw) times the [K x 64] matrix
-// whose row k is the input row of tap k -- 64 consecutive floats of the input as it lies in memory.  One wavefront
-// takes 16 output channels x 64 steps of one pixel at a time on the matrix cores (v_mfma_f32_16x16x4_f32: float32
-// operands, float32 accumulation) and walks along the image row, so neighbouring pixels find their shared input
-// rows in the cache; a wave-wide load is four input rows of 256 bytes, a wave-wide store four output rows.
+// the one the neuron kernels walk.  Here the tensors stay as they are.  Forward pass and input gradient run on the walking
+// kernel (synapse_walk.hip); this file has the one-pixel kernel for the geometries that it does not take, the
+// one-channel layers, the weight gradient and the entry points.
+//
+// One-pixel kernel: for an output pixel (n, h, w) and a tile of 64 time steps the [Co x 64] result is the [Co x K] weight matrix
+// (K = Ci * kh * kw) times the [K x 64] matrix whose row k is the input row of tap k -- 64 consecutive floats of the input as it
+// lies in memory.  One wavefront takes 16 output channels x 64 steps of one pixel at a time on the matrix cores
+// (v_mfma_f32_16x16x4_f32: float32 operands, float32 accumulation) and walks along the image row, so neighbouring pixels find
+// their shared input rows in the cache; a wave-wide load is four input rows of 256 bytes, a wave-wide store four output rows.
 //
 // Lane (kk, j) = (lane / 16, lane % 16) loads steps 4j .. 4j+3 of tap 4g + kk for tap group g: element e of that
 // quad is the B operand of the e-th of four matrix products, whose column j stands for step 4j + e; lane (q, j) of a
 // result then holds output channels 4q .. 4q+3 of step 4j + e, i.e. over e a quad of consecutive steps per channel.
-#include "common.h"
+#include "synapse.h"
 #include "split.h"
-#include "tile.h"
 
 namespace slayer {
 
 int launch_zero_fill(float* p, int64_t n, hipStream_t stream);          // li.hip
 
-typedef float syn_f4 __attribute__((ext_vector_type(4)));
-
-// Rows of any length (T >= 4): a quad of steps is a 16-byte access at a dword-aligned address, and the last quad of
-// a row may hold fewer than four steps (nv of them).  Such a quad is loaded four steps before the end of its row --
-// never beyond it -- and moved into place: element e of the result is element e + 4 - nv of what was loaded, zero
-// behind the row's end.  Stores leave the steps that do not exist out.
-struct SynQuad {
-    int t_load;                         // step the quad is loaded at
-    int nv;                             // steps of the quad that exist (<= 0: none, the lane loads nothing)
-    template <bool TAIL>
-    __device__ __forceinline__ void set(int t, int t_end) {
-        nv = t_end - t;
-        t_load = (TAIL && nv > 0 && nv < 4) ? t_end - 4 : t;
-    }
-    __device__ __forceinline__ bool any() const { return nv > 0; }
-    __device__ __forceinline__ bool partial() const { return nv > 0 && nv < 4; }
-    // TAIL: the rows are not whole quads (decided on the host: a test per load would sit between the loads)
-    template <bool TAIL>
-    __device__ __forceinline__ float4 place(float4 q) const {
-        if (!TAIL || !__any(partial())) return q;                        // only the tile that holds the end of the rows
-        const int d = partial() ? 4 - nv : 0;
-        const float a[4] = {q.x, q.y, q.z, q.w};
-        float r[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int i = e + d;
-            r[e] = i == 0 ? a[0] : (i == 1 ? a[1] : (i == 2 ? a[2] : (i == 3 ? a[3] : 0.f)));
-        }
-        return make_float4(r[0], r[1], r[2], r[3]);
-    }
-};
-// the quad v at byte offset off, of which the first nv elements exist (nv <= 0: nothing is stored)
-template <bool STREAM, bool TAIL>
-__device__ __forceinline__ void syn_store_quad(__amdgpu_buffer_rsrc_t dst, bool on, int off, int nv, float4 v) {
-    buf_store4<STREAM>(dst, (on && nv >= 4) ? off : kOutOfRange, v);
-    if (TAIL && __any(on && nv > 0 && nv < 4)) {                                 // only the tile that holds the end of the rows
-        const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 3; ++i) buf_store1<false>(dst, (on && nv < 4 && i < nv) ? off + 4 * i : kOutOfRange, e[i]);
-    }
-}
-
-// Workgroups are handed to the chip's eight XCDs round-robin by their index, and each XCD has an L2 of its own.
-// Neighbouring work items of the kernels below share most of what they read (an input row serves the output rows
-// above and below it and the neighbouring time shares of the weight gradient), so taken in index order every XCD
-// fetched nearly every row for itself: FETCH_SIZE read 5.0 x the input tensor for the forward kernel on
-// [32,8,32,32,300] -> 16 channels, 1.4 x with the permuted index below, by which XCD x gets the x-th contiguous eighth
-// of the work.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_contiguous(int b, int nb) {
-    const int x = b % kXcds, slot = b / kXcds, q = nb / kXcds, r = nb % kXcds;
-    return x * q + (x < r ? x : r) + slot;
-}
-
-constexpr int kSynTile = 64;            // time steps per tile
-constexpr int kSynWaves = 4;            // waves per workgroup: same output channels, same image row, different tiles
-
 constexpr int kSynChunk = 6;            // tap groups whose loads are in flight together (fewer for filters of a few taps)
-
-struct SynapseConv {
-    float* out;
-    const float* in;
-    const float* weight;                // [Co][Ci][kh_full][kw_full]
-    int N, Ci, Co, H, W, Ho, Wo, T;
-    int kh, kw, sh, sw, ph, pw, dh, dw; // ph, pw: may be negative (a window that begins inside the image)
-    int K, KG;                          // taps, groups of four taps (a whole number of chunks, padded with null taps)
-    int ttiles, wsplit;                 // tiles of 64 steps per row, pieces an image row is cut into
-    int items;                          // (tile, piece, output row) triples of one (batch entry, channel block)
-    // The taps may be a sub-lattice of a larger filter and the outputs a sub-lattice of a larger image (identity for
-    // a plain convolution): row iy of the kh x kw taps is row ky0 + iy * kys of the weight tensor's kh_full rows,
-    // output pixel (ho, wo) is pixel (oy0 + ho * oys, ox0 + wo * oxs) of a tensor [Co][Ho_full][Wo_full][T].
-    int kh_full, kw_full, ky0, kys, kx0, kxs;
-    int Ho_full, Wo_full, oy0, oys, ox0, oxs;
-    __device__ __forceinline__ int weight_index(int ci, int iy, int ix) const {
-        return (ci * kh_full + ky0 + iy * kys) * kw_full + kx0 + ix * kxs;
-    }
-    __device__ __forceinline__ int out_pixel(int ho, int wo) const {     // in pixels of the full output image
-        return (oy0 + ho * oys) * Wo_full + ox0 + wo * oxs;
-    }
-};
 
 // The gradient of the input of a convolution with strides (what conv_transpose3d computes, the ConvTranspose synapse
 // of synapse/layer.py:513-560 in the reference) is one plain convolution per residue class of the output pixels: the
@@ -199,374 +122,6 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_kernel(const S
             syn_store_quad<STREAM, TAIL>(dst, co < p.Co, co * (p.Ho_full * p.Wo_full * p.T * 4) + opix, nv,
                                    make_float4(acc[0][i], acc[1][i], acc[2][i], acc[3][i]));
         }
-    }
-}
-
-// The common case -- unit stride and dilation along the image row, KW taps per row -- takes PIX neighbouring
-// output pixels at a time: they share their input columns (PIX + KW - 1 of them instead of PIX * KW), so a group of
-// four (input channel, kernel row) pairs costs PIX + KW - 1 loads for PIX * KW * 4 matrix products.  Measured on
-// [32,8,32,32,300] -> 16 channels, 3x3: the one-pixel form is bound by what the caches deliver to the loads
-// (18 KB per pixel and tile of 64 steps), not by the matrix cores.
-// LDS: weights as above (tap k = pair * KW + x, pair = ci * kh + y), and per pair the byte offset of its input row
-// relative to the pixel block's own position and its row displacement.
-template <int KW, int PIX, bool STREAM, bool TAIL>
-__device__ __forceinline__ void synapse_conv_row(const SynapseConv& p) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int PG = p.KG;                                // groups of four pairs
-    const int Kp = PG * 4 * KW;
-    float* wt = lds;                                    // [Kp][16]
-    int* pair_off = reinterpret_cast<int*>(lds + Kp * 16);  // [4 PG] bytes
-    int* pair_dy = pair_off + 4 * PG;                   // [4 PG]
-
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int groups = (p.items + kSynWaves - 1) / kSynWaves;
-    int b = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int ig = b % groups; b /= groups;
-    const int cob = b % ((p.Co + 15) / 16);
-    const int n = b / ((p.Co + 15) / 16);
-    const int co0 = cob * 16;
-
-    const int64_t k_full = (int64_t)p.Ci * p.kh_full * p.kw_full;
-    // eight loads of a thread in flight at a time (one after the other they were a fifth of a workgroup's life)
-    for (int i0 = tid; i0 < Kp * 16; i0 += 8 * kSynWaves * kWave) {
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = i0 + u * kSynWaves * kWave;
-            const int k = i >> 4, m = i & 15;
-            const int pr = k / KW, x = k - pr * KW, ci = pr / p.kh, y = pr - ci * p.kh;
-            v[u] = (k < p.K && co0 + m < p.Co) ? p.weight[(int64_t)(co0 + m) * k_full + p.weight_index(ci, y, x)] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = i0 + u * kSynWaves * kWave;
-            if (i < Kp * 16) wt[i] = v[u];
-        }
-    }
-    for (int pr = tid; pr < 4 * PG; pr += kSynWaves * kWave) {
-        const int ci = pr / p.kh, y = pr - ci * p.kh;
-        const int dy = y * p.dh - p.ph;
-        pair_dy[pr] = pr < p.Ci * p.kh ? dy : (1 << 28);                 // a pair that does not exist: always outside
-        pair_off[pr] = (((ci * p.H + dy) * p.W) - p.pw) * p.T * 4;
-    }
-    __syncthreads();
-
-    const int item = ig * kSynWaves + wave;
-    if (item >= p.items) return;
-    const int tile = item % p.ttiles;
-    const int piece = (item / p.ttiles) % p.wsplit;
-    const int ho = item / (p.ttiles * p.wsplit);
-    const int t0 = tile * kSynTile;
-    const int kk = lane >> 4, j = lane & 15;
-    SynQuad tq;
-    tq.template set<TAIL>(t0 + 4 * j, p.T);
-    const int nv = tq.nv;
-    const bool t_ok = tq.any();
-    const int hin = ho * p.sh;
-    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
-    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
-    const int64_t out_plane = (int64_t)p.Co * p.Ho_full * p.Wo_full * p.T;
-    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
-    const int col = p.T * 4;                                             // bytes from a pixel to its right neighbour
-
-    const int per = ((p.Wo + p.wsplit - 1) / p.wsplit + PIX - 1) / PIX * PIX;
-    const int w_lo = piece * per, w_hi = (w_lo + per) < p.Wo ? (w_lo + per) : p.Wo;
-    for (int wo0 = w_lo; wo0 < w_hi; wo0 += PIX) {
-        const int pix = ((hin * p.W) + wo0) * col + tq.t_load * 4;
-        syn_f4 acc[PIX][4];
-#pragma unroll
-        for (int i = 0; i < PIX; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[i][e] = syn_f4{0.f, 0.f, 0.f, 0.f};
-        for (int g = 0; g < PG; ++g) {
-            const int pr = 4 * g + kk;
-            const bool row_ok = t_ok && (unsigned)(hin + pair_dy[pr]) < (unsigned)p.H;
-            const int base = pix + pair_off[pr];
-            float4 q[PIX + KW - 1];
-#pragma unroll
-            for (int c = 0; c < PIX + KW - 1; ++c) {
-                const bool ok = row_ok && (unsigned)(wo0 + c - p.pw) < (unsigned)p.W;
-                q[c] = tq.template place<TAIL>(buf_load4<false>(src, ok ? base + c * col : kOutOfRange));
-            }
-            float a[KW];
-#pragma unroll
-            for (int x = 0; x < KW; ++x) a[x] = wt[(pr * KW + x) * 16 + j];
-#pragma unroll
-            for (int x = 0; x < KW; ++x) {
-#pragma unroll
-                for (int i = 0; i < PIX; ++i) {
-                    acc[i][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], q[i + x].x, acc[i][0], 0, 0, 0);
-                    acc[i][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], q[i + x].y, acc[i][1], 0, 0, 0);
-                    acc[i][2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], q[i + x].z, acc[i][2], 0, 0, 0);
-                    acc[i][3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x], q[i + x].w, acc[i][3], 0, 0, 0);
-                }
-            }
-        }
-        // lane (kk, j): output channels co0 + 4 kk + i, steps t0 + 4 j + e
-#pragma unroll
-        for (int px = 0; px < PIX; ++px) {
-            const int opix = p.out_pixel(ho, wo0 + px) * col + (t0 + 4 * j) * 4;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int co = co0 + 4 * kk + i;
-                syn_store_quad<STREAM, TAIL>(dst, co < p.Co && wo0 + px < w_hi, co * (p.Ho_full * p.Wo_full * col) + opix, nv,
-                                       make_float4(acc[px][0][i], acc[px][1][i], acc[px][2][i], acc[px][3][i]));
-            }
-        }
-    }
-}
-
-// Rows of whole quads at five waves per SIMD (88 registers, no spills; four waves otherwise: 2-3 % slower); the
-// forms for rows that end inside a quad need a few registers more and keep the compiler's own choice.
-template <int KW, int PIX, bool STREAM>
-__global__ __launch_bounds__(kSynWaves * kWave) __attribute__((amdgpu_waves_per_eu(5)))
-void synapse_conv_row_kernel(const SynapseConv p) { synapse_conv_row<KW, PIX, STREAM, false>(p); }
-template <int KW, int PIX, bool STREAM>
-__global__ __launch_bounds__(kSynWaves * kWave) void synapse_conv_row_tail_kernel(const SynapseConv p) {
-    synapse_conv_row<KW, PIX, STREAM, true>(p);
-}
-
-// The row form on the bfloat16 matrix instruction, for layers with enough (input channel, kernel row) pairs to fill its 32
-// terms.  The float32 instruction bounds wide layers: 32 -> 64 channels on [16,32,16,16,300] 398 us forward (72 % of its
-// peak) and 429 us for the input gradient.  Operands are split into three parts (split.h) unless they are bfloat16
-// numbers as they are: the weights are looked at once per workgroup (those of an 8-bit quantiser always are), the input
-// once per column and group of 32 pairs (spikes are, gradients are not), and the products run to match: one for spikes
-// and quantised weights, three for one split operand, six for two.
-//
-// A wave walks the columns of its image row: lane (kk, j) loads steps 4j .. 4j+3 of pairs 32 g + 8 kk + {0 .. 7} at the
-// column, turns them into the operands of four products (one per step of the quad: eight pairs each), and uses these
-// for the KW output pixels the column meets, whose accumulators it keeps -- every column is loaded and split once.  A
-// pixel is complete, and stored, after its last column.  The next loads are on their way during the products.
-// The instruction rounds every sum it leaves, so the products of the lower parts, 2^-8 of the whole at most, are added up
-// from zero and join the sum in one addition: it is rounded twice for 32 terms, not up to six times.  The error against
-// float64 is 0.3 to 0.6 times that of the float32 form, sparse (graded) inputs included (96 pairs: real x real 1.0e-7 and
-// 2.9e-7, graded x real 0.7e-7 and 1.2e-7, real x quantised over 192 pairs 1.3e-7 and 4.2e-7; every product into the one sum:
-// 2.6e-7, 2.1e-7, 2.4e-7).
-// [16,32,16,16,300] -> 64 channels forward 402 -> 262 us, input gradient 418 -> 287 us with quantised weights, 357 without;
-// [32,8,32,32,300] -> 16 channels 352 -> 297 and 415 -> 328 us (168 registers, three waves per SIMD; five taps 213, two waves).
-// What bounds it now: the unaligned rows of the result (T = 300) for few channels, the vector instructions of the split
-// for gradients.
-//
-// A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
-// each of them is not infinity times their sum: a wave with a result that is not finite computes its row again from
-// the operands as they are, and so does every wave of a workgroup with such a weight.
-// LDS: the parts of the weights in the operand's layout, [group][tap][part][lane]; per wave the byte
-// offset of every pair's input row (or kOutOfRange).
-template <int KW, bool STREAM, bool TAIL>
-__global__ __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(KW <= 3 ? 3 : 2)))
-void synapse_conv_split_kernel(const SynapseConv p) {
-    extern __shared__ __attribute__((aligned(16))) float lds[];
-    const int G = p.KG;                                 // groups of 32 pairs
-    const int pairs = p.Ci * p.kh;
-    uint4* wt = reinterpret_cast<uint4*>(lds);
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), threads = blockDim.x, waves = threads / kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int* row_off = reinterpret_cast<int*>(wt + G * KW * 3 * kWave) + wave * G * 32;
-    // neighbouring workgroups take the channel blocks of the same items: they share the input rows
-    const int cobs = (p.Co + 15) / 16;
-    const int groups = (p.items + waves - 1) / waves;
-    int b = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int cob = b % cobs; b /= cobs;
-    const int ig = b % groups;
-    const int n = b / groups;
-    const int co0 = cob * 16;
-    const int kk = lane >> 4, j = lane & 15;
-
-    const int64_t k_full = (int64_t)p.Ci * p.kh_full * p.kw_full;
-    unsigned low = 0u;
-    bool odd = false;                                   // a weight that is not finite
-    for (int i = tid; i < G * KW * kWave; i += threads) {
-        const int l = i & (kWave - 1), x = (i >> 6) % KW, g = (i >> 6) / KW;
-        const int co = co0 + (l & 15);
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const int pr = 32 * g + 8 * (l >> 4) + e, ci = pr / p.kh, y = pr - ci * p.kh;
-            v[e] = (pr < pairs && co < p.Co) ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.0f;
-            low |= __float_as_uint(v[e]);
-            odd = odd || !(fabsf(v[e]) < __builtin_inff());
-            v[e] *= kSplitScale;
-        }
-        uint4* to = wt + (i >> 6) * 3 * kWave + l;
-        to[0] = round_eight(v);
-        to[kWave] = round_eight(v);
-        to[2 * kWave] = bf16_eight(v);
-    }
-    const int item = ig * waves + wave;
-    const bool on = item < p.items;
-    const int tile = item % p.ttiles;
-    const int piece = (item / p.ttiles) % p.wsplit;
-    const int ho = item / (p.ttiles * p.wsplit);
-    const int hin = ho * p.sh;
-    const int col = p.T * 4;                                             // bytes from a pixel to its right neighbour
-    for (int pr = lane; pr < 32 * G; pr += kWave) {
-        const int ci = pr / p.kh, row = hin + (pr - ci * p.kh) * p.dh - p.ph;
-        row_off[pr] = (pr < pairs && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
-    }
-    const bool split_w = __syncthreads_or((low & 0xffffu) != 0u);
-    const bool float_only = __syncthreads_or(odd);
-    if (!on) return;
-    const int t0 = tile * kSynTile;
-    SynQuad tq;
-    tq.template set<TAIL>(t0 + 4 * j, p.T);
-    const bool t_ok = tq.any();
-    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
-    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
-    const int64_t out_plane = (int64_t)p.Co * p.Ho_full * p.Wo_full * p.T;
-    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
-    const int per = (p.Wo + p.wsplit - 1) / p.wsplit;
-    const int w_lo = piece * per, w_hi = (w_lo + per) < p.Wo ? (w_lo + per) : p.Wo;
-    if (w_lo >= w_hi) return;
-
-    // column c (counted with the padding: tap x of output pixel wo lies at column wo + x) is image column c - pw
-    const int c_end = w_hi + KW - 1;
-    const int c_lo = w_lo > p.pw ? w_lo : p.pw;                          // the columns inside the image
-    const int c_hi = c_end < p.W + p.pw ? c_end : p.W + p.pw;
-    float4 raw[8];
-    auto fetch = [&](int c, int g) {
-        const int4* off = reinterpret_cast<const int4*>(row_off + 32 * g + 8 * kk);
-        const int4 o[2] = {off[0], off[1]};
-        const int at = (c - p.pw) * col + tq.t_load * 4;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            raw[4 * i] = buf_load4<false>(src, t_ok ? o[i].x + at : kOutOfRange);
-            raw[4 * i + 1] = buf_load4<false>(src, t_ok ? o[i].y + at : kOutOfRange);
-            raw[4 * i + 2] = buf_load4<false>(src, t_ok ? o[i].z + at : kOutOfRange);
-            raw[4 * i + 3] = buf_load4<false>(src, t_ok ? o[i].w + at : kOutOfRange);
-        }
-    };
-    // lane (kk, j): output channels co0 + 4 kk + i, steps t0 + 4 j + e
-    auto store = [&](int wo, const syn_f4 (&d)[4]) {
-        const int opix = p.out_pixel(ho, wo) * col + (t0 + 4 * j) * 4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int co = co0 + 4 * kk + i;
-            syn_store_quad<STREAM, TAIL>(dst, co < p.Co, co * (p.Ho_full * p.Wo_full * col) + opix, tq.nv,
-                                         make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
-        }
-    };
-    float stored = 0.f;                                                  // not finite once a result is not
-    syn_f4 acc[KW][4];
-    if (c_lo < c_hi) fetch(c_lo, 0);
-#pragma unroll
-    for (int x = 0; x < KW; ++x)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[x][e] = syn_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int c = w_lo; c < c_end; ++c) {                                 // tap x of column c goes to pixel c - x: acc[x]
-        if (c >= c_lo && c < c_hi) {
-#pragma unroll 1
-            for (int g = 0; g < G; ++g) {
-                float v[4][8];                                       // [step of the quad][pair]
-                unsigned bits = 0u;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float4 r = tq.template place<TAIL>(raw[i]);
-                    v[0][i] = r.x * kSplitScale; v[1][i] = r.y * kSplitScale;
-                    v[2][i] = r.z * kSplitScale; v[3][i] = r.w * kSplitScale;
-                    bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
-                }
-                const bool split_x = __any((bits & 0xffffu) != 0u);
-                const uint4* wg = wt + g * KW * 3 * kWave + lane;
-                const bool last = g + 1 == G;                            // the next loads are on their way during the products
-                if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
-                // kH steps of the quad at a time (the parts of all four do not fit beside the accumulators), and branches
-                // around the products of the lower parts only: around several copies of the whole they cost the compiler a
-                // second set of accumulators and spills.
-                constexpr int kH = KW == 5 ? 4 : 2;
-                const syn_f4 zero = syn_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int h = 0; h < 4; h += kH) {
-                    uint4 q[kH][3];
-#pragma unroll
-                    for (int e = 0; e < kH; ++e) {
-                        q[e][0] = bf16_eight(v[h + e]);
-                        if (split_x) {
-                            leave_eight(v[h + e], q[e][0]);
-                            q[e][1] = round_eight(v[h + e]);
-                            q[e][2] = bf16_eight(v[h + e]);
-                        }
-                    }
-#pragma unroll
-                    for (int x = 0; x < KW; ++x) {
-                        const uint4 w0 = wg[x * 3 * kWave];
-                        syn_f4 d[kH];
-                        if (split_x) {
-                            if (split_w) {
-                                const uint4 w1 = wg[(x * 3 + 1) * kWave], w2 = wg[(x * 3 + 2) * kWave];
-#pragma unroll
-                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
-#pragma unroll
-                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][1], d[e]);
-#pragma unroll
-                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][0], d[e]);
-#pragma unroll
-                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], d[e]);
-                            } else {
-#pragma unroll
-                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], zero);
-                            }
-#pragma unroll
-                            for (int e = 0; e < kH; ++e) acc[x][h + e] += mfma_bf16(w0, q[e][1], d[e]);
-                        } else if (split_w) {
-                            const uint4 w1 = wg[(x * 3 + 1) * kWave], w2 = wg[(x * 3 + 2) * kWave];
-#pragma unroll
-                            for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
-#pragma unroll
-                            for (int e = 0; e < kH; ++e) acc[x][h + e] += mfma_bf16(w1, q[e][0], d[e]);
-                        }
-#pragma unroll
-                        for (int e = 0; e < kH; ++e) acc[x][h + e] = mfma_bf16(w0, q[e][0], acc[x][h + e]);
-                    }
-                }
-            }
-        }
-        const int wo = c - (KW - 1);
-        if (wo >= w_lo) {
-            syn_f4 d[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                d[e] = acc[KW - 1][e];
-                stored += (d[e][0] + d[e][1]) + (d[e][2] + d[e][3]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) d[e][i] *= kSplitProductScale;
-            }
-            store(wo, d);
-        }
-#pragma unroll
-        for (int x = KW - 1; x >= 0; --x)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[x][e] = x > 0 ? acc[x - 1][e] : syn_f4{0.f, 0.f, 0.f, 0.f};
-    }
-    if (!float_only && !__any(!(fabsf(stored) < __builtin_inff()))) return;
-
-    // once more in float32 multiplications and additions, taps outside the image as products with zero like the float32 form
-#pragma unroll 1
-    for (int wo = w_lo; wo < w_hi; ++wo) {
-        syn_f4 d[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) d[e] = syn_f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-        for (int pr = 0; pr < pairs; ++pr) {
-            const int ci = pr / p.kh, y = pr - ci * p.kh, row = row_off[pr];
-#pragma unroll 1
-            for (int x = 0; x < KW; ++x) {
-                const int c = wo + x - p.pw;
-                const bool in = t_ok && row != kOutOfRange && (unsigned)c < (unsigned)p.W;
-                const float4 q = tq.template place<TAIL>(buf_load4<false>(src, in ? row + c * col + tq.t_load * 4 : kOutOfRange));
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int co = co0 + 4 * kk + i;
-                    const float w = co < p.Co ? p.weight[(int64_t)co * k_full + p.weight_index(ci, y, x)] : 0.f;
-                    d[0][i] = __fmaf_rn(w, q.x, d[0][i]);
-                    d[1][i] = __fmaf_rn(w, q.y, d[1][i]);
-                    d[2][i] = __fmaf_rn(w, q.z, d[2][i]);
-                    d[3][i] = __fmaf_rn(w, q.w, d[3][i]);
-                }
-            }
-        }
-        store(wo, d);
     }
 }
 
@@ -1133,57 +688,35 @@ using namespace slayer;
 
 namespace {
 
-#ifndef SLAYER_SYN_PIX
-#define SLAYER_SYN_PIX 4
-#endif
-
-// What a launch of the row kernels takes, in us: every wave walks its piece of an image row -- the columns of the split
-// form with 32 (input channel, kernel row) pairs to a group, the blocks of four pixels of the float32 form with four -- and a
-// group costs a wait for its loads and its share of the SIMD, which all waves there divide up.  Fitted to 1900 layers
-// (2, 3 and 5 taps, 17 to 192 pairs, 3 to 64 output channels, 1 to 64 samples of 8x8 to 34x34 pixels, 50 to 302 steps; real
-// values times real weights) with an error of 12 to 15 % for the split and 13 to 22 % for the float32 form.
-// Split form over float32 form for 500 layers of these ranges that it decides for the former, margins of the caller included,
-// mean / 95 % of the layers / largest:
-//            spikes x quantised     real x quantised       real x real
-//   2 taps   0.60 / 0.84 / 0.97     0.76 / 1.01 / 1.12     0.85 / 1.18 / 1.27
-//   3 taps   0.52 / 0.77 / 1.11     0.72 / 0.99 / 1.29     0.85 / 1.16 / 1.40
-//   5 taps   0.42 / 0.68 / 0.74     0.60 / 0.90 / 1.05     0.75 / 1.11 / 1.28
-// Taken always from 17 pairs on, the split form lost up to 2.8 times on single samples of small images, up to 1.7
-// times with badly filled groups (5x5, 40 pairs, real x real 195 us against 141).
-double row_form_time(bool split, const SynapseConv& p, int64_t row_tiles, int pieces) {
-    struct Cost { double launch, step, wait, rate, tail; };               // tail: rows that end inside a quad
-    static constexpr Cost costs[2][3] = {{{0.0, 2.0, 0.21, 0.645, 0.85}, {4.5, 0.0, 0.10, 0.96, 0.71}, {1.0, 3.25, 0.62, 1.26, 0.69}},
-                                         {{1.7, 0.54, 0.03, 1.10, 0.70}, {0.0, 0.51, 0.30, 1.14, 0.63}, {0.0, 0.38, 0.71, 1.28, 0.92}}};
-    const Cost& c = costs[split][p.kw == 5 ? 2 : p.kw - 2];
-    const int pixels = (p.Wo + pieces - 1) / pieces, pairs = p.Ci * p.kh;
-    const int steps = split ? pixels + p.kw - 1 : (pixels + 3) / 4;
-    const int groups = split ? (pairs + 31) / 32 : (pairs + 3) / 4;
-    const double load = (double)(row_tiles * pieces) / 1024;              // waves per SIMD
-    return c.launch + steps * (c.step + groups * (c.wait + c.rate * (load > 1 ? load : 1))) * (p.T % 4 ? 1 + c.tail : 1);
+// Whether a filter is one of those taken: its weights have to fit the LDS of a workgroup.
+bool filter_fits(const SynapseConv& p) {
+    const int64_t pairs = (int64_t)p.Ci * p.kh, K = pairs * p.kw;
+    if (p.sw == 1 && p.dw == 1 && (p.kw == 2 || p.kw == 3 || p.kw == 5) && p.Wo >= 4)
+        return (pairs + 31) / 32 * p.kw * 3 <= 96 || (pairs + 3) / 4 * 4 * (p.kw * 64 + 8) <= 64 * 1024;
+    const int64_t groups = (K + 3) / 4, chunk = groups <= 2 ? (groups < 1 ? 1 : groups) : kSynChunk;
+    return (groups + chunk - 1) / chunk * chunk * 4 * 76 <= 64 * 1024;
 }
 
 // One launch of the convolution kernels for the geometry in p (tensors, sizes, taps and sub-lattices filled in by the
-// caller): the row kernel for unit stride and dilation along the image row with 2, 3 or 5 taps per row, else the
-// one-pixel kernel with as many tap groups in flight as the filter has, up to six.  A filter without taps (K = 0)
-// clears its outputs.
+// caller): the walking kernel where it takes the geometry, else the one-pixel kernel with as many tap groups in flight as
+// the filter has, up to six.  A filter without taps (K = 0) clears its outputs.
 int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
+    if (!filter_fits(p)) return SLAYER_ERANGE;
+    int code = 0;
+    if (launch_synapse_walk(p, st, &code)) return code;
     // Non-temporal stores only for the classes of a transposed convolution, which leave every line they touch
     // unfinished for the next launch.  A plain convolution finishes the lines that two of its tiles share within
-    // microseconds, and the L2 puts the pieces together if it is allowed to keep them: [32,8,32,32,300] -> 16 channels
-    // forward 378 -> 329 us with cached stores (the transposed 4x4 stride-2 classes 251 -> 288 us).
+    // microseconds, and the L2 puts the pieces together if it is allowed to keep them.
     if (p.oys == 1 && p.oxs == 1) streaming = false;
-    constexpr int kRowPix = SLAYER_SYN_PIX;
     const int64_t K = (int64_t)p.Ci * p.kh * p.kw;
     p.K = (int)K;
     p.ttiles = (p.T + kSynTile - 1) / kSynTile;
-    // blocks of four neighbouring pixels that share their input columns: unit stride and dilation along the row
-    const bool rows = p.sw == 1 && p.dw == 1 && (p.kw == 2 || p.kw == 3 || p.kw == 5) && p.Wo >= kRowPix;
     // enough waves for four rounds of the chip (16 waves on each of 256 compute units), so that the last, partly
     // filled round weighs little; image rows cut into as few pieces as that takes
     const int64_t cobs = (p.Co + 15) / 16;
     const int64_t base = (int64_t)p.N * cobs * p.Ho * p.ttiles;
     int wsplit = 1;
-    while (base * wsplit < 16 * 1024 && wsplit * 2 * (rows ? kRowPix : 1) <= p.Wo) wsplit *= 2;
+    while (base * wsplit < 16 * 1024 && wsplit * 2 <= p.Wo) wsplit *= 2;
     p.wsplit = wsplit;
     const int64_t items = (int64_t)p.Ho * wsplit * p.ttiles;
     if (items > 0x7fffffffLL) return SLAYER_ERANGE;
@@ -1192,70 +725,10 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     if (blocks > 0x7fffffffLL) return SLAYER_ERANGE;
     const bool tail = (p.T % 4) != 0;                                     // rows that end inside a quad
     const dim3 grid((unsigned)blocks), block(kSynWaves * kWave);
-    // The split form where it is about as fast with both operands real, its worst case (row_form_time), from 17 pairs
-    // on, and if the parts of 16 channels' weights fit LDS.  A piece of an image row visits kw - 1 columns more than it has
-    // pixels: rows are cut while there are few waves, for five taps (two waves per SIMD) below 1024 only
-    // ([4,16,16,16,300] -> 64 channels 182 us with 2560 waves, 140 with 1280).
-    const int pairs = p.Ci * p.kh;
-    const int g32 = (pairs + 31) / 32;
-    const size_t split_lds = (size_t)g32 * p.kw * 3 * 1024;
-    const size_t row_lds = (size_t)((pairs + 3) / 4) * 4 * (p.kw * 16 * sizeof(float) + 2 * sizeof(int));
-    int pieces = 1;
-    while (base * pieces < (p.kw == 5 ? 1024 : 6144) && p.Wo >= 16 * pieces) pieces *= 2;
-    // In all but small launches a margin for what it gains with spikes and quantised weights, which the host cannot see:
-    // layers estimated at 1.0 to 1.1 of the float32 form take 0.5 to 0.7 of it with both, 0.8 to 1.0 with one, 1.0 to 1.15 with
-    // neither.
-    const bool small = base * pieces < 640;
-    const double margin = p.kw == 2 ? (small ? 1.1 : 1.2) : small ? 1.0 : p.kw == 3 ? 1.12 : 1.07;
-    if (rows && pairs > 16 && split_lds <= 96 * 1024 &&
-        (row_lds > 64 * 1024 || row_form_time(true, p, base, pieces) <= margin * row_form_time(false, p, base, wsplit))) {
-        // Workgroups of four waves: the registers hold three of them on a CU (five taps: two), but one of eight.  Eight where the
-        // LDS has room for one workgroup only and there are more than four waves to a CU.  Both operands real, us, float32
-        // form / four / eight waves: 3x3 on [5,43,31,31,64] -> 40 channels 127 / 153 / 192, [2,43,32,32,300] -> 27 144 / 159 /
-        // 215, 5x5 on [10,25,11,11,100] -> 2 97 / 98 / 128; with room for one, 5x5 on [1,33,35,35,300] -> 3 (700 waves)
-        // 249 / 166 / 220, 3x3 on [3,86,23,23,159] -> 47 (1242 waves) 758 / 1006 / 553.
-        const int waves = 2 * (split_lds + 4 * g32 * 32 * sizeof(int)) > 160 * 1024 && base * pieces > 4 * 256 ? 8 : 4;
-        p.wsplit = pieces;
-        p.KG = g32;
-        const int64_t all = (int64_t)p.Ho * pieces * p.ttiles;
-        const int64_t wgs = p.N * cobs * ((all + waves - 1) / waves);
-        if (all > 0x7fffffffLL || wgs * waves > 0x3fffffffLL) return SLAYER_ERANGE;
-        p.items = (int)all;
-        const dim3 sgrid((unsigned)wgs), sblock((unsigned)(waves * kWave));
-        const size_t bytes = split_lds + (size_t)waves * g32 * 32 * sizeof(int);
-#define SLAYER_SYN_SPLIT(KW)                                                                                        \
-        do {                                                                                                             \
-            if (tail) { if (streaming) hipLaunchKernelGGL((synapse_conv_split_kernel<KW, true, true>), sgrid, sblock, bytes, st, p); \
-                        else hipLaunchKernelGGL((synapse_conv_split_kernel<KW, false, true>), sgrid, sblock, bytes, st, p); } \
-            else { if (streaming) hipLaunchKernelGGL((synapse_conv_split_kernel<KW, true, false>), sgrid, sblock, bytes, st, p); \
-                   else hipLaunchKernelGGL((synapse_conv_split_kernel<KW, false, false>), sgrid, sblock, bytes, st, p); } \
-        } while (0)
-        if (p.kw == 2) SLAYER_SYN_SPLIT(2);
-        else if (p.kw == 3) { SLAYER_SYN_SPLIT(3); }
-        else SLAYER_SYN_SPLIT(5);
-#undef SLAYER_SYN_SPLIT
-        return (int)hipGetLastError();
-    }
-    if (rows) {
-        p.KG = (pairs + 3) / 4;                                           // groups of four (channel, kernel row) pairs
-        if (row_lds > 64 * 1024) return SLAYER_ERANGE;
-#define SLAYER_SYN_ROW_T(KERNEL, KW)                                                                      \
-        do {                                                                                             \
-            if (streaming) hipLaunchKernelGGL((KERNEL<KW, kRowPix, true>), grid, block, row_lds, st, p);  \
-            else hipLaunchKernelGGL((KERNEL<KW, kRowPix, false>), grid, block, row_lds, st, p);           \
-        } while (0)
-#define SLAYER_SYN_ROW(KW)                                                                                \
-        do { if (tail) SLAYER_SYN_ROW_T(synapse_conv_row_tail_kernel, KW); else SLAYER_SYN_ROW_T(synapse_conv_row_kernel, KW); } while (0)
-        if (p.kw == 2) SLAYER_SYN_ROW(2); else if (p.kw == 3) SLAYER_SYN_ROW(3); else SLAYER_SYN_ROW(5);
-#undef SLAYER_SYN_ROW_T
-#undef SLAYER_SYN_ROW
-        return (int)hipGetLastError();
-    }
     const int groups = (int)((K + 3) / 4);
     const int chunk = groups <= 1 ? 1 : (groups == 2 ? 2 : kSynChunk);
     p.KG = (groups + chunk - 1) / chunk * chunk;
     const size_t lds = (size_t)p.KG * 4 * (16 * sizeof(float) + 3 * sizeof(int));
-    if (lds > 64 * 1024) return SLAYER_ERANGE;
 #define SLAYER_SYN_ONE(S, TL, CH) hipLaunchKernelGGL((synapse_conv_kernel<S, TL, CH>), grid, block, lds, st, p)
 #define SLAYER_SYN_CH(S, TL) \
     do { if (chunk == 1) SLAYER_SYN_ONE(S, TL, 1); else if (chunk == 2) SLAYER_SYN_ONE(S, TL, 2); else SLAYER_SYN_ONE(S, TL, kSynChunk); } while (0)
@@ -1527,24 +1000,34 @@ extern "C" int slayer_conv_synapse_input_grad(float* grad_in, const float* grad_
         int code = 0;
         if (launch_synapse_plane(q, true, streaming, (hipStream_t)stream, &code)) return code;
     }
-    for (int ry = 0; ry < (int)stride_h && ry < (int)H; ++ry) {
+    // the plain convolution of one residue class
+    auto one_class = [&](int ry, int rx) {
         const TapClass cy = tap_class(ry, (int)kh, (int)stride_h, (int)pad_h, (int)dil_h);
-        for (int rx = 0; rx < (int)stride_w && rx < (int)W; ++rx) {
-            const TapClass cx = tap_class(rx, (int)kw, (int)stride_w, (int)pad_w, (int)dil_w);
-            p.oy0 = ry; p.ox0 = rx;
-            p.Ho = ((int)H - ry + (int)stride_h - 1) / (int)stride_h;
-            p.Wo = ((int)W - rx + (int)stride_w - 1) / (int)stride_w;
-            const bool none = cy.count == 0 || cx.count == 0;            // pixels no tap reaches: zeros
-            // the taps in the order of rising source coordinate: from the last one down, a step of
-            // step * dil / stride pixels of the source each
-            p.kh = none ? 0 : cy.count; p.kw = none ? 0 : cx.count;
-            p.ky0 = cy.y_last; p.kys = -cy.step; p.kx0 = cx.y_last; p.kxs = -cx.step;
-            p.dh = cy.count > 1 ? cy.step * (int)dil_h / (int)stride_h : 1;
-            p.dw = cx.count > 1 ? cx.step * (int)dil_w / (int)stride_w : 1;
-            p.ph = -cy.first; p.pw = -cx.first;
-            const int code = launch_synapse_conv(p, streaming, (hipStream_t)stream);
-            if (code != 0) return code;
-        }
+        const TapClass cx = tap_class(rx, (int)kw, (int)stride_w, (int)pad_w, (int)dil_w);
+        p.oy0 = ry; p.ox0 = rx;
+        p.Ho = ((int)H - ry + (int)stride_h - 1) / (int)stride_h;
+        p.Wo = ((int)W - rx + (int)stride_w - 1) / (int)stride_w;
+        const bool none = cy.count == 0 || cx.count == 0;                // pixels no tap reaches: zeros
+        // the taps in the order of rising source coordinate: from the last one down, a step of
+        // step * dil / stride pixels of the source each
+        p.kh = none ? 0 : cy.count; p.kw = none ? 0 : cx.count;
+        p.ky0 = cy.y_last; p.kys = -cy.step; p.kx0 = cx.y_last; p.kxs = -cx.step;
+        p.dh = cy.count > 1 ? cy.step * (int)dil_h / (int)stride_h : 1;
+        p.dw = cx.count > 1 ? cx.step * (int)dil_w / (int)stride_w : 1;
+        p.ph = -cy.first; p.pw = -cx.first;
+    };
+    const int classes_h = (int)(stride_h < H ? stride_h : H), classes_w = (int)(stride_w < W ? stride_w : W);
+    bool fits = true;
+    for (int r = 0; r < classes_h * classes_w; ++r) { one_class(r / classes_w, r % classes_w); fits = fits && filter_fits(p); }
+    if (!fits) return SLAYER_ERANGE;
+    int code = 0;
+    if (dil_h == 1 && dil_w == 1 && launch_synapse_walk_transposed(p, (int)kh, (int)kw, (int)stride_h, (int)stride_w, (int)pad_h, (int)pad_w,
+                                                                   (hipStream_t)stream, &code))
+        return code;
+    for (int r = 0; r < classes_h * classes_w; ++r) {
+        one_class(r / classes_w, r % classes_w);
+        code = launch_synapse_conv(p, streaming, (hipStream_t)stream);
+        if (code != 0) return code;
     }
     return 0;
 }

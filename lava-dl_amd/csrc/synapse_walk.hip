@@ -1,0 +1,574 @@
+// Convolution synapse on time-innermost tensors, products on the bfloat16 matrix instruction: forward pass, input gradient and
+// transposed convolution of every geometry with one to five taps along the axis that is walked.
+//
+// One axis of the image (the rows, where the filter allows) is walked, the other one and time are one "line" of positions: M
+// pixels of T steps, in memory one piece.  A wave owns 64 positions of the line and 16 or 32 output channels and walks the rows: a
+// step brings the input row (`ss` rows, the stride along the walk) at the line's XP taps, each loaded and split into bfloat16
+// parts once for all KS taps along the walk, whose sums are KS sets of accumulators; an output row is stored when its last
+// row has come.  Tiles are 64 positions of the line rather than of a pixel's row, so their stores fill whole 128-byte lines
+// whatever T is, and no tile is half empty: [32,8,32,32,300] -> 16 channels 300 -> 248 us (64 steps of one pixel a tile: rows of
+// 300 steps end inside a line, 20 of 320 positions idle), 31x30 pixels of 301 steps 283 -> 213.
+//
+// The terms of a product are (input channel, line tap, row of the step) triples, E to a lane and group (4 E to a group): as few loads
+// as the layer has triples, 24 of them are one group of six.  The rows of a product are (channel, pixel) pairs: XS neighbouring
+// pixels of the line of a layer with few channels share a position, and their taps, so that 8 channels of two pixels load four
+// taps where one pixel each would load six, and no row of the product is empty (input gradient [20,8,31,30,324], 5x5, 8 -> 4
+// channels 293 -> 126 us).  In a transposed convolution the pixels of a position are those of all residues modulo the stride,
+// and the classes of the walked axis are one launch: one read of the source instead of one per class, and lines written once
+// (4x4 stride 2, [32,16,16,16,300] -> 8 channels 245 -> 185 us, 13x11 pixels of 173 steps 139 -> 25).
+//
+// Steps that are not whole quads: a pixel's last quad is its last four steps, overlapping the one before; the steps they share are
+// computed twice, to the same bits, instead of being moved into place ([16,8,24,24,250] -> 16 channels, 5x5: 204 -> 114 us).
+//
+// Operands are split into three parts (split.h) unless they are bfloat16 numbers as they are: the weights are looked at once
+// per workgroup, the input once per group, and the products run to match: one for spikes and quantised weights, three for one
+// split operand, six for two.  The instruction rounds every sum it leaves, so the products of the lower parts, 2^-8 of
+// the whole at most, are added up from zero and join the sum in one addition: it is rounded twice for 32 terms, not up to
+// six times (error against float64 1.0e-7 real x real over 96 terms, float32 instruction 2.9e-7; every product into the one sum
+// 2.6e-7).
+//
+// What bounds it: with the products left out the forward pass of [32,8,32,32,300] -> 16 channels takes as long (254 us): a group
+// of loads has to arrive before its step, and 12 waves hold 72 KB of a CU's loads in flight.  Two blocks of channels to a wave
+// (MB) halve the loads and the splitting of wide layers: [16,32,16,16,300] -> 64 channels 262 -> 232 us, its input gradient 349 ->
+// 280, though two waves stay on a SIMD instead of three.
+//
+// A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
+// each of them is not infinity times their sum: a wave with a result that is not finite computes its piece again in
+// float32 multiplications and additions, and so does every wave of a workgroup with such a weight.
+//
+// LDS: the parts of the weights in the operand's layout, [group][tap][part][block][lane]; per triple its byte offset, its line tap
+// and row, its channel.
+#include "synapse.h"
+#include "split.h"
+
+namespace slayer {
+
+constexpr int kWalkQuads = 16;          // quads of steps to a tile
+
+// Rows of the result that take the same taps along the walk: all of them, or, in a transposed convolution, a residue class.
+struct WalkClass {
+    int s0;                             // weights: slide tap i of the launch is row s0 + i * WalkConv::sstep of the filter
+    int row0;                           // input row of step 0's first row
+    int S;                              // output rows
+    int c_lo, c_hi;                     // the steps that meet a row inside the image
+    int out0;                           // bytes to the first output row
+};
+
+struct WalkConv {
+    float* out;
+    const float* in;
+    const float* weight;                // [Co][Ci][...]
+    int N, Ci, Co, T;
+    int in_plane, out_plane;            // bytes of one sample
+    int in_ch, in_slide, in_line, out_ch, out_slide, out_line, out_rx;   // bytes
+    int Hs, Ws;                         // input rows along the walk, pixels along the line
+    int M, quads, line_quads;           // pixels along the line; quads of steps a pixel has, the line has
+    int ss, ls;                         // strides along walk and line
+    int XP, shift0, shift_step;         // line taps, the first one's shift, pixels from one to the next
+    int XS, line_full;                  // outputs that share a line position, pixels of the output's line
+    int pairs, groups;
+    int wslide, wline, nslide, nline;   // weights: strides and sizes of the filter's axes
+    int sstep, l0, lstep, lrx;          // filter row / column of a slide / line tap
+    int tiles, pieces, items, blocks;   // per sample, class and channel block; blocks of 16 MB channels
+    int MB;
+    int classes;
+    WalkClass cls[4];
+    // weight of output channel v = co * XS + rx, line tap x, slide tap i (of cls), or -1 where the filter has none
+    __device__ __forceinline__ int weight_at(int co, int rx, int ci, int x, int i, int s0) const {
+        const int y = s0 + i * sstep, l = l0 + x * lstep + rx * lrx;
+        if ((unsigned)y >= (unsigned)nslide || (unsigned)l >= (unsigned)nline) return -1;
+        return (co * Ci + ci) * (nslide * nline) + y * wslide + l * wline;
+    }
+};
+
+// KS: taps along the walk; E: triples to a lane and group; MB: blocks of 16 rows of the product to a wave.  Three waves per SIMD where
+// 168 registers do, else two.
+template <int KS, int E, int MB>
+__global__ __launch_bounds__(8 * kWave) __attribute__((amdgpu_waves_per_eu(KS <= 3 && MB == 1 ? 3 : 2)))
+void synapse_walk_kernel(const WalkConv p) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int G = p.groups;                             // groups of 4 E pairs
+    uint4* wt = reinterpret_cast<uint4*>(lds);          // [G][KS][3][MB][64]
+    int* pair_off = reinterpret_cast<int*>(wt + G * KS * 3 * MB * kWave);     // [G][4][E] bytes
+    int* pair_info = pair_off + G * 4 * E;              // line tap, row of the step << 8
+    int* pair_ch = pair_info + G * 4 * E;               // input channel
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), threads = blockDim.x, waves = threads / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int b = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int cb = b % (p.blocks * p.classes); b /= p.blocks * p.classes;
+    const int v0 = (cb % p.blocks) * 16 * MB;
+    const WalkClass cls = p.cls[cb / p.blocks];
+    const int groups = (p.items + waves - 1) / waves;
+    const int ig = b % groups;
+    const int n = b / groups;
+    const int kk = lane >> 4, j = lane & 15;
+
+    for (int i = tid; i < G * 4 * E; i += threads) {
+        const int e = i % E, q = (i / E) & 3, g = i / (4 * E);
+        const int pr = 4 * E * g + 4 * e + q;
+        const int ci = pr / (p.XP * p.ss), r = pr - ci * (p.XP * p.ss), x = r / p.ss, row = r - x * p.ss;
+        const bool is = pr < p.pairs;
+        pair_off[i] = is ? ci * p.in_ch + (p.shift0 + x * p.shift_step) * p.in_line + row * p.in_slide : kOutOfRange;
+        pair_info[i] = is ? x | row << 8 : 31;          // tap 31 is outside in every lane
+        pair_ch[i] = is ? ci : -1;
+    }
+    __syncthreads();
+    unsigned low = 0u;
+    bool odd = false;                                   // a weight that is not finite
+    for (int i = tid; i < G * KS * MB * kWave; i += threads) {
+        const int l = i & (kWave - 1), mb = (i >> 6) % MB, tap = (i >> 6) / MB % KS, g = (i >> 6) / (MB * KS);
+        const int vc = v0 + 16 * mb + (l & 15), co = vc / p.XS, rx = vc - co * p.XS;
+        float v[8];
+        int at[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (e >= E) { v[e] = 0.0f; at[e] = -1; continue; }
+            const int pr = (4 * g + (l >> 4)) * E + e, ci = pair_ch[pr], what = pair_info[pr];
+            at[e] = ci >= 0 && co < p.Co ? p.weight_at(co, rx, ci, what & 31, tap * p.ss + (what >> 8), cls.s0) : -1;
+            v[e] = p.weight[at[e] < 0 ? 0 : at[e]];
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            v[e] = at[e] < 0 ? 0.0f : v[e];
+            low |= __float_as_uint(v[e]);
+            odd = odd || !(fabsf(v[e]) < __builtin_inff());
+            v[e] *= kSplitScale;
+        }
+        uint4* to = wt + (((g * KS + tap) * 3) * MB + mb) * kWave + l;
+        to[0] = round_eight(v);
+        to[MB * kWave] = round_eight(v);
+        to[2 * MB * kWave] = bf16_eight(v);
+    }
+    const bool split_w = __syncthreads_or((low & 0xffffu) != 0u);
+    const bool float_only = __syncthreads_or(odd);
+    const int item = ig * waves + wave;
+    if (item >= p.items) return;
+    const int tile = item % p.tiles, piece = item / p.tiles;
+    const int per = (cls.S + p.pieces - 1) / p.pieces;
+    const int s_lo = piece * per, s_hi = (s_lo + per) < cls.S ? (s_lo + per) : cls.S;
+    if (s_lo >= s_hi) return;
+
+    // the lane's quad: pixel m of the line, steps t .. t + 3
+    const int quad = tile * kWalkQuads + j;
+    const bool on = quad < p.line_quads;
+    const int m = on ? quad / p.quads : 0;
+    // where a pixel's steps are not whole quads its last quad is the last four steps: those that it shares with the one before
+    // are computed, and stored, twice
+    int t = 4 * (quad - m * p.quads);
+    t = t < p.T - 4 ? t : p.T - 4;
+    unsigned taps = 0u;                                 // line taps inside the image
+    for (int x = 0; x < p.XP; ++x)
+        taps |= (on && (unsigned)(m * p.ls + p.shift0 + x * p.shift_step) < (unsigned)p.Ws) ? 1u << x : 0u;
+    const bool inner = __all(taps == (1u << p.XP) - 1u);   // no lane has a tap outside
+    const int lane_in = m * p.ls * p.in_line + t * 4;
+    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * (p.in_plane / 4), (unsigned)p.in_plane);
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * (p.out_plane / 4), (unsigned)p.out_plane);
+    int to[MB][4];                                      // where the lane's four channels go, row 0
+#pragma unroll
+    for (int i = 0; i < 4 * MB; ++i) {
+        const int vc = v0 + 16 * (i >> 2) + 4 * kk + (i & 3), co = vc / p.XS, rx = vc - co * p.XS;
+        to[i >> 2][i & 3] = (on && co < p.Co && m * p.XS + rx < p.line_full)
+                                ? co * p.out_ch + rx * p.out_rx + m * p.out_line + t * 4 + cls.out0 : kOutOfRange;
+    }
+
+    // step c brings rows c * ss + row0 .. + ss - 1: slide tap i of output row c - i
+    const int c_end = s_hi + KS - 1;
+    const int c_lo = s_lo > cls.c_lo ? s_lo : cls.c_lo;
+    const int c_hi = c_end < cls.c_hi ? c_end : cls.c_hi;
+    float4 raw[E];
+    auto fetch = [&](int c, int g) {
+        const int* off = pair_off + (4 * g + kk) * E;
+        const int row = c * p.ss + cls.row0;
+        const int at = lane_in + row * p.in_slide;
+        int o[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] = off[e] + at;
+        if (!inner || row < 0 || row + p.ss > p.Hs) {
+            const int* info = pair_info + (4 * g + kk) * E;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int what = info[e];
+                const bool in = (taps >> (what & 31) & 1u) != 0u && (unsigned)(row + (what >> 8)) < (unsigned)p.Hs;
+                o[e] = in ? o[e] : kOutOfRange;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) raw[e] = buf_load4<false>(src, o[e]);
+    };
+    // lane (kk, j): output channels v0 + 16 mb + 4 kk + i, steps t .. t + 3
+    auto store = [&](int s, int mb, const syn_f4 (&d)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            buf_store4<false>(dst, to[mb][i] != kOutOfRange ? to[mb][i] + s * p.out_slide : kOutOfRange,
+                              make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
+    };
+    float stored = 0.f;                                                  // not finite once a result is not
+    syn_f4 acc[MB][KS][4];
+    if (c_lo < c_hi) fetch(c_lo, 0);
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int x = 0; x < KS; ++x)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[b][x][e] = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = s_lo; c < c_end; ++c) {                                 // tap i of step c goes to row c - i: acc[i]
+        if (c >= c_lo && c < c_hi) {
+#pragma unroll 1
+            for (int g = 0; g < G; ++g) {
+                float v[4][8];                                           // [step of the quad][pair]
+                unsigned bits = 0u;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (i >= E) { v[0][i] = v[1][i] = v[2][i] = v[3][i] = 0.f; continue; }
+                    const float4 r = raw[i < E ? i : 0];
+                    v[0][i] = r.x * kSplitScale; v[1][i] = r.y * kSplitScale;
+                    v[2][i] = r.z * kSplitScale; v[3][i] = r.w * kSplitScale;
+                    bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
+                }
+                const bool split_x = __any((bits & 0xffffu) != 0u);
+                const uint4* wg = wt + g * KS * 3 * MB * kWave + lane;
+                const bool last = g + 1 == G;                            // the next loads are on their way during the products
+                if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
+                // kH steps of the quad at a time (the parts of all four do not fit beside the accumulators), and branches
+                // around the products of the lower parts only: around several copies of the whole they cost the compiler a
+                // second set of accumulators and spills.
+                constexpr int kH = KS == 5 ? 4 : 2;
+                const syn_f4 zero = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int h = 0; h < 4; h += kH) {
+                    uint4 q[kH][3];
+#pragma unroll
+                    for (int e = 0; e < kH; ++e) {
+                        q[e][0] = bf16_eight(v[h + e]);
+                        if (split_x) {
+                            leave_eight(v[h + e], q[e][0]);
+                            q[e][1] = round_eight(v[h + e]);
+                            q[e][2] = bf16_eight(v[h + e]);
+                        }
+                    }
+#pragma unroll
+                    for (int xb = 0; xb < KS * MB; ++xb) {
+                        const int x = xb / MB, mb = xb % MB;
+                        const uint4* wx = wg + (x * 3 * MB + mb) * kWave;
+                        const uint4 w0 = wx[0];
+                        syn_f4 d[kH];
+                        if (split_x) {
+                            if (split_w) {
+                                const uint4 w1 = wx[MB * kWave], w2 = wx[2 * MB * kWave];
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][1], d[e]);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w1, q[e][0], d[e]);
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], d[e]);
+                            } else {
+#pragma unroll
+                                for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w0, q[e][2], zero);
+                            }
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) acc[mb][x][h + e] += mfma_bf16(w0, q[e][1], d[e]);
+                        } else if (split_w) {
+                            const uint4 w1 = wx[MB * kWave], w2 = wx[2 * MB * kWave];
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) d[e] = mfma_bf16(w2, q[e][0], zero);
+#pragma unroll
+                            for (int e = 0; e < kH; ++e) acc[mb][x][h + e] += mfma_bf16(w1, q[e][0], d[e]);
+                        }
+#pragma unroll
+                        for (int e = 0; e < kH; ++e) acc[mb][x][h + e] = mfma_bf16(w0, q[e][0], acc[mb][x][h + e]);
+                    }
+                }
+            }
+        }
+        const int s = c - (KS - 1);
+        if (s >= s_lo) {
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                syn_f4 d[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    d[e] = acc[mb][KS - 1][e];
+                    stored += (d[e][0] + d[e][1]) + (d[e][2] + d[e][3]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) d[e][i] *= kSplitProductScale;
+                }
+                store(s, mb, d);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+#pragma unroll
+            for (int x = KS - 1; x >= 0; --x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[b][x][e] = x > 0 ? acc[b][x - 1][e] : syn_f4{0.f, 0.f, 0.f, 0.f};
+    }
+    if (!float_only && !__any(!(fabsf(stored) < __builtin_inff()))) return;
+
+    // once more in float32 multiplications and additions, taps outside the image as products with zero
+#pragma unroll 1
+    for (int sb = s_lo * MB; sb < s_hi * MB; ++sb) {
+        const int s = sb / MB, mb = sb % MB;
+        syn_f4 d[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[e] = syn_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int pr = 0; pr < p.pairs; ++pr) {
+            const int ci = pr / (p.XP * p.ss), r = pr - ci * (p.XP * p.ss), x = r / p.ss, sub = r - x * p.ss;
+            const int off = ci * p.in_ch + (p.shift0 + x * p.shift_step) * p.in_line + lane_in;
+#pragma unroll 1
+            for (int tap = 0; tap < KS; ++tap) {
+                const int row = (s + tap) * p.ss + cls.row0 + sub;
+                const bool in = (taps >> x & 1u) != 0u && (unsigned)row < (unsigned)p.Hs;
+                const float4 q = buf_load4<false>(src, in ? off + row * p.in_slide : kOutOfRange);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int vc = v0 + 16 * mb + 4 * kk + i, co = vc / p.XS, rx = vc - co * p.XS;
+                    const int at = co < p.Co ? p.weight_at(co, rx, ci, x, tap * p.ss + sub, cls.s0) : -1;
+                    if (at < 0) continue;
+                    const float w = p.weight[at];
+                    d[0][i] = __fmaf_rn(w, q.x, d[0][i]);
+                    d[1][i] = __fmaf_rn(w, q.y, d[1][i]);
+                    d[2][i] = __fmaf_rn(w, q.z, d[2][i]);
+                    d[3][i] = __fmaf_rn(w, q.w, d[3][i]);
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < MB; ++b)
+            if (b == mb) store(s, b, d);
+    }
+}
+
+namespace {
+
+constexpr int kMaxLineTaps = 31;        // bits of a lane's mask, less one
+constexpr size_t kWalkLds = 150 * 1024;
+
+struct Axis { int in, out, k, stride, pad, dil, k0, kstep, kfull, o0, ostep, ofull, wstride; };
+
+template <int KS, int MB>
+void launch_walk(int E, const WalkConv& w, unsigned wgs, int waves, size_t bytes, hipStream_t st) {
+    const dim3 grid(wgs), block((unsigned)(waves * kWave));
+    if (E == 2) hipLaunchKernelGGL((synapse_walk_kernel<KS, 2, MB>), grid, block, bytes, st, w);
+    else if (E == 4) hipLaunchKernelGGL((synapse_walk_kernel<KS, 4, MB>), grid, block, bytes, st, w);
+    else if (E == 6) hipLaunchKernelGGL((synapse_walk_kernel<KS, 6, MB>), grid, block, bytes, st, w);
+    else hipLaunchKernelGGL((synapse_walk_kernel<KS, 8, MB>), grid, block, bytes, st, w);
+}
+
+int slide_taps(int taps) { return taps == 4 ? 5 : taps; }              // those there are kernels for
+
+// The loads of one walk step for `pairs` (channel, line tap, row) triples: E to a lane and group, groups.
+struct Grouping { int E, groups; };
+Grouping grouping(int pairs) {
+    Grouping best = {8, (pairs + 31) / 32};
+    for (int e : {6, 4, 2}) {
+        const int g = (pairs + 4 * e - 1) / (4 * e);
+        if (g * (e + 4) < best.groups * (best.E + 4)) best = {e, g};
+    }
+    return best;
+}
+
+size_t walk_lds(const Grouping& g, int KS, int MB) { return (size_t)g.groups * (KS * 3 * 1024 * MB + 4 * g.E * 3 * sizeof(int)); }
+// Workgroups of four waves: the registers hold three of them on a CU (two with five taps or two blocks of channels), but one of eight.
+// Eight where the LDS has room for one workgroup only and there are more than four waves to a CU.
+int walk_waves(size_t lds, double waves) { return 2 * lds > 160 * 1024 && waves > 4 * 256 ? 8 : 4; }
+
+// What a launch takes, in us: a workgroup sets up its weights; a wave walks its piece of S rows, KS - 1 steps more than it
+// has rows; a group of loads is a wait or, where a SIMD has several waves, its share of the instructions; of what the last,
+// partly filled round of workgroups leaves idle, 0.44 is lost.  Fitted to 814 layers (3x3 and 5x5, strides 1 and 2, 4x4
+// transposed and its gradient, 2 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 50 to 350 steps), each cut in all the
+// ways below: what it decides for takes 1.02 times the least of them, in the mean.
+double walk_time(double waves, int S, int pieces, int KS, int MB, const Grouping& g) {
+    const size_t lds = walk_lds(g, KS, MB);
+    const double load = waves * pieces / 1024;                            // waves per SIMD
+    const double room = (double)(160 * 1024 / lds) * walk_waves(lds, waves * pieces) / 4;
+    const double slots = KS > 3 || MB == 2 ? (room < 2 ? room : 2) : (room < 3 ? room : 3);
+    const int steps = (S + pieces - 1) / pieces + KS - 1;
+    const auto round = [&](double l) {
+        const double busy = l * (0.38 * MB + 0.097 * g.groups * g.E), wait = 1.5 * g.groups;
+        return 0.4 * g.groups * KS * MB + steps * (busy > wait ? busy : wait);
+    };
+    if (load <= slots) return round(load);
+    const int full = (int)(load / slots);
+    const double left = load - full * slots;
+    return 0.56 * load / slots * round(slots) + 0.44 * (full * round(slots) + (left > 0.02 ? round(left) : 0.0));
+}
+
+bool beyond_cache(int64_t N, const WalkConv& w) { return N * ((int64_t)w.in_plane + w.out_plane) > 250000000; }
+
+// How a launch is cut: XS neighbouring pixels of the line share a position, Co channels of them being the rows of a product,
+// MB blocks of 16 rows to a wave, and the S rows are walked in pieces.  `step`: pixels come in whole multiples of it; taps(XS): the
+// line taps they have together; count: samples and classes; channels: of the input, times the rows a step brings.
+struct Cut { int XS, pieces, MB; };
+template <typename Taps>
+Cut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int channels, int step, bool together, bool large,
+               Taps taps) {
+    Cut best = {step, 1, 1};
+    double least = 1e30;
+    for (int XS = step; XS == step || (together && Co * XS <= 16 && XS < width + step); XS += step) {
+        const int XP = taps(XS);
+        if (XS > step && XP > kMaxLineTaps) break;
+        const Grouping g = grouping(channels * XP);
+        const int64_t tiles = ((int64_t)((width + XS - 1) / XS) * quads + kWalkQuads - 1) / kWalkQuads;
+        for (int MB = 1; MB <= 2; ++MB) {
+            if (MB == 2 && (KS > 3 || Co * XS <= 16)) continue;
+            if (walk_lds(g, KS, MB) > kWalkLds) continue;
+            const double waves = (double)(count * ((Co * XS + 16 * MB - 1) / (16 * MB)) * tiles);
+            for (int pieces = 1; pieces <= S && pieces <= 16; pieces *= 2) {
+                // tensors beyond the last-level cache: pieces of a line that does not lie in one piece cost more
+                const double t = walk_time(waves, S, pieces, KS, MB, g) * (large && XS > step ? 1.15 : 1.0);
+                if (t < least) { least = t; best = {XS, pieces, MB}; }
+            }
+        }
+    }
+    // ... and of these tensors pieces that leave less than a round and a half waves take longer than they should: gradient of a
+    // transposed 4x4 layer, [32,8,32,32,300] -> 16 channels, 176 us with 2400 waves, 157 with 4800
+    if (large && best.MB == 1) {
+        const int64_t tiles = ((int64_t)((width + best.XS - 1) / best.XS) * quads + kWalkQuads - 1) / kWalkQuads;
+        const int64_t waves = count * ((Co * best.XS + 15) / 16) * tiles;
+        while (waves * best.pieces < 4608 && S >= 16 * best.pieces) best.pieces *= 2;
+    }
+    return best;
+}
+
+// The launch of a WalkConv whose geometry is filled in; `taps` of the walk.  false: not one that the kernel takes.
+bool launch(WalkConv& w, int taps, hipStream_t st, int* code) {
+    const int KS = slide_taps(taps);
+    if (KS < 1 || KS > 5 || w.XP > kMaxLineTaps) return false;
+    const int64_t pairs = (int64_t)w.Ci * w.XP * w.ss;
+    if (pairs > 4096) return false;
+    w.pairs = (int)pairs;
+    const Grouping grp = grouping(w.pairs);
+    const int E = grp.E;
+    w.groups = grp.groups;
+    const size_t bytes = walk_lds(grp, KS, w.MB);
+    if (bytes > kWalkLds) return false;
+    w.quads = (w.T + 3) / 4;
+    if ((int64_t)w.M * w.quads > 0x3fffffffLL) return false;
+    w.line_quads = w.M * w.quads;
+    w.tiles = (w.line_quads + kWalkQuads - 1) / kWalkQuads;
+    w.blocks = (w.Co * w.XS + 16 * w.MB - 1) / (16 * w.MB);
+    const int64_t base = (int64_t)w.N * w.blocks * w.classes * w.tiles;
+    const int pieces = w.pieces;
+    const int64_t items = (int64_t)w.tiles * pieces;
+    const int waves = walk_waves(bytes, (double)(base * pieces));
+    const int64_t wgs = (int64_t)w.N * w.blocks * w.classes * ((items + waves - 1) / waves);
+    if (items > 0x7fffffffLL || wgs > 0x7fffffffLL / 8) return false;
+    w.items = (int)items;
+#define SLAYER_WALK(KS, MB) launch_walk<KS, MB>(E, w, (unsigned)wgs, waves, bytes, st)
+    if (w.MB == 2) { if (KS == 1) SLAYER_WALK(1, 2); else if (KS == 2) SLAYER_WALK(2, 2); else SLAYER_WALK(3, 2); }
+    else if (KS == 1) SLAYER_WALK(1, 1);
+    else if (KS == 2) SLAYER_WALK(2, 1);
+    else if (KS == 3) SLAYER_WALK(3, 1);
+    else SLAYER_WALK(5, 1);
+#undef SLAYER_WALK
+    *code = (int)hipGetLastError();
+    return true;
+}
+
+void steps_inside(WalkClass& c, int ss, int Hs) {
+    c.c_lo = c.row0 + ss - 1 >= 0 ? 0 : (-c.row0 - ss + 1 + ss - 1) / ss;
+    c.c_hi = Hs - 1 - c.row0 < 0 ? 0 : (Hs - 1 - c.row0) / ss + 1;
+}
+
+}  // namespace
+
+bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
+    if (p.kh < 1 || p.kw < 1) return false;
+    const Axis h = {p.H, p.Ho, p.kh, p.sh, p.ph, p.dh, p.ky0, p.kys, p.kh_full, p.oy0, p.oys, p.Ho_full, p.kw_full};
+    const Axis v = {p.W, p.Wo, p.kw, p.sw, p.pw, p.dw, p.kx0, p.kxs, p.kw_full, p.ox0, p.oxs, p.Wo_full, 1};
+    auto taps = [](const Axis& a) { return a.k == 1 || a.dil == 1 ? (a.k + a.stride - 1) / a.stride : 0; };
+    auto takes = [&](const Axis& a, const Axis& line) { return taps(a) >= 1 && taps(a) <= 5 && line.k <= kMaxLineTaps && a.stride <= 16; };
+    // along the rows of the image, so that the line is one piece of memory, unless the filter has more taps the other way
+    const bool down = takes(h, v), right = takes(v, h);
+    if (!down && !right) return false;
+    const bool use_h = down && (!right || taps(h) >= taps(v));
+    const Axis& s = use_h ? h : v;
+    const Axis& l = use_h ? v : h;
+    const int px = p.T * 4;
+    WalkConv w;
+    w.out = p.out; w.in = p.in; w.weight = p.weight;
+    w.N = p.N; w.Ci = p.Ci; w.Co = p.Co; w.T = p.T;
+    w.in_ch = p.H * p.W * px; w.in_plane = p.Ci * w.in_ch;
+    w.out_ch = p.Ho_full * p.Wo_full * px; w.out_plane = p.Co * w.out_ch;
+    w.in_slide = use_h ? p.W * px : px; w.in_line = use_h ? px : p.W * px;
+    w.out_slide = s.ostep * (use_h ? p.Wo_full * px : px); w.out_line = l.ostep * (use_h ? px : p.Wo_full * px);
+    w.out_rx = w.out_line;
+    w.Hs = s.in; w.Ws = l.in;
+    // pixels that lie together share their taps, unless these lie apart
+    const auto line_taps = [&](int XS) { return (XS - 1) * l.stride + l.k; };
+    const bool together = l.dil == 1 || l.k == 1;
+    const Cut cut = cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together, beyond_cache(p.N, w),
+                               [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
+    w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
+    w.out_line *= w.XS;
+    w.M = (l.out + w.XS - 1) / w.XS;
+    w.ss = s.stride; w.ls = l.stride * w.XS;
+    w.XP = w.XS > 1 ? line_taps(w.XS) : l.k; w.shift0 = -l.pad; w.shift_step = w.XS > 1 ? 1 : l.dil;
+    w.line_full = l.out;
+    w.wslide = s.wstride; w.wline = l.wstride; w.nslide = s.kfull; w.nline = l.kfull;
+    w.sstep = s.kstep; w.l0 = l.k0; w.lstep = l.kstep; w.lrx = -l.stride * l.kstep;
+    w.classes = 1;
+    WalkClass& c = w.cls[0];
+    c.s0 = s.k0; c.row0 = -s.pad; c.S = s.out;
+    c.out0 = (p.oy0 * p.Wo_full + p.ox0) * px;
+    steps_inside(c, w.ss, w.Hs);
+    return launch(w, taps(s), st, code);
+}
+
+bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh, int sw, int ph, int pw, hipStream_t st, int* code) {
+    const int H = p.Ho_full, W = p.Wo_full, px = p.T * 4;                // of the result
+    if (sh > 4) return false;
+    WalkConv w;
+    w.out = p.out; w.in = p.in; w.weight = p.weight;
+    w.N = p.N; w.Ci = p.Ci; w.Co = p.Co; w.T = p.T;
+    w.in_ch = p.H * p.W * px; w.in_plane = p.Ci * w.in_ch;
+    w.out_ch = H * W * px; w.out_plane = p.Co * w.out_ch;
+    w.in_slide = p.W * px; w.in_line = px;
+    int lo = 0, hi = 0;                                                  // shifts of the line taps, over the pixels together
+    const auto line_taps = [&](int XS) {
+        lo = 1 << 30; hi = -(1 << 30);
+        for (int r = 0; r < XS; ++r)
+            for (int x = 0; x < kw; ++x)
+                if ((r + pw - x) % sw == 0) {
+                    const int d = (r + pw - x) / sw;
+                    lo = d < lo ? d : lo;
+                    hi = d > hi ? d : hi;
+                }
+        return hi - lo + 1;
+    };
+    const Cut cut = cut_launch((int64_t)p.N * (sh < H ? sh : H), p.Co, W, (p.T + 3) / 4, (H + sh - 1) / sh, slide_taps((kh + sh - 1) / sh), p.Ci, sw, true,
+                               beyond_cache(p.N, w),
+                               line_taps);
+    w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
+    w.XP = line_taps(w.XS); w.shift0 = lo; w.shift_step = 1;
+    w.out_slide = sh * W * px; w.out_line = w.XS * px; w.out_rx = px;
+    w.Hs = p.H; w.Ws = p.W; w.M = (W + w.XS - 1) / w.XS; w.line_full = W;
+    w.ss = 1; w.ls = w.XS / sw;
+    w.wslide = kw; w.wline = 1; w.nslide = kh; w.nline = kw;
+    w.sstep = -sh; w.l0 = pw - lo * sw; w.lstep = -sw; w.lrx = 1;
+    w.classes = sh < H ? sh : H;
+    int taps = 1;
+    for (int r = 0; r < w.classes; ++r) {
+        WalkClass& c = w.cls[r];
+        int count = 0, last = 0;
+        for (int y = 0; y < kh; ++y)
+            if ((r + ph - y) % sh == 0) { ++count; last = y; }
+        taps = count > taps ? count : taps;
+        c.S = (H - r + sh - 1) / sh;
+        c.out0 = r * W * px;
+        if (count) {
+            c.s0 = last;
+            c.row0 = (r + ph - last) / sh;
+            steps_inside(c, 1, w.Hs);
+        } else {                                                         // rows that no tap reaches: zeros
+            c.s0 = -1; c.row0 = 0; c.c_lo = c.c_hi = 0;
+        }
+    }
+    return launch(w, taps, st, code);
+}
+
+}  // namespace slayer

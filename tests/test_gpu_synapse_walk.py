@@ -1,0 +1,93 @@
+"""The walking kernel of the convolution synapse (csrc/synapse_walk.hip) where it can go wrong: every number of taps along the
+walk, strides along either axis, pixels that share a position, two blocks of channels, rows cut into pieces, residue classes of
+a transposed convolution, and pixels whose steps are not whole quads.  The operands are small integers, so every sum is exact
+in float32 whatever its order and the results equal float64's, bit for bit."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from tests.util import dev
+
+pytestmark = pytest.mark.gpu
+
+# (batch, Ci, H, W, T), Co, kernel, stride, padding, dilation
+FORMS = [
+    ((1, 1, 1, 1, 4), 1, (1, 2), (1, 1), (0, 1), (1, 1)),
+    ((2, 3, 4, 5, 5), 2, (3, 3), (1, 1), (1, 1), (1, 1)),            # several pixels to a position, the last one alone
+    ((1, 2, 7, 9, 6), 1, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ((1, 8, 33, 6, 7), 8, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ((1, 8, 6, 33, 11), 3, (5, 5), (1, 1), (2, 2), (1, 1)),
+    ((1, 5, 6, 7, 64), 17, (3, 3), (1, 1), (0, 2), (1, 1)),          # two blocks of channels, the second of one
+    ((1, 32, 5, 5, 300), 64, (3, 3), (1, 1), (1, 1), (1, 1)),
+    ((300, 17, 4, 4, 9), 40, (2, 2), (1, 1), (1, 1), (1, 1)),        # enough waves for whole rows
+    ((1, 4, 9, 8, 13), 6, (4, 4), (1, 1), (1, 2), (1, 1)),           # four taps
+    ((2, 4, 9, 10, 10), 8, (3, 3), (2, 2), (1, 1), (1, 1)),          # rows of a step outside the image on one side
+    ((2, 3, 10, 9, 50), 4, (5, 5), (2, 3), (2, 1), (1, 1)),
+    ((1, 2, 11, 12, 8), 5, (4, 3), (3, 2), (0, 0), (1, 1)),
+    ((1, 3, 8, 9, 20), 16, (3, 3), (1, 1), (2, 2), (1, 2)),          # taps along the line that lie apart
+    ((1, 3, 9, 8, 20), 16, (3, 3), (1, 1), (2, 2), (2, 1)),          # walked along the other axis
+    ((1, 3, 9, 8, 20), 4, (3, 3), (1, 1), (2, 2), (2, 2)),           # not one that it takes
+    ((1, 3, 9, 9, 20), 4, (7, 7), (1, 1), (3, 3), (1, 1)),
+    ((1, 3, 3, 12, 21), 4, (1, 5), (1, 1), (0, 2), (1, 1)),
+    ((1, 20, 4, 5, 31), 20, (1, 1), (1, 1), (0, 0), (1, 1)),
+    ((2, 4, 9, 7, 17), 4, (2, 2), (3, 3), (0, 0), (1, 1)),           # transposed: classes without taps
+]
+
+
+def _integers(gen, shape, most):
+    return torch.randint(-most, most + 1, shape, generator=gen).float()
+
+
+@pytest.mark.parametrize('form', FORMS, ids=str)
+@pytest.mark.parametrize('parts', [1, 3])
+def test_integers_equal_float64(form, parts):
+    """parts = 1: both operands are bfloat16 numbers; 3: neither is (up to 2^11 times 2^9, a few hundred terms: below 2^31,
+    held exactly where a sum stays below 2^24, which few taps of sparse inputs do)."""
+    import lava_dl_amd.slayer as slayer
+    shape, co, kernel, stride, padding, dilation = form
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x = _integers(gen, shape, 3 if parts == 1 else 1025)
+    w = _integers(gen, (co, shape[1]) + kernel + (1,), 5 if parts == 1 else 517)
+    if parts == 3:                                                   # at most 2^24 / (1025 * 517) = 31 terms of one sum
+        x *= torch.rand(shape, generator=gen) < 0.5
+        w *= torch.rand(w.shape, generator=gen) < min(1.0, 16 / (shape[1] * kernel[0] * kernel[1]))
+        assert float((w != 0).sum((1, 2, 3, 4)).max()) <= 31
+    cfg = (stride + (1,), padding + (0,), dilation + (1,))
+    want = F.conv3d(x.double(), w.double(), None, *cfg)
+    got = slayer.synapse.conv_synapse(x.to(dev()), w.to(dev()), stride, padding, dilation)
+    assert torch.equal(got.cpu().double(), want), 'convolution'
+    up = [(shape[2 + i] - 1) * stride[i] - 2 * padding[i] + dilation[i] * (kernel[i] - 1) + 1 for i in (0, 1)]
+    if min(up) < 1:
+        return
+    wt = w.transpose(0, 1).contiguous()[:, :31]                      # [Ci, Co, ...]: sums over Ci
+    if parts == 3:
+        wt = wt * (torch.rand(wt.shape, generator=gen) < min(1.0, 16 / float((wt != 0).sum((0, 2, 3, 4)).max())))
+        if float((wt != 0).sum((0, 2, 3, 4)).max()) > 31:
+            return
+    want = F.conv_transpose3d(x.double(), wt.double(), None, cfg[0], cfg[1], 0, 1, cfg[2])
+    got = slayer.synapse.conv_transpose_synapse(x.to(dev()), wt.to(dev()), stride, padding, dilation)
+    assert torch.equal(got.cpu().double(), want), 'transposed convolution'
+
+
+@pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
+@pytest.mark.parametrize('form', [FORMS[i] for i in (1, 3, 9, 10, 11, 18)], ids=str)
+def test_a_value_that_is_not_finite_reaches_the_outputs_whose_taps_meet_it_and_no_others(form, value):
+    import lava_dl_amd.slayer as slayer
+    shape, co, kernel, stride, padding, dilation = form
+    gen = torch.Generator().manual_seed(5)
+    x = torch.randint(1, 4, shape, generator=gen).float()
+    x[0, 0, shape[2] // 2, shape[3] // 2, 1] = value
+    cfg = (stride + (1,), padding + (0,), dilation + (1,))
+    for transposed in (False, True):
+        w = torch.randint(1, 5, ((shape[1], co) if transposed else (co, shape[1])) + kernel + (1,), generator=gen).float()
+        op = slayer.synapse.conv_transpose_synapse if transposed else slayer.synapse.conv_synapse
+        met = torch.zeros(shape).masked_fill_(~x.isfinite(), 1.0)
+        if transposed:
+            reach = F.conv_transpose3d(met, w, None, cfg[0], cfg[1], 0, 1, cfg[2]) > 0
+            want = F.conv_transpose3d(torch.where(x.isfinite(), x, 0.0), w, None, cfg[0], cfg[1], 0, 1, cfg[2])
+        else:
+            reach = F.conv3d(met, w, None, *cfg) > 0
+            want = F.conv3d(torch.where(x.isfinite(), x, 0.0), w, None, *cfg)
+        got = op(x.to(dev()), w.to(dev()), stride, padding, dilation).cpu()
+        want = torch.where(reach, torch.full_like(want, value), want)
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
