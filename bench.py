@@ -670,7 +670,7 @@ class ConvSynapse(Cuba):
     name = 'Conv synapse (3x3, 8 -> 16 channels) -> fused CUBA neuron, fwd+bwd (input and weight gradients)'
     ops = [('conv_synapse', 'synapse_walk_kernel', 6), ('cuba_fwd', 'stream_kernel_staged<CubaFwd>', 16),
            ('cuba_bwd', 'cuba_bwd_scan_kernel', 16), ('conv_synapse_bwd', 'synapse_walk_kernel', 6),
-           ('conv_synapse_wgrad', 'synapse_wgrad_row_kernel', 6)]
+           ('conv_synapse_wgrad', 'synapse_wgrad_walk_kernel', 6)]
     weight_gradient = True
     note = Cuba.note + '; input spikes Bernoulli(0.05) on 8 channels, weights round(N(0, 0.3) * 64) / 64'
     in_channels = 8
@@ -790,7 +790,7 @@ class ConvTransposeSynapse(Workload):
     name = 'ConvTranspose synapse 4x4 stride 2, 16 -> 8 channels, 16x16 -> 32x32, fwd + input and weight gradients'
     shape = (32, 8, 32, 32, 300)
     ops = [('conv_transpose', 'synapse_walk_kernel', 6), ('conv_transpose_bwd', 'synapse_walk_kernel', 6),
-           ('conv_transpose_wgrad', 'synapse_wgrad_kernel', 6)]
+           ('conv_transpose_wgrad', 'synapse_wgrad_walk_kernel', 6)]
     note = 'input spikes Bernoulli(0.05) on 16 channels of 16x16, weights round(N(0, 0.3) * 64) / 64, upstream gradient N(0, 1)'
 
     def __init__(self, dev):

@@ -92,4 +92,24 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t stream, int* code);
 bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh, int sw, int ph, int pw, hipStream_t stream,
                                     int* code);
 
+// The weight gradient on the walking kernel (synapse_wgrad_walk.hip): the geometry as for the convolution, in bytes, the line
+// cut into shares of whole visits of eight quads, the rows into kSynWaves pieces or one.
+struct WgradWalk {
+    float* partial;                     // [N][blocks of 16 channels][shares][passes][KS npt][64] quads
+    const float* grad_out;
+    const float* in;
+    int N, Co, T;
+    int in_plane, out_plane;            // bytes of one sample
+    int in_ch, in_slide, in_line, out_ch, out_slide, out_line;           // bytes
+    int Hs, Ws;                         // input rows along the walk, pixels along the line
+    int quads, line_quads;              // quads of steps a pixel of the gradient has, its line has
+    int ss, ls;                         // strides along walk and line
+    int row0, S, c_lo, c_hi;            // input row of step 0, gradient rows, the steps that meet a row inside the image
+    int XP, shift0, shift_step;         // line taps, the first one's shift, pixels from one to the next
+    int pairs, npt, passes, KS;         // (channel, line tap, row of a step) triples, tiles of 16 of them a pass, taps along the walk
+    int shares, share_quads, pieces;
+    int kslide, kline, wslide, wline;   // the filter's axes: sizes and strides
+};
+int launch_synapse_wgrad_walk(const WgradWalk& w, hipStream_t stream);
+
 }  // namespace slayer

@@ -340,284 +340,13 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
                                       acc[tt][0][2] + acc[tt][1][2], acc[tt][0][3] + acc[tt][1][3]);
 }
 
-// The common case again (unit stride and dilation along the image row, KW taps per row): the taps of a tile are 16
-// (input channel, kernel row) pairs at one input column, and that column meets KW output pixels, one per tap of the
-// row -- so the wave walks the input columns of its image row, keeps the gradient of the last KW pixels in registers
-// (one new visit per column), and a column costs 1 + NPT visits for KW * NPT tiles.
-// Accumulator tile (x, pt): [16 channels x 16 pairs] for tap x.
-//
-// The float32 instruction (16 steps of time in 4 x 32 cycles) was one bound of wide layers: 32 -> 64 channels on
-// [16,32,16,16,300] 539 us, 84 % of its peak.  Here the products run on the bfloat16
-// instruction (32 steps in 16 cycles): the gradient split into three parts (split.h), the input as it is where its
-// values are bfloat16 numbers -- spikes, and pooled spikes, always are; a visit that brings anything else splits it, too,
-// and takes six products instead of three.  The parts of the gradient are formed once per visit and stay in the window.
-// The other bound was the L1: in the operand's layout neighbouring lanes lie in sixteen different rows, so a load
-// of 1 KB looks up 64 lines.  Eight lanes now read the 128-byte line of a row together, and the split values
-// reach the operand's layout through LDS of the wave's own.
-//
-// The instruction rounds its sums down, not to nearest: a bias of some 2^-27 a product that a sum over 10^4 of them
-// collects (relative error of the result 1e-6, float32 instruction 1.3e-7 .. 5.7e-7).  A visit's products therefore start
-// from zero, every other column with the input negated, and the vector units add or subtract them: the biases cancel,
-// and the error is 0.8e-7 .. 1.2e-7 over spikes, graded spikes and real values.
-//   [16,32,16,16,300] -> 64 channels 539 -> 271 us, [32,8,32,32,300] -> 16 channels 374 -> 340 us (3 waves per SIMD; 64
-// steps per visit leave 2: 335 and 368 us).  What bounds it now: lines of the unaligned rows (T = 300) that two visits
-// share and fetch twice, and the vector instructions of the split.
-//
-// What is not finite (or overflows when it is scaled or rounded) shows in a tile at the end: the wave then runs its
-// share again with the float32 instruction (float_products), whose results such inputs had before.
-constexpr int kWgPitch = 80;                   // bytes of LDS per row of 32 bfloat16: no two quarters of a read collide
-constexpr int kWgSlot = 16 * kWgPitch;         // one part of one tile of 16 rows
-
-template <int KW, int NPT, bool TAIL>
-struct WgradRow {
-    const SynapseWgrad& p;
-    static constexpr int kSlots = 3 + 3 * NPT; // three parts of the gradient and of every tile of the input
-    char* lds;                                 // kSlots slots of this wave
-    __amdgpu_buffer_rsrc_t src, grd;
-    int col, co0, ho, hin, pair0, t_lo, t_hi, lane;
-    syn_f4 acc[KW][NPT];
-
-    // byte offset of the gradient row of channel co0 + r / of the input row of pair pair0 + r at column 0, or none
-    __device__ __forceinline__ int grad_row(int r) const {
-        return co0 + r < p.Co ? ((co0 + r) * p.Ho + ho) * p.Wo * col : kOutOfRange;
-    }
-    __device__ __forceinline__ int pair_row(int r) const {
-        const int pr = pair0 + r, ci = pr / p.kh, row = hin + (pr - ci * p.kh) * p.dh - p.ph;
-        return (pr < p.Ci * p.kh && (unsigned)row < (unsigned)p.H) ? (ci * p.H + row) * p.W * col : kOutOfRange;
-    }
-    // steps t .. t + 3 of the pixel (or column) x of such a row, to be moved into place (SynQuad) where they are used
-    __device__ __forceinline__ float4 grad_at(int row, int wo, const SynQuad& tq) const {
-        return buf_load4<false>(
-            grd, (tq.any() && row != kOutOfRange && (unsigned)wo < (unsigned)p.Wo) ? row + wo * col + tq.t_load * 4 : kOutOfRange);
-    }
-    __device__ __forceinline__ float4 pair_at(int row, int c, const SynQuad& tq) const {
-        return buf_load4<false>(src, (tq.any() && row != kOutOfRange) ? row + c * col + tq.t_load * 4 : kOutOfRange);
-    }
-    __device__ __forceinline__ void clear() {
-#pragma unroll
-        for (int x = 0; x < KW; ++x)
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt) acc[x][pt] = syn_f4{0.f, 0.f, 0.f, 0.f};
-    }
-    // the wave's own LDS: its instructions run in order, the fences keep the compiler to that order
-    __device__ __forceinline__ static void settle() {
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
-    // Lane l holds a quad of steps 4 (l % 8) of row l / 8 (+ 8 in the second quad); the operand's lane (kk, j) takes
-    // steps 8 kk .. 8 kk + 7 of row j.
-    __device__ __forceinline__ void put(int slot, int half, uint2 v) const {
-        *reinterpret_cast<uint2*>(lds + slot * kWgSlot + ((lane >> 3) + 8 * half) * kWgPitch + (lane & 7) * 8) = v;
-    }
-    __device__ __forceinline__ uint4 get(int slot) const {
-        return *reinterpret_cast<const uint4*>(lds + slot * kWgSlot + (lane & 15) * kWgPitch + (lane >> 4) * 16);
-    }
-    __device__ __forceinline__ static float4 scaled(float4 v) {
-        return make_float4(v.x * kSplitScale, v.y * kSplitScale, v.z * kSplitScale, v.w * kSplitScale);
-    }
-    __device__ __forceinline__ void put_parts(int slot, const float4 (&raw)[2], const SynQuad& tq) const {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float4 v = scaled(tq.template place<TAIL>(raw[h]));
-            uint2 part;
-#pragma unroll
-            for (int t = 0; t < 3; ++t) {
-                part.x = t < 2 ? round_pair(v.x, v.y) : bf16_pair(v.x, v.y);
-                part.y = t < 2 ? round_pair(v.z, v.w) : bf16_pair(v.z, v.w);
-                put(slot + t, h, part);
-            }
-        }
-    }
-
-    __device__ __forceinline__ void split_products() {
-        clear();
-        int g_row[2], q_row[NPT][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            g_row[h] = grad_row((lane >> 3) + 8 * h);
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt) q_row[pt][h] = pair_row(16 * pt + (lane >> 3) + 8 * h);
-        }
-        for (int t0 = t_lo; t0 < t_hi; t0 += 32) {
-            SynQuad tq;
-            tq.template set<TAIL>(t0 + 4 * (lane & 7), t_hi);
-            float4 raw_g[2], raw_q[NPT][2];
-            auto fetch = [&](int c) {
-#pragma unroll
-                for (int h = 0; h < 2; ++h) raw_g[h] = grad_at(g_row[h], c + p.pw, tq);
-#pragma unroll
-                for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) raw_q[pt][h] = pair_at(q_row[pt][h], c, tq);
-            };
-            // gw[x]: the gradient at pixel c + pw - x for the column c at hand; gw[0] arrives with the column
-            uint4 gw[KW][3];
-            float4 first[KW][2];
-#pragma unroll
-            for (int x = KW - 1; x >= 1; --x)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) first[x][h] = grad_at(g_row[h], p.pw - x, tq);
-#pragma unroll
-            for (int x = KW - 1; x >= 1; --x) {
-                put_parts(0, first[x], tq);
-                settle();
-#pragma unroll
-                for (int t = 0; t < 3; ++t) gw[x][t] = get(t);
-                settle();
-            }
-            fetch(0);
-            for (int c = 0; c < p.W; ++c) {
-                const unsigned flip = (c & 1) ? 0x80008000u : 0u;
-                const float back = (c & 1) ? -kSplitProductScale : kSplitProductScale;
-                auto flipped = [&](uint4 v) { return make_uint4(v.x ^ flip, v.y ^ flip, v.z ^ flip, v.w ^ flip); };
-                put_parts(0, raw_g, tq);
-                unsigned low = 0u;
-#pragma unroll
-                for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const float4 v = raw_q[pt][h] = tq.template place<TAIL>(raw_q[pt][h]);
-                        low |= __float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w);
-                    }
-                const bool more = __any((low & 0xffffu) != 0u);          // more than bfloat16 holds
-#pragma unroll
-                for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        float4 v = scaled(raw_q[pt][h]);
-                        if (!more) {
-                            put(3 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
-                        } else {
-                            uint2 part;
-                            part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
-                            put(3 + 3 * pt, h, part);
-                            part.x = round_pair(v.x, v.y); part.y = round_pair(v.z, v.w);
-                            put(4 + 3 * pt, h, part);
-                            put(5 + 3 * pt, h, make_uint2(bf16_pair(v.x, v.y), bf16_pair(v.z, v.w)));
-                        }
-                    }
-                settle();
-                if (c + 1 < p.W) fetch(c + 1);                           // on its way during the products
-#pragma unroll
-                for (int t = 0; t < 3; ++t) gw[0][t] = get(t);
-#pragma unroll
-                for (int pt = 0; pt < NPT; ++pt) {
-                    const uint4 q = flipped(get(3 + 3 * pt));
-                    syn_f4 d[KW];
-#pragma unroll
-                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][2], q, syn_f4{0.f, 0.f, 0.f, 0.f});
-                    if (more) {
-                        const uint4 q1 = flipped(get(4 + 3 * pt)), q2 = flipped(get(5 + 3 * pt));
-#pragma unroll
-                        for (int x = 0; x < KW; ++x) {
-                            d[x] = mfma_bf16(gw[x][0], q2, d[x]);
-                            d[x] = mfma_bf16(gw[x][1], q1, d[x]);
-                            d[x] = mfma_bf16(gw[x][0], q1, d[x]);
-                        }
-                    }
-#pragma unroll
-                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][1], q, d[x]);
-#pragma unroll
-                    for (int x = 0; x < KW; ++x) d[x] = mfma_bf16(gw[x][0], q, d[x]);
-#pragma unroll
-                    for (int x = 0; x < KW; ++x)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[x][pt][i] = __fmaf_rn(back, d[x][i], acc[x][pt][i]);
-                }
-                settle();
-#pragma unroll
-                for (int x = KW - 1; x >= 1; --x)
-#pragma unroll
-                    for (int t = 0; t < 3; ++t) gw[x][t] = gw[x - 1][t];
-            }
-        }
-    }
-    // the same sums on the float32 instruction, 16 steps at a time
-    __device__ __forceinline__ void float_products() {
-        clear();
-        const int g_row = grad_row(lane & 15);
-        int q_row[NPT];
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt) q_row[pt] = pair_row(16 * pt + (lane & 15));
-        for (int t0 = t_lo; t0 < t_hi; t0 += 16) {
-            SynQuad tq;
-            tq.template set<TAIL>(t0 + 4 * (lane >> 4), t_hi);
-            for (int c = 0; c < p.W; ++c) {
-#pragma unroll
-                for (int x = 0; x < KW; ++x) {
-                    const float4 g = tq.template place<TAIL>(grad_at(g_row, c + p.pw - x, tq));
-#pragma unroll
-                    for (int pt = 0; pt < NPT; ++pt) {
-                        const float4 q = tq.template place<TAIL>(pair_at(q_row[pt], c, tq));
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.x, q.x, acc[x][pt], 0, 0, 0);
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.y, q.y, acc[x][pt], 0, 0, 0);
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.z, q.z, acc[x][pt], 0, 0, 0);
-                        acc[x][pt] = __builtin_amdgcn_mfma_f32_16x16x4f32(g.w, q.w, acc[x][pt], 0, 0, 0);
-                    }
-                }
-            }
-        }
-    }
-    __device__ __forceinline__ bool not_finite() const {
-        bool bad = false;
-#pragma unroll
-        for (int x = 0; x < KW; ++x)
-#pragma unroll
-            for (int pt = 0; pt < NPT; ++pt)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) bad = bad || !(fabsf(acc[x][pt][i]) < __builtin_inff());
-        return __any(bad);
-    }
-};
-
-template <int KW, int NPT, bool TAIL>
-__global__ __launch_bounds__(kSynWaves * kWave) __attribute__((amdgpu_waves_per_eu(KW == 3 || NPT == 1 ? 3 : 2)))
-void synapse_wgrad_row_kernel(const SynapseWgrad p) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int cobs = (p.Co + 15) / 16;
-    // The waves of a workgroup, and neighbouring workgroups, take the channel blocks and passes of one share: they read
-    // the same input rows and gradient rows at about the same time and find them in the L1 and L2.
-    int b = xcd_contiguous(blockIdx.x, gridDim.x) * kSynWaves + wave;
-    const int cob = b % cobs; b /= cobs;
-    const int pass = b % p.passes; b /= p.passes;
-    const int item = b % p.items;
-    const int n = b / p.items;
-    if (n >= p.N) return;
-    const int co0 = cob * 16;
-    const int tpart = item % p.tparts;
-    const int ho = item / p.tparts;
-    __shared__ __attribute__((aligned(16))) char lds[kSynWaves][WgradRow<KW, NPT, TAIL>::kSlots * kWgSlot];
-    const int64_t in_plane = (int64_t)p.Ci * p.H * p.W * p.T;
-    const int64_t out_plane = (int64_t)p.Co * p.Ho * p.Wo * p.T;
-    WgradRow<KW, NPT, TAIL> w{p};
-    w.lds = lds[wave];
-    w.src = make_rsrc(p.in + (int64_t)n * in_plane, (unsigned)(in_plane * 4));
-    w.grd = make_rsrc(p.grad_out + (int64_t)n * out_plane, (unsigned)(out_plane * 4));
-    w.col = p.T * 4;
-    w.lane = lane;
-    w.co0 = co0; w.ho = ho; w.hin = ho * p.sh;
-    w.pair0 = pass * NPT * 16;
-    w.t_lo = tpart * p.tlen;
-    w.t_hi = (w.t_lo + p.tlen) < p.T ? (w.t_lo + p.tlen) : p.T;
-    w.split_products();
-    if (w.not_finite()) w.float_products();
-    // lane (q, j) of tile (x, pt): channels co0 + 4 q + i, pair 16 (pass NPT + pt) + j, tap x of its row
-    float4* dst = reinterpret_cast<float4*>(p.partial) +
-                  ((((int64_t)(n * cobs + cob) * p.items + item) * p.passes + pass) * (KW * NPT)) * kWave + lane;
-#pragma unroll
-    for (int x = 0; x < KW; ++x)
-#pragma unroll
-        for (int pt = 0; pt < NPT; ++pt)
-            dst[(x * NPT + pt) * kWave] = make_float4(w.acc[x][pt][0], w.acc[x][pt][1], w.acc[x][pt][2], w.acc[x][pt][3]);
-}
-
 // grad_w[co][k] = sum over batch entries and items of the waves' tiles, in double, in a fixed order, in two
 // launches: block (tile, chunk) adds the tiles of its chunk of the (batch entry, item) pairs -- sixteen partial sums
 // (every sixteenth pair each), then those in turn -- into stage[chunk][tile]; the second launch adds the chunks and
 // writes the gradient.  `tiles` tiles per wave and pass; tile tl holds taps k = 16 (pass tiles + tl) + j
-// (row_kw == 0) or, for the row kernel, pairs 16 (pass npt + tl % npt) + j at tap x = tl / npt of their row:
-// k = pair * row_kw + x.
+// (map.npt == 0) or, for the walking kernel, triples (channel, line tap, row of the step) 16 (pass npt + tl % npt) + j at tap
+// tl / npt of the walk.
+struct WgradMap { int npt, pairs, XP, ss, kslide, wslide, wline; };
 constexpr int kWgradParts = 16;
 constexpr int kWgradChunks = 32;
 __global__ __launch_bounds__(kWgradParts * kWave) void synapse_wgrad_reduce_kernel(
@@ -654,20 +383,20 @@ __global__ __launch_bounds__(kWgradParts * kWave) void synapse_wgrad_reduce_kern
 
 __global__ __launch_bounds__(kWave) void synapse_wgrad_final_kernel(float* __restrict__ grad_w,
                                                                      const double* __restrict__ stage, int Co, int K,
-                                                                     int passes, int tiles, int row_kw, int npt) {
+                                                                     int passes, int tiles, const WgradMap map) {
     const int lane = threadIdx.x, q = lane >> 4, j = lane & 15;
     const int tl = blockIdx.x % tiles;
     int b = blockIdx.x / tiles;
     const int pass = b % passes;
     const int cob = b / passes;
     int k;
-    if (row_kw == 0) {
+    if (map.npt == 0) {
         k = (pass * tiles + tl) * 16 + j;
     } else {
-        const int x = tl / npt, pt = tl - x * npt;
-        const int pair = (pass * npt + pt) * 16 + j;
-        k = pair * row_kw + x;
-        if (pair * row_kw >= K) k = K;                                   // a pair that does not exist
+        const int tap = tl / map.npt, pr = (pass * map.npt + tl - tap * map.npt) * 16 + j;
+        const int ci = pr / (map.XP * map.ss), r = pr - ci * (map.XP * map.ss), x = r / map.ss;
+        const int y = tap * map.ss + r - x * map.ss;
+        k = pr < map.pairs && y < map.kslide ? ci * map.XP * map.kslide + y * map.wslide + x * map.wline : K;   // or no tap
     }
     double tot[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c = 0; c < kWgradChunks; ++c) {
@@ -835,9 +564,9 @@ extern "C" int slayer_conv_synapse(float* out, const float* in, const float* wei
 
 namespace {
 
-// The form of the weight-gradient kernels for a geometry: the row kernel (tiles of 16 (channel, kernel row) pairs,
-// row_kw taps each) for unit stride and dilation along the image row with 3 or 5 taps per row, else tiles of 16
-// taps; `tiles` accumulator tiles per wave and pass; the shares the time axis is cut into.
+// The tiles of sums that the workspace of a geometry holds (`tiles` per wave and pass) and the one-pixel kernel's shares of the
+// time axis.  row_kw: 3 or 5 taps along the image row without stride or dilation, tiles of 16 (channel, kernel row) pairs; that
+// the walking kernel cuts its line into no more shares than these have is what bounds its workspace.
 struct WgradForm { int row_kw, npt, tiles; };
 WgradForm wgrad_form(int64_t Ci, int64_t kh, int64_t kw, int64_t stride_w, int64_t dil_w) {
     WgradForm f;
@@ -858,14 +587,8 @@ void wgrad_shape(int64_t N, int64_t Ci, int64_t Co, int64_t Ho, int64_t T, int64
                  SynapseWgrad& p) {
     if (f.row_kw) p.passes = (int)((Ci * kh + 16 * f.npt - 1) / (16 * f.npt));
     else p.passes = (int)((Ci * kh * kw + 16 * f.tiles - 1) / (16 * f.tiles));
-    // Shares of whole visits of 32 steps, about eight thousand waves: a wave's set-up (the gradient window) is paid once per
-    // share ([16,32,16,16,300] -> 64 channels 310 us with 4096 waves, 285 with 8192).  A row of up to 16 pairs has few
-    // products to a visit and is bound by its loads, and a line that two visits of one share have in common is gone
-    // from the caches when the second one comes, while the waves of neighbouring shares find it there: one visit a
-    // share, up to 32768 waves (float32 kernel before / 8192 / 32768 waves: [32,4,32,32,300] -> 16 channels 237 / 280 / 206 us,
-    // [64,1,32,32,300] -> 16 383 / 445 / 313, [8,4,64,64,300] -> 64 904 / 1008 / 685, 5x5 [32,2,32,32,300] -> 16
-    // 303 / 260 / 198, and where rows are whole lines [32,4,32,32,256] -> 16 147 / 147 / 146, [128,4,32,32,64] -> 16
-    // 167 / 176 / 177).
+    // Shares of whole visits of 32 steps, about eight thousand waves, since a wave's start is paid once per share; layers of up to
+    // 16 pairs, which have few products to a visit and are bound by their loads, one visit a share up to 32768 waves.
     const int64_t waves = f.npt == 1 ? 32768 : 8192;
     const int64_t base = N * ((Co + 15) / 16) * Ho;
     const int64_t visits = (T + 31) / 32;
@@ -875,6 +598,51 @@ void wgrad_shape(int64_t N, int64_t Ci, int64_t Co, int64_t Ho, int64_t T, int64
     p.tparts = (int)((T + len - 1) / len);
     p.tlen = (int)len;
     p.items = (int)(Ho * p.tparts);
+}
+
+// The walking form of a geometry ([0]: rows, [1]: columns) in a workspace of `floats`, or false.  w: tensors, N, Co and T filled in.
+bool wgrad_walk(WgradWalk& w, int Ci, const int (&k)[2], const int (&stride)[2], const int (&pad)[2], const int (&dil)[2],
+                const int (&in)[2], const int (&out)[2], int64_t floats) {
+    const int px = w.T * 4;
+    auto taps = [&](int a) { return (k[a] == 1 || dil[a] == 1) && stride[a] <= 16 ? (k[a] + stride[a] - 1) / stride[a] : 0; };
+    const bool down = taps(0) >= 1 && taps(0) <= 5, right = taps(1) >= 1 && taps(1) <= 5;
+    if (!down && !right) return false;
+    const int s = down && (!right || taps(0) >= taps(1)) ? 0 : 1, l = 1 - s;
+    w.KS = taps(s) == 4 ? 5 : taps(s);
+    w.in_ch = in[0] * in[1] * px; w.in_plane = Ci * w.in_ch;
+    w.out_ch = out[0] * out[1] * px; w.out_plane = w.Co * w.out_ch;
+    w.in_slide = s == 0 ? in[1] * px : px; w.in_line = s == 0 ? px : in[1] * px;
+    w.out_slide = s == 0 ? out[1] * px : px; w.out_line = s == 0 ? px : out[1] * px;
+    w.Hs = in[s]; w.Ws = in[l];
+    w.quads = (w.T + 3) / 4;
+    if ((int64_t)out[l] * w.quads > 0x3fffffffLL) return false;
+    w.line_quads = out[l] * w.quads;
+    w.ss = stride[s]; w.ls = stride[l];
+    w.row0 = -pad[s]; w.S = out[s];
+    w.c_lo = w.row0 + w.ss - 1 >= 0 ? 0 : -w.row0 / w.ss;
+    w.c_hi = w.Hs - 1 - w.row0 < 0 ? 0 : (w.Hs - 1 - w.row0) / w.ss + 1;
+    w.XP = k[l]; w.shift0 = -pad[l]; w.shift_step = dil[l];
+    w.kslide = k[s]; w.kline = k[l];
+    w.wslide = s == 0 ? k[1] : 1; w.wline = s == 0 ? 1 : k[1];
+    w.pairs = Ci * w.XP * w.ss;
+    w.npt = w.pairs <= 16 ? 1 : 2;
+    w.passes = (w.pairs + 16 * w.npt - 1) / (16 * w.npt);
+    // as many waves as the workspace has room for, and no more than the line has visits; few waves: pieces of the rows
+    const int64_t cobs = (w.Co + 15) / 16;
+    const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N;
+    if (room < 1) return false;
+    const int64_t visits = (w.line_quads + 7) / 8;
+    const int64_t each = (visits + room - 1) / room;
+    w.share_quads = (int)(8 * each);
+    w.shares = (int)((visits + each - 1) / each);
+    // The rows in pieces where that is fewer steps for the chip, which two waves to a SIMD fill: a piece has KS - 1 steps more than
+    // it has rows, and its start is worth about three.
+    auto steps = [&](int pieces) {
+        const double load = (double)(w.N * cobs * w.passes * w.shares * pieces) / 2250;
+        return ((w.S + pieces - 1) / pieces + w.KS + 2) * (load > 1 ? load : 1);
+    };
+    w.pieces = steps(kSynWaves) < steps(1) ? kSynWaves : 1;
+    return true;
 }
 
 }  // namespace
@@ -921,49 +689,52 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     if (Ci * H * W * T * 4 >= lim || Co * Ho * Wo * T * 4 >= lim || K > 4096 || pad_h > 4096 || pad_w > 4096 ||
         H * stride_h > (1 << 20) || W * stride_w > (1 << 20) || Ho > (1 << 20) || T > (1 << 24))
         return SLAYER_ERANGE;
+    const int64_t cobs = (Co + 15) / 16;
+    const int64_t floats = slayer_conv_synapse_wgrad_workspace(N, Ci, Co, H, W, T, kh, kw, stride_h, pad_h, dil_h);
+    auto reduce = [&](int items, int passes, int tiles, const WgradMap& map) {
+        double* stage = reinterpret_cast<double*>(workspace + N * cobs * items * passes * tiles * 256);
+        const unsigned tile_blocks = (unsigned)(cobs * passes * tiles);
+        hipLaunchKernelGGL(synapse_wgrad_reduce_kernel, dim3(tile_blocks, kWgradChunks), dim3(kWgradParts * kWave), 0, st, stage,
+                           workspace, (int)N, (int)Co, items, passes, tiles);
+        hipLaunchKernelGGL(synapse_wgrad_final_kernel, dim3(tile_blocks), dim3(kWave), 0, st, grad_weight, stage, (int)Co, (int)K,
+                           passes, tiles, map);
+        return (int)hipGetLastError();
+    };
+    WgradWalk w;
+    w.partial = workspace; w.grad_out = grad_out; w.in = in;
+    w.N = (int)N; w.Co = (int)Co; w.T = (int)T;
+    const int ker[2] = {(int)kh, (int)kw}, str[2] = {(int)stride_h, (int)stride_w}, pad[2] = {(int)pad_h, (int)pad_w};
+    const int dil[2] = {(int)dil_h, (int)dil_w}, size[2] = {(int)H, (int)W}, size_out[2] = {(int)Ho, (int)Wo};
+    if (wgrad_walk(w, (int)Ci, ker, str, pad, dil, size, size_out, floats)) {
+        if (workspace_floats < (N * w.shares + 2 * kWgradChunks) * cobs * w.passes * w.KS * w.npt * 256) return SLAYER_ERANGE;
+        const int code = launch_synapse_wgrad_walk(w, st);
+        if (code != 0) return code;
+        return reduce(w.shares, w.passes, w.KS * w.npt, {w.npt, w.pairs, w.XP, w.ss, w.kslide, w.wslide, w.wline});
+    }
     SynapseWgrad p;
     p.partial = workspace; p.grad_out = grad_out; p.in = in;
     p.N = (int)N; p.Ci = (int)Ci; p.Co = (int)Co; p.H = (int)H; p.W = (int)W; p.Ho = (int)Ho; p.Wo = (int)Wo; p.T = (int)T;
     p.kh = (int)kh; p.kw = (int)kw; p.sh = (int)stride_h; p.sw = (int)stride_w; p.ph = (int)pad_h; p.pw = (int)pad_w;
     p.dh = (int)dil_h; p.dw = (int)dil_w;
     p.K = (int)K;
-    const WgradForm f = wgrad_form(Ci, kh, kw, stride_w, dil_w);
+    const WgradForm f = wgrad_form(Ci, kh, kw, 2, 1);                     // tiles of 16 taps
     wgrad_shape(N, Ci, Co, Ho, T, kh, kw, f, p);
-    const int64_t cobs = (Co + 15) / 16;
     // the waves' tiles, then the chunk sums of the first reduction launch (doubles)
-    const int64_t tile_floats = N * cobs * p.items * p.passes * f.tiles * 256;
-    const int64_t stage_floats = 2 * kWgradChunks * cobs * p.passes * f.tiles * 256;
-    if (workspace_floats < tile_floats + stage_floats) return SLAYER_ERANGE;
-    double* stage = reinterpret_cast<double*>(workspace + tile_floats);
+    if (workspace_floats < (N * p.items + 2 * kWgradChunks) * cobs * p.passes * f.tiles * 256) return SLAYER_ERANGE;
     const int64_t blocks = N * cobs * ((p.items + kSynWaves - 1) / kSynWaves);
     if (blocks > 0x7fffffffLL || p.passes > 65535) return SLAYER_ERANGE;
-    const int64_t row_blocks = (N * cobs * p.items * p.passes + kSynWaves - 1) / kSynWaves;
-    if (row_blocks > 0x7fffffffLL / kSynWaves) return SLAYER_ERANGE;
-    const dim3 grid((unsigned)blocks, (unsigned)p.passes), row_grid((unsigned)row_blocks), block(kSynWaves * kWave);
+    const dim3 grid((unsigned)blocks, (unsigned)p.passes), block(kSynWaves * kWave);
     const bool tail = (T % 4) != 0;                                       // rows that end inside a quad
 #define SLAYER_WGRAD(NTT)                                                                                              \
     do {                                                                                                               \
         if (tail) hipLaunchKernelGGL((synapse_wgrad_kernel<NTT, true>), grid, block, NTT * 16 * 3 * sizeof(int), st, p); \
         else hipLaunchKernelGGL((synapse_wgrad_kernel<NTT, false>), grid, block, NTT * 16 * 3 * sizeof(int), st, p);    \
     } while (0)
-#define SLAYER_WGRAD_ROW(KW, NPT)                                                                                      \
-    do {                                                                                                               \
-        if (tail) hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, true>), row_grid, block, 0, st, p);             \
-        else hipLaunchKernelGGL((synapse_wgrad_row_kernel<KW, NPT, false>), row_grid, block, 0, st, p);                 \
-    } while (0)
-    if (f.row_kw == 3) { if (f.npt == 1) SLAYER_WGRAD_ROW(3, 1); else SLAYER_WGRAD_ROW(3, 2); }
-    else if (f.row_kw == 5) { if (f.npt == 1) SLAYER_WGRAD_ROW(5, 1); else SLAYER_WGRAD_ROW(5, 2); }
-    else if (f.tiles == 1) SLAYER_WGRAD(1);
+    if (f.tiles == 1) SLAYER_WGRAD(1);
     else if (f.tiles == 2) SLAYER_WGRAD(2);
     else SLAYER_WGRAD(5);
-#undef SLAYER_WGRAD_ROW
 #undef SLAYER_WGRAD
-    const unsigned tile_blocks = (unsigned)(cobs * p.passes * f.tiles);
-    hipLaunchKernelGGL(synapse_wgrad_reduce_kernel, dim3(tile_blocks, kWgradChunks), dim3(kWgradParts * kWave), 0, st,
-                       stage, workspace, (int)N, (int)Co, p.items, p.passes, f.tiles);
-    hipLaunchKernelGGL(synapse_wgrad_final_kernel, dim3(tile_blocks), dim3(kWave), 0, st, grad_weight, stage, (int)Co,
-                       (int)K, p.passes, f.tiles, f.row_kw, f.npt);
-    return (int)hipGetLastError();
+    return reduce(p.items, p.passes, f.tiles, {0, 0, 1, 1, 0, 0, 0});
 }
 
 // The gradient of the input of slayer_conv_synapse for any stride (and, read as a layer of its own, the transposed

@@ -1,4 +1,4 @@
-"""The walking kernel of the convolution synapse (csrc/synapse_walk.hip) where it can go wrong: every number of taps along the
+"""The walking kernels of the convolution synapse (csrc/synapse_walk.hip, synapse_wgrad_walk.hip) where they can go wrong: every number of taps along the
 walk, strides along either axis, pixels that share a position, two blocks of channels, rows cut into pieces, residue classes of
 a transposed convolution, and pixels whose steps are not whole quads.  The operands are small integers, so every sum is exact
 in float32 whatever its order and the results equal float64's, bit for bit."""
@@ -67,6 +67,28 @@ def test_integers_equal_float64(form, parts):
     want = F.conv_transpose3d(x.double(), wt.double(), None, cfg[0], cfg[1], 0, 1, cfg[2])
     got = slayer.synapse.conv_transpose_synapse(x.to(dev()), wt.to(dev()), stride, padding, dilation)
     assert torch.equal(got.cpu().double(), want), 'transposed convolution'
+
+
+@pytest.mark.parametrize('form', FORMS + [((1, 3, 33, 3, 12), 16, (3, 3), (1, 1), (1, 1), (1, 1)),          # rows in four pieces
+                                          ((1, 2, 9, 4, 70), 4, (3, 3), (1, 1), (1, 1), (1, 1)),            # ... of two or three
+                                          ((40, 8, 8, 8, 300), 16, (3, 3), (1, 1), (1, 1), (1, 1))], ids=str)   # whole rows
+@pytest.mark.parametrize('split', ['neither', 'gradient', 'input'])
+def test_weight_gradient_of_integers_equals_float64(form, split):
+    """Up to 2^18 terms of at most 3 * 3, or at most 31 of an operand that takes several parts: below 2^24."""
+    from lava_dl_amd.slayer.synapse import layer
+    shape, co, kernel, stride, padding, dilation = form
+    gen = torch.Generator().manual_seed(sum(shape) + co + 1)
+    out = [(shape[2 + i] + 2 * padding[i] - dilation[i] * (kernel[i] - 1) - 1) // stride[i] + 1 for i in (0, 1)]
+    x, g = _integers(gen, shape, 3), _integers(gen, (shape[0], co, *out, shape[4]), 3)
+    if split != 'neither':
+        big = g if split == 'gradient' else x
+        keep = torch.rand(big.shape, generator=gen) < 16 / (big.numel() / big.shape[1])
+        big.copy_(_integers(gen, big.shape, 60001) * keep)
+        assert float((big != 0).sum((0, 2, 3, 4)).max()) <= 31       # 31 * 60001 * 3 < 2^24
+    wd = torch.zeros((co, shape[1]) + kernel + (1,), dtype=torch.float64).requires_grad_()
+    F.conv3d(x.double(), wd, None, stride + (1,), padding + (0,), dilation + (1,)).backward(g.double())
+    got = layer._weight_gradient(x.to(dev()), wd.shape, g.to(dev()), stride, padding, dilation)
+    assert torch.equal(got.cpu().double(), wd.grad)
 
 
 @pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
