@@ -341,9 +341,9 @@ int slayer_conv_synapse(float *out, const float *in, const float *weight,
  *                           grad_out[n][co][(h + pad_h - y * dil_h) / stride_h][(w + pad_w - x * dil_w) / stride_w][t]
  * over the taps whose two quotients are exact and lie inside grad_out's [Ho][Wo].  N, Ci, Co, H, W, kh ... dil_w are
  * those of the forward call; weight_t is [Ci][Co][kh][kw] (the forward weights with the channel axes exchanged,
- * not flipped).  One launch per residue class of the pixels modulo the strides (stride_h * stride_w launches, each
- * a plain convolution over the taps that class meets); a single launch on the vector units when Ci = Co = 1 (the
- * pooling layers).  SLAYER_ERANGE as for slayer_conv_synapse, and for strides above 16 or images beyond 65535
+ * not flipped).  One launch without dilation and for strides along the rows of up to 4 (and, on the vector units, when
+ * Ci = Co = 1: the pooling layers), else one per residue class of the pixels modulo the strides (stride_h * stride_w
+ * launches, each a plain convolution over the taps that class meets).  SLAYER_ERANGE as for slayer_conv_synapse, and for strides above 16 or images beyond 65535
  * pixels a side. */
 int slayer_conv_synapse_input_grad(float *grad_in, const float *grad_out, const float *weight_t,
                                    int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
@@ -601,6 +601,12 @@ int slayer_recurrent_steps_bwd(float *grad_z, const float *grad_spikes, const fl
                                const float *rec, float spike_threshold, float tau_rho, float scale_rho, int graded,
                                int64_t N, int64_t C, int64_t T,
                                float *workspace, int64_t workspace_floats, void *stream);
+
+/* The operands of the recurrent weight gradient, [C][N * (T-1)] times [N * (T-1)][C] (utils/recurrent.py:85-112):
+ * grad_rows[c][n * (T-1) + t] = grad[n][c][t+1], spike_rows[n * (T-1) + t][c] = spikes[n][c][t], t < T-1.  Nothing is written for
+ * T < 2. */
+int slayer_recurrent_operands(float *grad_rows, float *spike_rows, const float *grad, const float *spikes, int64_t N, int64_t C,
+                              int64_t T, void *stream);
 
 /* ---- weight quantiser ------------------------------------------------------------------------- */
 

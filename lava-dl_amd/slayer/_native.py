@@ -82,6 +82,7 @@ _SIGNATURES = {
     'slayer_recurrent_steps_workspace': (_I64, [_I64, _I64, _I64, _INT]),
     'slayer_cuba_recurrent_steps_fwd': (_INT, [_P] * 10 + [_F, _INT, _F, _INT] + [_I64] * 7 + [_P, _I64, _P]),
     'slayer_alif_recurrent_steps_fwd': (_INT, [_P] * 17 + [_F, _I64, _INT, _F, _INT] + [_I64] * 11 + [_P, _I64, _P]),
+    'slayer_recurrent_operands': (_INT, [_P] * 4 + [_I64] * 3 + [_P]),
     'slayer_quantize': (_INT, [_P] * 3 + [_F] * 4 + [_I64, _P]),
     'slayer_rf_limit': (_INT, [_P] * 2 + [_F, _I64, _P]),
     'slayer_quantize_bwd': (_INT, [_P] * 3 + [_F, _I64, _P]),

@@ -11,6 +11,9 @@ that multiplies the matrix with the whole batch; any other neuron runs the refer
 import torch
 
 from .. import _native as N
+from .quantize import takes_kernel
+
+_ERANGE = -3
 
 
 def _recurrent_matrix(recurrent_synapse):
@@ -124,8 +127,28 @@ class CustomRecurrent(torch.autograd.Function):
         return grad_z, None, _weight_gradient(grad_z, ctx.x)
 
 
+def _operands(grad_z, x):
+    """The two operands of _weight_gradient in one launch, or None where somebody wants to see the single operations or they are
+    not float32 tensors on one GPU as they lie in memory."""
+    if not (takes_kernel(grad_z) and takes_kernel(x) and grad_z.device == x.device and grad_z.shape == x.shape
+            and x.shape[-1] > 1 and not (torch.is_grad_enabled() and (grad_z.requires_grad or x.requires_grad))):
+        return None
+    n, c, t = x.shape
+    grad_rows, spike_rows = x.new_empty(c, n * (t - 1)), x.new_empty(n * (t - 1), c)
+    with N.device_guard(x.device):
+        code = N.lib().slayer_recurrent_operands(N.ptr(grad_rows), N.ptr(spike_rows), N.ptr(grad_z), N.ptr(x), n, c, t,
+                                                 N.stream_handle())
+    if code == _ERANGE:
+        return None
+    N.check(code)
+    return grad_rows, spike_rows
+
+
 def _weight_gradient(grad_z, x):
     """grad R = sum over batch and time of grad_feedback[t] (outer) spike[t-1]."""
+    operands = _operands(grad_z, x)
+    if operands is not None:
+        return torch.matmul(*operands)
     grad_output = grad_z[..., 1:].transpose(0, 1).reshape(grad_z.shape[1], -1)
     spikes_in = x[..., :-1].transpose(1, 2).reshape(-1, x.shape[1])
     return torch.matmul(grad_output, spikes_in)
