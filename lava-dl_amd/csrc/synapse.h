@@ -95,7 +95,7 @@ bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh
 // The weight gradient on the walking kernel (synapse_wgrad_walk.hip): the geometry as for the convolution, in bytes, the line
 // cut into shares of whole visits of eight quads, the rows into kSynWaves pieces or one.
 struct WgradWalk {
-    float* partial;                     // [N][blocks of 16 channels][shares][passes][KS npt][64] quads
+    float* partial;                     // [N][blocks of 16 channels][sets][passes][KS npt][64] quads
     const float* grad_out;
     const float* in;
     int N, Co, T;
@@ -107,7 +107,7 @@ struct WgradWalk {
     int row0, S, c_lo, c_hi;            // input row of step 0, gradient rows, the steps that meet a row inside the image
     int XP, shift0, shift_step;         // line taps, the first one's shift, pixels from one to the next
     int pairs, npt, passes, KS;         // (channel, line tap, row of a step) triples, tiles of 16 of them a pass, taps along the walk
-    int shares, share_quads, pieces;
+    int shares, share_quads, pieces, sets;   // sets of tiles: one a share, or one for the shares of a workgroup
     int kslide, kline, wslide, wline;   // the filter's axes: sizes and strides
 };
 int launch_synapse_wgrad_walk(const WgradWalk& w, hipStream_t stream);

@@ -629,7 +629,13 @@ bool wgrad_walk(WgradWalk& w, int Ci, const int (&k)[2], const int (&stride)[2],
     w.passes = (w.pairs + 16 * w.npt - 1) / (16 * w.npt);
     // as many waves as the workspace has room for, and no more than the line has visits; few waves: pieces of the rows
     const int64_t cobs = (w.Co + 15) / 16;
-    const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N;
+    // The waves of a workgroup take neighbouring shares and leave one set of tiles: a quarter of the tiles to write and add, and
+    // room for shares of one visit, which leaves no line to two visits of one wave.  [32,8,32,32,300] -> 16 channels 330 -> 290 us
+    // (cold caches), 4x4 stride 2 194 -> 184, [16,16,20,18,128] -> 32 97 -> 86, 5x5 [16,32,12,12,150] -> 64 280 -> 252.  With many
+    // blocks of channels and passes these are what the waves of a workgroup had better share: [16,32,16,16,300] -> 64, twelve
+    // of them, 296 us with the same operands in a workgroup, 307 without; five taps have enough products a load.
+    const int merged = cobs * w.passes <= 8 || w.KS == 5 ? kSynWaves : 1;
+    const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N * merged;
     if (room < 1) return false;
     const int64_t visits = (w.line_quads + 7) / 8;
     const int64_t each = (visits + room - 1) / room;
@@ -641,7 +647,8 @@ bool wgrad_walk(WgradWalk& w, int Ci, const int (&k)[2], const int (&stride)[2],
         const double load = (double)(w.N * cobs * w.passes * w.shares * pieces) / 2250;
         return ((w.S + pieces - 1) / pieces + w.KS + 2) * (load > 1 ? load : 1);
     };
-    w.pieces = steps(kSynWaves) < steps(1) ? kSynWaves : 1;
+    w.pieces = w.shares <= room / merged && steps(kSynWaves) < steps(1) ? kSynWaves : 1;
+    w.sets = w.pieces == 1 ? (w.shares + merged - 1) / merged : w.shares;
     return true;
 }
 
@@ -706,10 +713,10 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     const int ker[2] = {(int)kh, (int)kw}, str[2] = {(int)stride_h, (int)stride_w}, pad[2] = {(int)pad_h, (int)pad_w};
     const int dil[2] = {(int)dil_h, (int)dil_w}, size[2] = {(int)H, (int)W}, size_out[2] = {(int)Ho, (int)Wo};
     if (wgrad_walk(w, (int)Ci, ker, str, pad, dil, size, size_out, floats)) {
-        if (workspace_floats < (N * w.shares + 2 * kWgradChunks) * cobs * w.passes * w.KS * w.npt * 256) return SLAYER_ERANGE;
+        if (workspace_floats < (N * w.sets + 2 * kWgradChunks) * cobs * w.passes * w.KS * w.npt * 256) return SLAYER_ERANGE;
         const int code = launch_synapse_wgrad_walk(w, st);
         if (code != 0) return code;
-        return reduce(w.shares, w.passes, w.KS * w.npt, {w.npt, w.pairs, w.XP, w.ss, w.kslide, w.wslide, w.wline});
+        return reduce(w.sets, w.passes, w.KS * w.npt, {w.npt, w.pairs, w.XP, w.ss, w.kslide, w.wslide, w.wline});
     }
     SynapseWgrad p;
     p.partial = workspace; p.grad_out = grad_out; p.in = in;

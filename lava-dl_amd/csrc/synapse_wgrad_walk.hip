@@ -21,8 +21,8 @@
 // start from zero, every other step with the input negated, and the vector units add or subtract them: the biases cancel,
 // and the error against float64 is 0.5e-7 .. 1.0e-7.
 //
-// Few waves: the rows are cut into four pieces, the waves of one workgroup, whose sums are added in double before they are
-// written.  What is not finite (or overflows when it is scaled or rounded) shows in a tile at the end: the wave then runs its
+// The sums of a workgroup's waves are added in double before they are written; where waves are few, these are four pieces of the
+// rows.  What is not finite (or overflows when it is scaled or rounded) shows in a tile at the end: the wave then runs its
 // share again with the float32 instruction (float_products).
 #include "synapse.h"
 #include "split.h"
@@ -289,18 +289,18 @@ void synapse_wgrad_walk_kernel(const WgradWalk p) {
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int cobs = (p.Co + 15) / 16;
-    // Whole rows: the waves of a workgroup, and neighbouring workgroups, take the channel blocks and passes of one share: they
-    // read the same input rows and gradient rows at about the same time and find them in the L1 and L2.  In pieces: the
-    // waves of a workgroup take the pieces of one share, and their sums are one set of tiles.
-    const bool together = p.pieces > 1;
+    // The waves of a workgroup take neighbouring shares, or the pieces of one, and their sums are one set of tiles; or, with many
+    // channel blocks and passes, these of one share: they read the same input rows and gradient rows at about the same time
+    // and find them in the L1 and L2.
+    const bool together = p.pieces > 1 || p.sets < p.shares;
     int b = xcd_contiguous(blockIdx.x, gridDim.x);
     if (!together) b = b * kSynWaves + wave;
     const int cob = b % cobs; b /= cobs;
     const int pass = b % p.passes; b /= p.passes;
-    const int share = b % p.shares;
-    const int n = b / p.shares;
-    if (n >= p.N) return;                               // (never in pieces: those are whole workgroups)
-    const int piece = together ? wave : 0;
+    const int set = b % p.sets;
+    const int n = b / p.sets;
+    if (n >= p.N) return;                               // (never together: those are whole workgroups)
+    const int share = p.sets < p.shares ? set * kSynWaves + wave : set, piece = p.pieces > 1 ? wave : 0;
     const int per = (p.S + p.pieces - 1) / p.pieces;
     __shared__ __attribute__((aligned(16))) char lds[kSynWaves][WgradWave<KS, NPT>::kSlots * kWgSlot];
     WgradWave<KS, NPT> w{p};
@@ -318,7 +318,7 @@ void synapse_wgrad_walk_kernel(const WgradWalk p) {
     if (w.not_finite()) w.float_products();
     // lane (q, j) of tile (x, pt): channels co0 + 4 q + i, pair 16 (pass NPT + pt) + j, tap x of the walk
     float4* dst = reinterpret_cast<float4*>(p.partial) +
-                  ((((int64_t)(n * cobs + cob) * p.shares + share) * p.passes + pass) * (KS * NPT)) * kWave + lane;
+                  ((((int64_t)(n * cobs + cob) * p.sets + set) * p.passes + pass) * (KS * NPT)) * kWave + lane;
     if (!together) {
 #pragma unroll
         for (int x = 0; x < KS; ++x)
@@ -349,8 +349,8 @@ void synapse_wgrad_walk_kernel(const WgradWalk p) {
 }
 
 int launch_synapse_wgrad_walk(const WgradWalk& w, hipStream_t st) {
-    const int64_t sets = (int64_t)w.N * ((w.Co + 15) / 16) * w.shares * w.passes;        // of tiles
-    const int64_t blocks = w.pieces > 1 ? sets : (sets + kSynWaves - 1) / kSynWaves;
+    const int64_t sets = (int64_t)w.N * ((w.Co + 15) / 16) * w.sets * w.passes;          // of tiles
+    const int64_t blocks = w.pieces > 1 || w.sets < w.shares ? sets : (sets + kSynWaves - 1) / kSynWaves;
     if (blocks > 0x7fffffffLL / kSynWaves) return SLAYER_ERANGE;
     const dim3 grid((unsigned)blocks), block(kSynWaves * kWave);
 #define SLAYER_WGRAD_WALK(KS)                                                                                   \
