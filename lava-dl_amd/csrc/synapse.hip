@@ -17,7 +17,6 @@
 // quad is the B operand of the e-th of four matrix products, whose column j stands for step 4j + e; lane (q, j) of a
 // result then holds output channels 4q .. 4q+3 of step 4j + e, i.e. over e a quad of consecutive steps per channel.
 #include "synapse.h"
-#include "split.h"
 
 namespace slayer {
 

@@ -6,7 +6,7 @@
 // step brings the input row (`ss` rows, the stride along the walk) at the line's XP taps, each loaded and split into bfloat16
 // parts once for all KS taps along the walk, whose sums are KS sets of accumulators; an output row is stored when its last
 // row has come.  Tiles are 64 positions of the line rather than of a pixel's row, so their stores fill whole 128-byte lines
-// whatever T is, and no tile is half empty: [32,8,32,32,300] -> 16 channels 300 -> 248 us (64 steps of one pixel a tile: rows of
+// whatever T is, and no tile is half empty: [32,8,32,32,300] -> 16 channels 313 -> 247 us (64 steps of one pixel a tile: rows of
 // 300 steps end inside a line, 20 of 320 positions idle), 31x30 pixels of 301 steps 283 -> 213.
 //
 // The terms of a product are (input channel, line tap, row of the step) triples, E to a lane and group (4 E to a group): as few loads
@@ -29,8 +29,8 @@
 //
 // What bounds it: with the products left out the forward pass of [32,8,32,32,300] -> 16 channels takes as long (254 us): a group
 // of loads has to arrive before its step, and 12 waves hold 72 KB of a CU's loads in flight.  Two blocks of channels to a wave
-// (MB) halve the loads and the splitting of wide layers: [16,32,16,16,300] -> 64 channels 262 -> 232 us, its input gradient 349 ->
-// 280, though two waves stay on a SIMD instead of three.
+// (MB) halve the loads and the splitting of wide layers: [16,32,16,16,300] -> 64 channels 259 -> 220 us, its input gradient 355 ->
+// 280 (both 296 and 337 with the kernel before), though two waves stay on a SIMD instead of three.
 //
 // A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
 // each of them is not infinity times their sum: a wave with a result that is not finite computes its piece again in

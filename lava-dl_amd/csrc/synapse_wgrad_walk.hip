@@ -7,9 +7,10 @@
 // of the step) triples; a step brings one gradient row and its input rows, the gradient of the last KS rows stays in
 // registers, so a visit and step costs 1 + NPT loads for KS NPT tiles of sums.  With tiles of one pixel's steps (the form before) a
 // line was fetched by the two tiles that met in it (rows of 300 steps: 2.0 x the tensors read) and strided layers, among them
-// every transposed one, had the float32 instruction.  [32,8,32,32,300] -> 16 channels 340 -> 290 us, [16,32,16,16,300] -> 64
-// 300 -> 262, 4x4 stride 2 between [32,8,32,32,300] and 16 channels 268 -> 160; 220 layers (3x3, 5x5, strides 1 and 2, 4x4
-// transposed): 0.65 of the time before in the mean.
+// every transposed one, had the float32 instruction.  [32,8,32,32,300] -> 16 channels 338 -> 243 us between the layer's other passes
+// (400 -> 291 with the caches swept; it fetches 1.02 x the tensors now), [16,32,16,16,300] -> 64 336 -> 296, 4x4 stride 2 between
+// [32,8,32,32,300] and 16 channels 327 -> 184; 220 layers (3x3, 5x5, strides 1 and 2, 4x4 transposed): 0.64 of the time before
+// in the mean.
 //
 // Neighbouring lanes of the operand's layout lie in sixteen different rows, so a load of 1 KB would look up 64 lines: eight
 // lanes read the 128 bytes of a row together, and the split values reach the operand's layout through LDS of the wave's own.
