@@ -29,8 +29,8 @@
 //
 // What bounds it: with the products left out the forward pass of [32,8,32,32,300] -> 16 channels takes as long (254 us): a group
 // of loads has to arrive before its step, and 12 waves hold 72 KB of a CU's loads in flight.  Two blocks of channels to a wave
-// (MB) halve the loads and the splitting of wide layers: [16,32,16,16,300] -> 64 channels 259 -> 220 us, its input gradient 355 ->
-// 280 (both 296 and 337 with the kernel before), though two waves stay on a SIMD instead of three.
+// (MB) halve the loads and the splitting of wide layers: [16,32,16,16,300] -> 64 channels 259 -> 216 us, its input gradient 355 ->
+// 260 (both 296 and 337 with the kernel before), though two waves stay on a SIMD instead of three.
 //
 // A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
 // each of them is not infinity times their sum: a wave with a result that is not finite computes its piece again in
@@ -230,10 +230,11 @@ void synapse_walk_kernel(const WalkConv p) {
                 const uint4* wg = wt + g * KS * 3 * MB * kWave + lane;
                 const bool last = g + 1 == G;                            // the next loads are on their way during the products
                 if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
-                // kH steps of the quad at a time (the parts of all four do not fit beside the accumulators), and branches
-                // around the products of the lower parts only: around several copies of the whole they cost the compiler a
-                // second set of accumulators and spills.
-                constexpr int kH = KS == 5 ? 4 : 2;
+                // kH steps of the quad at a time, so that a part of the weights is read once for them: all four where two waves stay on
+                // a SIMD (gradient of [16,32,16,16,300] -> 64 channels 273 -> 260 us) or the accumulators leave room, two for
+                // three taps and one block (four: [32,8,32,32,300] 312 -> 341 us, registers).  Branches around the products of the
+                // lower parts only: around several copies of the whole they cost the compiler a second set of accumulators.
+                constexpr int kH = KS == 3 && MB == 1 ? 2 : 4;
                 const syn_f4 zero = syn_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int h = 0; h < 4; h += kH) {
