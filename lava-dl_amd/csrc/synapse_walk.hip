@@ -74,10 +74,10 @@ struct WalkConv {
     int classes;
     WalkClass cls[4];
     // weight of output channel v = co * XS + rx, line tap x, slide tap i (of cls), or -1 where the filter has none
-    __device__ __forceinline__ int weight_at(int co, int rx, int ci, int x, int i, int s0) const {
+    __device__ __forceinline__ int64_t weight_at(int co, int rx, int ci, int x, int i, int s0) const {
         const int y = s0 + i * sstep, l = l0 + x * lstep + rx * lrx;
         if ((unsigned)y >= (unsigned)nslide || (unsigned)l >= (unsigned)nline) return -1;
-        return (co * Ci + ci) * (nslide * nline) + y * wslide + l * wline;
+        return ((int64_t)co * Ci + ci) * (nslide * nline) + y * wslide + l * wline;
     }
 };
 
@@ -119,7 +119,7 @@ void synapse_walk_kernel(const WalkConv p) {
         const int l = i & (kWave - 1), mb = (i >> 6) % MB, tap = (i >> 6) / MB % KS, g = (i >> 6) / (MB * KS);
         const int vc = v0 + 16 * mb + (l & 15), co = vc / p.XS, rx = vc - co * p.XS;
         float v[8];
-        int at[8];
+        int64_t at[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (e >= E) { v[e] = 0.0f; at[e] = -1; continue; }
@@ -327,7 +327,7 @@ void synapse_walk_kernel(const WalkConv p) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int vc = v0 + 16 * mb + 4 * kk + i, co = vc / p.XS, rx = vc - co * p.XS;
-                    const int at = co < p.Co ? p.weight_at(co, rx, ci, x, tap * p.ss + sub, cls.s0) : -1;
+                    const int64_t at = co < p.Co ? p.weight_at(co, rx, ci, x, tap * p.ss + sub, cls.s0) : -1;
                     if (at < 0) continue;
                     const float w = p.weight[at];
                     d[0][i] = __fmaf_rn(w, q.x, d[0][i]);
