@@ -508,15 +508,16 @@ bool launch_synapse_plane(const SynapseConv& p, bool spread, bool streaming, hip
 
 // the taps y of a filter row that output pixels of residue r (mod stride) meet in a transposed convolution:
 // (r + pad - y * dil) divisible by stride; they are y_last, y_last - step, ... (count of them), and the source
-// coordinate of y_last for the first pixel of the class, (r + pad - y_last * dil) / stride, is `first`
+// coordinate of y_last for the first pixel of the class, (r + pad - y_last * dil) / stride, is `first`.  `step` is what
+// lies between any two of them, also for a class of one: a step beyond either end of a class is outside the filter, by
+// which the walking kernel tells the taps that a pixel does not have
 struct TapClass { int count, y_last, step, first; };
 TapClass tap_class(int r, int k, int stride, int pad, int dil) {
-    TapClass c{0, 0, 1, 0};
-    int y_first = -1;
+    int both = stride, rest = dil;                                        // their greatest common divisor
+    while (rest) { const int next = both % rest; both = rest; rest = next; }
+    TapClass c{0, 0, stride / both, 0};
     for (int y = 0; y < k; ++y) {
         if ((r + pad - y * dil) % stride != 0) continue;
-        if (c.count == 0) y_first = y;
-        else if (c.count == 1) c.step = y - y_first;
         c.y_last = y;
         ++c.count;
     }

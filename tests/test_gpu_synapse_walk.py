@@ -113,3 +113,29 @@ def test_a_value_that_is_not_finite_reaches_the_outputs_whose_taps_meet_it_and_n
         got = op(x.to(dev()), w.to(dev()), stride, padding, dilation).cpu()
         want = torch.where(reach, torch.full_like(want, value), want)
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+# (batch, Ci, H, W, T) -> Co, kernel, stride, padding, dilation: a launch per residue class, pixels together, classes of one tap
+CLASSES = [((16, 4, 16, 16, 50), 1, (5, 5), (5, 5), (0, 0), (1, 1)),         # as many taps as the stride
+           ((16, 4, 16, 16, 50), 1, (8, 8), (8, 8), (0, 0), (1, 1)),
+           ((64, 4, 16, 16, 12), 1, (7, 7), (5, 5), (0, 0), (1, 1)),         # classes of one tap and of two
+           ((64, 4, 16, 16, 12), 1, (3, 3), (2, 2), (1, 1), (2, 1)),
+           ((64, 4, 16, 16, 13), 2, (2, 2), (2, 2), (0, 0), (3, 3)),
+           ((64, 4, 16, 16, 12), 1, (5, 3), (5, 2), (0, 0), (1, 1)),
+           ((8, 16, 16, 16, 100), 2, (3, 3), (2, 2), (1, 1), (2, 1))]
+
+
+@pytest.mark.parametrize('form', CLASSES, ids=str)
+def test_a_pixel_meets_the_taps_of_its_own_class(form):
+    """Terms of at most 15 in a sum of at most 16 * 9 of them."""
+    import lava_dl_amd.slayer as slayer
+    shape, co, kernel, stride, padding, dilation = form
+    gen = torch.Generator().manual_seed(sum(shape) + co)
+    x, w = _integers(gen, shape, 3), _integers(gen, (shape[1], co) + kernel + (1,), 5)
+    cfg = (stride + (1,), padding + (0,), dilation + (1,))
+    want = F.conv_transpose3d(x, w, None, cfg[0], cfg[1], 0, 1, cfg[2])
+    got = slayer.synapse.conv_transpose_synapse(x.to(dev()), w.to(dev()), stride, padding, dilation)
+    assert torch.equal(got.cpu(), want), 'transposed convolution'
+    image = torch.zeros(want.shape, device=dev()).requires_grad_()
+    slayer.synapse.conv_synapse(image, w.to(dev()), stride, padding, dilation).backward(x.to(dev()))
+    assert torch.equal(image.grad.cpu(), want), 'input gradient'
