@@ -34,7 +34,9 @@
 //
 // A value that is not finite, or overflows when it is scaled or rounded, leaves parts of either sign, and infinity times
 // each of them is not infinity times their sum: a wave with a result that is not finite computes its piece again in
-// float32 multiplications and additions, and so does every wave of a workgroup with such a weight.
+// float32 multiplications and additions, and so does every wave of a workgroup with such a weight.  Of the input's, the sums replace
+// results that are not finite and no others: a finite one has met no such value, and the quad that shares its steps may be
+// another wave's.  A weight that is not finite is met outside the image too, and by every wave that stores these channels.
 //
 // LDS: the parts of the weights in the operand's layout, [group][tap][part][block][lane]; per triple its byte offset, its line tap
 // and row, its channel.
@@ -308,7 +310,9 @@ void synapse_walk_kernel(const WalkConv p) {
     }
     if (!float_only && !__any(!(fabsf(stored) < __builtin_inff()))) return;
 
-    // once more in float32 multiplications and additions, taps outside the image as products with zero
+    // Once more in float32 multiplications and additions, taps outside the image as products with zero, for the results that are
+    // not finite, or all of them: a wave's own stores are in place when it loads them, and of steps that another wave stores as
+    // well either one's result is what the other one would put there.
 #pragma unroll 1
     for (int sb = s_lo * MB; sb < s_hi * MB; ++sb) {
         const int s = sb / MB, mb = sb % MB;
@@ -338,8 +342,18 @@ void synapse_walk_kernel(const WalkConv p) {
             }
         }
 #pragma unroll
-        for (int b = 0; b < MB; ++b)
-            if (b == mb) store(s, b, d);
+        for (int b = 0; b < MB; ++b) {
+            if (b != mb) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float4 was = buf_load4<false>(dst, to[b][i] != kOutOfRange ? to[b][i] + s * p.out_slide : kOutOfRange);
+                d[0][i] = !float_only && fabsf(was.x) < __builtin_inff() ? was.x : d[0][i];
+                d[1][i] = !float_only && fabsf(was.y) < __builtin_inff() ? was.y : d[1][i];
+                d[2][i] = !float_only && fabsf(was.z) < __builtin_inff() ? was.z : d[2][i];
+                d[3][i] = !float_only && fabsf(was.w) < __builtin_inff() ? was.w : d[3][i];
+            }
+            store(s, b, d);
+        }
     }
 }
 

@@ -139,3 +139,22 @@ def test_a_pixel_meets_the_taps_of_its_own_class(form):
     image = torch.zeros(want.shape, device=dev()).requires_grad_()
     slayer.synapse.conv_synapse(image, w.to(dev()), stride, padding, dilation).backward(x.to(dev()))
     assert torch.equal(image.grad.cpu(), want), 'input gradient'
+
+
+@pytest.mark.parametrize('transposed', [False, True])
+@pytest.mark.parametrize('steps', [66, 67, 131])
+def test_finite_results_are_those_of_the_call_without_the_infinite_value(transposed, steps):
+    """The last two quads of a pixel share steps and may lie in two waves: 17 or 33 quads of a pixel, 16 in a wave."""
+    import lava_dl_amd.slayer as slayer
+    gen = torch.Generator().manual_seed(steps)
+    x = torch.randn(2, 3, 5, 4, steps, generator=gen)
+    w = torch.randn(*((3, 18) if transposed else (18, 3)), 3, 3, 1, generator=gen)
+    op = slayer.synapse.conv_transpose_synapse if transposed else slayer.synapse.conv_synapse
+    want = op(x.to(dev()), w.to(dev()), 1, 1, 1)
+    x[0, 1, 2, 1, 10] = float('inf')
+    x[1, 0, 0, 0, steps - 3] = float('inf')
+    got = [op(x.to(dev()), w.to(dev()), 1, 1, 1) for _ in range(2)]
+    finite = got[0].isfinite()
+    assert not finite.all() and finite.sum() > finite.numel() // 4
+    assert torch.equal(got[0][finite], want[finite])
+    assert torch.equal(got[0].nan_to_num(7.0, 8.0, 9.0), got[1].nan_to_num(7.0, 8.0, 9.0))
