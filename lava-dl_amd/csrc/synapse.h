@@ -63,6 +63,10 @@ __device__ __forceinline__ int xcd_contiguous(int b, int nb) {
 constexpr int kSynTile = 64;            // time steps per tile
 constexpr int kSynWaves = 4;            // waves per workgroup: same output channels, same image row, different tiles
 
+// How a launch of the walking kernel is cut: XS neighbouring pixels of the line share a position, their channels being the rows of a
+// product, MB blocks of 16 rows to a wave, and the rows of the image are walked in pieces.
+struct WalkCut { int XS, MB, pieces; };
+
 struct SynapseConv {
     float* out;
     const float* in;
@@ -77,6 +81,7 @@ struct SynapseConv {
     // output pixel (ho, wo) is pixel (oy0 + ho * oys, ox0 + wo * oxs) of a tensor [Co][Ho_full][Wo_full][T].
     int kh_full, kw_full, ky0, kys, kx0, kxs;
     int Ho_full, Wo_full, oy0, oys, ox0, oxs;
+    const WalkCut* want;                // the cut of the walking kernel and no other kernel, or null: what takes least
     __device__ __forceinline__ int weight_index(int ci, int iy, int ix) const {
         return (ci * kh_full + ky0 + iy * kys) * kw_full + kx0 + ix * kxs;
     }

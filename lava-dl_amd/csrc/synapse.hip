@@ -432,6 +432,7 @@ int launch_synapse_conv(SynapseConv p, bool streaming, hipStream_t st) {
     if (!filter_fits(p)) return SLAYER_ERANGE;
     int code = 0;
     if (launch_synapse_walk(p, st, &code)) return code;
+    if (p.want && p.kh > 0 && p.kw > 0) return SLAYER_ERANGE;
     // Non-temporal stores only for the classes of a transposed convolution, which leave every line they touch
     // unfinished for the next launch.  A plain convolution finishes the lines that two of its tiles share within
     // microseconds, and the L2 puts the pieces together if it is allowed to keep them.
@@ -528,12 +529,9 @@ TapClass tap_class(int r, int k, int stride, int pad, int dil) {
     return c;
 }
 
-}  // namespace
-
-extern "C" int slayer_conv_synapse(float* out, const float* in, const float* weight,
-                                   int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
-                                   int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
-                                   int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w, void* stream) {
+int conv_synapse(float* out, const float* in, const float* weight, int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
+                 int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w,
+                 const WalkCut* want, void* stream) {
     if (N < 0 || Ci < 1 || Co < 1 || H < 1 || W < 1 || T < 0 || kh < 1 || kw < 1 || stride_h < 1 || stride_w < 1 ||
         pad_h < 0 || pad_w < 0 || dil_h < 1 || dil_w < 1)
         return SLAYER_EINVAL;
@@ -556,13 +554,79 @@ extern "C" int slayer_conv_synapse(float* out, const float* in, const float* wei
     p.dh = (int)dil_h; p.dw = (int)dil_w;
     p.kh_full = p.kh; p.kw_full = p.kw; p.ky0 = p.kx0 = 0; p.kys = p.kxs = 1;
     p.Ho_full = p.Ho; p.Wo_full = p.Wo; p.oy0 = p.ox0 = 0; p.oys = p.oxs = 1;
+    p.want = want;
     const bool streaming = N * Co * Ho * Wo * T * 4 > ((int64_t)64 << 20);
     int code = 0;
-    if (launch_synapse_plane(p, false, streaming, (hipStream_t)stream, &code)) return code;
+    if (!want && launch_synapse_plane(p, false, streaming, (hipStream_t)stream, &code)) return code;
     return launch_synapse_conv(p, streaming, (hipStream_t)stream);
 }
 
-namespace {
+// The gradient of the input of slayer_conv_synapse for any stride (and, read as a layer of its own, the transposed
+// convolution): one plain convolution per residue class of the pixels of grad_in, see SynapseConv.
+int conv_synapse_input_grad(float* grad_in, const float* grad_out, const float* weight_t, int64_t N, int64_t Ci, int64_t Co, int64_t H,
+                            int64_t W, int64_t T, int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
+                            int64_t dil_h, int64_t dil_w, const WalkCut* want, bool by_class, void* stream) {
+    if (N < 0 || Ci < 1 || Co < 1 || H < 1 || W < 1 || T < 0 || kh < 1 || kw < 1 || stride_h < 1 || stride_w < 1 ||
+        pad_h < 0 || pad_w < 0 || dil_h < 1 || dil_w < 1)
+        return SLAYER_EINVAL;
+    const int64_t Ho = (H + 2 * pad_h - dil_h * (kh - 1) - 1) / stride_h + 1;
+    const int64_t Wo = (W + 2 * pad_w - dil_w * (kw - 1) - 1) / stride_w + 1;
+    if (Ho < 1 || Wo < 1) return SLAYER_EINVAL;
+    if (N == 0 || T == 0) return 0;
+    if (!grad_in || !grad_out || !weight_t) return SLAYER_ENULL;
+    if (T < 4) return SLAYER_ERANGE;
+    const int64_t K = Co * kh * kw, lim = (int64_t)1 << 31;
+    if (Ci * H * W * T * 4 >= lim || Co * Ho * Wo * T * 4 >= lim || K > 4096 || pad_h > 4096 || pad_w > 4096 ||
+        dil_h > 4096 || dil_w > 4096 || H + pad_h >= (1 << 16) || W + pad_w >= (1 << 16) || stride_h > 16 || stride_w > 16)
+        return SLAYER_ERANGE;
+    SynapseConv p;
+    p.out = grad_in; p.in = grad_out; p.weight = weight_t;
+    // in the kernels' names: the source is the gradient of the output, the result the gradient of the input
+    p.N = (int)N; p.Ci = (int)Co; p.Co = (int)Ci; p.H = (int)Ho; p.W = (int)Wo; p.T = (int)T;
+    p.sh = p.sw = 1;
+    p.kh_full = (int)kh; p.kw_full = (int)kw; p.Ho_full = (int)H; p.Wo_full = (int)W;
+    p.oys = (int)stride_h; p.oxs = (int)stride_w;
+    p.want = want;
+    const bool streaming = N * Ci * H * W * T * 4 > ((int64_t)64 << 20);
+    if (!want) {
+        SynapseConv q = p;                                                // one channel: every class in one launch
+        q.Ho = (int)H; q.Wo = (int)W; q.kh = (int)kh; q.kw = (int)kw; q.sh = (int)stride_h; q.sw = (int)stride_w;
+        q.ph = (int)pad_h; q.pw = (int)pad_w; q.dh = (int)dil_h; q.dw = (int)dil_w;
+        int code = 0;
+        if (launch_synapse_plane(q, true, streaming, (hipStream_t)stream, &code)) return code;
+    }
+    // the plain convolution of one residue class
+    auto one_class = [&](int ry, int rx) {
+        const TapClass cy = tap_class(ry, (int)kh, (int)stride_h, (int)pad_h, (int)dil_h);
+        const TapClass cx = tap_class(rx, (int)kw, (int)stride_w, (int)pad_w, (int)dil_w);
+        p.oy0 = ry; p.ox0 = rx;
+        p.Ho = ((int)H - ry + (int)stride_h - 1) / (int)stride_h;
+        p.Wo = ((int)W - rx + (int)stride_w - 1) / (int)stride_w;
+        const bool none = cy.count == 0 || cx.count == 0;                // pixels no tap reaches: zeros
+        // the taps in the order of rising source coordinate: from the last one down, a step of
+        // step * dil / stride pixels of the source each
+        p.kh = none ? 0 : cy.count; p.kw = none ? 0 : cx.count;
+        p.ky0 = cy.y_last; p.kys = -cy.step; p.kx0 = cx.y_last; p.kxs = -cx.step;
+        p.dh = cy.count > 1 ? cy.step * (int)dil_h / (int)stride_h : 1;
+        p.dw = cx.count > 1 ? cx.step * (int)dil_w / (int)stride_w : 1;
+        p.ph = -cy.first; p.pw = -cx.first;
+    };
+    const int classes_h = (int)(stride_h < H ? stride_h : H), classes_w = (int)(stride_w < W ? stride_w : W);
+    bool fits = true;
+    for (int r = 0; r < classes_h * classes_w; ++r) { one_class(r / classes_w, r % classes_w); fits = fits && filter_fits(p); }
+    if (!fits) return SLAYER_ERANGE;
+    int code = 0;
+    if (!by_class && dil_h == 1 && dil_w == 1 &&
+        launch_synapse_walk_transposed(p, (int)kh, (int)kw, (int)stride_h, (int)stride_w, (int)pad_h, (int)pad_w, (hipStream_t)stream, &code))
+        return code;
+    for (int r = 0; r < classes_h * classes_w; ++r) {
+        one_class(r / classes_w, r % classes_w);
+        code = launch_synapse_conv(p, streaming, (hipStream_t)stream);
+        if (code != 0) return code;
+    }
+    return 0;
+}
+
 
 // The tiles of sums that the workspace of a geometry holds (`tiles` per wave and pass) and the one-pixel kernel's shares of the
 // time axis.  row_kw: 3 or 5 taps along the image row without stride or dilation, tiles of 16 (channel, kernel row) pairs; that
@@ -744,68 +808,30 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     return reduce(p.items, p.passes, f.tiles, {0, 0, 1, 1, 0, 0, 0});
 }
 
-// The gradient of the input of slayer_conv_synapse for any stride (and, read as a layer of its own, the transposed
-// convolution): one plain convolution per residue class of the pixels of grad_in, see SynapseConv.
+extern "C" int slayer_conv_synapse(float* out, const float* in, const float* weight,
+                                   int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
+                                   int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
+                                   int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w, void* stream) {
+    return conv_synapse(out, in, weight, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, nullptr, stream);
+}
+
 extern "C" int slayer_conv_synapse_input_grad(float* grad_in, const float* grad_out, const float* weight_t,
                                               int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
                                               int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
                                               int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w, void* stream) {
-    if (N < 0 || Ci < 1 || Co < 1 || H < 1 || W < 1 || T < 0 || kh < 1 || kw < 1 || stride_h < 1 || stride_w < 1 ||
-        pad_h < 0 || pad_w < 0 || dil_h < 1 || dil_w < 1)
-        return SLAYER_EINVAL;
-    const int64_t Ho = (H + 2 * pad_h - dil_h * (kh - 1) - 1) / stride_h + 1;
-    const int64_t Wo = (W + 2 * pad_w - dil_w * (kw - 1) - 1) / stride_w + 1;
-    if (Ho < 1 || Wo < 1) return SLAYER_EINVAL;
-    if (N == 0 || T == 0) return 0;
-    if (!grad_in || !grad_out || !weight_t) return SLAYER_ENULL;
-    if (T < 4) return SLAYER_ERANGE;
-    const int64_t K = Co * kh * kw, lim = (int64_t)1 << 31;
-    if (Ci * H * W * T * 4 >= lim || Co * Ho * Wo * T * 4 >= lim || K > 4096 || pad_h > 4096 || pad_w > 4096 ||
-        dil_h > 4096 || dil_w > 4096 || H + pad_h >= (1 << 16) || W + pad_w >= (1 << 16) || stride_h > 16 || stride_w > 16)
-        return SLAYER_ERANGE;
-    SynapseConv p;
-    p.out = grad_in; p.in = grad_out; p.weight = weight_t;
-    // in the kernels' names: the source is the gradient of the output, the result the gradient of the input
-    p.N = (int)N; p.Ci = (int)Co; p.Co = (int)Ci; p.H = (int)Ho; p.W = (int)Wo; p.T = (int)T;
-    p.sh = p.sw = 1;
-    p.kh_full = (int)kh; p.kw_full = (int)kw; p.Ho_full = (int)H; p.Wo_full = (int)W;
-    p.oys = (int)stride_h; p.oxs = (int)stride_w;
-    const bool streaming = N * Ci * H * W * T * 4 > ((int64_t)64 << 20);
-    {
-        SynapseConv q = p;                                                // one channel: every class in one launch
-        q.Ho = (int)H; q.Wo = (int)W; q.kh = (int)kh; q.kw = (int)kw; q.sh = (int)stride_h; q.sw = (int)stride_w;
-        q.ph = (int)pad_h; q.pw = (int)pad_w; q.dh = (int)dil_h; q.dw = (int)dil_w;
-        int code = 0;
-        if (launch_synapse_plane(q, true, streaming, (hipStream_t)stream, &code)) return code;
-    }
-    // the plain convolution of one residue class
-    auto one_class = [&](int ry, int rx) {
-        const TapClass cy = tap_class(ry, (int)kh, (int)stride_h, (int)pad_h, (int)dil_h);
-        const TapClass cx = tap_class(rx, (int)kw, (int)stride_w, (int)pad_w, (int)dil_w);
-        p.oy0 = ry; p.ox0 = rx;
-        p.Ho = ((int)H - ry + (int)stride_h - 1) / (int)stride_h;
-        p.Wo = ((int)W - rx + (int)stride_w - 1) / (int)stride_w;
-        const bool none = cy.count == 0 || cx.count == 0;                // pixels no tap reaches: zeros
-        // the taps in the order of rising source coordinate: from the last one down, a step of
-        // step * dil / stride pixels of the source each
-        p.kh = none ? 0 : cy.count; p.kw = none ? 0 : cx.count;
-        p.ky0 = cy.y_last; p.kys = -cy.step; p.kx0 = cx.y_last; p.kxs = -cx.step;
-        p.dh = cy.count > 1 ? cy.step * (int)dil_h / (int)stride_h : 1;
-        p.dw = cx.count > 1 ? cx.step * (int)dil_w / (int)stride_w : 1;
-        p.ph = -cy.first; p.pw = -cx.first;
-    };
-    const int classes_h = (int)(stride_h < H ? stride_h : H), classes_w = (int)(stride_w < W ? stride_w : W);
-    bool fits = true;
-    for (int r = 0; r < classes_h * classes_w; ++r) { one_class(r / classes_w, r % classes_w); fits = fits && filter_fits(p); }
-    if (!fits) return SLAYER_ERANGE;
-    int code = 0;
-    if (dil_h == 1 && dil_w == 1 && launch_synapse_walk_transposed(p, (int)kh, (int)kw, (int)stride_h, (int)stride_w, (int)pad_h, (int)pad_w,
-                                                                   (hipStream_t)stream, &code))
-        return code;
-    for (int r = 0; r < classes_h * classes_w; ++r) {
-        one_class(r / classes_w, r % classes_w);
-        code = launch_synapse_conv(p, streaming, (hipStream_t)stream);
-        if (code != 0) return code;
-    }
-    return 0;
+    return conv_synapse_input_grad(grad_in, grad_out, weight_t, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w,
+                                   nullptr, false, stream);
+}
+
+extern "C" int slayer_conv_synapse_cut(float* out, const float* in, const float* weight,
+                                       int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
+                                       int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
+                                       int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w,
+                                       int input_grad, int by_class, int64_t pixels, int64_t blocks, int64_t pieces, void* stream) {
+    if (pixels < 1 || blocks < 1 || pieces < 1) return SLAYER_EINVAL;
+    if (pixels > 64 || blocks > 2 || pieces > 1024) return SLAYER_ERANGE;
+    const WalkCut want = {(int)pixels, (int)blocks, (int)pieces};
+    if (!input_grad) return conv_synapse(out, in, weight, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &want, stream);
+    return conv_synapse_input_grad(out, in, weight, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &want,
+                                   by_class != 0, stream);
 }

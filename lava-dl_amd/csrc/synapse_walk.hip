@@ -414,14 +414,12 @@ double walk_time(double waves, int S, int pieces, int KS, int MB, const Grouping
 
 bool beyond_cache(int64_t N, const WalkConv& w) { return N * ((int64_t)w.in_plane + w.out_plane) > 250000000; }
 
-// How a launch is cut: XS neighbouring pixels of the line share a position, Co channels of them being the rows of a product,
-// MB blocks of 16 rows to a wave, and the S rows are walked in pieces.  `step`: pixels come in whole multiples of it; taps(XS): the
-// line taps they have together; count: samples and classes; channels: of the input, times the rows a step brings.
-struct Cut { int XS, pieces, MB; };
+// The cut that takes least.  `step`: pixels come in whole multiples of it; taps(XS): the line taps they have together; count:
+// samples and classes; channels: of the input, times the rows a step brings.
 template <typename Taps>
-Cut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int channels, int step, bool together, bool large,
+WalkCut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int channels, int step, bool together, bool large,
                Taps taps) {
-    Cut best = {step, 1, 1};
+    WalkCut best = {step, 1, 1};
     double least = 1e30;
     for (int XS = step; XS == step || (together && Co * XS <= 16 && XS < width + step); XS += step) {
         const int XP = taps(XS);
@@ -435,7 +433,7 @@ Cut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int c
             for (int pieces = 1; pieces <= S && pieces <= 16; pieces *= 2) {
                 // tensors beyond the last-level cache: pieces of a line that does not lie in one piece cost more
                 const double t = walk_time(waves, S, pieces, KS, MB, g) * (large && XS > step ? 1.15 : 1.0);
-                if (t < least) { least = t; best = {XS, pieces, MB}; }
+                if (t < least) { least = t; best = {XS, MB, pieces}; }
             }
         }
     }
@@ -447,6 +445,12 @@ Cut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int c
         while (waves * best.pieces < 4608 && S >= 16 * best.pieces) best.pieces *= 2;
     }
     return best;
+}
+
+// Whether a cut that was asked for is one there is
+bool may_cut(const WalkCut& c, int step, bool together, int KS) {
+    return c.XS >= step && c.XS % step == 0 && c.XS <= 64 && (c.XS == step || together) && (c.MB == 1 || (c.MB == 2 && KS <= 3)) &&
+           c.pieces >= 1 && c.pieces <= 1024;
 }
 
 // The launch of a WalkConv whose geometry is filled in; `taps` of the walk.  false: not one that the kernel takes.
@@ -516,8 +520,10 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
     // pixels that lie together share their taps, unless these lie apart
     const auto line_taps = [&](int XS) { return (XS - 1) * l.stride + l.k; };
     const bool together = l.dil == 1 || l.k == 1;
-    const Cut cut = cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together, beyond_cache(p.N, w),
-                               [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
+    if (p.want && !may_cut(*p.want, 1, together, slide_taps(taps(s)))) return false;
+    const WalkCut cut = p.want ? *p.want
+                               : cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together,
+                                            beyond_cache(p.N, w), [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
     w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
     w.out_line *= w.XS;
     w.M = (l.out + w.XS - 1) / w.XS;
@@ -555,9 +561,11 @@ bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh
                 }
         return hi - lo + 1;
     };
-    const Cut cut = cut_launch((int64_t)p.N * (sh < H ? sh : H), p.Co, W, (p.T + 3) / 4, (H + sh - 1) / sh, slide_taps((kh + sh - 1) / sh), p.Ci, sw, true,
-                               beyond_cache(p.N, w),
-                               line_taps);
+    const int most = slide_taps((kh + sh - 1) / sh);
+    if (p.want && !may_cut(*p.want, sw, true, most)) return false;
+    const WalkCut cut = p.want ? *p.want
+                               : cut_launch((int64_t)p.N * (sh < H ? sh : H), p.Co, W, (p.T + 3) / 4, (H + sh - 1) / sh, most, p.Ci, sw, true,
+                                            beyond_cache(p.N, w), line_taps);
     w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
     w.XP = line_taps(w.XS); w.shift0 = lo; w.shift_step = 1;
     w.out_slide = sh * W * px; w.out_line = w.XS * px; w.out_rx = px;

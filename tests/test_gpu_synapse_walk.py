@@ -1,7 +1,10 @@
 """The walking kernels of the convolution synapse (csrc/synapse_walk.hip, synapse_wgrad_walk.hip) where they can go wrong: every number of taps along the
 walk, strides along either axis, pixels that share a position, two blocks of channels, rows cut into pieces, residue classes of
 a transposed convolution, and pixels whose steps are not whole quads.  The operands are small integers, so every sum is exact
-in float32 whatever its order and the results equal float64's, bit for bit."""
+in float32 whatever its order and the results equal float64's, bit for bit.
+
+The layers are small, and for such the library takes few pixels to a position, one block of channels and many pieces: the tests
+below that give the cut themselves take every layer through the others too."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -13,13 +16,13 @@ pytestmark = pytest.mark.gpu
 # (batch, Ci, H, W, T), Co, kernel, stride, padding, dilation
 FORMS = [
     ((1, 1, 1, 1, 4), 1, (1, 2), (1, 1), (0, 1), (1, 1)),
-    ((2, 3, 4, 5, 5), 2, (3, 3), (1, 1), (1, 1), (1, 1)),            # several pixels to a position, the last one alone
+    ((2, 3, 4, 5, 5), 2, (3, 3), (1, 1), (1, 1), (1, 1)),            # five pixels: with two or three to a position some are alone
     ((1, 2, 7, 9, 6), 1, (3, 3), (1, 1), (1, 1), (1, 1)),
     ((1, 8, 33, 6, 7), 8, (3, 3), (1, 1), (1, 1), (1, 1)),
     ((1, 8, 6, 33, 11), 3, (5, 5), (1, 1), (2, 2), (1, 1)),
-    ((1, 5, 6, 7, 64), 17, (3, 3), (1, 1), (0, 2), (1, 1)),          # two blocks of channels, the second of one
+    ((1, 5, 6, 7, 64), 17, (3, 3), (1, 1), (0, 2), (1, 1)),          # two blocks of channels, the second of one channel
     ((1, 32, 5, 5, 300), 64, (3, 3), (1, 1), (1, 1), (1, 1)),
-    ((300, 17, 4, 4, 9), 40, (2, 2), (1, 1), (1, 1), (1, 1)),        # enough waves for whole rows
+    ((300, 17, 4, 4, 9), 40, (2, 2), (1, 1), (1, 1), (1, 1)),        # many samples
     ((1, 4, 9, 8, 13), 6, (4, 4), (1, 1), (1, 2), (1, 1)),           # four taps
     ((2, 4, 9, 10, 10), 8, (3, 3), (2, 2), (1, 1), (1, 1)),          # rows of a step outside the image on one side
     ((2, 3, 10, 9, 50), 4, (5, 5), (2, 3), (2, 1), (1, 1)),
@@ -158,3 +161,63 @@ def test_finite_results_are_those_of_the_call_without_the_infinite_value(transpo
     assert not finite.all() and finite.sum() > finite.numel() // 4
     assert torch.equal(got[0][finite], want[finite])
     assert torch.equal(got[0].nan_to_num(7.0, 8.0, 9.0), got[1].nan_to_num(7.0, 8.0, 9.0))
+
+
+# ------------------------------------------------------------------ the cut given
+def _cut(input_grad, x, w, out_shape, stride, padding, dilation, by_class, pixels, blocks, pieces):
+    """The call with the cut given, or None where there is no such cut.  w: [Co, Ci, kh, kw], Co the channels of the result."""
+    from lava_dl_amd.slayer import _native as N
+    out = torch.full(out_shape, -12345.0, device=dev())
+    big, small = (out_shape, x.shape) if input_grad else (x.shape, out_shape)            # of the plain convolution
+    with N.device_guard(x.device):
+        code = N.lib().slayer_conv_synapse_cut(N.ptr(out), N.ptr(x), N.ptr(w), big[0], big[1], small[1], *big[2:], *w.shape[2:], *stride,
+                                               *padding, *dilation, int(input_grad), int(by_class), pixels, blocks, pieces,
+                                               N.stream_handle())
+    if code == -3:
+        return None
+    N.check(code)
+    return out
+
+
+@pytest.mark.parametrize('form', FORMS + CLASSES[3:5], ids=str)
+def test_every_cut_of_a_layer_gives_the_same(form):
+    """Terms of at most 15, a few hundred of them."""
+    shape, co, kernel, stride, padding, dilation = form
+    shape = (min(shape[0], 3),) + shape[1:]
+    gen = torch.Generator().manual_seed(sum(shape) + co + 2)
+    x, w = _integers(gen, shape, 3), _integers(gen, (co, shape[1]) + kernel, 5)
+    cfg = (stride + (1,), padding + (0,), dilation + (1,))
+    want = F.conv3d(x, w[..., None], None, *cfg)
+    up = [(shape[2 + i] - 1) * stride[i] - 2 * padding[i] + dilation[i] * (kernel[i] - 1) + 1 for i in (0, 1)]
+    cases = [(False, False, x.to(dev()), w.to(dev()), want)]
+    if min(up) >= 1:
+        want = F.conv_transpose3d(x, w.transpose(0, 1)[..., None], None, cfg[0], cfg[1], 0, 1, cfg[2])
+        cases += [(True, by_class, x.to(dev()), w.to(dev()), want) for by_class in (False, True)]
+    taken = [0, 0]
+    for input_grad, by_class, xd, wd, want in cases:
+        for pixels in (1, 2, 3, 4, 6, 8):
+            for blocks in (1, 2):
+                for pieces in (1, 2, 3, 16):
+                    got = _cut(input_grad, xd, wd, want.shape, stride, padding, dilation, by_class, pixels, blocks, pieces)
+                    assert got is None or torch.equal(got.cpu(), want), (input_grad, by_class, pixels, blocks, pieces)
+                    taken[pixels > 1] += got is not None
+    if max(kernel) < 6 and 1 in dilation:
+        assert taken[0]
+    if max(kernel) < 6 and dilation == (1, 1):
+        assert taken[1]
+
+
+@pytest.mark.parametrize('split', ['input', 'neither'])
+@pytest.mark.parametrize('blocks', [1, 2])
+@pytest.mark.parametrize('channels', [5, 12, 20, 30, 70])            # two, four, six, eight loads to a lane; more groups than one
+@pytest.mark.parametrize('taps', [1, 2, 3, 4, 5])
+def test_every_form_of_the_walking_kernel(taps, channels, blocks, split):
+    """`taps` along the walk and one along the line: as many triples as channels.  At most 5 * 70 terms of 1025 * 5: below 2^24."""
+    gen = torch.Generator().manual_seed(100 * taps + channels)
+    x, w = _integers(gen, (2, channels, 7, 3, 18), 3), _integers(gen, (40, channels, taps, 1), 5)
+    if split == 'input':
+        x = _integers(gen, x.shape, 1025)
+    want = F.conv3d(x.double(), w[..., None].double(), None, 1, (taps // 2, 0, 0))
+    got = _cut(False, x.to(dev()), w.to(dev()), want.shape, (1, 1), (taps // 2, 0), (1, 1), False, 1, blocks, 2)
+    assert (got is None) == (blocks == 2 and taps > 3)
+    assert got is None or torch.equal(got.cpu().double(), want)
