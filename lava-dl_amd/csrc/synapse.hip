@@ -416,7 +416,9 @@ using namespace slayer;
 
 namespace {
 
-// Whether a filter is one of those taken: its weights have to fit the LDS of a workgroup.
+// Whether a filter is one of those taken, by its size alone: about 860 taps, 960 to 1024 of two, three or five columns without stride
+// or dilation along the row.  The walking kernel takes 150 KB of LDS for them; the one-pixel kernel, where that does not take the
+// geometry, at most 78 KB of a workgroup's 160.
 bool filter_fits(const SynapseConv& p) {
     const int64_t pairs = (int64_t)p.Ci * p.kh, K = pairs * p.kw;
     if (p.sw == 1 && p.dw == 1 && (p.kw == 2 || p.kw == 3 || p.kw == 5) && p.Wo >= 4)

@@ -501,43 +501,46 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
     const Axis v = {p.W, p.Wo, p.kw, p.sw, p.pw, p.dw, p.kx0, p.kxs, p.kw_full, p.ox0, p.oxs, p.Wo_full, 1};
     auto taps = [](const Axis& a) { return a.k == 1 || a.dil == 1 ? (a.k + a.stride - 1) / a.stride : 0; };
     auto takes = [&](const Axis& a, const Axis& line) { return taps(a) >= 1 && taps(a) <= 5 && line.k <= kMaxLineTaps && a.stride <= 16; };
-    // along the rows of the image, so that the line is one piece of memory, unless the filter has more taps the other way
-    const bool down = takes(h, v), right = takes(v, h);
+    // along the rows of the image, so that the line is one piece of memory, unless the filter has more taps the other way; along
+    // the other axis where the weights do not fit LDS this way (9x2, stride 8 along the rows, 56 channels: 183 KB and 98)
+    const bool down = takes(h, v), right = takes(v, h), rows_first = down && (!right || taps(h) >= taps(v));
     if (!down && !right) return false;
-    const bool use_h = down && (!right || taps(h) >= taps(v));
-    const Axis& s = use_h ? h : v;
-    const Axis& l = use_h ? v : h;
-    const int px = p.T * 4;
-    WalkConv w;
-    w.out = p.out; w.in = p.in; w.weight = p.weight;
-    w.N = p.N; w.Ci = p.Ci; w.Co = p.Co; w.T = p.T;
-    w.in_ch = p.H * p.W * px; w.in_plane = p.Ci * w.in_ch;
-    w.out_ch = p.Ho_full * p.Wo_full * px; w.out_plane = p.Co * w.out_ch;
-    w.in_slide = use_h ? p.W * px : px; w.in_line = use_h ? px : p.W * px;
-    w.out_slide = s.ostep * (use_h ? p.Wo_full * px : px); w.out_line = l.ostep * (use_h ? px : p.Wo_full * px);
-    w.out_rx = w.out_line;
-    w.Hs = s.in; w.Ws = l.in;
-    // pixels that lie together share their taps, unless these lie apart
-    const auto line_taps = [&](int XS) { return (XS - 1) * l.stride + l.k; };
-    const bool together = l.dil == 1 || l.k == 1;
-    if (p.want && !may_cut(*p.want, 1, together, slide_taps(taps(s)))) return false;
-    const WalkCut cut = p.want ? *p.want
-                               : cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together,
-                                            beyond_cache(p.N, w), [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
-    w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
-    w.out_line *= w.XS;
-    w.M = (l.out + w.XS - 1) / w.XS;
-    w.ss = s.stride; w.ls = l.stride * w.XS;
-    w.XP = w.XS > 1 ? line_taps(w.XS) : l.k; w.shift0 = -l.pad; w.shift_step = w.XS > 1 ? 1 : l.dil;
-    w.line_full = l.out;
-    w.wslide = s.wstride; w.wline = l.wstride; w.nslide = s.kfull; w.nline = l.kfull;
-    w.sstep = s.kstep; w.l0 = l.k0; w.lstep = l.kstep; w.lrx = -l.stride * l.kstep;
-    w.classes = 1;
-    WalkClass& c = w.cls[0];
-    c.s0 = s.k0; c.row0 = -s.pad; c.S = s.out;
-    c.out0 = (p.oy0 * p.Wo_full + p.ox0) * px;
-    steps_inside(c, w.ss, w.Hs);
-    return launch(w, taps(s), st, code);
+    const auto along = [&](bool use_h) {
+        const Axis& s = use_h ? h : v;
+        const Axis& l = use_h ? v : h;
+        const int px = p.T * 4;
+        WalkConv w;
+        w.out = p.out; w.in = p.in; w.weight = p.weight;
+        w.N = p.N; w.Ci = p.Ci; w.Co = p.Co; w.T = p.T;
+        w.in_ch = p.H * p.W * px; w.in_plane = p.Ci * w.in_ch;
+        w.out_ch = p.Ho_full * p.Wo_full * px; w.out_plane = p.Co * w.out_ch;
+        w.in_slide = use_h ? p.W * px : px; w.in_line = use_h ? px : p.W * px;
+        w.out_slide = s.ostep * (use_h ? p.Wo_full * px : px); w.out_line = l.ostep * (use_h ? px : p.Wo_full * px);
+        w.out_rx = w.out_line;
+        w.Hs = s.in; w.Ws = l.in;
+        // pixels that lie together share their taps, unless these lie apart
+        const auto line_taps = [&](int XS) { return (XS - 1) * l.stride + l.k; };
+        const bool together = l.dil == 1 || l.k == 1;
+        if (p.want && !may_cut(*p.want, 1, together, slide_taps(taps(s)))) return false;
+        const WalkCut cut = p.want ? *p.want
+                                   : cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together,
+                                                beyond_cache(p.N, w), [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
+        w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
+        w.out_line *= w.XS;
+        w.M = (l.out + w.XS - 1) / w.XS;
+        w.ss = s.stride; w.ls = l.stride * w.XS;
+        w.XP = w.XS > 1 ? line_taps(w.XS) : l.k; w.shift0 = -l.pad; w.shift_step = w.XS > 1 ? 1 : l.dil;
+        w.line_full = l.out;
+        w.wslide = s.wstride; w.wline = l.wstride; w.nslide = s.kfull; w.nline = l.kfull;
+        w.sstep = s.kstep; w.l0 = l.k0; w.lstep = l.kstep; w.lrx = -l.stride * l.kstep;
+        w.classes = 1;
+        WalkClass& c = w.cls[0];
+        c.s0 = s.k0; c.row0 = -s.pad; c.S = s.out;
+        c.out0 = (p.oy0 * p.Wo_full + p.ox0) * px;
+        steps_inside(c, w.ss, w.Hs);
+        return launch(w, taps(s), st, code);
+    };
+    return along(rows_first) || (down && right && along(!rows_first));
 }
 
 bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh, int sw, int ph, int pw, hipStream_t st, int* code) {

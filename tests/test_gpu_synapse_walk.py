@@ -219,5 +219,19 @@ def test_every_form_of_the_walking_kernel(taps, channels, blocks, split):
         x = _integers(gen, x.shape, 1025)
     want = F.conv3d(x.double(), w[..., None].double(), None, 1, (taps // 2, 0, 0))
     got = _cut(False, x.to(dev()), w.to(dev()), want.shape, (1, 1), (taps // 2, 0), (1, 1), False, 1, blocks, 2)
-    assert (got is None) == (blocks == 2 and taps > 3)
-    assert got is None or torch.equal(got.cpu().double(), want)
+    assert got is not None and torch.equal(got.cpu().double(), want)    # five taps and two blocks: walked along the other axis
+
+
+@pytest.mark.parametrize('form', [((2, 56, 16, 9, 9), 16, (9, 2), (8, 1), (0, 0), (1, 1)),      # weights beyond LDS along the rows
+                                  ((2, 16, 45, 8, 9), 8, (32, 2), (1, 1), (0, 0), (1, 1)),      # 1024 taps on the one-pixel kernel
+                                  ((2, 12, 45, 8, 9), 8, (16, 5), (1, 1), (0, 0), (1, 1))], ids=str)
+def test_filters_of_the_most_taps(form):
+    import lava_dl_amd.slayer as slayer
+    shape, co, kernel, stride, padding, dilation = form
+    gen = torch.Generator().manual_seed(shape[1])
+    x, w = _integers(gen, shape, 3), _integers(gen, (co, shape[1]) + kernel, 5)
+    want = F.conv3d(x, w[..., None], None, stride + (1,), padding + (0,), dilation + (1,))
+    assert torch.equal(slayer.synapse.layer._launch(x.to(dev()), w.to(dev()), stride, padding, dilation).cpu(), want)
+    if stride == (8, 1):
+        got = _cut(False, x.to(dev()), w.to(dev()), want.shape, stride, padding, dilation, False, 1, 1, 4)
+        assert got is not None and torch.equal(got.cpu(), want)
