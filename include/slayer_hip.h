@@ -353,13 +353,13 @@ int slayer_conv_synapse_input_grad(float *grad_in, const float *grad_out, const 
 /* Either of the two above (input_grad: the second, by_class: a launch per residue class where one would do) on the kernel that
  * walks the rows, cut as told instead of as is estimated to take least: `pixels` neighbouring pixels of the line share a position
  * (a multiple of the stride in a launch for all classes), `blocks` (1 or 2) blocks of 16 rows of the product to a wave, the rows of
- * the image walked in `pieces`.  The results differ in the order of their sums.  What it is for: tests, and measuring what the
+ * the image walked in `pieces`; whole: every row of the result by itself, from all the rows it meets.  The results differ in the order of their sums.  What it is for: tests, and measuring what the
  * choice costs.  SLAYER_ERANGE where that kernel does not take the layer or the cut is not one it has. */
 int slayer_conv_synapse_cut(float *out, const float *in, const float *weight,
                             int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
                             int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
                             int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w,
-                            int input_grad, int by_class, int64_t pixels, int64_t blocks, int64_t pieces, void *stream);
+                            int input_grad, int by_class, int64_t pixels, int64_t blocks, int64_t pieces, int whole, void *stream);
 
 /* The gradient of the synapse's weights (what autograd obtains from conv3d's backward, synapse/layer.py:297-323):
  * grad_weight[co][ci][y][x] = sum over n, ho, wo, t of grad_out[n][co][ho][wo][t] *

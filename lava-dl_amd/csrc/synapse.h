@@ -60,12 +60,28 @@ __device__ __forceinline__ int xcd_contiguous(int b, int nb) {
     return x * q + (x < r ? x : r) + slot;
 }
 
+// Division of a number below 2^31 by one that the host knows, as a multiplication (a division of integers is some thirty
+// instructions, a chain of them in front of a kernel's first load): with 2^shift >= d, n / d = (n + n mul / 2^32) / 2^shift for
+// mul = 2^32 (2^shift - d) / d + 1, rounded down.
+struct Divisor {
+    unsigned d, mul;
+    int shift;
+    Divisor() = default;
+    Divisor(int by) : d((unsigned)by), shift(0) {
+        while ((1ull << shift) < d) ++shift;
+        mul = (unsigned)((1ull << 32) * ((1ull << shift) - d) / d + 1);
+    }
+    __device__ __forceinline__ int of(int n) const { return (int)((__umulhi((unsigned)n, mul) + (unsigned)n) >> shift); }
+    __device__ __forceinline__ int rest(int n) const { return n - of(n) * (int)d; }
+};
+
 constexpr int kSynTile = 64;            // time steps per tile
 constexpr int kSynWaves = 4;            // waves per workgroup: same output channels, same image row, different tiles
 
 // How a launch of the walking kernel is cut: XS neighbouring pixels of the line share a position, their channels being the rows of a
-// product, MB blocks of 16 rows to a wave, and the rows of the image are walked in pieces.
-struct WalkCut { int XS, MB, pieces; };
+// product, MB blocks of 16 rows to a wave, and the rows of the image are walked in pieces.  whole: a step brings all the input rows that
+// its output row meets, as terms of one product, instead of `stride` rows that several output rows meet.
+struct WalkCut { int XS, MB, pieces; bool whole; };
 
 struct SynapseConv {
     float* out;

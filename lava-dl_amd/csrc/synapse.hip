@@ -829,10 +829,11 @@ extern "C" int slayer_conv_synapse_cut(float* out, const float* in, const float*
                                        int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
                                        int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
                                        int64_t pad_h, int64_t pad_w, int64_t dil_h, int64_t dil_w,
-                                       int input_grad, int by_class, int64_t pixels, int64_t blocks, int64_t pieces, void* stream) {
+                                       int input_grad, int by_class, int64_t pixels, int64_t blocks, int64_t pieces, int whole,
+                                       void* stream) {
     if (pixels < 1 || blocks < 1 || pieces < 1) return SLAYER_EINVAL;
     if (pixels > 64 || blocks > 2 || pieces > 1024) return SLAYER_ERANGE;
-    const WalkCut want = {(int)pixels, (int)blocks, (int)pieces};
+    const WalkCut want = {(int)pixels, (int)blocks, (int)pieces, whole != 0};
     if (!input_grad) return conv_synapse(out, in, weight, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &want, stream);
     return conv_synapse_input_grad(out, in, weight, N, Ci, Co, H, W, T, kh, kw, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w, &want,
                                    by_class != 0, stream);

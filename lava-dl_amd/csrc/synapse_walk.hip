@@ -39,7 +39,8 @@
 // another wave's.  A weight that is not finite is met outside the image too, and by every wave that stores these channels.
 //
 // LDS: the parts of the weights in the operand's layout, [group][tap][part][block][lane]; per triple its byte offset, its line tap
-// and row, its channel.
+// and row, its channel; what the waves' weights are; where lanes store that have no registers for it.
+#include <cmath>
 #include "synapse.h"
 #include "split.h"
 
@@ -51,7 +52,7 @@ constexpr int kWalkQuads = 16;          // quads of steps to a tile
 struct WalkClass {
     int s0;                             // weights: slide tap i of the launch is row s0 + i * WalkConv::sstep of the filter
     int row0;                           // input row of step 0's first row
-    int S;                              // output rows
+    int S, per;                         // output rows, of a piece
     int c_lo, c_hi;                     // the steps that meet a row inside the image
     int out0;                           // bytes to the first output row
 };
@@ -66,6 +67,7 @@ struct WalkConv {
     int Hs, Ws;                         // input rows along the walk, pixels along the line
     int M, quads, line_quads;           // pixels along the line; quads of steps a pixel has, the line has
     int ss, ls;                         // strides along walk and line
+    int rows;                           // input rows of a step: ss, or all that an output row meets (KS = 1)
     int XP, shift0, shift_step;         // line taps, the first one's shift, pixels from one to the next
     int XS, line_full;                  // outputs that share a line position, pixels of the output's line
     int pairs, groups;
@@ -74,6 +76,9 @@ struct WalkConv {
     int tiles, pieces, items, blocks;   // per sample, class and channel block; blocks of 16 MB channels
     int MB;
     int classes;
+    int waves;                          // of a workgroup
+    Divisor by_cb, by_blocks, by_wgs, by_tiles, by_quads, by_XS, by_triples, by_rows;   // blocks * classes, blocks, workgroups of items,
+                                                                                          // tiles, quads, XS, XP * rows, rows
     WalkClass cls[4];
     // weight of output channel v = co * XS + rx, line tap x, slide tap i (of cls), or -1 where the filter has none
     __device__ __forceinline__ int64_t weight_at(int co, int rx, int ci, int x, int i, int s0) const {
@@ -82,6 +87,10 @@ struct WalkConv {
         return ((int64_t)co * Ci + ci) * (nslide * nline) + y * wslide + l * wline;
     }
 };
+
+// Whether a lane keeps in registers where it stores: three taps and eight loads leave none, and a register that comes back from
+// memory waits for the loads of the next step (three channels of two pixels, [11,32,27,27,248] -> 2 channels 70 -> 81 us), so LDS has it
+constexpr bool walk_keeps(int KS, int E, int MB) { return KS != 3 || E < 8 || MB > 1; }
 
 // KS: taps along the walk; E: triples to a lane and group; MB: blocks of 16 rows of the product to a wave.  Three waves per SIMD where
 // 168 registers do, else two.
@@ -94,39 +103,83 @@ void synapse_walk_kernel(const WalkConv p) {
     int* pair_off = reinterpret_cast<int*>(wt + G * KS * 3 * MB * kWave);     // [G][4][E] bytes
     int* pair_info = pair_off + G * 4 * E;              // line tap, row of the step << 8
     int* pair_ch = pair_info + G * 4 * E;               // input channel
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), threads = blockDim.x, waves = threads / kWave;
+    int* flags = pair_ch + G * 4 * E;                   // [8]: what a wave's weights are
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), waves = p.waves, threads = waves * kWave;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     int b = xcd_contiguous(blockIdx.x, gridDim.x);
-    const int cb = b % (p.blocks * p.classes); b /= p.blocks * p.classes;
-    const int v0 = (cb % p.blocks) * 16 * MB;
-    const WalkClass cls = p.cls[cb / p.blocks];
-    const int groups = (p.items + waves - 1) / waves;
-    const int ig = b % groups;
-    const int n = b / groups;
+    const int rest = p.by_cb.of(b), cb = b - rest * p.blocks * p.classes, which = p.by_blocks.of(cb);
+    const int v0 = (cb - which * p.blocks) * 16 * MB;
+    const WalkClass cls = p.cls[which];
+    const int n = p.by_wgs.of(rest), ig = p.by_wgs.rest(rest);
     const int kk = lane >> 4, j = lane & 15;
 
+    const int item = ig * waves + wave;
+    const int piece = p.by_tiles.of(item), tile = item - piece * p.tiles;
+    const int s_lo = piece * cls.per, s_hi = (s_lo + cls.per) < cls.S ? (s_lo + cls.per) : cls.S;
+    const bool idle = item >= p.items || s_lo >= s_hi;
+
+    // the lane's quad: pixel m of the line, steps t .. t + 3
+    const int quad = tile * kWalkQuads + j;
+    const bool on = quad < p.line_quads;
+    const int m = on ? p.by_quads.of(quad) : 0;
+    // where a pixel's steps are not whole quads its last quad is the last four steps: those that it shares with the one before
+    // are computed, and stored, twice
+    int t = 4 * (quad - m * p.quads);
+    t = t < p.T - 4 ? t : p.T - 4;
+    unsigned taps = 0u;                                 // line taps inside the image
+    for (int x = 0; x < p.XP; ++x)
+        taps |= (on && (unsigned)(m * p.ls + p.shift0 + x * p.shift_step) < (unsigned)p.Ws) ? 1u << x : 0u;
+    const bool inner = __all(taps == (1u << p.XP) - 1u);   // no lane has a tap outside
+    const int lane_in = m * p.ls * p.in_line + t * 4;
+    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * (p.in_plane / 4), (unsigned)p.in_plane);
+    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * (p.out_plane / 4), (unsigned)p.out_plane);
+    // step c brings rows c * ss + row0 .. + rows - 1: slide tap i of output row c - i
+    const int c_end = s_hi + KS - 1;
+    const int c_lo = s_lo > cls.c_lo ? s_lo : cls.c_lo;
+    const int c_hi = c_end < cls.c_hi ? c_end : cls.c_hi;
+    float4 raw[E];
+    auto fetch = [&](int c, int g) {
+        const int* off = pair_off + (4 * g + kk) * E;
+        const int row = c * p.ss + cls.row0;
+        const int at = lane_in + row * p.in_slide;
+        int o[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] = off[e] + at;
+        if (!inner || row < 0 || row + p.rows > p.Hs) {
+            const int* info = pair_info + (4 * g + kk) * E;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int what = info[e];
+                const bool in = (taps >> (what & 31) & 1u) != 0u && (unsigned)(row + (what >> 8)) < (unsigned)p.Hs;
+                o[e] = in ? o[e] : kOutOfRange;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) raw[e] = buf_load4<false>(src, o[e]);
+    };
     for (int i = tid; i < G * 4 * E; i += threads) {
         const int e = i % E, q = (i / E) & 3, g = i / (4 * E);
         const int pr = 4 * E * g + 4 * e + q;
-        const int ci = pr / (p.XP * p.ss), r = pr - ci * (p.XP * p.ss), x = r / p.ss, row = r - x * p.ss;
+        const int ci = p.by_triples.of(pr), r = pr - ci * (p.XP * p.rows), x = p.by_rows.of(r), row = r - x * p.rows;
         const bool is = pr < p.pairs;
         pair_off[i] = is ? ci * p.in_ch + (p.shift0 + x * p.shift_step) * p.in_line + row * p.in_slide : kOutOfRange;
         pair_info[i] = is ? x | row << 8 : 31;          // tap 31 is outside in every lane
         pair_ch[i] = is ? ci : -1;
     }
     __syncthreads();
+    if (!idle && c_lo < c_hi) fetch(c_lo, 0);           // on its way while the weights are set up
     unsigned low = 0u;
     bool odd = false;                                   // a weight that is not finite
     for (int i = tid; i < G * KS * MB * kWave; i += threads) {
         const int l = i & (kWave - 1), mb = (i >> 6) % MB, tap = (i >> 6) / MB % KS, g = (i >> 6) / (MB * KS);
-        const int vc = v0 + 16 * mb + (l & 15), co = vc / p.XS, rx = vc - co * p.XS;
+        const int vc = v0 + 16 * mb + (l & 15), co = p.by_XS.of(vc), rx = vc - co * p.XS;
         float v[8];
         int64_t at[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (e >= E) { v[e] = 0.0f; at[e] = -1; continue; }
             const int pr = (4 * g + (l >> 4)) * E + e, ci = pair_ch[pr], what = pair_info[pr];
-            at[e] = ci >= 0 && co < p.Co ? p.weight_at(co, rx, ci, what & 31, tap * p.ss + (what >> 8), cls.s0) : -1;
+            at[e] = ci >= 0 && co < p.Co ? p.weight_at(co, rx, ci, what & 31, tap * p.rows + (what >> 8), cls.s0) : -1;
             v[e] = p.weight[at[e] < 0 ? 0 : at[e]];
         }
 #pragma unroll
@@ -141,72 +194,41 @@ void synapse_walk_kernel(const WalkConv p) {
         to[MB * kWave] = round_eight(v);
         to[2 * MB * kWave] = bf16_eight(v);
     }
-    const bool split_w = __syncthreads_or((low & 0xffffu) != 0u);
-    const bool float_only = __syncthreads_or(odd);
-    const int item = ig * waves + wave;
-    if (item >= p.items) return;
-    const int tile = item % p.tiles, piece = item / p.tiles;
-    const int per = (cls.S + p.pieces - 1) / p.pieces;
-    const int s_lo = piece * per, s_hi = (s_lo + per) < cls.S ? (s_lo + per) : cls.S;
-    if (s_lo >= s_hi) return;
-
-    // the lane's quad: pixel m of the line, steps t .. t + 3
-    const int quad = tile * kWalkQuads + j;
-    const bool on = quad < p.line_quads;
-    const int m = on ? quad / p.quads : 0;
-    // where a pixel's steps are not whole quads its last quad is the last four steps: those that it shares with the one before
-    // are computed, and stored, twice
-    int t = 4 * (quad - m * p.quads);
-    t = t < p.T - 4 ? t : p.T - 4;
-    unsigned taps = 0u;                                 // line taps inside the image
-    for (int x = 0; x < p.XP; ++x)
-        taps |= (on && (unsigned)(m * p.ls + p.shift0 + x * p.shift_step) < (unsigned)p.Ws) ? 1u << x : 0u;
-    const bool inner = __all(taps == (1u << p.XP) - 1u);   // no lane has a tap outside
-    const int lane_in = m * p.ls * p.in_line + t * 4;
-    const __amdgpu_buffer_rsrc_t src = make_rsrc(p.in + (int64_t)n * (p.in_plane / 4), (unsigned)p.in_plane);
-    const __amdgpu_buffer_rsrc_t dst = make_rsrc(p.out + (int64_t)n * (p.out_plane / 4), (unsigned)p.out_plane);
+    // bit 0: a weight has lower parts, bit 1: one is not finite
+    const int mine = (__any((low & 0xffffu) != 0u) ? 1 : 0) | (__any(odd) ? 2 : 0);
+    if (lane == 0) flags[wave] = mine;
+    __syncthreads();
+    if (idle) return;
+    const int seen = lane < waves ? flags[lane] : 0;
+    const bool split_w = __any((seen & 1) != 0), float_only = __any((seen & 2) != 0);
     int to[MB][4];                                      // where the lane's four channels go, row 0
 #pragma unroll
     for (int i = 0; i < 4 * MB; ++i) {
-        const int vc = v0 + 16 * (i >> 2) + 4 * kk + (i & 3), co = vc / p.XS, rx = vc - co * p.XS;
+        const int vc = v0 + 16 * (i >> 2) + 4 * kk + (i & 3), co = p.by_XS.of(vc), rx = vc - co * p.XS;
         to[i >> 2][i & 3] = (on && co < p.Co && m * p.XS + rx < p.line_full)
                                 ? co * p.out_ch + rx * p.out_rx + m * p.out_line + t * 4 + cls.out0 : kOutOfRange;
     }
-
-    // step c brings rows c * ss + row0 .. + ss - 1: slide tap i of output row c - i
-    const int c_end = s_hi + KS - 1;
-    const int c_lo = s_lo > cls.c_lo ? s_lo : cls.c_lo;
-    const int c_hi = c_end < cls.c_hi ? c_end : cls.c_hi;
-    float4 raw[E];
-    auto fetch = [&](int c, int g) {
-        const int* off = pair_off + (4 * g + kk) * E;
-        const int row = c * p.ss + cls.row0;
-        const int at = lane_in + row * p.in_slide;
-        int o[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = off[e] + at;
-        if (!inner || row < 0 || row + p.ss > p.Hs) {
-            const int* info = pair_info + (4 * g + kk) * E;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int what = info[e];
-                const bool in = (taps >> (what & 31) & 1u) != 0u && (unsigned)(row + (what >> 8)) < (unsigned)p.Hs;
-                o[e] = in ? o[e] : kOutOfRange;
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) raw[e] = buf_load4<false>(src, o[e]);
+    constexpr bool kKept = walk_keeps(KS, E, MB);
+    int4* kept = reinterpret_cast<int4*>(flags + 8) + wave * kWave + lane;
+    if (!kKept) {
+        *kept = make_int4(to[0][0], to[0][1], to[0][2], to[0][3]);
+        asm volatile("" ::: "memory");
+    }
+    auto place = [&](int mb, int (&at)[4]) {
+        at[0] = to[mb][0]; at[1] = to[mb][1]; at[2] = to[mb][2]; at[3] = to[mb][3];
+        if (!kKept) { const int4 k = *kept; at[0] = k.x; at[1] = k.y; at[2] = k.z; at[3] = k.w; }
     };
     // lane (kk, j): output channels v0 + 16 mb + 4 kk + i, steps t .. t + 3
     auto store = [&](int s, int mb, const syn_f4 (&d)[4]) {
+        int at[4];
+        place(mb, at);
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            buf_store4<false>(dst, to[mb][i] != kOutOfRange ? to[mb][i] + s * p.out_slide : kOutOfRange,
+            buf_store4<false>(dst, at[i] != kOutOfRange ? at[i] + s * p.out_slide : kOutOfRange,
                               make_float4(d[0][i], d[1][i], d[2][i], d[3][i]));
     };
     float stored = 0.f;                                                  // not finite once a result is not
     syn_f4 acc[MB][KS][4];
-    if (c_lo < c_hi) fetch(c_lo, 0);
 #pragma unroll
     for (int b = 0; b < MB; ++b)
 #pragma unroll
@@ -229,7 +251,9 @@ void synapse_walk_kernel(const WalkConv p) {
                     bits |= __float_as_uint(r.x) | __float_as_uint(r.y) | __float_as_uint(r.z) | __float_as_uint(r.w);
                 }
                 const bool split_x = __any((bits & 0xffffu) != 0u);
-                const uint4* wg = wt + g * KS * 3 * MB * kWave + lane;
+                int here = lane;
+                if (!walk_keeps(KS, E, MB)) asm("" : "+v"(here));        // the address is worked out here, not kept
+                const uint4* wg = wt + g * KS * 3 * MB * kWave + here;
                 const bool last = g + 1 == G;                            // the next loads are on their way during the products
                 if (!last || c + 1 < c_hi) fetch(last ? c + 1 : c, last ? 0 : g + 1);
                 // kH steps of the quad at a time, so that a part of the weights is read once for them: all four where two waves stay on
@@ -313,6 +337,8 @@ void synapse_walk_kernel(const WalkConv p) {
     // Once more in float32 multiplications and additions, taps outside the image as products with zero, for the results that are
     // not finite, or all of them: a wave's own stores are in place when it loads them, and of steps that another wave stores as
     // well either one's result is what the other one would put there.
+    int kq = kk;                                         // (nothing of this loop is kept in registers during the one before)
+    asm("" : "+v"(kq));
 #pragma unroll 1
     for (int sb = s_lo * MB; sb < s_hi * MB; ++sb) {
         const int s = sb / MB, mb = sb % MB;
@@ -321,7 +347,7 @@ void synapse_walk_kernel(const WalkConv p) {
         for (int e = 0; e < 4; ++e) d[e] = syn_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
         for (int pr = 0; pr < p.pairs; ++pr) {
-            const int ci = pr / (p.XP * p.ss), r = pr - ci * (p.XP * p.ss), x = r / p.ss, sub = r - x * p.ss;
+            const int ci = p.by_triples.of(pr), r = pr - ci * (p.XP * p.rows), x = p.by_rows.of(r), sub = r - x * p.rows;
             const int off = ci * p.in_ch + (p.shift0 + x * p.shift_step) * p.in_line + lane_in;
 #pragma unroll 1
             for (int tap = 0; tap < KS; ++tap) {
@@ -330,8 +356,8 @@ void synapse_walk_kernel(const WalkConv p) {
                 const float4 q = buf_load4<false>(src, in ? off + row * p.in_slide : kOutOfRange);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int vc = v0 + 16 * mb + 4 * kk + i, co = vc / p.XS, rx = vc - co * p.XS;
-                    const int64_t at = co < p.Co ? p.weight_at(co, rx, ci, x, tap * p.ss + sub, cls.s0) : -1;
+                    const int vc = v0 + 16 * mb + 4 * kq + i, co = p.by_XS.of(vc), rx = vc - co * p.XS;
+                    const int64_t at = co < p.Co ? p.weight_at(co, rx, ci, x, tap * p.rows + sub, cls.s0) : -1;
                     if (at < 0) continue;
                     const float w = p.weight[at];
                     d[0][i] = __fmaf_rn(w, q.x, d[0][i]);
@@ -344,9 +370,11 @@ void synapse_walk_kernel(const WalkConv p) {
 #pragma unroll
         for (int b = 0; b < MB; ++b) {
             if (b != mb) continue;
+            int at[4];
+            place(b, at);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float4 was = buf_load4<false>(dst, to[b][i] != kOutOfRange ? to[b][i] + s * p.out_slide : kOutOfRange);
+                const float4 was = buf_load4<false>(dst, at[i] != kOutOfRange ? at[i] + s * p.out_slide : kOutOfRange);
                 d[0][i] = !float_only && fabsf(was.x) < __builtin_inff() ? was.x : d[0][i];
                 d[1][i] = !float_only && fabsf(was.y) < __builtin_inff() ? was.y : d[1][i];
                 d[2][i] = !float_only && fabsf(was.z) < __builtin_inff() ? was.z : d[2][i];
@@ -386,16 +414,19 @@ Grouping grouping(int pairs) {
     return best;
 }
 
-size_t walk_lds(const Grouping& g, int KS, int MB) { return (size_t)g.groups * (KS * 3 * 1024 * MB + 4 * g.E * 3 * sizeof(int)); }
+// of a workgroup of four waves
+size_t walk_lds(const Grouping& g, int KS, int MB) {
+    return (size_t)g.groups * (KS * 3 * 1024 * MB + 4 * g.E * 3 * sizeof(int)) + 8 * sizeof(int) +
+           (walk_keeps(KS, g.E, MB) ? 0 : 4 * kWave * sizeof(int4));
+}
 // Workgroups of four waves: the registers hold three of them on a CU (two with five taps or two blocks of channels), but one of eight.
 // Eight where the LDS has room for one workgroup only and there are more than four waves to a CU.
 int walk_waves(size_t lds, double waves) { return 2 * lds > 160 * 1024 && waves > 4 * 256 ? 8 : 4; }
 
-// What a launch takes, in us: a workgroup sets up its weights; a wave walks its piece of S rows, KS - 1 steps more than it
-// has rows; a group of loads is a wait or, where a SIMD has several waves, its share of the instructions; of what the last,
-// partly filled round of workgroups leaves idle, 0.44 is lost.  Fitted to 814 layers (3x3 and 5x5, strides 1 and 2, 4x4
-// transposed and its gradient, 2 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 50 to 350 steps), each cut in all the
-// ways below: what it decides for takes 1.02 times the least of them, in the mean.
+// What a launch of the walking form takes, in us: a workgroup sets up its weights; a wave walks its piece of S rows, KS - 1 steps more
+// than it has rows; a group of loads is a wait or, where a SIMD has several waves, its share of the instructions; of what the last,
+// partly filled round of workgroups leaves idle, 0.44 is lost.  Fitted to 814 layers (3x3 and 5x5, strides 1 and 2, 4x4 transposed
+// and its gradient, 2 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 50 to 350 steps), each cut in all the ways below.
 double walk_time(double waves, int S, int pieces, int KS, int MB, const Grouping& g) {
     const size_t lds = walk_lds(g, KS, MB);
     const double load = waves * pieces / 1024;                            // waves per SIMD
@@ -412,34 +443,68 @@ double walk_time(double waves, int S, int pieces, int KS, int MB, const Grouping
     return 0.56 * load / slots * round(slots) + 0.44 * (full * round(slots) + (left > 0.02 ? round(left) : 0.0));
 }
 
+// What a short launch of either form takes: also the start of a wave, the products, and that compute units with fewer workgroups than
+// others wait for these with 0.34 to 0.57 of what they have less.  Fitted to 3408 passes (forward and input gradient of 860
+// layers: 1x1 to 5x5, strides 1 and 2, transposed, 1 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 20 to 350 steps, spikes x
+// 8-bit and real x real), each cut in all the ways below.  What it decides for below kShort takes 0.87 times what walk_time decides
+// for, in the mean (2.3 % of these passes: more than 1.03 times).  Above, the two differ by less than what either misses, and
+// walk_time stays (0.90 in the mean between 20 and 60 us, but up to 1.39 times, 0.95 and up to 1.35 times beyond), unless
+// the `whole` form is estimated at less than 0.85 of it.
+constexpr double kShort = 20.0;
+double short_walk_time(double waves, int steps, int KS, int MB, const Grouping& g) {
+    const size_t lds = walk_lds(g, KS, MB);
+    const double unit = walk_waves(lds, waves) / 4, load = waves / 1024;                  // waves per SIMD: of a workgroup, of all
+    const double room = (double)(160 * 1024 / lds) * unit;
+    const int held = KS == 1 && MB == 1 && g.E <= 4 ? 4 : (KS == 1 || (KS <= 3 && MB == 1) || (KS == 2 && g.E == 2) ? 3 : 2);
+    const double slots = room < held ? room : held;                       // by LDS and by the registers of the kernel
+    const auto round = [&](double l) {
+        const double uneven = l + (g.groups > 1 ? 0.336 : 0.573) * (std::ceil(l / unit - 1e-9) * unit - l);
+        const double busy = uneven * (0.306 * MB + 0.081 * g.groups * g.E + 0.024 * g.groups * KS * MB + (KS == 5 ? 0.025 : 0.0));
+        const double wait = 0.426 + 1.308 * g.groups;
+        return 0.443 + 0.182 * g.groups * KS * MB + steps * (busy > wait ? busy : wait);
+    };
+    if (load <= slots) return round(load);
+    const int full = (int)(load / slots);
+    const double left = load - full * slots;
+    return 0.5 * load / slots * round(slots) + 0.5 * (full * round(slots) + (left > 0.02 ? round(left) : 0.0));
+}
+
 bool beyond_cache(int64_t N, const WalkConv& w) { return N * ((int64_t)w.in_plane + w.out_plane) > 250000000; }
 
 // The cut that takes least.  `step`: pixels come in whole multiples of it; taps(XS): the line taps they have together; count:
-// samples and classes; channels: of the input, times the rows a step brings.
+// samples and classes; Ci channels of the input, of which a step brings `stride` rows or all `k` that an output row meets; large:
+// tensors beyond the last-level cache.
 template <typename Taps>
-WalkCut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, int channels, int step, bool together, bool large,
-               Taps taps) {
-    WalkCut best = {step, 1, 1};
-    double least = 1e30;
+WalkCut cut_launch(int64_t count, int Co, int width, int quads, int S, int taps_walked, int Ci, int stride, int k, int step, bool together,
+                   bool large, Taps taps) {
+    WalkCut best = {step, 1, 1, false}, best_short = best;
+    double least = 1e30, least_short = 1e30, kept = 1e30;                 // kept: the short estimate of `best`
     for (int XS = step; XS == step || (together && Co * XS <= 16 && XS < width + step); XS += step) {
         const int XP = taps(XS);
         if (XS > step && XP > kMaxLineTaps) break;
-        const Grouping g = grouping(channels * XP);
         const int64_t tiles = ((int64_t)((width + XS - 1) / XS) * quads + kWalkQuads - 1) / kWalkQuads;
-        for (int MB = 1; MB <= 2; ++MB) {
-            if (MB == 2 && (KS > 3 || Co * XS <= 16)) continue;
+        for (int form = 0; form < 4; ++form) {
+            const bool whole = (form & 1) != 0;
+            const int MB = 1 + form / 2, KS = whole ? 1 : taps_walked;
+            const Grouping g = grouping(Ci * (whole ? k : stride) * XP);
+            if (KS > 5 || (MB == 2 && (KS > 3 || Co * XS <= 16))) continue;
             if (walk_lds(g, KS, MB) > kWalkLds) continue;
             const double waves = (double)(count * ((Co * XS + 16 * MB - 1) / (16 * MB)) * tiles);
-            for (int pieces = 1; pieces <= S && pieces <= 16; pieces *= 2) {
-                // tensors beyond the last-level cache: pieces of a line that does not lie in one piece cost more
-                const double t = walk_time(waves, S, pieces, KS, MB, g) * (large && XS > step ? 1.15 : 1.0);
-                if (t < least) { least = t; best = {XS, MB, pieces}; }
+            for (int cut = 1; cut <= 32 && (cut == 1 || cut < 2 * S); cut *= 2) {
+                const int per = (S + cut - 1) / cut, pieces = (S + per - 1) / per;
+                double t = short_walk_time(waves * pieces, per + KS - 1, KS, MB, g);
+                if (t < least_short) { least_short = t; best_short = {XS, MB, pieces, whole}; }
+                if (whole || cut > 16 || cut > S) continue;
+                // large tensors: pieces of a line that does not lie in one piece cost more (8 of 274 passes, 0.99 times the time without)
+                t = walk_time(waves, S, cut, KS, MB, g) * (large && XS > step ? 1.15 : 1.0);
+                if (t < least) { least = t; best = {XS, MB, cut, false}; kept = short_walk_time(waves * pieces, per + KS - 1, KS, MB, g); }
             }
         }
     }
-    // ... and of these tensors pieces that leave less than a round and a half waves take longer than they should: gradient of a
-    // transposed 4x4 layer, [32,8,32,32,300] -> 16 channels, 176 us with 2400 waves, 157 with 4800
-    if (large && best.MB == 1) {
+    if (least < kShort || least == 1e30 || (best_short.whole && least_short < 0.85 * kept)) return best_short;
+    // ... and large tensors' pieces that leave less than a round and a half waves take longer than they should: 54 of 274 passes with
+    // up to three taps, 0.98 times the time without, in the mean (0.74 to 1.20); with five taps it would be 1.1
+    if (large && best.MB == 1 && taps_walked <= 3) {
         const int64_t tiles = ((int64_t)((width + best.XS - 1) / best.XS) * quads + kWalkQuads - 1) / kWalkQuads;
         const int64_t waves = count * ((Co * best.XS + 15) / 16) * tiles;
         while (waves * best.pieces < 4608 && S >= 16 * best.pieces) best.pieces *= 2;
@@ -448,22 +513,22 @@ WalkCut cut_launch(int64_t count, int Co, int width, int quads, int S, int KS, i
 }
 
 // Whether a cut that was asked for is one there is
-bool may_cut(const WalkCut& c, int step, bool together, int KS) {
-    return c.XS >= step && c.XS % step == 0 && c.XS <= 64 && (c.XS == step || together) && (c.MB == 1 || (c.MB == 2 && KS <= 3)) &&
+bool may_cut(const WalkCut& c, int step, bool together, int taps_walked) {
+    const int KS = c.whole ? 1 : taps_walked;
+    return KS <= 5 && c.XS >= step && c.XS % step == 0 && c.XS <= 64 && (c.XS == step || together) && (c.MB == 1 || (c.MB == 2 && KS <= 3)) &&
            c.pieces >= 1 && c.pieces <= 1024;
 }
 
-// The launch of a WalkConv whose geometry is filled in; `taps` of the walk.  false: not one that the kernel takes.
-bool launch(WalkConv& w, int taps, hipStream_t st, int* code) {
-    const int KS = slide_taps(taps);
+// The launch of a WalkConv whose geometry is filled in; KS taps along the walk.  false: not one that the kernel takes.
+bool launch(WalkConv& w, int KS, hipStream_t st, int* code) {
     if (KS < 1 || KS > 5 || w.XP > kMaxLineTaps) return false;
-    const int64_t pairs = (int64_t)w.Ci * w.XP * w.ss;
+    const int64_t pairs = (int64_t)w.Ci * w.XP * w.rows;
     if (pairs > 4096) return false;
     w.pairs = (int)pairs;
     const Grouping grp = grouping(w.pairs);
     const int E = grp.E;
     w.groups = grp.groups;
-    const size_t bytes = walk_lds(grp, KS, w.MB);
+    size_t bytes = walk_lds(grp, KS, w.MB);
     if (bytes > kWalkLds) return false;
     w.quads = (w.T + 3) / 4;
     if ((int64_t)w.M * w.quads > 0x3fffffffLL) return false;
@@ -475,8 +540,13 @@ bool launch(WalkConv& w, int taps, hipStream_t st, int* code) {
     const int64_t items = (int64_t)w.tiles * pieces;
     const int waves = walk_waves(bytes, (double)(base * pieces));
     const int64_t wgs = (int64_t)w.N * w.blocks * w.classes * ((items + waves - 1) / waves);
-    if (items > 0x7fffffffLL || wgs > 0x7fffffffLL / 8) return false;
+    if (!walk_keeps(KS, E, w.MB)) bytes += (waves - 4) * kWave * sizeof(int4);
+    if (items > 0x3fffffffLL || wgs > 0x7fffffffLL / 8) return false;
     w.items = (int)items;
+    w.waves = waves;
+    w.by_cb = w.blocks * w.classes; w.by_blocks = w.blocks; w.by_wgs = (w.items + waves - 1) / waves; w.by_tiles = w.tiles;
+    w.by_quads = w.quads; w.by_XS = w.XS; w.by_triples = w.XP * w.rows; w.by_rows = w.rows;
+    for (int i = 0; i < w.classes; ++i) w.cls[i].per = (w.cls[i].S + pieces - 1) / pieces;
 #define SLAYER_WALK(KS, MB) launch_walk<KS, MB>(E, w, (unsigned)wgs, waves, bytes, st)
     if (w.MB == 2) { if (KS == 1) SLAYER_WALK(1, 2); else if (KS == 2) SLAYER_WALK(2, 2); else SLAYER_WALK(3, 2); }
     else if (KS == 1) SLAYER_WALK(1, 1);
@@ -488,8 +558,8 @@ bool launch(WalkConv& w, int taps, hipStream_t st, int* code) {
     return true;
 }
 
-void steps_inside(WalkClass& c, int ss, int Hs) {
-    c.c_lo = c.row0 + ss - 1 >= 0 ? 0 : (-c.row0 - ss + 1 + ss - 1) / ss;
+void steps_inside(WalkClass& c, int ss, int rows, int Hs) {
+    c.c_lo = c.row0 + rows - 1 >= 0 ? 0 : (-c.row0 - rows + 1 + ss - 1) / ss;
     c.c_hi = Hs - 1 - c.row0 < 0 ? 0 : (Hs - 1 - c.row0) / ss + 1;
 }
 
@@ -504,7 +574,9 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
     // along the rows of the image, so that the line is one piece of memory, unless the filter has more taps the other way; along
     // the other axis where the weights do not fit LDS this way (9x2, stride 8 along the rows, 56 channels: 183 KB and 98)
     const bool down = takes(h, v), right = takes(v, h), rows_first = down && (!right || taps(h) >= taps(v));
-    if (!down && !right) return false;
+    // filters of more rows than a line has taps (40x3) bring them all in one step
+    const bool tall = !down && !right && h.dil == 1 && h.k > kMaxLineTaps && v.k <= 5;
+    if (!down && !right && !tall) return false;
     const auto along = [&](bool use_h) {
         const Axis& s = use_h ? h : v;
         const Axis& l = use_h ? v : h;
@@ -521,11 +593,13 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
         // pixels that lie together share their taps, unless these lie apart
         const auto line_taps = [&](int XS) { return (XS - 1) * l.stride + l.k; };
         const bool together = l.dil == 1 || l.k == 1;
-        if (p.want && !may_cut(*p.want, 1, together, slide_taps(taps(s)))) return false;
+        const int KS = slide_taps(taps(s));
+        if (p.want && !may_cut(*p.want, 1, together, KS)) return false;
         const WalkCut cut = p.want ? *p.want
-                                   : cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, slide_taps(taps(s)), p.Ci * s.stride, 1, together,
+                                   : cut_launch(p.N, p.Co, l.out, (p.T + 3) / 4, s.out, KS, p.Ci, s.stride, s.k, 1, together,
                                                 beyond_cache(p.N, w), [&](int XS) { return XS > 1 ? line_taps(XS) : l.k; });
         w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
+        w.rows = cut.whole ? s.k : s.stride;
         w.out_line *= w.XS;
         w.M = (l.out + w.XS - 1) / w.XS;
         w.ss = s.stride; w.ls = l.stride * w.XS;
@@ -537,10 +611,10 @@ bool launch_synapse_walk(const SynapseConv& p, hipStream_t st, int* code) {
         WalkClass& c = w.cls[0];
         c.s0 = s.k0; c.row0 = -s.pad; c.S = s.out;
         c.out0 = (p.oy0 * p.Wo_full + p.ox0) * px;
-        steps_inside(c, w.ss, w.Hs);
-        return launch(w, taps(s), st, code);
+        steps_inside(c, w.ss, w.rows, w.Hs);
+        return launch(w, cut.whole ? 1 : KS, st, code);
     };
-    return along(rows_first) || (down && right && along(!rows_first));
+    return along(rows_first || tall) || (down && right && along(!rows_first));
 }
 
 bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh, int sw, int ph, int pw, hipStream_t st, int* code) {
@@ -564,37 +638,36 @@ bool launch_synapse_walk_transposed(const SynapseConv& p, int kh, int kw, int sh
                 }
         return hi - lo + 1;
     };
-    const int most = slide_taps((kh + sh - 1) / sh);
-    if (p.want && !may_cut(*p.want, sw, true, most)) return false;
+    const int most = (kh + sh - 1) / sh, KS = slide_taps(most);              // taps of a class
+    if (KS > 5) return false;
+    if (p.want && !may_cut(*p.want, sw, true, KS)) return false;
     const WalkCut cut = p.want ? *p.want
-                               : cut_launch((int64_t)p.N * (sh < H ? sh : H), p.Co, W, (p.T + 3) / 4, (H + sh - 1) / sh, most, p.Ci, sw, true,
+                               : cut_launch((int64_t)p.N * (sh < H ? sh : H), p.Co, W, (p.T + 3) / 4, (H + sh - 1) / sh, KS, p.Ci, 1, most, sw, true,
                                             beyond_cache(p.N, w), line_taps);
     w.XS = cut.XS; w.pieces = cut.pieces; w.MB = cut.MB;
     w.XP = line_taps(w.XS); w.shift0 = lo; w.shift_step = 1;
     w.out_slide = sh * W * px; w.out_line = w.XS * px; w.out_rx = px;
     w.Hs = p.H; w.Ws = p.W; w.M = (W + w.XS - 1) / w.XS; w.line_full = W;
-    w.ss = 1; w.ls = w.XS / sw;
+    w.ss = 1; w.ls = w.XS / sw; w.rows = cut.whole ? most : 1;
     w.wslide = kw; w.wline = 1; w.nslide = kh; w.nline = kw;
     w.sstep = -sh; w.l0 = pw - lo * sw; w.lstep = -sw; w.lrx = 1;
     w.classes = sh < H ? sh : H;
-    int taps = 1;
     for (int r = 0; r < w.classes; ++r) {
         WalkClass& c = w.cls[r];
         int count = 0, last = 0;
         for (int y = 0; y < kh; ++y)
             if ((r + ph - y) % sh == 0) { ++count; last = y; }
-        taps = count > taps ? count : taps;
         c.S = (H - r + sh - 1) / sh;
         c.out0 = r * W * px;
         if (count) {
             c.s0 = last;
             c.row0 = (r + ph - last) / sh;
-            steps_inside(c, 1, w.Hs);
+            steps_inside(c, 1, w.rows, w.Hs);
         } else {                                                         // rows that no tap reaches: zeros
             c.s0 = -1; c.row0 = 0; c.c_lo = c.c_hi = 0;
         }
     }
-    return launch(w, taps, st, code);
+    return launch(w, cut.whole ? 1 : KS, st, code);
 }
 
 }  // namespace slayer

@@ -59,7 +59,7 @@ _SIGNATURES = {
     'slayer_delay_bwd': (_INT, [_P, _P, _P, _P, _P, _I64, _F, _P, _I64, _I64, _I64, _P]),
     'slayer_conv_synapse': (_INT, [_P, _P, _P] + [_I64] * 14 + [_P]),
     'slayer_conv_synapse_input_grad': (_INT, [_P, _P, _P] + [_I64] * 14 + [_P]),
-    'slayer_conv_synapse_cut': (_INT, [_P, _P, _P] + [_I64] * 14 + [_INT] * 2 + [_I64] * 3 + [_P]),
+    'slayer_conv_synapse_cut': (_INT, [_P, _P, _P] + [_I64] * 14 + [_INT] * 2 + [_I64] * 3 + [_INT] + [_P]),
     'slayer_conv_synapse_wgrad_workspace': (_I64, [_I64] * 11),
     'slayer_conv_synapse_wgrad': (_INT, [_P, _P, _P] + [_I64] * 14 + [_P, _I64, _P]),
     'slayer_conv': (_INT, [_P, _P, _P, _I64, _F, _I64, _I64, _P]),

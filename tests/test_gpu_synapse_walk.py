@@ -34,6 +34,7 @@ FORMS = [
     ((1, 3, 3, 12, 21), 4, (1, 5), (1, 1), (0, 2), (1, 1)),
     ((1, 20, 4, 5, 31), 20, (1, 1), (1, 1), (0, 0), (1, 1)),
     ((2, 4, 9, 7, 17), 4, (2, 2), (3, 3), (0, 0), (1, 1)),           # transposed: classes without taps
+    ((2, 3, 36, 5, 9), 4, (33, 3), (1, 1), (2, 1), (1, 1)),          # more rows than a line has taps
 ]
 
 
@@ -164,14 +165,14 @@ def test_finite_results_are_those_of_the_call_without_the_infinite_value(transpo
 
 
 # ------------------------------------------------------------------ the cut given
-def _cut(input_grad, x, w, out_shape, stride, padding, dilation, by_class, pixels, blocks, pieces):
+def _cut(input_grad, x, w, out_shape, stride, padding, dilation, by_class, pixels, blocks, pieces, whole=False):
     """The call with the cut given, or None where there is no such cut.  w: [Co, Ci, kh, kw], Co the channels of the result."""
     from lava_dl_amd.slayer import _native as N
     out = torch.full(out_shape, -12345.0, device=dev())
     big, small = (out_shape, x.shape) if input_grad else (x.shape, out_shape)            # of the plain convolution
     with N.device_guard(x.device):
         code = N.lib().slayer_conv_synapse_cut(N.ptr(out), N.ptr(x), N.ptr(w), big[0], big[1], small[1], *big[2:], *w.shape[2:], *stride,
-                                               *padding, *dilation, int(input_grad), int(by_class), pixels, blocks, pieces,
+                                               *padding, *dilation, int(input_grad), int(by_class), pixels, blocks, pieces, int(whole),
                                                N.stream_handle())
     if code == -3:
         return None
@@ -197,9 +198,9 @@ def test_every_cut_of_a_layer_gives_the_same(form):
     for input_grad, by_class, xd, wd, want in cases:
         for pixels in (1, 2, 3, 4, 6, 8):
             for blocks in (1, 2):
-                for pieces in (1, 2, 3, 16):
-                    got = _cut(input_grad, xd, wd, want.shape, stride, padding, dilation, by_class, pixels, blocks, pieces)
-                    assert got is None or torch.equal(got.cpu(), want), (input_grad, by_class, pixels, blocks, pieces)
+                for pieces, whole in ((1, False), (2, False), (3, False), (16, False), (1, True), (3, True), (16, True)):
+                    got = _cut(input_grad, xd, wd, want.shape, stride, padding, dilation, by_class, pixels, blocks, pieces, whole)
+                    assert got is None or torch.equal(got.cpu(), want), (input_grad, by_class, pixels, blocks, pieces, whole)
                     taken[pixels > 1] += got is not None
     if max(kernel) < 6 and 1 in dilation:
         assert taken[0]
