@@ -130,7 +130,8 @@ struct WgradWalk {
     int pairs, npt, passes, KS;         // (channel, line tap, row of a step) triples, tiles of 16 of them a pass, taps along the walk
     int shares, share_quads, pieces, sets;   // sets of tiles: one a share, or one for the shares of a workgroup
     int kslide, kline, wslide, wline;   // the filter's axes: sizes and strides
+    Divisor by_cobs, by_passes, by_sets, by_quads, by_triples, by_ss;    // blocks of channels, passes, sets, quads, XP * ss, ss
 };
-int launch_synapse_wgrad_walk(const WgradWalk& w, hipStream_t stream);
+int launch_synapse_wgrad_walk(WgradWalk& w, hipStream_t stream);
 
 }  // namespace slayer

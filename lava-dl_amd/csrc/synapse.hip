@@ -342,14 +342,35 @@ __global__ __launch_bounds__(kSynWaves * kWave) void synapse_wgrad_kernel(const 
 // grad_w[co][k] = sum over batch entries and items of the waves' tiles, in double, in a fixed order, in two
 // launches: block (tile, chunk) adds the tiles of its chunk of the (batch entry, item) pairs -- sixteen partial sums
 // (every sixteenth pair each), then those in turn -- into stage[chunk][tile]; the second launch adds the chunks and
-// writes the gradient.  `tiles` tiles per wave and pass; tile tl holds taps k = 16 (pass tiles + tl) + j
-// (map.npt == 0) or, for the walking kernel, triples (channel, line tap, row of the step) 16 (pass npt + tl % npt) + j at tap
-// tl / npt of the walk.
-struct WgradMap { int npt, pairs, XP, ss, kslide, wslide, wline; };
+// writes the gradient.  Up to kWgradFew pairs are one chunk, and its launch writes the gradient.  `tiles` tiles per wave and pass;
+// tile tl holds taps k = 16 (pass tiles + tl) + j (map.npt == 0) or, for the walking kernel, triples (channel, line tap, row of the
+// step) 16 (pass npt + tl % npt) + j at tap tl / npt of the walk.
+struct WgradMap {
+    int npt, pairs, XP, ss, kslide, wslide, wline;
+    // tap of lane j of tile tl of a pass, or K where there is none
+    __device__ __forceinline__ int tap(int K, int pass, int tiles, int tl, int j) const {
+        if (npt == 0) return (pass * tiles + tl) * 16 + j;
+        const int walked = tl / npt, pr = (pass * npt + tl - walked * npt) * 16 + j;
+        const int ci = pr / (XP * ss), r = pr - ci * (XP * ss), x = r / ss;
+        const int y = walked * ss + r - x * ss;
+        return pr < pairs && y < kslide ? ci * XP * kslide + y * wslide + x * wline : K;
+    }
+    __device__ __forceinline__ void write(float* grad_w, const double (&tot)[4], int Co, int K, int cob, int pass, int tiles, int tl,
+                                          int lane) const {
+        const int k = tap(K, pass, tiles, tl, lane & 15);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int co = cob * 16 + 4 * (lane >> 4) + i;
+            if (co < Co && k < K) grad_w[(int64_t)co * K + k] = (float)tot[i];
+        }
+    }
+};
 constexpr int kWgradParts = 16;
 constexpr int kWgradChunks = 32;
+constexpr int kWgradFew = 96;           // six a thread: one launch less, 12 of 15 us of small layers; 16 a thread were up to 1.15 times as long
 __global__ __launch_bounds__(kWgradParts * kWave) void synapse_wgrad_reduce_kernel(
-        double* __restrict__ stage, const float* __restrict__ partial, int N, int Co, int items, int passes, int tiles) {
+        double* __restrict__ stage, float* __restrict__ grad_w, const float* __restrict__ partial, int N, int Co, int K, int items,
+        int passes, int tiles, const WgradMap map) {
     __shared__ double sums[kWgradParts][kWave][4];
     const int lane = threadIdx.x & (kWave - 1), part = threadIdx.x >> 6;
     const int tl = blockIdx.x % tiles;
@@ -360,54 +381,46 @@ __global__ __launch_bounds__(kWgradParts * kWave) void synapse_wgrad_reduce_kern
     double s[4] = {0.0, 0.0, 0.0, 0.0};
     const float4* src = reinterpret_cast<const float4*>(partial);
     const int64_t total = (int64_t)N * items;
-    const int64_t per = (total + kWgradChunks - 1) / kWgradChunks;
+    const int64_t per = (total + gridDim.y - 1) / gridDim.y;
     const int64_t lo = blockIdx.y * per, hi = (lo + per) < total ? (lo + per) : total;
     for (int64_t at = lo + part; at < hi; at += kWgradParts) {
-        const int64_t n = at / items, item = at - n * items;
-        const float4 v = src[((((n * cobs + cob) * items + item) * passes + pass) * tiles + tl) * kWave + lane];
+        // pair `at` of this block of channels: the blocks lie between the batch entries
+        const int64_t row = cobs == 1 ? at : at + (at / items * (cobs - 1) + cob) * items;
+        const float4 v = src[((row * passes + pass) * tiles + tl) * kWave + lane];
         s[0] += v.x; s[1] += v.y; s[2] += v.z; s[3] += v.w;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) sums[part][lane][i] = s[i];
     __syncthreads();
     if (part != 0) return;
+    double tot[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int pp = 0; pp < kWgradParts; ++pp)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tot[i] += sums[pp][lane][i];
+    if (gridDim.y == 1) {
+        map.write(grad_w, tot, Co, K, cob, pass, tiles, tl, lane);
+        return;
+    }
     double* dst = stage + (((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kWave + lane) * 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        double tot = 0.0;
-        for (int pp = 0; pp < kWgradParts; ++pp) tot += sums[pp][lane][i];
-        dst[i] = tot;
-    }
+    for (int i = 0; i < 4; ++i) dst[i] = tot[i];
 }
 
 __global__ __launch_bounds__(kWave) void synapse_wgrad_final_kernel(float* __restrict__ grad_w,
                                                                      const double* __restrict__ stage, int Co, int K,
                                                                      int passes, int tiles, const WgradMap map) {
-    const int lane = threadIdx.x, q = lane >> 4, j = lane & 15;
+    const int lane = threadIdx.x;
     const int tl = blockIdx.x % tiles;
     int b = blockIdx.x / tiles;
     const int pass = b % passes;
     const int cob = b / passes;
-    int k;
-    if (map.npt == 0) {
-        k = (pass * tiles + tl) * 16 + j;
-    } else {
-        const int tap = tl / map.npt, pr = (pass * map.npt + tl - tap * map.npt) * 16 + j;
-        const int ci = pr / (map.XP * map.ss), r = pr - ci * (map.XP * map.ss), x = r / map.ss;
-        const int y = tap * map.ss + r - x * map.ss;
-        k = pr < map.pairs && y < map.kslide ? ci * map.XP * map.kslide + y * map.wslide + x * map.wline : K;   // or no tap
-    }
     double tot[4] = {0.0, 0.0, 0.0, 0.0};
     for (int c = 0; c < kWgradChunks; ++c) {
         const double* src = stage + (((int64_t)c * gridDim.x + blockIdx.x) * kWave + lane) * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) tot[i] += src[i];
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int co = cob * 16 + 4 * q + i;
-        if (co < Co && k < K) grad_w[(int64_t)co * K + k] = (float)tot[i];
-    }
+    map.write(grad_w, tot, Co, K, cob, pass, tiles, tl, lane);
 }
 
 }  // namespace slayer
@@ -701,20 +714,26 @@ bool wgrad_walk(WgradWalk& w, int Ci, const int (&k)[2], const int (&stride)[2],
     // blocks of channels and passes these are what the waves of a workgroup had better share: [16,32,16,16,300] -> 64, twelve
     // of them, 296 us with the same operands in a workgroup, 307 without; five taps have enough products a load.
     const int merged = cobs * w.passes <= 8 || w.KS == 5 ? kSynWaves : 1;
-    const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N * merged;
+    const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N;   // sets of tiles
     if (room < 1) return false;
     const int64_t visits = (w.line_quads + 7) / 8;
-    const int64_t each = (visits + room - 1) / room;
-    w.share_quads = (int)(8 * each);
-    w.shares = (int)((visits + each - 1) / each);
     // The rows in pieces where that is fewer steps for the chip, which two waves to a SIMD fill: a piece has KS - 1 steps more than
-    // it has rows, and its start is worth about three.
-    auto steps = [&](int pieces) {
-        const double load = (double)(w.N * cobs * w.passes * w.shares * pieces) / 2250;
-        return ((w.S + pieces - 1) / pieces + w.KS + 2) * (load > 1 ? load : 1);
-    };
-    w.pieces = w.shares <= room / merged && steps(kSynWaves) < steps(1) ? kSynWaves : 1;
-    w.sets = w.pieces == 1 ? (w.shares + merged - 1) / merged : w.shares;
+    // it has rows, its start is worth about three, and every set of tiles is written and added.  800 layers like those of short_walk_time, spikes
+    // and real values: what it decides for takes 1.02 times the better of the two in the mean.
+    double least = 1e30;
+    for (int pieces : {1, kSynWaves}) {
+        const int64_t most = pieces == 1 ? room * merged : room, each = (visits + most - 1) / most, shares = (visits + each - 1) / each;
+        const double load = (double)(w.N * cobs * w.passes * shares * pieces) / 2250;
+        const int64_t sets = pieces == 1 ? (shares + merged - 1) / merged : shares;
+        const double steps = (double)each * ((w.S + pieces - 1) / pieces + w.KS + 2) * (load > 1 ? load : 1) +
+                             0.0003 * w.N * sets * cobs * w.passes * w.KS * w.npt;
+        if (steps >= least) continue;
+        least = steps;
+        w.share_quads = (int)(8 * each);
+        w.shares = (int)shares;
+        w.pieces = pieces;
+        w.sets = (int)sets;
+    }
     return true;
 }
 
@@ -739,6 +758,19 @@ extern "C" int64_t slayer_conv_synapse_wgrad_workspace(int64_t N, int64_t Ci, in
         const int64_t floats = (N * p.items + 2 * kWgradChunks) * ((Co + 15) / 16) * p.passes * f.tiles * 256;
         need = floats > need ? floats : need;
     }
+    // ... and for the walking form of few waves, a set of its tiles for every visit of the line, or 4096 of them in all: small layers have
+    // more of these than the forms above have waves, and longer shares are a longer way for each wave ([1,1,16,15,168] -> 32 channels,
+    // 2x2: 38 us with the shares that fit before)
+    const auto walked = [&](int64_t KS, int64_t pairs, int64_t pixels) {
+        if (KS < 1 || KS > 5) return;
+        KS = KS == 4 ? 5 : KS;
+        const int64_t npt = pairs <= 16 ? 1 : 2, passes = (pairs + 16 * npt - 1) / (16 * npt), cobs = (Co + 15) / 16;
+        const int64_t visits = (pixels * ((T + 3) / 4) + 7) / 8, waves = N * cobs * passes, most = (4096 + waves - 1) / (waves < 1 ? 1 : waves);
+        const int64_t floats = (N * (visits < most ? visits : most) + 2 * kWgradChunks) * cobs * passes * KS * npt * 256;
+        need = floats > need ? floats : need;
+    };
+    if (kh == 1 || dil_h == 1) walked((kh + stride_h - 1) / stride_h, Ci * kw * stride_h, W);   // the rows walked, the line of about W pixels
+    walked(kw, Ci * kh, Ho);                                                                    // the columns, with stride 1
     return need;
 }
 
@@ -767,8 +799,10 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     auto reduce = [&](int items, int passes, int tiles, const WgradMap& map) {
         double* stage = reinterpret_cast<double*>(workspace + N * cobs * items * passes * tiles * 256);
         const unsigned tile_blocks = (unsigned)(cobs * passes * tiles);
-        hipLaunchKernelGGL(synapse_wgrad_reduce_kernel, dim3(tile_blocks, kWgradChunks), dim3(kWgradParts * kWave), 0, st, stage,
-                           workspace, (int)N, (int)Co, items, passes, tiles);
+        const bool few = N * items <= kWgradFew;
+        hipLaunchKernelGGL(synapse_wgrad_reduce_kernel, dim3(tile_blocks, few ? 1 : kWgradChunks), dim3(kWgradParts * kWave), 0, st, stage,
+                           grad_weight, workspace, (int)N, (int)Co, (int)K, items, passes, tiles, map);
+        if (few) return (int)hipGetLastError();
         hipLaunchKernelGGL(synapse_wgrad_final_kernel, dim3(tile_blocks), dim3(kWave), 0, st, grad_weight, stage, (int)Co, (int)K,
                            passes, tiles, map);
         return (int)hipGetLastError();

@@ -45,7 +45,7 @@ struct WgradWave {
 
     struct Pair { int off, shift, row; };      // offset of its input row at step 0, line shift, row of the step; off none: no such pair
     __device__ __forceinline__ Pair pair(int r) const {
-        const int pr = pair0 + r, ci = pr / (p.XP * p.ss), rem = pr - ci * (p.XP * p.ss), x = rem / p.ss, row = rem - x * p.ss;
+        const int pr = pair0 + r, ci = p.by_triples.of(pr), rem = pr - ci * (p.XP * p.ss), x = p.by_ss.of(rem), row = rem - x * p.ss;
         const int shift = p.shift0 + x * p.shift_step;
         if (pr >= p.pairs) return {kOutOfRange, 0, 0};
         return {ci * p.in_ch + shift * p.in_line + row * p.in_slide, shift, row};
@@ -57,7 +57,7 @@ struct WgradWave {
     __device__ __forceinline__ Place place(int quad) const {
         Place a;
         a.on = quad < q_hi;
-        a.m = a.on ? quad / p.quads : 0;
+        a.m = a.on ? p.by_quads.of(quad) : 0;
         a.t = 4 * (quad - a.m * p.quads);
         a.repeats = a.on && a.t > p.T - 4 ? a.t - (p.T - 4) : 0;
         a.t -= a.repeats;
@@ -296,10 +296,9 @@ void synapse_wgrad_walk_kernel(const WgradWalk p) {
     const bool together = p.pieces > 1 || p.sets < p.shares;
     int b = xcd_contiguous(blockIdx.x, gridDim.x);
     if (!together) b = b * kSynWaves + wave;
-    const int cob = b % cobs; b /= cobs;
-    const int pass = b % p.passes; b /= p.passes;
-    const int set = b % p.sets;
-    const int n = b / p.sets;
+    const int cob = p.by_cobs.rest(b); b = p.by_cobs.of(b);
+    const int pass = p.by_passes.rest(b); b = p.by_passes.of(b);
+    const int set = p.by_sets.rest(b), n = p.by_sets.of(b);
     if (n >= p.N) return;                               // (never together: those are whole workgroups)
     const int share = p.sets < p.shares ? set * kSynWaves + wave : set, piece = p.pieces > 1 ? wave : 0;
     const int per = (p.S + p.pieces - 1) / p.pieces;
@@ -349,7 +348,8 @@ void synapse_wgrad_walk_kernel(const WgradWalk p) {
     }
 }
 
-int launch_synapse_wgrad_walk(const WgradWalk& w, hipStream_t st) {
+int launch_synapse_wgrad_walk(WgradWalk& w, hipStream_t st) {
+    w.by_cobs = (w.Co + 15) / 16; w.by_passes = w.passes; w.by_sets = w.sets; w.by_quads = w.quads; w.by_triples = w.XP * w.ss; w.by_ss = w.ss;
     const int64_t sets = (int64_t)w.N * ((w.Co + 15) / 16) * w.sets * w.passes;          // of tiles
     const int64_t blocks = w.pieces > 1 || w.sets < w.shares ? sets : (sets + kSynWaves - 1) / kSynWaves;
     if (blocks > 0x7fffffffLL / kSynWaves) return SLAYER_ERANGE;
