@@ -18,14 +18,18 @@
 // (4x4 stride 2, [32,16,16,16,300] -> 8 channels 245 -> 185 us, 13x11 pixels of 173 steps 139 -> 25).
 //
 // Steps that are not whole quads: a pixel's last quad is its last four steps, overlapping the one before; the steps they share are
-// computed twice, to the same bits, instead of being moved into place ([16,8,24,24,250] -> 16 channels, 5x5: 204 -> 114 us).
+// computed and stored twice, to the same bits (also beside results that are not finite, see below), instead of being moved into place ([16,8,24,24,250] -> 16 channels, 5x5: 204 -> 114 us).
 //
 // Operands are split into three parts (split.h) unless they are bfloat16 numbers as they are: the weights are looked at once
 // per workgroup, the input once per group, and the products run to match: one for spikes and quantised weights, three for one
 // split operand, six for two.  The instruction rounds every sum it leaves, so the products of the lower parts, 2^-8 of
 // the whole at most, are added up from zero and join the sum in one addition: it is rounded twice for 32 terms, not up to
 // six times (error against float64 1.0e-7 real x real over 96 terms, float32 instruction 2.9e-7; every product into the one sum
-// 2.6e-7).
+// 2.6e-7; over 8 to 24 terms 0.31e-7 .. 0.48e-7, float32 instruction 0.45e-7 .. 0.89e-7).  The last addition rounds down as well: the mean of
+// the errors, with sign, is -0.9e-8 of the mean result over 8 terms, -0.3e-8 over 800, a quarter of their spread or less.
+//
+// The walk loads the rows that an output row meets one after another.  Short launches, which wait for their loads, take all of them in
+// one step instead, as terms of one product (WalkCut::whole): [9,1,13,13,132] -> 2 channels, real values, 14.4 -> 5.8 us.
 //
 // What bounds it: with the products left out the forward pass of [32,8,32,32,300] -> 16 channels takes as long (254 us): a group
 // of loads has to arrive before its step, and 12 waves hold 72 KB of a CU's loads in flight.  Two blocks of channels to a wave
@@ -40,7 +44,6 @@
 //
 // LDS: the parts of the weights in the operand's layout, [group][tap][part][block][lane]; per triple its byte offset, its line tap
 // and row, its channel; what the waves' weights are; where lanes store that have no registers for it.
-#include <cmath>
 #include "synapse.h"
 #include "split.h"
 
@@ -423,51 +426,57 @@ size_t walk_lds(const Grouping& g, int KS, int MB) {
 // Eight where the LDS has room for one workgroup only and there are more than four waves to a CU.
 int walk_waves(size_t lds, double waves) { return 2 * lds > 160 * 1024 && waves > 4 * 256 ? 8 : 4; }
 
-// What a launch of the walking form takes, in us: a workgroup sets up its weights; a wave walks its piece of S rows, KS - 1 steps more
-// than it has rows; a group of loads is a wait or, where a SIMD has several waves, its share of the instructions; of what the last,
-// partly filled round of workgroups leaves idle, 0.44 is lost.  Fitted to 814 layers (3x3 and 5x5, strides 1 and 2, 4x4 transposed
-// and its gradient, 2 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 50 to 350 steps), each cut in all the ways below.
-double walk_time(double waves, int S, int pieces, int KS, int MB, const Grouping& g) {
-    const size_t lds = walk_lds(g, KS, MB);
-    const double load = waves * pieces / 1024;                            // waves per SIMD
-    const double room = (double)(160 * 1024 / lds) * walk_waves(lds, waves * pieces) / 4;
-    const double slots = KS > 3 || MB == 2 ? (room < 2 ? room : 2) : (room < 3 ? room : 3);
-    const int steps = (S + pieces - 1) / pieces + KS - 1;
-    const auto round = [&](double l) {
-        const double busy = l * (0.38 * MB + 0.097 * g.groups * g.E), wait = 1.5 * g.groups;
-        return 0.4 * g.groups * KS * MB + steps * (busy > wait ? busy : wait);
-    };
-    if (load <= slots) return round(load);
-    const int full = (int)(load / slots);
-    const double left = load - full * slots;
-    return 0.56 * load / slots * round(slots) + 0.44 * (full * round(slots) + (left > 0.02 ? round(left) : 0.0));
-}
+// What the launches of one form (KS, MB, the groups) take, in us: a workgroup sets up its weights; a wave walks its piece, KS - 1 steps
+// more than it has rows; a group of loads is a wait or, where a SIMD has several waves, its share of the instructions; of what the
+// last, partly filled round of workgroups leaves idle, some is lost.  load: waves per SIMD.  (A layer has some hundred cuts: what
+// is the same for all of a form is worked out once.)
+struct WalkTime {
+    bool wide;                          // LDS has room for one workgroup only
+    float room, held;                   // workgroups of four waves that LDS, waves that the registers of a SIMD hold
+    float start, busy, wait, slots;
+    float short_start, short_busy, short_wait, part;
 
-// What a short launch of either form takes: also the start of a wave, the products, and that compute units with fewer workgroups than
-// others wait for these with 0.34 to 0.57 of what they have less.  Fitted to 3408 passes (forward and input gradient of 860
-// layers: 1x1 to 5x5, strides 1 and 2, transposed, 1 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 20 to 350 steps, spikes x
-// 8-bit and real x real), each cut in all the ways below.  What it decides for below kShort takes 0.87 times what walk_time decides
-// for, in the mean (2.3 % of these passes: more than 1.03 times).  Above, the two differ by less than what either misses, and
-// walk_time stays (0.90 in the mean between 20 and 60 us, but up to 1.39 times, 0.95 and up to 1.35 times beyond), unless
-// the `whole` form is estimated at less than 0.85 of it.
-constexpr double kShort = 20.0;
-double short_walk_time(double waves, int steps, int KS, int MB, const Grouping& g) {
-    const size_t lds = walk_lds(g, KS, MB);
-    const double unit = walk_waves(lds, waves) / 4, load = waves / 1024;                  // waves per SIMD: of a workgroup, of all
-    const double room = (double)(160 * 1024 / lds) * unit;
-    const int held = KS == 1 && MB == 1 && g.E <= 4 ? 4 : (KS == 1 || (KS <= 3 && MB == 1) || (KS == 2 && g.E == 2) ? 3 : 2);
-    const double slots = room < held ? room : held;                       // by LDS and by the registers of the kernel
-    const auto round = [&](double l) {
-        const double uneven = l + (g.groups > 1 ? 0.336 : 0.573) * (std::ceil(l / unit - 1e-9) * unit - l);
-        const double busy = uneven * (0.306 * MB + 0.081 * g.groups * g.E + 0.024 * g.groups * KS * MB + (KS == 5 ? 0.025 : 0.0));
-        const double wait = 0.426 + 1.308 * g.groups;
-        return 0.443 + 0.182 * g.groups * KS * MB + steps * (busy > wait ? busy : wait);
-    };
-    if (load <= slots) return round(load);
-    const int full = (int)(load / slots);
-    const double left = load - full * slots;
-    return 0.5 * load / slots * round(slots) + 0.5 * (full * round(slots) + (left > 0.02 ? round(left) : 0.0));
-}
+    WalkTime(int KS, int MB, const Grouping& g) {
+        const size_t lds = walk_lds(g, KS, MB);
+        const float terms = (float)(g.groups * g.E), taps = (float)(g.groups * KS * MB);
+        wide = 2 * lds > 160 * 1024;
+        room = (float)(160 * 1024 / lds);
+        start = 0.4f * taps; busy = 0.38f * MB + 0.097f * terms; wait = 1.5f * g.groups; slots = KS > 3 || MB == 2 ? 2.f : 3.f;
+        held = KS == 1 && MB == 1 && g.E <= 4 ? 4.f : (KS == 1 || (KS <= 3 && MB == 1) || (KS == 2 && g.E == 2) ? 3.f : 2.f);
+        short_start = 0.443f + 0.182f * taps;
+        short_busy = 0.306f * MB + 0.081f * terms + 0.024f * taps + (KS == 5 ? 0.025f : 0.f);
+        short_wait = 0.426f + 1.308f * g.groups;
+        part = g.groups > 1 ? 0.336f : 0.573f;
+    }
+    static float rounds(float load, float slots, float lost, float one, float left_over) {   // a full round; what is left over
+        const float all = load / slots, full = (float)(int)all;
+        return (1.f - lost) * all * one + lost * (full * one + (load - full * slots > 0.02f ? left_over : 0.f));
+    }
+    // Fitted to 814 layers (3x3 and 5x5, strides 1 and 2, 4x4 transposed and its gradient, 2 to 64 channels, 1 to 32 samples of 4x4 to
+    // 34x34 pixels, 50 to 350 steps), each walked in all the ways below.
+    float walk(float load, int steps) const {
+        const float by_lds = room * (wide && load > 1.f ? 2.f : 1.f), most = by_lds < slots ? by_lds : slots;
+        const auto round = [&](float l) { return start + steps * (l * busy > wait ? l * busy : wait); };
+        return load <= most ? round(load) : rounds(load, most, 0.44f, round(most), round(load - (float)(int)(load / most) * most));
+    }
+    // Short launches of either form: also the start of a wave, the products, and that compute units with fewer workgroups than others
+    // wait for these with 0.34 to 0.57 of what they have less.  Fitted to 3408 passes (forward and input gradient of 860 layers: 1x1 to
+    // 5x5, strides 1 and 2, transposed, 1 to 64 channels, 1 to 32 samples of 4x4 to 34x34 pixels, 20 to 350 steps, spikes x 8-bit and
+    // real x real), each cut in all the ways below.  What it decides for below kShort takes 0.87 times what walk() decides for, in the
+    // mean (2.3 % of these passes: more than 1.03 times).  Above, the two differ by less than what either misses, and walk()
+    // stays (0.90 in the mean between 20 and 60 us, but up to 1.39 times, 0.95 and up to 1.35 times beyond), unless the `whole` form
+    // is estimated at less than 0.85 of it.
+    float brief(float load, int steps) const {
+        const float unit = wide && load > 1.f ? 2.f : 1.f, by_lds = room * unit, most = by_lds < held ? by_lds : held;
+        const auto round = [&](float l) {
+            const float units = l / unit, whole = (float)(int)units, full = (units - whole > 1e-6f ? whole + 1.f : whole) * unit;
+            const float b = (l + part * (full - l)) * short_busy;
+            return short_start + steps * (b > short_wait ? b : short_wait);
+        };
+        return load <= most ? round(load) : rounds(load, most, 0.5f, round(most), round(load - (float)(int)(load / most) * most));
+    }
+};
+constexpr float kShort = 20.f;
 
 bool beyond_cache(int64_t N, const WalkConv& w) { return N * ((int64_t)w.in_plane + w.out_plane) > 250000000; }
 
@@ -478,30 +487,34 @@ template <typename Taps>
 WalkCut cut_launch(int64_t count, int Co, int width, int quads, int S, int taps_walked, int Ci, int stride, int k, int step, bool together,
                    bool large, Taps taps) {
     WalkCut best = {step, 1, 1, false}, best_short = best;
-    double least = 1e30, least_short = 1e30, kept = 1e30;                 // kept: the short estimate of `best`
+    constexpr float none = 1e30f;
+    float least = none, least_short = none, kept = none;                  // kept: the short estimate of `best`
     for (int XS = step; XS == step || (together && Co * XS <= 16 && XS < width + step); XS += step) {
         const int XP = taps(XS);
         if (XS > step && XP > kMaxLineTaps) break;
         const int64_t tiles = ((int64_t)((width + XS - 1) / XS) * quads + kWalkQuads - 1) / kWalkQuads;
-        for (int form = 0; form < 4; ++form) {
+        const bool wide = Co * XS > 16;
+        for (int form = 0; form < (wide ? 4 : 2); ++form) {
             const bool whole = (form & 1) != 0;
             const int MB = 1 + form / 2, KS = whole ? 1 : taps_walked;
+            if (KS > 5 || (MB == 2 && KS > 3)) continue;
             const Grouping g = grouping(Ci * (whole ? k : stride) * XP);
-            if (KS > 5 || (MB == 2 && (KS > 3 || Co * XS <= 16))) continue;
             if (walk_lds(g, KS, MB) > kWalkLds) continue;
-            const double waves = (double)(count * ((Co * XS + 16 * MB - 1) / (16 * MB)) * tiles);
+            const WalkTime time(KS, MB, g);
+            const float loads = (float)(count * ((Co * XS + 16 * MB - 1) / (16 * MB)) * tiles) * (1.f / 1024.f);
+            const float apart = large && XS > step ? 1.15f : 1.f;
             for (int cut = 1; cut <= 32 && (cut == 1 || cut < 2 * S); cut *= 2) {
                 const int per = (S + cut - 1) / cut, pieces = (S + per - 1) / per;
-                double t = short_walk_time(waves * pieces, per + KS - 1, KS, MB, g);
-                if (t < least_short) { least_short = t; best_short = {XS, MB, pieces, whole}; }
+                const float brief = time.brief(loads * pieces, per + KS - 1);
+                if (brief < least_short) { least_short = brief; best_short = {XS, MB, pieces, whole}; }
                 if (whole || cut > 16 || cut > S) continue;
                 // large tensors: pieces of a line that does not lie in one piece cost more (8 of 274 passes, 0.99 times the time without)
-                t = walk_time(waves, S, cut, KS, MB, g) * (large && XS > step ? 1.15 : 1.0);
-                if (t < least) { least = t; best = {XS, MB, cut, false}; kept = short_walk_time(waves * pieces, per + KS - 1, KS, MB, g); }
+                const float t = time.walk(loads * cut, per + KS - 1) * apart;
+                if (t < least) { least = t; best = {XS, MB, cut, false}; kept = brief; }
             }
         }
     }
-    if (least < kShort || least == 1e30 || (best_short.whole && least_short < 0.85 * kept)) return best_short;
+    if (least < kShort || least == none || (best_short.whole && least_short < 0.85f * kept)) return best_short;
     // ... and large tensors' pieces that leave less than a round and a half waves take longer than they should: 54 of 274 passes with
     // up to three taps, 0.98 times the time without, in the mean (0.74 to 1.20); with five taps it would be 1.1
     if (large && best.MB == 1 && taps_walked <= 3) {
