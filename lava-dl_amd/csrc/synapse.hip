@@ -27,8 +27,9 @@ constexpr int kSynChunk = 6;            // tap groups whose loads are in flight 
 // The gradient of the input of a convolution with strides (what conv_transpose3d computes, the ConvTranspose synapse
 // of synapse/layer.py:513-560 in the reference) is one plain convolution per residue class of the output pixels: the
 // pixels (ry + m sh, rx + m' sw) meet only the taps y with (ry + ph - y dh) divisible by sh (x likewise), and over
-// m, m' those taps slide across the source with unit stride.  Each class is a launch of the kernels below on its
-// sub-lattices of taps and of outputs (slayer_conv_synapse_input_grad), a fraction 1 / (sh sw) of the taps each.
+// m, m' those taps slide across the source with unit stride.  The walking kernel takes all classes in one launch where there
+// is no dilation and up to four classes of rows; otherwise each class is a launch of its own on its sub-lattices of taps and of outputs,
+// of the walking kernel or of the one below, a fraction 1 / (sh sw) of the taps each.
 //
 // LDS: the weights of this workgroup's 16 output channels, tap-major (row k holds the 16 channels), and per tap the
 // offset of its input row relative to the pixel's own position and its (row, column) displacement in the image.
@@ -367,7 +368,9 @@ struct WgradMap {
 };
 constexpr int kWgradParts = 16;
 constexpr int kWgradChunks = 32;
-constexpr int kWgradFew = 96;           // six a thread: one launch less, 12 of 15 us of small layers; 16 a thread were up to 1.15 times as long
+// six a thread, a launch less ([1,3,8,5,201] -> 10 channels, 3x3: 14.2 -> 10.3 us with its shares); 16 a thread took up to 1.15 times
+// as long as two launches
+constexpr int kWgradFew = 96;
 __global__ __launch_bounds__(kWgradParts * kWave) void synapse_wgrad_reduce_kernel(
         double* __restrict__ stage, float* __restrict__ grad_w, const float* __restrict__ partial, int N, int Co, int K, int items,
         int passes, int tiles, const WgradMap map) {
@@ -577,7 +580,7 @@ int conv_synapse(float* out, const float* in, const float* weight, int64_t N, in
 }
 
 // The gradient of the input of slayer_conv_synapse for any stride (and, read as a layer of its own, the transposed
-// convolution): one plain convolution per residue class of the pixels of grad_in, see SynapseConv.
+// convolution): one launch, or one plain convolution per residue class of the pixels of grad_in, see SynapseConv.
 int conv_synapse_input_grad(float* grad_in, const float* grad_out, const float* weight_t, int64_t N, int64_t Ci, int64_t Co, int64_t H,
                             int64_t W, int64_t T, int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w, int64_t pad_h, int64_t pad_w,
                             int64_t dil_h, int64_t dil_w, const WalkCut* want, bool by_class, void* stream) {
@@ -643,9 +646,10 @@ int conv_synapse_input_grad(float* grad_in, const float* grad_out, const float* 
 }
 
 
-// The tiles of sums that the workspace of a geometry holds (`tiles` per wave and pass) and the one-pixel kernel's shares of the
-// time axis.  row_kw: 3 or 5 taps along the image row without stride or dilation, tiles of 16 (channel, kernel row) pairs; that
-// the walking kernel cuts its line into no more shares than these have is what bounds its workspace.
+// What a workspace holds at least, so that the sizes of layers that fill the chip stay what they were: `tiles` of sums per wave and
+// pass and the shares of the time axis, of the one-pixel kernel (row_kw 0; these it runs with) or, for 3 or 5 taps along the image
+// row without stride or dilation, of tiles of 16 (channel, kernel row) pairs, which no kernel has: the walking kernel cuts its line
+// to what there is room for.
 struct WgradForm { int row_kw, npt, tiles; };
 WgradForm wgrad_form(int64_t Ci, int64_t kh, int64_t kw, int64_t stride_w, int64_t dil_w) {
     WgradForm f;
@@ -749,7 +753,7 @@ extern "C" int64_t slayer_conv_synapse_wgrad_workspace(int64_t N, int64_t Ci, in
     if (Ho < 1) return SLAYER_EINVAL;
     const int64_t K = Ci * kh * kw;
     if (K > 4096 || Ho > (1 << 20) || T > (1 << 24)) return SLAYER_ERANGE;
-    // enough for either form of the kernel (which one runs depends on stride and dilation along the image row)
+    // enough for either form (stride and dilation along the image row are not known here)
     int64_t need = 0;
     for (int64_t stride_w : {1, 2}) {
         const WgradForm f = wgrad_form(Ci, kh, kw, stride_w, 1);
@@ -760,7 +764,7 @@ extern "C" int64_t slayer_conv_synapse_wgrad_workspace(int64_t N, int64_t Ci, in
     }
     // ... and for the walking form of few waves, a set of its tiles for every visit of the line, or 4096 of them in all: small layers have
     // more of these than the forms above have waves, and longer shares are a longer way for each wave ([1,1,16,15,168] -> 32 channels,
-    // 2x2: 38 us with the shares that fit before)
+    // 2x2: 38 us with the shares that fit these forms, the kernel before the walk 15)
     const auto walked = [&](int64_t KS, int64_t pairs, int64_t pixels) {
         if (KS < 1 || KS > 5) return;
         KS = KS == 4 ? 5 : KS;
@@ -812,7 +816,8 @@ extern "C" int slayer_conv_synapse_wgrad(float* grad_weight, const float* grad_o
     w.N = (int)N; w.Co = (int)Co; w.T = (int)T;
     const int ker[2] = {(int)kh, (int)kw}, str[2] = {(int)stride_h, (int)stride_w}, pad[2] = {(int)pad_h, (int)pad_w};
     const int dil[2] = {(int)dil_h, (int)dil_w}, size[2] = {(int)H, (int)W}, size_out[2] = {(int)Ho, (int)Wo};
-    if (wgrad_walk(w, (int)Ci, ker, str, pad, dil, size, size_out, floats)) {
+    // (a workspace of fewer floats than are asked for now is cut to as far as it goes)
+    if (wgrad_walk(w, (int)Ci, ker, str, pad, dil, size, size_out, workspace_floats < floats ? workspace_floats : floats)) {
         if (workspace_floats < (N * w.sets + 2 * kWgradChunks) * cobs * w.passes * w.KS * w.npt * 256) return SLAYER_ERANGE;
         const int code = launch_synapse_wgrad_walk(w, st);
         if (code != 0) return code;

@@ -97,6 +97,25 @@ def test_weight_gradient_of_integers_equals_float64(form, split):
     assert torch.equal(got.cpu().double(), wd.grad)
 
 
+@pytest.mark.parametrize('sets', [1, 5, 38])
+def test_a_smaller_workspace_is_cut_to(sets):
+    """[1,1,16,15,168] -> 32 channels, 2x2: tiles of 256 floats for `sets` sums of each block of 16 channels, beside 64 for the
+    reduction.  At most 17 * 16 * 168 terms of 9."""
+    from lava_dl_amd.slayer import _native as N
+    gen = torch.Generator().manual_seed(sets)
+    x, g = _integers(gen, (1, 1, 16, 15, 168), 3), _integers(gen, (1, 32, 17, 16, 168), 3)
+    wd = torch.zeros((32, 1, 2, 2, 1), dtype=torch.float64).requires_grad_()
+    F.conv3d(x.double(), wd, None, 1, (1, 1, 0)).backward(g.double())
+    floats = (sets + 64) * 2 * 256 * 2
+    assert floats < N.lib().slayer_conv_synapse_wgrad_workspace(1, 1, 32, 16, 15, 168, 2, 2, 1, 1, 1)
+    x, g, workspace = x.to(dev()), g.to(dev()), torch.empty(floats, device=dev())
+    got = torch.empty(32, 1, 2, 2, 1, device=dev())
+    with N.device_guard(x.device):
+        N.check(N.lib().slayer_conv_synapse_wgrad(N.ptr(got), N.ptr(g), N.ptr(x), 1, 1, 32, 16, 15, 168, 2, 2, 1, 1, 1, 1, 1, 1,
+                                                  N.ptr(workspace), floats, N.stream_handle()))
+    assert torch.equal(got.cpu().double(), wd.grad)
+
+
 @pytest.mark.parametrize('value', [float('inf'), float('-inf'), float('nan')])
 @pytest.mark.parametrize('form', [FORMS[i] for i in (1, 3, 9, 10, 11, 18)], ids=str)
 def test_a_value_that_is_not_finite_reaches_the_outputs_whose_taps_meet_it_and_no_others(form, value):
