@@ -343,8 +343,8 @@ int slayer_conv_synapse(float *out, const float *in, const float *weight,
  * those of the forward call; weight_t is [Ci][Co][kh][kw] (the forward weights with the channel axes exchanged,
  * not flipped).  One launch without dilation and for strides along the rows of up to 4 (and, on the vector units, when
  * Ci = Co = 1: the pooling layers), else one per residue class of the pixels modulo the strides (stride_h * stride_w
- * launches, each a plain convolution over the taps that class meets).  SLAYER_ERANGE as for slayer_conv_synapse, and for strides above 16 or images beyond 65535
- * pixels a side. */
+ * launches, each a plain convolution over the taps that class meets).  SLAYER_ERANGE as for slayer_conv_synapse, and for
+ * strides above 16 or images beyond 65535 pixels a side. */
 int slayer_conv_synapse_input_grad(float *grad_in, const float *grad_out, const float *weight_t,
                                    int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
                                    int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,
@@ -353,8 +353,9 @@ int slayer_conv_synapse_input_grad(float *grad_in, const float *grad_out, const 
 /* Either of the two above (input_grad: the second, by_class: a launch per residue class where one would do) on the kernel that
  * walks the rows, cut as told instead of as is estimated to take least: `pixels` neighbouring pixels of the line share a position
  * (a multiple of the stride in a launch for all classes), `blocks` (1 or 2) blocks of 16 rows of the product to a wave, the rows of
- * the image walked in `pieces`; whole: every row of the result by itself, from all the rows it meets.  The results differ in the order of their sums.  What it is for: tests, and measuring what the
- * choice costs.  SLAYER_ERANGE where that kernel does not take the layer or the cut is not one it has. */
+ * the image walked in `pieces`; whole: every row of the result by itself, from all the rows it meets.  The results differ in the
+ * order of their sums.  What it is for: tests, and measuring what the choice costs.  SLAYER_ERANGE where that kernel does not take
+ * the layer or the cut is not one it has. */
 int slayer_conv_synapse_cut(float *out, const float *in, const float *weight,
                             int64_t N, int64_t Ci, int64_t Co, int64_t H, int64_t W, int64_t T,
                             int64_t kh, int64_t kw, int64_t stride_h, int64_t stride_w,

@@ -3,10 +3,11 @@
 // out <= 2^-27).  The products of parts are exact in float32; of two split factors the products part i x part j with
 // i + j <= 2 are taken, what is left out is below 2^-26 of the product.
 //   A value that is not finite leaves a NaN (so does a finite one beyond the largest bfloat16, 3.3895e38): callers
-// either treat it (conv.hip) or recognise a result that is not finite and compute it again in float32 (synapse.hip).
+// either treat it (conv.hip) or recognise a result that is not finite and compute it again in float32 (synapse_walk.hip,
+// synapse_wgrad_walk.hip).
 //   Parts below the smallest normal number are lost: a value under 3e-33 enters with an absolute error of 1e-38.  Every
 // float32 is a multiple of 2^-149, and so is what its parts leave: multiplied by kSplitScale first (exact), every part of
-// every value is zero or a normal number.  synapse.hip scales both operands; values from 1e31 on then overflow, like
+// every value is zero or a normal number.  These two scale both operands; values from 1e31 on then overflow, like
 // values that are not finite.
 #pragma once
 #include <hip/hip_runtime.h>

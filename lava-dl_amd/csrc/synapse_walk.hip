@@ -25,8 +25,8 @@
 // split operand, six for two.  The instruction rounds every sum it leaves, so the products of the lower parts, 2^-8 of
 // the whole at most, are added up from zero and join the sum in one addition: it is rounded twice for 32 terms, not up to
 // six times (error against float64 1.0e-7 real x real over 96 terms, float32 instruction 2.9e-7; every product into the one sum
-// 2.6e-7; over 8 to 24 terms 0.31e-7 .. 0.48e-7, float32 instruction 0.45e-7 .. 0.89e-7).  The last addition rounds down as well: the mean of
-// the errors, with sign, is -0.9e-8 of the mean result over 8 terms, -0.3e-8 over 800, a quarter of their spread or less.
+// 2.6e-7; over 8 to 24 terms 0.30e-7 .. 0.37e-7, float32 instruction 0.45e-7 .. 0.89e-7).  The last addition rounds down as well: the mean of
+// the errors, with sign, is -1.1e-8 of the mean result over 8 terms, -0.3e-8 over 800, a third of their spread or less.
 //
 // The walk loads the rows that an output row meets one after another.  Short launches, which wait for their loads, take all of them in
 // one step instead, as terms of one product (WalkCut::whole): [9,1,13,13,132] -> 2 channels, real values, 14.4 -> 5.8 us.

@@ -1,6 +1,6 @@
-"""How the weight gradient of a convolution cuts the time axis (the workspace holds 256 floats per tile and wave, and 64 more
-sets of tiles for the reduction): layers of up to 16 (channel, kernel row) pairs take 32 steps a wave until there are
-32768 waves, wider ones about 8192 waves."""
+"""What the workspace of a convolution's weight gradient holds: 256 floats per tile of sums, for 64 sets of tiles for the reduction
+and for as many more as shares of 32 steps of a row give up to 32768 of them (layers of up to 16 (channel, kernel row) pairs) or
+some 8192 (wider ones).  The kernel cuts the line it walks to the room there is (test_gpu_synapse_walk.py)."""
 import pytest
 
 # (N, Ci, Co, H, W, T), kernel, padding -> shares of the time axis, tiles of a wave
