@@ -711,16 +711,17 @@ bool wgrad_walk(WgradWalk& w, int Ci, const int (&k)[2], const int (&stride)[2],
     w.npt = w.pairs <= 16 ? 1 : 2;
     w.passes = (w.pairs + 16 * w.npt - 1) / (16 * w.npt);
     // as many waves as the workspace has room for, and no more than the line has visits; few waves: pieces of the rows
-    const int64_t cobs = (w.Co + 15) / 16;
+    const int64_t cobs = (w.Co + 15) / 16, visits = (w.line_quads + 7) / 8;
     // The waves of a workgroup take neighbouring shares and leave one set of tiles: a quarter of the tiles to write and add, and
     // room for shares of one visit, which leaves no line to two visits of one wave.  [32,8,32,32,300] -> 16 channels 330 -> 290 us
     // (cold caches), 4x4 stride 2 194 -> 184, [16,16,20,18,128] -> 32 97 -> 86, 5x5 [16,32,12,12,150] -> 64 280 -> 252.  With many
-    // blocks of channels and passes these are what the waves of a workgroup had better share: [16,32,16,16,300] -> 64, twelve
-    // of them, 296 us with the same operands in a workgroup, 307 without; five taps have enough products a load.
-    const int merged = cobs * w.passes <= 8 || w.KS == 5 ? kSynWaves : 1;
+    // blocks of channels and passes, and visits enough for all of them, these are what the waves of a workgroup had better share:
+    // [16,32,16,16,300] -> 64, twelve of them, 268 us with the same operands in a workgroup, 274 without (cold caches 294, 307).  154
+    // passes of nine blocks and passes or more: 1.00 of the time in the mean from 720 visits on (0.94 to 1.06), 1.03 to 1.32 with
+    // fewer; up to eight 1.01 to 1.04 and five taps, which have enough products a load, 1.04 to 1.23 in all sizes.
+    const int merged = cobs * w.passes <= 8 || w.KS == 5 || w.N * visits < 640 ? kSynWaves : 1;
     const int64_t room = (floats / (256 * cobs * w.passes * w.KS * w.npt) - 2 * kWgradChunks) / w.N;   // sets of tiles
     if (room < 1) return false;
-    const int64_t visits = (w.line_quads + 7) / 8;
     // The rows in pieces where that is fewer steps for the chip, which two waves to a SIMD fill: a piece has KS - 1 steps more than
     // it has rows, its start is worth about three, and every set of tiles is written and added.  800 layers like those of short_walk_time, spikes
     // and real values: what it decides for takes 1.02 times the better of the two in the mean.

@@ -77,6 +77,7 @@ def test_integers_equal_float64(form, parts):
                                           ((1, 2, 9, 4, 70), 4, (3, 3), (1, 1), (1, 1), (1, 1)),            # ... of two or three
                                           ((3, 2, 6, 5, 9), 20, (3, 3), (1, 1), (1, 1), (1, 1)),            # few sets, two blocks of channels
                                           ((1, 2, 12, 16, 40), 3, (2, 2), (1, 1), (0, 0), (1, 1)),
+                                          ((330, 17, 4, 4, 9), 80, (2, 2), (1, 1), (0, 0), (1, 1)),         # a set of sums to a wave
                                           ((40, 8, 8, 8, 300), 16, (3, 3), (1, 1), (1, 1), (1, 1))], ids=str)   # whole rows
 @pytest.mark.parametrize('split', ['neither', 'gradient', 'input'])
 def test_weight_gradient_of_integers_equals_float64(form, split):
