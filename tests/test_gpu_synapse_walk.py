@@ -169,20 +169,32 @@ def test_a_pixel_meets_the_taps_of_its_own_class(form):
 
 @pytest.mark.parametrize('transposed', [False, True])
 @pytest.mark.parametrize('steps', [66, 67, 131])
-def test_finite_results_are_those_of_the_call_without_the_infinite_value(transposed, steps):
+@pytest.mark.parametrize('cut', [None, (1, 1, 2, False), (2, 2, 2, False), (1, 1, 2, True)], ids=str)
+def test_finite_results_are_those_of_the_call_without_the_infinite_value(transposed, steps, cut):
     """The last two quads of a pixel share steps and may lie in two waves: 17 or 33 quads of a pixel, 16 in a wave."""
     import lava_dl_amd.slayer as slayer
     gen = torch.Generator().manual_seed(steps)
     x = torch.randn(2, 3, 5, 4, steps, generator=gen)
     w = torch.randn(*((3, 18) if transposed else (18, 3)), 3, 3, 1, generator=gen)
     op = slayer.synapse.conv_transpose_synapse if transposed else slayer.synapse.conv_synapse
+    if cut is not None:
+        def op(x, w, *_):
+            w = (w.transpose(0, 1) if transposed else w)[..., 0].contiguous()
+            return _cut(transposed, x, w, (2, 18, 5, 4, steps), (1, 1), (1, 1), (1, 1), False, *cut)
     want = op(x.to(dev()), w.to(dev()), 1, 1, 1)
     x[0, 1, 2, 1, 10] = float('inf')
     x[1, 0, 0, 0, steps - 3] = float('inf')
     got = [op(x.to(dev()), w.to(dev()), 1, 1, 1) for _ in range(2)]
     finite = got[0].isfinite()
+    met = torch.zeros_like(x).masked_fill_(~x.isfinite(), 1.0)
+    conv = F.conv_transpose3d if transposed else F.conv3d
+    assert torch.equal(finite.cpu(), conv(met, torch.ones_like(w), None, 1, (1, 1, 0)) == 0)
     assert not finite.all() and finite.sum() > finite.numel() // 4
-    assert torch.equal(got[0][finite], want[finite])
+    if cut is None or cut[0] == 1:
+        assert torch.equal(got[0][finite], want[finite])
+    else:       # pixels together have each other's taps as products with zero: a result beside it may be a float32 sum of 27 terms, too
+        terms = conv(x.nan_to_num(0.0, 0.0, 0.0).abs(), w.abs(), None, 1, (1, 1, 0)).to(dev())       # and each sum within 28 * 2^-24 of these
+        assert bool(((got[0] - want).abs() <= 2 * 28 * 2.0 ** -24 * terms)[finite].all())
     assert torch.equal(got[0].nan_to_num(7.0, 8.0, 9.0), got[1].nan_to_num(7.0, 8.0, 9.0))
 
 
